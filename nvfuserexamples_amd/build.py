@@ -33,6 +33,14 @@ HIP_FLAGS = [
     "-fno-honor-nans",
     "-Wno-unused-command-line-argument",
 ]
+FREE_MFMA_FORM = object()  # marks a translation unit that is compiled without -amdgpu-mfma-vgpr-form
+
+
+def _flags(defs):
+    if FREE_MFMA_FORM not in defs:
+        return HIP_FLAGS + EXTRA + defs
+    at = HIP_FLAGS.index("-amdgpu-mfma-vgpr-form")
+    return HIP_FLAGS[:at - 1] + HIP_FLAGS[at + 1:] + EXTRA + [f for f in defs if f is not FREE_MFMA_FORM]
 
 
 def _tus():
@@ -46,6 +54,11 @@ def _tus():
                 defs = [f"-DFMHA_TU_BF16={bf}", f"-DFMHA_TU_D={d}", f"-DFMHA_TU_STRIDED={strided}"]
                 tus.append(("fmha_fwd.hip", f"fmha_fwd_{tag}.o", defs))
                 tus.append(("fmha_bwd.hip", f"fmha_bwd_{tag}.o", defs))
+                if d != 256:
+                    # At head dim 128 the dK / dV kernel runs one wave per SIMD on both halves of the register file and
+                    # wants its accumulators in the accumulation half; the compiler finds that split by itself only
+                    # where it is free to choose the form of every matrix instruction.
+                    tus.append(("fmha_bwd_pipe.hip", f"fmha_bwd_pipe_{tag}.o", defs + [FREE_MFMA_FORM]))
     return tus
 
 
@@ -68,7 +81,7 @@ def build_hip(jobs=None, verbose=True):
         objs.append(o)
         if only and os.path.exists(o) and not re.search(only, obj):
             continue
-        cmds.append([HIPCC, *HIP_FLAGS, *EXTRA, *defs, "-c", os.path.join(CSRC, src), "-o", o])
+        cmds.append([HIPCC, *_flags(defs), "-c", os.path.join(CSRC, src), "-o", o])
     with cf.ThreadPoolExecutor(jobs) as ex:
         for out in ex.map(_run, cmds):
             if verbose and out.strip():

@@ -30,6 +30,7 @@
 #define FMHA_CAT3(a, b, c) a##b##_d##c
 #endif
 #define FMHA_NAME(t, d) FMHA_CAT3(bwd_dispatch_, t, d)
+#define FMHA_PIPE_NAME(t, d) FMHA_CAT3(bwd_pipe_launch_, t, d)
 
 namespace fmha {
 namespace {
@@ -44,27 +45,70 @@ template <typename K> int set_lds(K kern, int bytes) {
                              bytes) == hipSuccess ? 0 : 2;
 }
 
-template <int MASK, bool CAUSAL, int DROP> int launch(BwdArgs &a, int pair, hipStream_t s) {
-  constexpr int kLdsQ = BwdCfg<FMHA_TU_D, bwd_dq_tile_rows<FMHA_TU_D>()>::LDS_BYTES;
-  auto kq = fmha_bwd_dq_kernel<FMHA_TU_T, FMHA_TU_D, kQB, kNW, MASK, CAUSAL, DROP, kStrided>;
+// The pipelined kernels (fmha_bwd_pipe.hip) take everything but full mask tensors and head dim 256 -- at head dim 128 from
+// a number of queries on: their prologue costs more, and a causal head's streams are cut short by its diagonal (us,
+// pipelined against phase by phase, causal: S 128 110 / 95, S 256 121 / 116, S 384 130 / 129, S 512 153 / 163;
+// dropout: S 61 116 / 110, S 128 99 / 101, S 256 121 / 130).  And one exception: dK / dV at head dim 128 without causal
+// mask and dropout, where 32-row tiles at two waves per SIMD overlap one workgroup's start and stores with another's
+// arithmetic (BH 256 S 1024: 335 against 343; causal 462 against 429, with dropout 197 against 169 the other way round).
+template <int MASK, bool CAUSAL, int DROP> constexpr bool pipe_built() { return FMHA_TU_D != 256 && MASK != kMaskFull; }
+template <bool CAUSAL> bool pipe_wanted(const BwdArgs &a) { return FMHA_TU_D == 64 || a.sq >= (CAUSAL ? 384 : 128); }
+
+template <typename K> int launch_one(K kern, BwdArgs &a, long long nblk, int threads, int lds, hipStream_t s) {
+  if (nblk > 0x7fffffffLL) return 2;
+  hipLaunchKernelGGL(kern, dim3((unsigned)nblk), dim3(threads), lds, s, a);
+  return hipGetLastError() == hipSuccess ? 0 : 2;
+}
+
+template <int MASK, bool CAUSAL, int DROP> int launch_dq(BwdArgs &a, const BwdVariant &v, long long nblk, hipStream_t s) {
+#if FMHA_TU_D != 256
+  if constexpr (pipe_built<MASK, CAUSAL, DROP>()) {
+    if (pipe_wanted<CAUSAL>(a)) return FMHA_PIPE_NAME(FMHA_TU_TNAME, FMHA_TU_D)(a, v, false, nblk, s);
+  }
+#endif
+  if constexpr (!(pipe_built<MASK, CAUSAL, DROP>() && FMHA_TU_D == 64)) { // (there the pipelined kernel takes all)
+    constexpr int kLds = BwdCfg<FMHA_TU_D, bwd_dq_tile_rows<FMHA_TU_D>()>::LDS_BYTES;
+    static_assert(kLds <= 160 * 1024, "tiles do not fit the LDS of a compute unit");
+    auto kern = fmha_bwd_dq_kernel<FMHA_TU_T, FMHA_TU_D, kQB, kNW, MASK, CAUSAL, DROP, kStrided>;
+    static const int attr = set_lds(kern, kLds);
+    return attr ? 2 : launch_one(kern, a, nblk, kNW * 64, kLds, s);
+  }
+  return 1;
+}
+
+template <int MASK, bool CAUSAL, int DROP> int launch_dkdv(BwdArgs &a, const BwdVariant &v, long long nblk, hipStream_t s) {
 #if FMHA_TU_WIDE
   // head dim 256: the dK / dV work of a key block is split between two waves (fmha_bwd_wide.h; at head
   // dims 128 and 64 the same kernel measured level with and a third slower than the one-wave kernel)
-  using CfgK = BwdWideCfg<FMHA_TU_D, MASK>;
-  constexpr int kLdsK = CfgK::LDS_BYTES;
-  constexpr int kNWK = CfgK::NW, KT = CfgK::KT;
-  auto kk = fmha_bwd_dkdv_wide_kernel<FMHA_TU_T, FMHA_TU_D, MASK, CAUSAL, DROP, kStrided>;
+  using Cfg = BwdWideCfg<FMHA_TU_D, MASK>;
+  static_assert(Cfg::LDS_BYTES <= 160 * 1024, "tiles do not fit the LDS of a compute unit");
+  auto kern = fmha_bwd_dkdv_wide_kernel<FMHA_TU_T, FMHA_TU_D, MASK, CAUSAL, DROP, kStrided>;
+  static const int attr = set_lds(kern, Cfg::LDS_BYTES);
+  return attr ? 2 : launch_one(kern, a, nblk, Cfg::NW * 64, Cfg::LDS_BYTES, s);
 #else
-  using CfgK = BwdCfg<FMHA_TU_D, bwd_dkdv_tile_rows<FMHA_TU_D, CAUSAL, DROP>()>;
-  constexpr int kLdsK = CfgK::LDS_BYTES + (MASK == kMaskFull ? CfgK::MASK_BYTES : 0);
-  constexpr int kNWK = kNW, KT = kNW * kKB * 32;
-  auto kk = fmha_bwd_dkdv_kernel<FMHA_TU_T, FMHA_TU_D, kKB, kNW, MASK, CAUSAL, DROP, kStrided>;
+  constexpr bool kPipe = pipe_built<MASK, CAUSAL, DROP>() && !bwd_dkdv_small_tiles<FMHA_TU_D, CAUSAL, DROP>();
+  if constexpr (kPipe) {
+    if (pipe_wanted<CAUSAL>(a)) return FMHA_PIPE_NAME(FMHA_TU_TNAME, FMHA_TU_D)(a, v, true, nblk, s);
+  }
+  if constexpr (!(kPipe && FMHA_TU_D == 64)) {
+    using Cfg = BwdCfg<FMHA_TU_D, bwd_dkdv_tile_rows<FMHA_TU_D, CAUSAL, DROP>()>;
+    constexpr int kLds = Cfg::LDS_BYTES + (MASK == kMaskFull ? Cfg::MASK_BYTES : 0);
+    static_assert(kLds <= 160 * 1024, "tiles do not fit the LDS of a compute unit");
+    auto kern = fmha_bwd_dkdv_kernel<FMHA_TU_T, FMHA_TU_D, kKB, kNW, MASK, CAUSAL, DROP, kStrided>;
+    static const int attr = set_lds(kern, kLds);
+    return attr ? 2 : launch_one(kern, a, nblk, kNW * 64, kLds, s);
+  }
+  return 1;
 #endif
-  static_assert(kLdsQ <= 160 * 1024 && kLdsK <= 160 * 1024, "tiles do not fit the LDS of a compute unit");
-  static const int attr = set_lds(kq, kLdsQ) | set_lds(kk, kLdsK);
-  if (attr) return 2;
+}
+
+template <int MASK, bool CAUSAL, int DROP> int launch(BwdArgs &a, const BwdVariant &v, hipStream_t s) {
+#if FMHA_TU_WIDE
+  constexpr int KT = BwdWideCfg<FMHA_TU_D, MASK>::KT;
+#else
+  constexpr int KT = kNW * kKB * 32;
+#endif
   constexpr int QT = kNW * kQB * 32;
-  // dQ first: it also writes delta, which the dK/dV kernel reads (same stream => ordered)
   // causal: workgroups take pairs of tiles (see the kernels) when that leaves at least two
   // rounds of workgroups for the device
   static const int cus = [] {
@@ -73,22 +117,16 @@ template <int MASK, bool CAUSAL, int DROP> int launch(BwdArgs &a, int pair, hipS
       n = 0;
     return n;
   }();
-  a.ntile = (a.sq + QT - 1) / QT;
-  auto want_pair = [&](int ntile) {
-    if (!CAUSAL) return false;
-    return pair >= 0 ? pair != 0 : (long long)a.bh * ((ntile + 1) / 2) >= 4LL * cus;
+  auto blocks = [&](int ntile) -> long long {
+    a.ntile = ntile;
+    a.pair = CAUSAL && (v.pair >= 0 ? v.pair != 0 : (long long)a.bh * ((ntile + 1) / 2) >= 4LL * cus);
+    return (long long)a.bh * (a.pair ? (ntile + 1) / 2 : ntile);
   };
-  a.pair = want_pair(a.ntile);
-  long long nblk = (long long)a.bh * (a.pair ? (a.ntile + 1) / 2 : a.ntile);
-  if (nblk > 0x7fffffffLL) return 2;
-  hipLaunchKernelGGL(kq, dim3((unsigned)nblk), dim3(kNW * 64), kLdsQ, s, a);
-  if (hipGetLastError() != hipSuccess) return 2;
-  a.ntile = (a.sk + KT - 1) / KT;
-  a.pair = want_pair(a.ntile);
-  nblk = (long long)a.bh * (a.pair ? (a.ntile + 1) / 2 : a.ntile);
-  if (nblk > 0x7fffffffLL) return 2;
-  hipLaunchKernelGGL(kk, dim3((unsigned)nblk), dim3(kNWK * 64), kLdsK, s, a);
-  return hipGetLastError() == hipSuccess ? 0 : 2;
+  // dQ first: it also writes delta, which the dK/dV kernel reads (same stream => ordered)
+  const long long nq = blocks((a.sq + QT - 1) / QT);
+  if (const int rc = launch_dq<MASK, CAUSAL, DROP>(a, v, nq, s)) return rc;
+  const long long nk = blocks((a.sk + KT - 1) / KT);
+  return launch_dkdv<MASK, CAUSAL, DROP>(a, v, nk, s);
 }
 
 #if FMHA_TU_SHORT
@@ -104,8 +142,8 @@ template <int DROP, int SMAX, bool CAUSAL> int launch_short(BwdArgs &a, hipStrea
 #endif
 
 template <int MASK, bool CAUSAL> int by_drop(BwdArgs &a, const BwdVariant &v, hipStream_t s) {
-  if (v.drop == 0) return launch<MASK, CAUSAL, 0>(a, v.pair, s);
-  if (v.drop == 1) return launch<MASK, CAUSAL, 1>(a, v.pair, s);
+  if (v.drop == 0) return launch<MASK, CAUSAL, 0>(a, v, s);
+  if (v.drop == 1) return launch<MASK, CAUSAL, 1>(a, v, s);
   return 1;
 }
 

@@ -1,0 +1,808 @@
+// Software-pipelined backward kernels for head dims 64 and 128 (no mask or a per-key mask; full mask tensors stay on
+// fmha_bwd_kernel.h).  Mathematics, register layouts and the extra contraction step are those of fmha_bwd_kernel.h, whose
+// header describes them; what changes is the order of work and how tiles arrive:
+//
+//   * 32-row tiles, four resident per operand.  The copies of tile t + 3 are spread over iteration t, one instruction
+//     every few matrix instructions (in one burst behind the barrier they stall the issuing waves: 226 -> 216 us for dQ at
+//     BH 256 S 1024 D 128), and are waited for two iterations later with a count (`vmcnt(N)`), so no iteration waits for
+//     memory it has just asked for.  Tiles past the end re-read the last row instead of being skipped: every iteration
+//     issues the same number of copies and the counts are constants.  The first tiles are asked for before anything else.
+//   * Iteration t is one hand-ordered stream: the first products of tile t + 1 beside the exponentials of tile t (two sets
+//     of score / dP accumulators), then the gradient products of tile t, with the Philox call of tile t + 1 beside them.
+//     LDS operands are requested three or four matrix instructions ahead.  A scheduling barrier closes every slot and
+//     values are pinned to theirs (the compiler sinks exponentials towards their use otherwise).
+//   * Causal: a wave leaves out the tiles on the masked side of its own diagonal, and only the tile on it compares indexes.
+//   * The per-key mask terms (dQ) and the rows (-LSE, -delta) (dK / dV) of the whole head are staged in LDS once, in
+//     segments of 4096 keys / 1024 queries, instead of per tile through registers: a load that the compiler waits for
+//     would also wait for every copy issued ahead of it.
+//   * Gradients leave as whole rows (store_acc_rows).
+//
+// Measured against the two-stage, phase-by-phase kernels (us, dQ / dK+dV): BH 64 S 2048 D 64 without dropout
+// 114.9 / 146.0 -> 107.5 / 139.5, with dropout 140.4 / 190.1 -> 135.2 / 174.5; BH 192 S 1024 D 64 causal 78.0 / 92.1 -> 63.8 / 83.3;
+// BH 512 S 1024 D 128 causal bf16 289 / 462 -> 259 / 429; BH 32 S 4096 D 128 causal 273 / 334 -> 208 / 287.
+// What bounds them: at head dim 64 the issue slots (a matrix instruction takes the vector pipe for about 21 cycles, a
+// vector instruction for 2.5, and the sum of both is what two waves per SIMD need); at head dim 128 the board's power
+// (dQ on random data: 1.57 GHz, on zeros 2.19 GHz) and, for dK / dV at one wave per SIMD, the start and the stores of
+// workgroups that all compute units run in step (without stores 328 -> 255 us at BH 256 S 1024).
+#pragma once
+#include "fmha_bwd_kernel.h"
+
+namespace fmha {
+
+FMHA_DEV void bwd_lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+template <int N> FMHA_DEV void bwd_vm_wait() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
+
+template <int D> struct BwdPipeCfg {
+  static constexpr int BT = 32, NST = 4; // rows per tile, tiles resident per operand
+  static constexpr int KS = D / 16, DB = D / 32;
+  static constexpr int TILEB = BT * D * 2, STAGEB = 2 * TILEB;
+  static constexpr int OFF_X = NST * STAGEB;
+  static_assert(4 * RowStore<D>::BYTES <= OFF_X, "the output rows are turned in the tiles' LDS");
+  static constexpr int MSEG = 4096;             // per-key mask terms staged at once
+  static constexpr int QSEG = 1024;             // queries whose extra-step rows are staged at once (dK / dV)
+  static int dkdv_lds_bytes(int drop, int sq) { return OFF_X + 64 + (sq < QSEG ? (16 + (drop ? 4 : 0)) * ((sq + 31) / 32 * 32) : (16 + (drop ? 8 : 0)) * QSEG); }
+  static int dq_lds_bytes(int mask, int sk) { return OFF_X + (mask == kMaskPerKey ? 4 * (sk < MSEG ? (sk + 31) / 32 * 32 : MSEG) : 0) + 64; }
+};
+
+// Copies of 32-row tiles of a row-major [rows][D] matrix into swizzled LDS tiles, one instruction at a time so that
+// they can be spread over an instruction stream: rows past the end re-read the last one (a minimum on the byte offset,
+// no branch), so tiles that do not exist may be asked for and every tile costs the same number of copies.  Columns a
+// row does not have are filled with its first ones: they meet zeros in the register operand, or land in output columns
+// that are not stored.
+template <typename T, int D, int NT> struct PipeCopy {
+  static constexpr int BT = 32, CPT = BT * D / 8 / NT;
+  static_assert(CPT * NT * 8 == BT * D, "tile must divide evenly over the workgroup");
+  uint32_t voff[CPT], lim[CPT], dst;
+  uint32_t tile_step; // bytes between the first rows of consecutive tiles
+  FMHA_DEV void init(int tid, int64_t row_stride, int rend, int dv) {
+    const uint32_t ss2 = (uint32_t)row_stride * 2u;
+    tile_step = ss2 * BT;
+    dst = (uint32_t)__builtin_amdgcn_readfirstlane(tid >> 6) * 1024u;
+#pragma unroll
+    for (int i = 0; i < CPT; ++i) {
+      int row, col;
+      TileCopy<T, D, BT, NT>::slot(tid + i * NT, row, col);
+      const uint32_t cb = col * 8 < dv ? (uint32_t)col * 16u : 0u;
+      voff[i] = (uint32_t)row * ss2 + cb;
+      lim[i] = (uint32_t)(rend - 1) * ss2 + cb;
+    }
+  }
+  FMHA_DEV void issue(const T *base, int tile, uint32_t lds_tile, int i) const {
+    const uint32_t o = voff[i] + (uint32_t)tile * tile_step;
+    dma_global_to_lds_b128(base, o < lim[i] ? o : lim[i], lds_tile + dst + (uint32_t)(i * NT * 16));
+  }
+};
+
+// One Philox4x32-10 call in slices that can be spread over an instruction stream.
+struct PhiloxSlices {
+  uint32_t c[4];
+  FMHA_DEV void start(const DropCtx &d, uint32_t bh, uint32_t q4, uint32_t k4) {
+    const uint64_t blk = ((uint64_t)bh * d.qb4 + q4) * d.kb4 + k4;
+    c[0] = d.off_lo;
+    c[1] = d.off_hi;
+    c[2] = (uint32_t)blk;
+    c[3] = (uint32_t)(blk >> 32);
+  }
+  FMHA_DEV void round(const DropCtx &d, int r) {
+    const uint32_t k0 = d.seed_lo + (uint32_t)r * Philox::W0, k1 = d.seed_hi + (uint32_t)r * Philox::W1;
+    const uint64_t p0 = (uint64_t)Philox::M0 * c[0], p1 = (uint64_t)Philox::M1 * c[2];
+    const uint32_t n0 = __builtin_amdgcn_bitop3_b32((uint32_t)(p1 >> 32), c[1], k0, 0x96);
+    const uint32_t n2 = __builtin_amdgcn_bitop3_b32((uint32_t)(p0 >> 32), c[3], k1, 0x96);
+    c[0] = n0;
+    c[1] = (uint32_t)p1;
+    c[2] = n2;
+    c[3] = (uint32_t)p0;
+  }
+};
+
+// ------------------------------------------------------------------------------ dQ
+template <typename T, int D, int NW, int MASK, bool CAUSAL, int DROP, bool STRIDED>
+__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void fmha_bwd_dq_pipe_kernel(const BwdArgs a) {
+  using RW = Rows<STRIDED, D>;
+  using E = Elem<T>;
+  using v8 = typename E::v8;
+  using C = BwdPipeCfg<D>;
+  constexpr int BT = C::BT, NST = C::NST, KS = C::KS, DB = C::DB, TILEB = C::TILEB, STAGEB = C::STAGEB;
+  constexpr int NT = NW * 64, QT = NW * 32;
+  constexpr float NEG_INF = -__builtin_inff();
+  constexpr float BIGNEG = -60000.f;
+  static_assert(MASK != kMaskFull, "full mask tensors: fmha_bwd_dq_kernel");
+  // Rank-one terms: at head dim 64 the vector pipe is the busier one and they ride in an extra contraction step (XS, GS);
+  // at head dim 128 it is the matrix pipe, and a subtraction per element costs less: there only a per-key mask does.
+  constexpr bool XS = D == 64 || MASK == kMaskPerKey, GS = D == 64, LS = D == 64; // (LS: the LSE rides in the extra step)
+
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  uint32_t *ldsM = (uint32_t *)(lds + C::OFF_X + 64); // (mask_hi, mask_lo) per key of the current segment
+  int *ldsR = (int *)(lds + C::OFF_X);
+
+  const int tid = threadIdx.x;
+  const int w = tid >> 6, l = tid & 63, ql = l & 31, h = l >> 5;
+
+  int bid = blockIdx.x;
+  const int nb = gridDim.x;
+  if ((nb & 7) == 0) bid = (bid & 7) * (nb >> 3) + (bid >> 3);
+  const bool paired = CAUSAL && a.pair;
+  const int npair = paired ? (a.ntile + 1) / 2 : a.ntile;
+  const int bh = bid / npair;
+  const int pi = bid - bh * npair;
+  const int npass = (paired && a.ntile - 1 - pi != pi) ? 2 : 1;
+
+  const T *Qb = (const T *)a.q + RW::head(a.mq, bh, a.sq);
+  const T *Ob = (const T *)a.o + RW::head(a.mo, bh, a.sq);
+  const T *dOb = (const T *)a.dout + RW::head(a.mdo, bh, a.sq);
+  const T *Kb = (const T *)a.k + RW::head(a.mk, bh, a.sk);
+  const T *Vb = (const T *)a.v + RW::head(a.mv, bh, a.sk);
+  const T *mkey = (MASK == kMaskPerKey) ? (const T *)a.mask + (size_t)(bh / a.mask_div) * a.mask_sb : nullptr;
+  const int skv0 = bwd_valid_keys(a, bh);
+  int skv = skv0; // keys worth visiting
+
+  // Terms of a segment of the mask row -> LDS; returns (uniform) the number of keys up to the last one that is not
+  // hard-masked.
+  auto stage_mask = [&](int seg0) -> int {
+    constexpr float kHardMask = -9000.f * FMHA_LOG2E;
+    const int n = a.sk - seg0 < C::MSEG ? a.sk - seg0 : C::MSEG;
+    int last = -1;
+    for (int base = 0; base < n; base += 4 * NT) {
+      T v[4];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const int key = seg0 + base + c * NT + tid;
+        v[c] = mkey[key < a.sk ? key : a.sk - 1];
+      }
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const int i = base + c * NT + tid;
+        float mk = fmaf((float)v[c], a.mask_a, a.mask_b);
+        const bool live = i < n && mk > kHardMask;
+        const unsigned long long bal = __builtin_amdgcn_ballot_w64(live);
+        if (bal) last = base + c * NT + (tid & ~63) + 63 - __builtin_clzll(bal);
+        if (seg0 + i >= skv0) mk = BIGNEG;
+        T hl[2];
+        split_hi_lo<T>(mk, hl[0], hl[1]);
+        if (i < (n + 31) / 32 * 32) ldsM[i] = __builtin_bit_cast(uint32_t, *(const __attribute__((ext_vector_type(2))) T *)hl);
+      }
+    }
+    if ((tid & 63) == 0) ldsR[w] = last;
+    __syncthreads();
+    int top = -1;
+#pragma unroll
+    for (int ww = 0; ww < NW; ++ww) top = ldsR[ww] > top ? ldsR[ww] : top;
+    return __builtin_amdgcn_readfirstlane(top) + 1;
+  };
+
+  for (int pass = 0; pass < npass; ++pass) {
+    const int qt = CAUSAL ? (pass == 0 ? a.ntile - 1 - pi : pi) : pi;
+    const int q0w = qt * QT + w * 32;
+    const int q = q0w + ql;
+
+    // ---- tiles 0..2 on their way, ahead of everything that waits for memory
+    const uint32_t lds_base = lds_address(lds);
+    PipeCopy<T, D, NT> tcopy;
+    tcopy.init(tid, RW::ss(a.mk), a.sk, RW::cols(a));
+    constexpr int VPT = 2 * PipeCopy<T, D, NT>::CPT; // copies per tile pair and wave
+    auto dma_one = [&](int kt, int i) { // copy i of the K and V tiles kt
+      const uint32_t dst = lds_base + (uint32_t)(kt & (NST - 1)) * STAGEB;
+      if (i < VPT / 2) tcopy.issue(Kb, kt, dst, i);
+      else tcopy.issue(Vb, kt, dst + TILEB, i - VPT / 2);
+    };
+    auto dma_kv = [&](int kt) {
+#pragma unroll
+      for (int i = 0; i < VPT; ++i) dma_one(kt, i);
+    };
+#pragma unroll
+    for (int t = 0; t < NST - 1; ++t) dma_kv(t);
+
+    // ---- per-row operands (all loads unconditional, see fmha_bwd_dq_kernel)
+    v8 qreg[KS], doreg[KS], bxs, bxd;
+    float delta, nlse;
+    {
+      const int qc = q < a.sq ? q : a.sq - 1;
+      u32x4 tq[KS], td[KS], to[KS];
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        const size_t col = ks * 16 + h * 8 < RW::cols(a) ? ks * 16 + h * 8 : 0;
+        tq[ks] = *(const u32x4 *)(Qb + (size_t)qc * RW::ss(a.mq) + col);
+        td[ks] = *(const u32x4 *)(dOb + (size_t)qc * RW::ss(a.mdo) + col);
+        to[ks] = *(const u32x4 *)(Ob + (size_t)qc * RW::ss(a.mo) + col);
+      }
+      const float lse_q = a.lse[(size_t)bh * a.sq + qc];
+      if (MASK == kMaskPerKey && pass == 0) {
+        const int n = stage_mask(0); // (its loads share the trip to memory)
+        const bool trim = a.sk > 128 && a.sk <= C::MSEG && !(a.flags & kBwdFlagNoTrim);
+        if (trim && n > 0 && n < skv) skv = n; // a row without any live key keeps all its keys
+      }
+      float dsum = 0.f;
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        const bool live = ks * 16 + h * 8 < RW::cols(a);
+        const v8 qraw = as_v8<T>(chunk_or_zero(tq[ks], live));
+        const v8 doraw = as_v8<T>(chunk_or_zero(td[ks], live));
+        const v8 ov = as_v8<T>(to[ks]);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          qreg[ks][j] = (T)((float)qraw[j] * a.scale_l2);
+          doreg[ks][j] = DROP == 1 ? (T)((float)doraw[j] * a.drop_scale) : doraw[j];
+          dsum = fmaf((float)doraw[j], (float)ov[j], dsum);
+        }
+      }
+      dsum = xhalf_sum(dsum);
+      delta = dsum;
+      float nl = BIGNEG; // rows past the end and fully masked rows get P = 0
+      if (q < a.sq) {
+        if (lse_q != NEG_INF) nl = -lse_q * FMHA_LOG2E;
+        if (h == 0) a.delta[(size_t)bh * a.sq + q] = dsum;
+      }
+      nlse = nl;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        bxs[j] = (T)0.f;
+        bxd[j] = (T)0.f;
+      }
+      if (h == 0) {
+        T hi, lo;
+        split_hi_lo<T>(LS ? nl : 0.f, hi, lo);
+        bxs[0] = hi;
+        bxs[1] = lo;
+        bxs[2] = (T)1.f;
+        bxs[3] = (T)1.f;
+        split_hi_lo<T>(-dsum, hi, lo);
+        bxd[0] = hi;
+        bxd[1] = lo;
+      }
+    }
+
+    int nkt = (skv + BT - 1) / BT;
+    if (nkt < 1) nkt = 1;
+    if (CAUSAL) {
+      int qmax = qt * QT + QT - 1;
+      if (qmax > a.sq - 1) qmax = a.sq - 1;
+      const int need = qmax / BT + 1;
+      if (need < nkt) nkt = need;
+    }
+    const int kend = nkt * BT < skv ? nkt * BT : skv;
+    const int last_key = CAUSAL && q < kend - 1 ? q : kend - 1; // of this lane's row
+    // causal: tiles past the one that holds this wave's own diagonal are all masked for it
+    const int ws = __builtin_amdgcn_readfirstlane(w);
+    int nktw = nkt;
+    if (CAUSAL) {
+      const int own = (qt * QT + ws * 32) / BT + 1;
+      nktw = own < nkt ? own : nkt;
+    }
+
+    PanelLane pl;
+    pl.init(l);
+    constexpr uint32_t ONES = std::is_same<T, _Float16>::value ? 0x3c003c00u : 0x3f803f80u;
+    constexpr uint32_t BIGPAIR = std::is_same<T, _Float16>::value ? 0x0000fb53u : 0x0000c76au; // (-60000 in T, 0)
+    auto hl_of = [&](int kt) -> uint32_t { // (mask_hi, mask_lo) of key (l % 32) of a tile
+      const int key = kt * BT + ql;
+      if (MASK == kMaskPerKey) {
+        const uint32_t m = ldsM[key & (C::MSEG - 1)];
+        return key < kend ? m : BIGPAIR;
+      }
+      return key < kend ? 0u : BIGPAIR;
+    };
+    auto xa_of = [&](uint32_t hl) -> v8 { return as_v8<T>(u32x4{ONES, hl, 0u, 0u}); };
+
+    f32x16 dq[DB];
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) dq[db][r] = 0.f;
+
+    f32x16 xA, gA, xB, gB;
+    uint32_t wdA[4], wdB[4];
+    PhiloxSlices ph;
+
+    // The stream of one tile: first products of tile kt + 1 into (xn, gn) beside the softmax of tile kt (xc, gc),
+    // then dQ^T += K(kt)^T.dS(kt)^T; the Philox call of tile kt + 1 behind the softmax.
+    auto step = [&](auto next_tag, auto guard_tag, int kt, uint32_t hl, const f32x16 &xc, const f32x16 &gc,
+                    const uint32_t (&wc)[4], f32x16 &xn, f32x16 &gn, uint32_t (&wn)[4]) {
+      constexpr bool NEXT = decltype(next_tag)::value, GUARD = decltype(guard_tag)::value;
+      constexpr int NX = NEXT ? (XS ? 1 : 0) + (GS ? 1 : 0) : 0, NA = NEXT ? 2 * KS : 0, NC = 2 * DB, NO = NA + NC, NM = NX + NO;
+      constexpr int AHEAD = 3;
+      constexpr int NS = 10;                                  // softmax slots: 8 pairs, two to drain
+      constexpr int NP = DROP == 1 && NEXT ? 14 : 0;          // Philox slots
+      constexpr int JS = NEXT ? NX + NA : 0;                  // the softmax is done before matrix instruction JS
+      const char *ldsN = lds + ((kt + 1) & (NST - 1)) * STAGEB;
+      const char *ldsC = lds + (kt & (NST - 1)) * STAGEB;
+      const int k0 = kt * BT;
+      auto fetch = [&](int j) -> v8 {
+        if (j < NA) return panel_read_rows<T, BT>(ldsN + (j & 1) * TILEB, pl, 0, j >> 1);
+        const int i = j - NA;
+        return panel_read_transposed<T, BT>(ldsC, pl, 0, i % DB, i / DB);
+      };
+      float p[16];
+      bool keep[16];
+      v8 frag[2];
+      auto softmax = [&](int s) {
+        if (s < 8) {
+#pragma unroll
+          for (int e = 2 * s; e < 2 * s + 2; ++e) {
+            float xv = xc[e];
+            if (!LS) xv += nlse;
+            if (GUARD) xv = (k0 + 8 * (e / 4) + 4 * h + e % 4 <= last_key) ? xv : BIGNEG;
+            p[e] = fast_exp2(xv);
+            asm volatile("" : "+v"(p[e])); // (stays in this slot: left alone the compiler sinks it towards its use)
+            if (DROP == 1) keep[e] = drop_keep_byte(wc[e / 4], e % 4, a.drop.thr); // (used one slot on: no wait for it)
+          }
+        }
+        if (s >= 1 && s < 9) {
+#pragma unroll
+          for (int e = 2 * (s - 1); e < 2 * s; ++e) {
+            float gv = gc[e];
+            if (DROP == 1) gv = keep[e] ? gv : (GS ? -delta : 0.f);
+            if (!GS) gv -= delta;
+            p[e] *= gv;
+            asm volatile("" : "+v"(p[e]));
+          }
+        }
+        if (s >= 2) {
+#pragma unroll
+          for (int e = 2 * (s - 2); e < 2 * (s - 1); ++e) frag[e / 8][e % 8] = (T)p[e];
+        }
+      };
+      auto philox = [&](int s) {
+        if (s == 0) ph.start(a.drop, (uint32_t)bh, (uint32_t)q >> 2, (uint32_t)((k0 + BT) >> 2) + (uint32_t)h + 2u * ((uint32_t)l & 3u));
+        else if (s <= 10) ph.round(a.drop, s - 1);
+        else if (s == 11) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) wn[i] = ph.c[i];
+          quad_transpose4(wn, l);
+        }
+      };
+      v8 opnd[NO];
+#pragma unroll
+      for (int j = 0; j < AHEAD && j < NO; ++j) opnd[j] = fetch(j);
+      int done = 0;
+      if (!NEXT) {
+#pragma unroll
+        for (; done < NS; ++done) softmax(done);
+      }
+#pragma unroll
+      for (int m = 0; m < NM; ++m) {
+        if (m < NX) {
+          const v8 xa = xa_of(hl);
+          f32x16 z;
+#pragma unroll
+          for (int r = 0; r < 16; ++r) z[r] = 0.f;
+          if (XS && m == 0) xn = E::mfma(xa, bxs, z);
+          else gn = E::mfma(xa, bxd, z);
+        } else {
+          const int j = m - NX;
+          if (j + AHEAD < NO) opnd[j + AHEAD] = fetch(j + AHEAD);
+          if (j < NA) {
+            f32x16 z;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) z[r] = 0.f;
+            if ((j & 1) == 0) xn = E::mfma(opnd[j], qreg[j >> 1], !XS && j == 0 ? z : xn);
+            else gn = E::mfma(opnd[j], doreg[j >> 1], !GS && j == 1 ? z : gn);
+          } else {
+            const int i = j - NA;
+            dq[i % DB] = E::mfma(opnd[j], frag[i / DB], dq[i % DB]);
+          }
+        }
+        if (m % (NM / VPT) == NM / VPT - 1 && m / (NM / VPT) < VPT) dma_one(kt + NST - 1, m / (NM / VPT));
+        const int upto = m < JS ? (m + 1) * NS / (JS ? JS : 1) : NS + (m - JS + 1) * NP / (NM - JS);
+#pragma unroll
+        for (; done < upto; ++done) {
+          if (done < NS) softmax(done);
+          else philox(done - NS);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    using Yes = std::true_type;
+    using No = std::false_type;
+
+    // ---- first products of tile 0 (its wait covers the loads above too: they are younger than its copies)
+    bwd_vm_wait<0>();
+    bwd_lds_barrier();
+    auto first = [&](f32x16 &x, f32x16 &g) {
+      const v8 xa = xa_of(hl_of(0));
+      f32x16 z;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) z[r] = 0.f;
+      x = XS ? E::mfma(xa, bxs, z) : z;
+      g = GS ? E::mfma(xa, bxd, z) : z;
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        x = E::mfma(panel_read_rows<T, BT>(lds, pl, 0, ks), qreg[ks], x);
+        g = E::mfma(panel_read_rows<T, BT>(lds + TILEB, pl, 0, ks), doreg[ks], g);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    // top of the iteration of tile kt: tile kt + 1 has landed, tile kt + 3 goes on its way
+    auto turn = [&](int kt) -> uint32_t {
+      if (MASK == kMaskPerKey && ((kt + 1) * BT & (C::MSEG - 1)) == 0 && kt + 1 < nkt) stage_mask((kt + 1) * BT); // (4096 keys on)
+      const uint32_t hl = hl_of(kt + 1);
+      bwd_vm_wait<(NST - 3) * VPT>();
+      bwd_lds_barrier(); // ... everybody's part of it, and tile kt - 1 is no longer read
+      return hl;
+    };
+    auto mid = [&](int kt, const f32x16 &xc, const f32x16 &gc, const uint32_t (&wc)[4], f32x16 &xn, f32x16 &gn, uint32_t (&wn)[4]) {
+      const uint32_t hl = turn(kt);
+      step(Yes{}, No{}, kt, hl, xc, gc, wc, xn, gn, wn);
+    };
+    int kt = 0;
+    const int nmid = nktw - 1;
+    if (nmid & 1) {
+      if (DROP == 1) drop_words_q(a.drop, (uint32_t)bh, (uint32_t)q, 0u, h, l, wdB);
+      first(xB, gB);
+      mid(0, xB, gB, wdB, xA, gA, wdA);
+      kt = 1;
+    } else {
+      if (DROP == 1) drop_words_q(a.drop, (uint32_t)bh, (uint32_t)q, 0u, h, l, wdA);
+      first(xA, gA);
+    }
+    for (; kt < nmid; kt += 2) {
+      mid(kt, xA, gA, wdA, xB, gB, wdB);
+      mid(kt + 1, xB, gB, wdB, xA, gA, wdA);
+    }
+    {
+      turn(kt);
+      step(No{}, std::integral_constant<bool, CAUSAL || !XS>{}, kt, 0u, xA, gA, wdA, xB, gB, wdB);
+      for (++kt; kt < nkt; ++kt) {
+        turn(kt);
+        dma_kv(kt + NST - 1);
+      } // (causal: tiles that only later waves of the workgroup need)
+    }
+
+    bwd_vm_wait<0>(); // no copy may still be on its way into LDS when the wave ends, or the next pass starts
+    bwd_lds_barrier(); // (every wave is done with the tiles: their LDS turns the output rows)
+    {
+      T *dQb = (T *)a.dq + RW::head(a.mdq, bh, a.sq) + (size_t)q0w * RW::ss(a.mdq);
+      store_acc_rows<T, D>(lds + w * RowStore<D>::BYTES, dq, a.scale, dQb, RW::ss(a.mdq), a.sq - q0w, RW::cols(a), l);
+    }
+    __syncthreads(); // the next pass refills the tiles
+  }
+}
+
+// --------------------------------------------------------------------------- dK, dV
+template <int D> constexpr int bwd_dkdv_pipe_occ() { return D == 64 ? 2 : 1; }
+
+template <typename T, int D, int NW, int MASK, bool CAUSAL, int DROP, bool STRIDED>
+__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(bwd_dkdv_pipe_occ<D>(), bwd_dkdv_pipe_occ<D>()))) void fmha_bwd_dkdv_pipe_kernel(const BwdArgs a) {
+  using RW = Rows<STRIDED, D>;
+  using E = Elem<T>;
+  using v8 = typename E::v8;
+  using C = BwdPipeCfg<D>;
+  constexpr int BT = C::BT, NST = C::NST, KS = C::KS, DB = C::DB, TILEB = C::TILEB, STAGEB = C::STAGEB;
+  constexpr int NT = NW * 64, KT = NW * 32;
+  constexpr float NEG_INF = -__builtin_inff();
+  constexpr float BIGNEG = -60000.f;
+  static_assert(MASK != kMaskFull, "full mask tensors: fmha_bwd_dkdv_kernel");
+
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  int *ldsR = (int *)(lds + C::OFF_X);
+  u32x4 *ldsX = (u32x4 *)(lds + C::OFF_X + 64); // per query of the segment: (-L_hi, -L_lo, 1, 1, -delta_hi, -delta_lo, 0, 0)
+  const int nseg = a.sq < C::QSEG ? (a.sq + 31) / 32 * 32 : C::QSEG;
+  float *ldsD = (float *)(ldsX + nseg);         // -delta (dropout)
+
+  const int tid = threadIdx.x;
+  const int w = tid >> 6, l = tid & 63, kl = l & 31, h = l >> 5;
+
+  int bid = blockIdx.x;
+  const int nb = gridDim.x;
+  if ((nb & 7) == 0) bid = (bid & 7) * (nb >> 3) + (bid >> 3);
+  const bool paired = CAUSAL && a.pair;
+  const int npair = paired ? (a.ntile + 1) / 2 : a.ntile;
+  const int bh = bid / npair;
+  const int pi = bid - bh * npair;
+  const int npass = (paired && a.ntile - 1 - pi != pi) ? 2 : 1;
+
+  const T *Qb = (const T *)a.q + RW::head(a.mq, bh, a.sq);
+  const T *dOb = (const T *)a.dout + RW::head(a.mdo, bh, a.sq);
+  const T *Kb = (const T *)a.k + RW::head(a.mk, bh, a.sk);
+  const T *Vb = (const T *)a.v + RW::head(a.mv, bh, a.sk);
+  const float *lseb = a.lse + (size_t)bh * a.sq;
+  const float *delb = a.delta + (size_t)bh * a.sq;
+  const int skv = bwd_valid_keys(a, bh); // keys at or past it are invalid: their dK, dV rows are zero
+  MaskTail<T, NT> tail;
+  int live_keys = a.sk;
+  if (MASK == kMaskPerKey) tail.issue(a, (const T *)a.mask + (size_t)(bh / a.mask_div) * a.mask_sb, tid);
+
+  auto stage_rows = [&](int seg0) { // extra-step rows of queries seg0 .. seg0 + nseg - 1
+    for (int base = 0; base < nseg; base += 4 * NT) {
+      float lr[4], dr[4];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const int q = seg0 + base + c * NT + tid, qc = q < a.sq ? q : a.sq - 1;
+        lr[c] = lseb[qc];
+        dr[c] = delb[qc];
+      }
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const int i = base + c * NT + tid;
+        const bool ok = seg0 + i < a.sq && lr[c] != NEG_INF; // rows past the end and fully masked rows: P = 0
+        const float nl = ok ? -lr[c] * FMHA_LOG2E : BIGNEG, nd = ok ? -dr[c] : 0.f;
+        v8 x;
+        split_hi_lo<T>(nl, ((T *)&x)[0], ((T *)&x)[1]);
+        x[2] = (T)1.f;
+        x[3] = (T)1.f;
+        split_hi_lo<T>(nd, ((T *)&x)[4], ((T *)&x)[5]);
+        x[6] = (T)0.f;
+        x[7] = (T)0.f;
+        if (i < nseg) {
+          ldsX[i] = as_u32x4(x);
+          if (DROP == 1) ldsD[(seg0 + i) & (2 * C::QSEG - 1)] = nd; // (the previous segment's stay: its last tile is still to come)
+        }
+      }
+    }
+  };
+
+  for (int pass = 0; pass < npass; ++pass) {
+    const int ktile = pass == 0 ? pi : a.ntile - 1 - pi;
+    const int k0w = ktile * KT + w * 32;
+    const int key = k0w + kl;
+    const int nqt = (a.sq + BT - 1) / BT;
+    const int qt0 = CAUSAL ? ktile * KT / BT : 0; // first query tile that sees any of these keys
+
+    // ---- the first three tiles on their way
+    const uint32_t lds_base = lds_address(lds);
+    PipeCopy<T, D, NT> qcopy, dcopy; // Q and dO rows need not be equally far apart
+    qcopy.init(tid, RW::ss(a.mq), a.sq, RW::cols(a));
+    dcopy.init(tid, RW::ss(a.mdo), a.sq, RW::cols(a));
+    constexpr int VPT = 2 * PipeCopy<T, D, NT>::CPT;
+    auto dma_one = [&](int qt, int i) {
+      const uint32_t dst = lds_base + (uint32_t)(qt & (NST - 1)) * STAGEB;
+      if (i < VPT / 2) qcopy.issue(Qb, qt, dst, i);
+      else dcopy.issue(dOb, qt, dst + TILEB, i - VPT / 2);
+    };
+    auto dma_qdo = [&](int qt) {
+#pragma unroll
+      for (int i = 0; i < VPT; ++i) dma_one(qt, i);
+    };
+#pragma unroll
+    for (int t = 0; t < NST - 1; ++t) dma_qdo(qt0 + t);
+
+    // ---- per-key operands
+    v8 kreg[KS], vreg[KS], bxs, bxd;
+    {
+      const int kc = key < a.sk ? key : a.sk - 1;
+      u32x4 tk[KS], tv[KS];
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        const size_t col = ks * 16 + h * 8 < RW::cols(a) ? ks * 16 + h * 8 : 0;
+        tk[ks] = *(const u32x4 *)(Kb + (size_t)kc * RW::ss(a.mk) + col);
+        tv[ks] = *(const u32x4 *)(Vb + (size_t)kc * RW::ss(a.mv) + col);
+      }
+      T mraw = (T)0.f;
+      if (MASK == kMaskPerKey) mraw = ((const T *)a.mask)[(size_t)(bh / a.mask_div) * a.mask_sb + kc];
+      if (pass == 0 || a.sq > C::QSEG) stage_rows(qt0 * BT / C::QSEG * C::QSEG);
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        const bool live = ks * 16 + h * 8 < RW::cols(a);
+        const v8 kraw = as_v8<T>(chunk_or_zero(tk[ks], live));
+        const v8 vraw = as_v8<T>(chunk_or_zero(tv[ks], live));
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          kreg[ks][j] = (T)((float)kraw[j] * a.scale_l2);
+          vreg[ks][j] = DROP == 1 ? (T)((float)vraw[j] * a.drop_scale) : vraw[j];
+        }
+      }
+      float mk = 0.f;
+      if (MASK == kMaskPerKey) mk = fmaf((float)mraw, a.mask_a, a.mask_b);
+      if (key >= skv) mk = BIGNEG;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        bxs[j] = (T)0.f;
+        bxd[j] = (T)0.f;
+      }
+      if (h == 0) {
+        bxs[0] = (T)1.f;
+        bxs[1] = (T)1.f;
+        T hi, lo;
+        split_hi_lo<T>(mk, hi, lo);
+        bxs[2] = hi;
+        bxs[3] = lo;
+        bxd[4] = (T)1.f;
+        bxd[5] = (T)1.f;
+      }
+    }
+    if (MASK == kMaskPerKey && pass == 0) live_keys = tail.finish(a, ldsR, tid);
+    const bool dead = ktile * KT >= (live_keys < skv ? live_keys : skv); // the whole key tile is invalid
+
+    f32x16 dk[DB], dv[DB];
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        dk[db][r] = 0.f;
+        dv[db][r] = 0.f;
+      }
+
+    PanelLane pl;
+    pl.init(l);
+    f32x16 xA, gA, xB, gB;
+    uint32_t rbA[4], rbB[4];
+    PhiloxSlices ph;
+    const uint32_t sel1 = (l & 1) ? 0x03070105u : 0x06020400u, sel2 = (l & 2) ? 0x03020706u : 0x05040100u; // see drop_bytes_k
+
+    auto xrow = [&](int qt) -> v8 { return as_v8<T>(ldsX[(qt * BT + kl) & (C::QSEG - 1)]); };
+    auto step = [&](auto next_tag, auto guard_tag, int qt, const f32x16 &xc, const f32x16 &gc, const uint32_t (&rc)[4],
+                    f32x16 &xn, f32x16 &gn, uint32_t (&rn)[4]) {
+      constexpr bool NEXT = decltype(next_tag)::value, GUARD = decltype(guard_tag)::value;
+      constexpr int NX = NEXT ? 2 : 0, NA = NEXT ? 2 * KS : 0, NC = 4 * DB, NO = NA + NC, NM = NX + NO;
+      constexpr int AHEAD = D == 128 ? 4 : 3;
+      constexpr bool SWAP = D == 128;
+      constexpr int NS = 10;
+      constexpr int NP = DROP == 1 && NEXT ? 15 : 0;
+      constexpr int JS = NEXT ? NX + NA : 0;
+      const char *ldsN = lds + ((qt + 1) & (NST - 1)) * STAGEB;
+      const char *ldsC = lds + (qt & (NST - 1)) * STAGEB;
+      const int q0 = qt * BT;
+      auto fetch = [&](int j) -> v8 {
+        if (j < NA) return panel_read_rows<T, BT>(ldsN + (j & 1) * TILEB, pl, 0, j >> 1);
+        const int i = j - NA; // dO^T and Q^T alternate
+        return panel_read_transposed<T, BT>(ldsC + ((i & 1) ^ 1) * TILEB, pl, 0, (i >> 1) % DB, (i >> 1) / DB);
+      };
+      float p[16], ds[16];
+      bool keep[16];
+      f32x4 Dl[4];
+      v8 pf[2], df[2];
+      auto softmax = [&](int s) {
+        if (s < 8) {
+          if (DROP == 1 && s % 2 == 0) Dl[s / 2] = *(const f32x4 *)(ldsD + ((q0 + 8 * (s / 2) + 4 * h) & (2 * C::QSEG - 1)));
+#pragma unroll
+          for (int e = 2 * s; e < 2 * s + 2; ++e) {
+            float xv = xc[e];
+            if (GUARD) xv = (key <= q0 + 8 * (e / 4) + 4 * h + e % 4) ? xv : BIGNEG;
+            p[e] = fast_exp2(xv);
+            asm volatile("" : "+v"(p[e])); // (stays in this slot)
+            if (DROP == 1) keep[e] = drop_keep_byte(rc[e % 4], e / 4, a.drop.thr);
+          }
+        }
+        if (s >= 1 && s < 9) {
+#pragma unroll
+          for (int e = 2 * (s - 1); e < 2 * s; ++e) {
+            float gv = gc[e];
+            if (DROP == 1) gv = keep[e] ? gv : Dl[e / 4][e % 4];
+            ds[e] = p[e] * gv;
+            if (DROP == 1) p[e] = keep[e] ? p[e] : 0.f; // (drop_scale multiplies dV once, on store)
+            asm volatile("" : "+v"(ds[e]), "+v"(p[e]));
+          }
+        }
+        if (s >= 2) {
+#pragma unroll
+          for (int e = 2 * (s - 2); e < 2 * (s - 1); ++e) {
+            pf[e / 8][e % 8] = (T)p[e];
+            df[e / 8][e % 8] = (T)ds[e];
+          }
+        }
+      };
+      auto philox = [&](int s) {
+        if (s == 0) ph.start(a.drop, (uint32_t)bh, (uint32_t)((q0 + BT) >> 2) + (uint32_t)h + 2u * ((uint32_t)l & 3u), (uint32_t)key >> 2);
+        else if (s <= 10) ph.round(a.drop, s - 1);
+        else {
+          const int t = s - 11;
+          const uint32_t a1 = __builtin_amdgcn_perm(quad_perm<0xB1>(ph.c[t]), ph.c[t], sel1);
+          rn[t] = __builtin_amdgcn_perm(quad_perm<0x4E>(a1), a1, sel2);
+        }
+      };
+      v8 opnd[NO], xa;
+      if (NEXT) xa = xrow(qt + 1);
+#pragma unroll
+      for (int j = 0; j < AHEAD && j < NO; ++j) opnd[j] = fetch(j);
+      int done = 0;
+      if (!NEXT) {
+#pragma unroll
+        for (; done < NS; ++done) softmax(done);
+      }
+#pragma unroll
+      for (int m = 0; m < NM; ++m) {
+        if (m < NX) {
+          f32x16 z;
+#pragma unroll
+          for (int r = 0; r < 16; ++r) z[r] = 0.f;
+          if (m == 0) xn = E::mfma(xa, bxs, z);
+          else gn = E::mfma(xa, bxd, z);
+        } else {
+          const int j = m - NX;
+          if (j + AHEAD < NO) opnd[j + AHEAD] = fetch(j + AHEAD);
+          const int u = SWAP ? j ^ 1 : j; // (the later one of a pair first: its wait covers the other)
+          if (u < NA) {
+            if ((u & 1) == 0) xn = E::mfma(opnd[u], kreg[u >> 1], xn);
+            else gn = E::mfma(opnd[u], vreg[u >> 1], gn);
+          } else {
+            const int i = u - NA, db = (i >> 1) % DB, c = (i >> 1) / DB;
+            f32x16 &acc = (i & 1) ? dk[db] : dv[db];
+            const v8 fr = (i & 1) ? df[c] : pf[c];
+            acc = E::mfma(opnd[u], fr, acc);
+          }
+        }
+        if (m % (NM / VPT) == NM / VPT - 1 && m / (NM / VPT) < VPT) dma_one(qt + NST - 1, m / (NM / VPT));
+        const int upto = m < JS ? (m + 1) * NS / (JS ? JS : 1) : NS + (m - JS + 1) * NP / (NM - JS);
+#pragma unroll
+        for (; done < upto; ++done) {
+          if (done < NS) softmax(done);
+          else philox(done - NS);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    using Yes = std::true_type;
+    using No = std::false_type;
+    using Guard = std::integral_constant<bool, CAUSAL>;
+
+    auto first = [&](int qt, f32x16 &x, f32x16 &g, uint32_t (&rb)[4]) {
+      const char *t = lds + (qt & (NST - 1)) * STAGEB;
+      if (DROP == 1) drop_bytes_k(a.drop, (uint32_t)bh, (uint32_t)(qt * BT), (uint32_t)key, h, l, rb);
+      const v8 xa = xrow(qt);
+      f32x16 z;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) z[r] = 0.f;
+      x = E::mfma(xa, bxs, z);
+      g = E::mfma(xa, bxd, z);
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        x = E::mfma(panel_read_rows<T, BT>(t, pl, 0, ks), kreg[ks], x);
+        g = E::mfma(panel_read_rows<T, BT>(t + TILEB, pl, 0, ks), vreg[ks], g);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    // top of the iteration of tile qt: tile qt + 1 has landed, tile qt - 1 is no longer read
+    auto turn = [&](int qt) {
+      if (a.sq > C::QSEG && ((qt + 1) * BT & (C::QSEG - 1)) == 0 && qt + 1 < nqt) { // the next segment's extra-step rows
+        bwd_lds_barrier();
+        stage_rows((qt + 1) * BT);
+      }
+      bwd_vm_wait<(NST - 3) * VPT>();
+      bwd_lds_barrier();
+    };
+    bwd_vm_wait<0>();
+    bwd_lds_barrier();
+    if (!dead && qt0 < nqt) {
+      // causal: query tiles ahead of the one that holds this wave's own diagonal see none of its keys
+      int t0 = qt0;
+      if (CAUSAL) {
+        const int own = (ktile * KT + __builtin_amdgcn_readfirstlane(w) * 32) / BT;
+        const int stop = own < nqt ? own : nqt; // (no query at all may see them)
+        for (; t0 < stop; ++t0) {
+          turn(t0);
+          dma_qdo(t0 + NST - 1);
+        }
+      }
+      if (t0 < nqt) {
+        const int nmid = nqt - 1 - t0;
+        int qt = t0;
+        if (nmid & 1) {
+          first(qt, xB, gB, rbB);
+          turn(qt);
+          step(Yes{}, Guard{}, qt, xB, gB, rbB, xA, gA, rbA);
+          ++qt;
+        } else {
+          first(qt, xA, gA, rbA);
+          if (CAUSAL && nmid > 0) {
+            turn(qt);
+            step(Yes{}, Guard{}, qt, xA, gA, rbA, xB, gB, rbB);
+            turn(qt + 1);
+            step(Yes{}, No{}, qt + 1, xB, gB, rbB, xA, gA, rbA);
+            qt += 2;
+          }
+        }
+        for (; qt < nqt - 1; qt += 2) {
+          turn(qt);
+          step(Yes{}, No{}, qt, xA, gA, rbA, xB, gB, rbB);
+          turn(qt + 1);
+          step(Yes{}, No{}, qt + 1, xB, gB, rbB, xA, gA, rbA);
+        }
+        turn(qt);
+        if (CAUSAL && nmid == 0) step(No{}, Guard{}, qt, xA, gA, rbA, xB, gB, rbB);
+        else step(No{}, No{}, qt, xA, gA, rbA, xB, gB, rbB);
+      }
+    }
+    bwd_vm_wait<0>(); // no copy may still be on its way into LDS when the wave ends, or the next pass starts
+
+    bwd_lds_barrier(); // (every wave is done with the tiles: their LDS turns the output rows)
+    {
+      T *dKb = (T *)a.dk + RW::head(a.mdk, bh, a.sk) + (size_t)k0w * RW::ss(a.mdk);
+      T *dVb = (T *)a.dv + RW::head(a.mdv, bh, a.sk) + (size_t)k0w * RW::ss(a.mdv);
+      char *scratch = lds + w * RowStore<D>::BYTES;
+      store_acc_rows<T, D>(scratch, dk, a.scale, dKb, RW::ss(a.mdk), a.sk - k0w, RW::cols(a), l);
+      store_acc_rows<T, D>(scratch, dv, DROP == 1 ? a.drop_scale : 1.f, dVb, RW::ss(a.mdv), a.sk - k0w, RW::cols(a), l);
+    }
+    __syncthreads(); // the next pass refills the tiles
+  }
+}
+
+} // namespace fmha

@@ -1,0 +1,63 @@
+// Instantiates the software-pipelined backward kernels for one (element type, head dim, row layout kind) triple, chosen
+// with -DFMHA_TU_BF16={0,1} -DFMHA_TU_D={64,128} -DFMHA_TU_STRIDED={0,1}, and exports their launcher.
+#include "fmha_launch.h"
+#include "fmha_bwd_pipe.h"
+#ifndef FMHA_TU_STRIDED
+#define FMHA_TU_STRIDED 0
+#endif
+
+#if FMHA_TU_BF16
+#define FMHA_TU_T __bf16
+#define FMHA_TU_TNAME bf16
+#else
+#define FMHA_TU_T _Float16
+#define FMHA_TU_TNAME f16
+#endif
+#if FMHA_TU_STRIDED
+#define FMHA_CAT3(a, b, c) a##b##_d##c##_strided
+#else
+#define FMHA_CAT3(a, b, c) a##b##_d##c
+#endif
+#define FMHA_PIPE_NAME(t, d) FMHA_CAT3(bwd_pipe_launch_, t, d)
+
+namespace fmha {
+namespace {
+
+constexpr int kNW = 4;
+constexpr bool kStrided = FMHA_TU_STRIDED != 0;
+using Cfg = BwdPipeCfg<FMHA_TU_D>;
+
+template <int MASK, bool CAUSAL, int DROP> int launch(const BwdArgs &a, bool dkdv, long long nblk, hipStream_t s) {
+  if (dkdv) {
+    if constexpr (bwd_dkdv_small_tiles<FMHA_TU_D, CAUSAL, DROP>()) return 1; // stays on fmha_bwd_dkdv_kernel
+    else {
+      static const bool ready = hipFuncSetAttribute(reinterpret_cast<const void *>(fmha_bwd_dkdv_pipe_kernel<FMHA_TU_T, FMHA_TU_D, kNW, MASK, CAUSAL, DROP, kStrided>),
+                                                    hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::dkdv_lds_bytes(DROP, Cfg::QSEG)) == hipSuccess;
+      if (!ready || nblk > 0x7fffffffLL) return 2;
+      hipLaunchKernelGGL((fmha_bwd_dkdv_pipe_kernel<FMHA_TU_T, FMHA_TU_D, kNW, MASK, CAUSAL, DROP, kStrided>), dim3((unsigned)nblk),
+                         dim3(kNW * 64), Cfg::dkdv_lds_bytes(DROP, a.sq), s, a);
+    }
+  } else {
+    static const bool ready = hipFuncSetAttribute(reinterpret_cast<const void *>(fmha_bwd_dq_pipe_kernel<FMHA_TU_T, FMHA_TU_D, kNW, MASK, CAUSAL, DROP, kStrided>),
+                                                  hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::dq_lds_bytes(MASK, Cfg::MSEG)) == hipSuccess;
+    if (!ready || nblk > 0x7fffffffLL) return 2;
+    hipLaunchKernelGGL((fmha_bwd_dq_pipe_kernel<FMHA_TU_T, FMHA_TU_D, kNW, MASK, CAUSAL, DROP, kStrided>), dim3((unsigned)nblk),
+                       dim3(kNW * 64), Cfg::dq_lds_bytes(MASK, a.sk), s, a);
+  }
+  return hipGetLastError() == hipSuccess ? 0 : 2;
+}
+
+template <int MASK> int by_mask(const BwdArgs &a, const BwdVariant &v, bool dkdv, long long nblk, hipStream_t s) {
+  if (v.causal) return v.drop ? launch<MASK, true, 1>(a, dkdv, nblk, s) : launch<MASK, true, 0>(a, dkdv, nblk, s);
+  return v.drop ? launch<MASK, false, 1>(a, dkdv, nblk, s) : launch<MASK, false, 0>(a, dkdv, nblk, s);
+}
+
+} // namespace
+
+int FMHA_PIPE_NAME(FMHA_TU_TNAME, FMHA_TU_D)(const BwdArgs &a, const BwdVariant &v, bool dkdv, long long nblk, hipStream_t s) {
+  if (v.mask == kMaskPerKey) return by_mask<kMaskPerKey>(a, v, dkdv, nblk, s);
+  if (v.mask == kMaskNone) return by_mask<kMaskNone>(a, v, dkdv, nblk, s);
+  return 1;
+}
+
+} // namespace fmha

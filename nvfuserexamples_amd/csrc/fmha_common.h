@@ -327,6 +327,42 @@ template <typename T> FMHA_DEV void store_acc_block_row(T *dst_row, const f32x16
   }
 }
 
+// Store of a wave's 32 (rows = lanes) x D accumulator block as whole rows.  store_acc_block_row writes 32-byte pieces of
+// 32 different rows per instruction; here the block is turned in a wave-private LDS scratch first (its accesses execute
+// in order, no barrier) and leaves as 16 bytes per lane along the rows: every instruction writes complete cache lines.
+template <int D> struct RowStore {
+  static constexpr int PITCH = D * 2 + 16, BYTES = 32 * PITCH; // of LDS per wave, 16-byte aligned
+  static constexpr int LPR = D / 8, RPI = 64 / LPR;             // lanes per row, rows per instruction
+};
+// base: row 0 of the block; rows [0, nrows) and columns [0, ncol) exist (ncol a multiple of 8)
+template <typename T, int D>
+FMHA_DEV void store_acc_rows(char *scratch, const f32x16 (&acc)[D / 32], float scale, T *base, uint32_t ss, int nrows, int ncol, int l) {
+  using R = RowStore<D>;
+  char *w = scratch + (l & 31) * R::PITCH + (l >> 5) * 8;
+#pragma unroll
+  for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      typename Elem<T>::v4 x;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) x[i] = (T)(acc[db][4 * g + i] * scale);
+      Pack8 p;
+      if constexpr (__is_same(T, _Float16)) p.h = x;
+      else p.b = x;
+      *(u32x2 *)(w + db * 64 + g * 16) = p.u;
+    }
+  __builtin_amdgcn_wave_barrier();
+  asm volatile("" ::: "memory"); // (the compiler keeps the two layouts' accesses apart)
+  const int row = l / R::LPR, col = (l % R::LPR) * 8;
+#pragma unroll
+  for (int i = 0; i < 32 / R::RPI; ++i) {
+    const int r = i * R::RPI + row;
+    const u32x4 v = *(const u32x4 *)(scratch + r * R::PITCH + col * 2);
+    if (r < nrows && col < ncol) *(u32x4 *)(base + (uint32_t)r * ss + col) = v;
+  }
+  asm volatile("" ::: "memory");
+}
+
 // ---------------------------------------------------------------- row <-> accumulator layout
 // A wave's 32 x KEYS block of a [.., sq, sk] tensor (mask, dropout tensor, saved outputs) moves
 // to and from global memory as whole row segments: 16 bytes (8 keys) per lane, KEYS/8 lanes per

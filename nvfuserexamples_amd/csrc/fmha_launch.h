@@ -58,6 +58,17 @@ int bwd_dispatch_f16_d128_strided(BwdArgs &a, const BwdVariant &v, hipStream_t s
 int bwd_dispatch_bf16_d64_strided(BwdArgs &a, const BwdVariant &v, hipStream_t s);
 int bwd_dispatch_bf16_d128_strided(BwdArgs &a, const BwdVariant &v, hipStream_t s);
 
+// One launch of the software-pipelined backward (fmha_bwd_pipe.hip): the dQ kernel, or the dK / dV kernel; a.ntile and
+// a.pair as for the general kernels.
+int bwd_pipe_launch_f16_d64(const BwdArgs &a, const BwdVariant &v, bool dkdv, long long nblk, hipStream_t s);
+int bwd_pipe_launch_f16_d128(const BwdArgs &a, const BwdVariant &v, bool dkdv, long long nblk, hipStream_t s);
+int bwd_pipe_launch_bf16_d64(const BwdArgs &a, const BwdVariant &v, bool dkdv, long long nblk, hipStream_t s);
+int bwd_pipe_launch_bf16_d128(const BwdArgs &a, const BwdVariant &v, bool dkdv, long long nblk, hipStream_t s);
+int bwd_pipe_launch_f16_d64_strided(const BwdArgs &a, const BwdVariant &v, bool dkdv, long long nblk, hipStream_t s);
+int bwd_pipe_launch_f16_d128_strided(const BwdArgs &a, const BwdVariant &v, bool dkdv, long long nblk, hipStream_t s);
+int bwd_pipe_launch_bf16_d64_strided(const BwdArgs &a, const BwdVariant &v, bool dkdv, long long nblk, hipStream_t s);
+int bwd_pipe_launch_bf16_d128_strided(const BwdArgs &a, const BwdVariant &v, bool dkdv, long long nblk, hipStream_t s);
+
 // e4m3 forward (fmha_fwd_fp8.hip): 0 ok, 1 not built, 2 launch failed
 struct Fp8Args;
 int fwd_fp8_dispatch(const Fp8Args &a, int d, bool out_bf16, bool causal, hipStream_t s);

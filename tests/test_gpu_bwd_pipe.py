@@ -1,0 +1,50 @@
+"""The software-pipelined backward kernels at the edges of their tiles, segments and pipelines, against the CPU oracle:
+one to a few 32-row tiles, ragged ends, more than one segment of staged queries (1024) and mask terms (4096), causal
+heads whose keys outnumber the queries and the other way round."""
+import pytest
+import torch
+
+import oracle
+from nvfuserexamples_amd import capi
+from conftest import f32, make_qkv, pad_mask, rel_to_max
+
+pytestmark = pytest.mark.gpu
+
+TDT = {"fp16": torch.float16, "bf16": torch.bfloat16}
+TOL = {"fp16": 1e-2, "bf16": 3e-2}
+
+CASES = [
+    # bh, sq, sk, d, dtype, pad mask, causal, p
+    (2, 1, 300, 64, "fp16", False, False, 0.1),
+    (2, 300, 1, 64, "fp16", False, False, 0.0),
+    (2, 257, 33, 64, "bf16", True, False, 0.1),
+    (2, 31, 289, 64, "fp16", True, True, 0.1),
+    (2, 290, 64, 64, "fp16", False, True, 0.0),
+    (1, 33, 33, 128, "fp16", False, False, 0.1),
+    (1, 96, 128, 128, "bf16", True, True, 0.0),
+    (1, 130, 97, 128, "fp16", False, True, 0.1),
+    (2, 161, 95, 96, "fp16", True, False, 0.1),       # columns that rows do not have
+    (1, 1100, 96, 64, "fp16", False, False, 0.1),     # queries in two segments
+    (1, 2081, 40, 128, "fp16", False, False, 0.1),    # ... in three
+    (1, 1056, 1056, 128, "bf16", False, True, 0.1),   # ... under a causal mask
+    (1, 40, 4200, 64, "fp16", True, False, 0.0),      # mask terms in two segments
+]
+
+
+@pytest.mark.parametrize("bh,sq,sk,d,dtype,pad,causal,p", CASES)
+def test_pipelined_backward_at_its_edges(bh, sq, sk, d, dtype, pad, causal, p):
+    q, k, v, do = make_qkv(bh, sq, sk, d, seed=sq + sk, std=0.7, dtype=dtype, with_dout=True)
+    m = pad_mask(1, sk, max(1, sk // 2), sk, seed=5).to(TDT[dtype]) if pad else None
+    kw = dict(causal=causal)
+    okw = dict(causal=causal)
+    if p > 0:
+        kw.update(drop_kind=capi.DROP_PHILOX, p_drop=p, seed=99, offset=12)
+        okw.update(philox=True, p_drop=p, seed=99, offset=12)
+    qc, kc, vc, mc = q.cuda(), k.cuda(), v.cuda(), (None if m is None else m.cuda())
+    o, lse, _, _ = capi.fwd(qc, kc, vc, mask=mc, want_lse=True, **kw)
+    got = capi.bwd(do.cuda(), qc, kc, vc, o, lse, mask=mc, **kw)
+    torch.cuda.synchronize()
+    ref = oracle.attention(f32(q), f32(k), f32(v), mask=None if m is None else f32(m), dout=f32(do),
+                           want=("dq", "dk", "dv"), **okw)
+    for name, t in zip(("dq", "dk", "dv"), got):
+        assert rel_to_max(f32(t.cpu()), ref[name], floor=1e-2) <= TOL[dtype], name
