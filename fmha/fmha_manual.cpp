@@ -15,8 +15,11 @@
 // (common/manual_scheduled_kernel.h:13-41) has no counterpart: nothing is compiled
 // at run time, so the ops are stateless and re-entrant.
 #include <ATen/DeviceGuard.h>
+#include <ATen/hip/EmptyTensor.h>
 #include <c10/hip/HIPStream.h>
-#include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/function.h>
+#include <torch/csrc/autograd/functions/utils.h>
+#include <torch/csrc/autograd/saved_variable.h>
 #include <torch/extension.h>
 
 #include <algorithm>
@@ -35,6 +38,12 @@ struct MaskLayout {
 
 void *current_stream(const at::Tensor &t) {
   return static_cast<void *>(c10::hip::getCurrentHIPStream(t.device().index()).stream());
+}
+
+// A new dense tensor on t's device, straight from the caching allocator: through the dispatcher (at::empty) the same
+// allocation takes about 0.6 us longer, and an operator call makes two to five of them.
+at::Tensor new_tensor(at::IntArrayRef sizes, const at::Tensor &t, at::ScalarType dtype) {
+  return at::Tensor(at::detail::empty_cuda(sizes, dtype, t.device(), c10::nullopt));
 }
 
 int dtype_code(const at::Tensor &t) {
@@ -62,20 +71,17 @@ MaskLayout mask_layout(const at::Tensor &mask_in, const at::Tensor &q, int64_t b
                        const char *what) {
   TORCH_CHECK(mask_in.is_cuda() && mask_in.device() == q.device(), "mha_manual: ", what, " must be on q's device");
   TORCH_CHECK(mask_in.scalar_type() == q.scalar_type(), "mha_manual: ", what, " must have q's dtype");
-  at::Tensor m = mask_in;
-  if (m.dim() == 4) {
-    TORCH_CHECK(m.size(1) == 1, "mha_manual: 4-d ", what, " must be [B,1,Sq|1,Sk]");
-    m = m.reshape({m.size(0), m.size(2), m.size(3)});
-  }
-  TORCH_CHECK(m.dim() == 3 && m.size(2) == sk && (m.size(1) == 1 || m.size(1) == sq) && m.size(0) >= 1 &&
-                  bh % m.size(0) == 0,
+  const int64_t nd = mask_in.dim(); // (a 4-d mask's second dimension is 1: the same memory as the 3-d one)
+  TORCH_CHECK(nd != 4 || mask_in.size(1) == 1, "mha_manual: 4-d ", what, " must be [B,1,Sq|1,Sk]");
+  TORCH_CHECK((nd == 3 || nd == 4) && mask_in.size(nd - 1) == sk && (mask_in.size(nd - 2) == 1 || mask_in.size(nd - 2) == sq) &&
+                  mask_in.size(0) >= 1 && bh % mask_in.size(0) == 0,
               "mha_manual: ", what, " of shape ", mask_in.sizes(), " does not broadcast over [", bh, ",", sq, ",",
               sk, "]");
   MaskLayout L;
-  L.t = m.contiguous();
-  L.bh_div = bh / m.size(0);
-  L.stride_b = m.size(1) * sk;
-  L.stride_q = m.size(1) == 1 ? 0 : sk;
+  L.t = mask_in.contiguous();
+  L.bh_div = bh / mask_in.size(0);
+  L.stride_b = mask_in.size(nd - 2) * sk;
+  L.stride_q = mask_in.size(nd - 2) == 1 ? 0 : sk;
   return L;
 }
 
@@ -111,7 +117,7 @@ at::Tensor fmha_nvfuser(const at::Tensor &input, const at::Tensor &qk, const at:
   check_qkv(input, qk, v);
   at::DeviceGuard guard(input.device());
   MaskLayout m = mask_layout(amask, input, input.size(0), input.size(1), qk.size(1), "amask");
-  at::Tensor o = at::empty_like(input);
+  at::Tensor o = new_tensor(input.sizes(), input, input.scalar_type());
   fmha_fwd_params p = {};
   p.struct_bytes = sizeof p;
   fill_common(p, input, qk, v, o, default_scale(input));
@@ -141,7 +147,7 @@ std::vector<at::Tensor> train_forward(const at::Tensor &input, const at::Tensor 
                   dropout_mask.size(0) == bh && dropout_mask.size(1) == sq && dropout_mask.size(2) == sk,
               "mha_manual: dropout_mask must be a [BH,Sq,Sk] tensor of q's dtype on q's device");
   at::Tensor dm = dropout_mask.contiguous();
-  at::Tensor o = at::empty_like(input);
+  at::Tensor o = new_tensor(input.sizes(), input, input.scalar_type());
   fmha_fwd_params p = {};
   p.struct_bytes = sizeof p;
   fill_common(p, input, qk, v, o, default_scale(input));
@@ -156,10 +162,10 @@ std::vector<at::Tensor> train_forward(const at::Tensor &input, const at::Tensor 
   std::vector<at::Tensor> out{o};
   at::Tensor lse; // scratch: with it the library derives the saved outputs from one forward launch
   if (save) {
-    lse = at::empty({bh, sq}, input.options().dtype(at::kFloat));
+    lse = new_tensor({bh, sq}, input, at::kFloat);
     p.lse = lse.data_ptr<float>();
-    at::Tensor sm = at::empty({bh, sq, sk}, input.options());
-    at::Tensor dr = at::empty({bh, sq, sk}, input.options());
+    at::Tensor sm = new_tensor({bh, sq, sk}, input, input.scalar_type());
+    at::Tensor dr = new_tensor({bh, sq, sk}, input, input.scalar_type());
     p.save_softmax = sm.data_ptr();
     p.save_dropout = dr.data_ptr();
     out.push_back(sm);
@@ -220,15 +226,15 @@ RowsOf rows_of(const at::Tensor &x, const char *what) {
 // A new tensor of x's shape with x's order of dimensions in memory, but dense: a [B,H,S,D] view of
 // [B,S,H,D] memory (or of a slice of a packed projection) gets fresh [B,S,H,D] memory.
 at::Tensor empty_like_rows(const at::Tensor &x) {
-  if (x.dim() != 4) return at::empty(x.sizes(), x.options());
-  std::vector<int64_t> order{0, 1, 2, 3};
-  std::stable_sort(order.begin(), order.end(), [&](int64_t a, int64_t b) { return x.stride(a) > x.stride(b); });
-  std::vector<int64_t> sizes(4), inv(4);
-  for (int i = 0; i < 4; ++i) {
-    sizes[i] = x.size(order[i]);
-    inv[order[i]] = i;
+  if (x.dim() != 4) return new_tensor(x.sizes(), x, x.scalar_type());
+  int order[4] = {0, 1, 2, 3};
+  std::stable_sort(order, order + 4, [&](int a, int b) { return x.stride(a) > x.stride(b); });
+  int64_t strides[4], step = 1;
+  for (int i = 3; i >= 0; --i) {
+    strides[order[i]] = step;
+    step *= x.size(order[i]);
   }
-  return at::empty(sizes, x.options()).permute(inv);
+  return at::Tensor(at::detail::empty_strided_cuda(x.sizes(), strides, x.scalar_type(), x.device()));
 }
 
 // The kernels copy K and V tiles with one set of offsets: where their rows are not equally far
@@ -323,8 +329,8 @@ std::tuple<at::Tensor, at::Tensor> fmha_fwd(const at::Tensor &q_, const at::Tens
   at::DeviceGuard guard(q.t.device());
   at::Tensor o = empty_like_rows(q.t);
   const RowsOf orow = rows_of(o, "o");
-  at::Tensor lse = q.heads ? at::empty({q_.size(0), q_.size(1), q.s}, q.t.options().dtype(at::kFloat))
-                           : at::empty({q.bh, q.s}, q.t.options().dtype(at::kFloat));
+  at::Tensor lse = q.heads ? new_tensor({q_.size(0), q_.size(1), q.s}, q.t, at::kFloat)
+                           : new_tensor({q.bh, q.s}, q.t, at::kFloat);
   fmha_fwd_params p = {};
   p.struct_bytes = sizeof p;
   p.q = q.t.data_ptr();
@@ -352,7 +358,7 @@ std::tuple<at::Tensor, at::Tensor> fmha_fwd(const at::Tensor &q_, const at::Tens
   // results the library cuts the key range into pieces and fills the whole chip.
   at::Tensor workspace;
   if (const uint64_t need = fmha_fwd_workspace_bytes(&p); need > 0) {
-    workspace = at::empty({static_cast<int64_t>(need)}, q.t.options().dtype(at::kByte));
+    workspace = new_tensor({static_cast<int64_t>(need)}, q.t, at::kByte);
     p.workspace = workspace.data_ptr();
     p.workspace_bytes = need;
   }
@@ -392,7 +398,7 @@ fmha_bwd(const at::Tensor &dout_, const at::Tensor &q_, const at::Tensor &k_, co
   at::Tensor lsec = lse.contiguous();
   at::Tensor dq = empty_like_rows(q.t), dk = empty_like_rows(k.t), dv = empty_like_rows(v.t);
   const RowsOf dqr = rows_of(dq, "dq"), dkr = rows_of(dk, "dk"), dvr = rows_of(dv, "dv");
-  at::Tensor delta = at::empty_like(lsec);
+  at::Tensor delta = new_tensor(lsec.sizes(), lsec, at::kFloat);
   fmha_bwd_params p = {};
   p.struct_bytes = sizeof p;
   p.q = q.t.data_ptr();
@@ -444,8 +450,8 @@ std::tuple<at::Tensor, at::Tensor> fmha_fwd_fp8(const at::Tensor &q8, const at::
               "mha_manual: shapes must be q [BH,Sq,D], k [BH,Sk,D], v [BH,Sk,D]");
   at::DeviceGuard guard(q8.device());
   const auto odt = out_bf16 ? at::kBFloat16 : at::kHalf;
-  at::Tensor o = at::empty(q8.sizes(), q8.options().dtype(odt));
-  at::Tensor lse = at::empty({q8.size(0), q8.size(1)}, q8.options().dtype(at::kFloat));
+  at::Tensor o = new_tensor(q8.sizes(), q8, odt);
+  at::Tensor lse = new_tensor({q8.size(0), q8.size(1)}, q8, at::kFloat);
   fmha_fwd_fp8_params p = {};
   p.struct_bytes = sizeof p;
   p.q = q8.data_ptr();
@@ -475,7 +481,7 @@ std::tuple<at::Tensor, at::Tensor> fmha_fwd_fp8(const at::Tensor &q8, const at::
   at::Tensor kv_keep, workspace;
   set_kv_len(p, kv_len, q8.size(0), kv_keep);
   if (const uint64_t need = fmha_fwd_fp8_workspace_bytes(&p); need > 0) {
-    workspace = at::empty({static_cast<int64_t>(need)}, q8.options().dtype(at::kByte));
+    workspace = new_tensor({static_cast<int64_t>(need)}, q8, at::kByte);
     p.workspace = workspace.data_ptr();
     p.workspace_bytes = need;
   }
@@ -489,7 +495,7 @@ at::Tensor philox_keep_mask_op(const at::Tensor &like, int64_t bh, int64_t sq, i
                                  int64_t seed, int64_t offset) {
   TORCH_CHECK(like.is_cuda(), "mha_manual: `like` must live on the GPU");
   at::DeviceGuard guard(like.device());
-  at::Tensor out = at::empty({bh, sq, sk}, like.options().dtype(at::kByte));
+  at::Tensor out = new_tensor({bh, sq, sk}, like, at::kByte);
   const int rc = fmha_philox_keep_mask(static_cast<uint64_t>(seed), static_cast<uint64_t>(offset),
                                        static_cast<float>(p_drop), static_cast<int32_t>(bh),
                                        static_cast<int32_t>(sq), static_cast<int32_t>(sk),
@@ -502,41 +508,34 @@ at::Tensor philox_keep_mask_op(const at::Tensor &like, int64_t bh, int64_t sq, i
 // are under no_grad): O is differentiable in q, k and v; the row log-sum-exp, the mask and the key counts
 // are not.  Nothing of size S x S is kept for the backward: it recomputes P from the saved LSE and
 // regenerates the dropout decisions from the same (seed, offset).
-class FmhaFunction : public torch::autograd::Function<FmhaFunction> {
- public:
-  static torch::autograd::variable_list forward(torch::autograd::AutogradContext *ctx, const at::Tensor &q,
-                                                const at::Tensor &k, const at::Tensor &v,
-                                                const c10::optional<at::Tensor> &mask, double scale, bool is_causal,
-                                                double p_drop, int64_t seed, int64_t offset,
-                                                const c10::optional<at::Tensor> &kv_len) {
-    at::AutoDispatchBelowADInplaceOrView below;
-    auto [o, lse] = fmha_fwd(q, k, v, mask, scale, is_causal, p_drop, seed, offset, kv_len);
-    const bool has_mask = mask.has_value() && mask->defined(), has_len = kv_len.has_value() && kv_len->defined();
-    ctx->save_for_backward({q, k, v, o, lse, has_mask ? *mask : at::empty({0}, q.options()),
-                            has_len ? *kv_len : at::empty({0}, q.options().dtype(at::kInt))});
-    ctx->saved_data["has_mask"] = has_mask;
-    ctx->saved_data["has_len"] = has_len;
-    ctx->saved_data["scale"] = scale;
-    ctx->saved_data["is_causal"] = is_causal;
-    ctx->saved_data["p_drop"] = p_drop;
-    ctx->saved_data["seed"] = seed;
-    ctx->saved_data["offset"] = offset;
-    ctx->mark_non_differentiable({lse});
-    return {o, lse};
+//
+// A plain graph node with typed members: the generic custom-function wrapper keeps its scalars in a dictionary and looks
+// every one of them up by name, which costs several microseconds per step.
+struct FmhaBackward : public torch::autograd::Node {
+  torch::autograd::SavedVariable q, k, v, o, lse, mask, kv_len;
+  double scale = 0, p_drop = 0;
+  bool is_causal = false, has_mask = false, has_len = false;
+  int64_t seed = 0, offset = 0;
+
+  std::string name() const override { return "FmhaBackward"; }
+  void release_variables() override {
+    std::lock_guard<std::mutex> lock(mutex_);
+    for (torch::autograd::SavedVariable *s : {&q, &k, &v, &o, &lse, &mask, &kv_len}) s->reset_data();
   }
-  static torch::autograd::variable_list backward(torch::autograd::AutogradContext *ctx,
-                                                 torch::autograd::variable_list grads) {
-    const auto saved = ctx->get_saved_variables();
-    const at::Tensor &q = saved[0], &k = saved[1], &v = saved[2], &o = saved[3], &lse = saved[4];
-    const at::Tensor dout = grads[0].defined() ? grads[0] : at::zeros_like(o);
-    c10::optional<at::Tensor> mask, kv_len;
-    if (ctx->saved_data["has_mask"].toBool()) mask = saved[5];
-    if (ctx->saved_data["has_len"].toBool()) kv_len = saved[6];
-    auto [dq, dk, dv] = fmha_bwd(dout, q, k, v, o, lse, mask, ctx->saved_data["scale"].toDouble(),
-                                 ctx->saved_data["is_causal"].toBool(), ctx->saved_data["p_drop"].toDouble(),
-                                 ctx->saved_data["seed"].toInt(), ctx->saved_data["offset"].toInt(), kv_len);
-    at::Tensor none;
-    return {dq, dk, dv, none, none, none, none, none, none, none};
+  torch::autograd::variable_list apply(torch::autograd::variable_list &&grads) override {
+    std::lock_guard<std::mutex> lock(mutex_);
+    const at::Tensor ot = o.unpack(shared_from_this());
+    const at::Tensor dout = grads[0].defined() ? grads[0] : at::zeros_like(ot);
+    c10::optional<at::Tensor> m, n;
+    if (has_mask) m = mask.unpack();
+    if (has_len) n = kv_len.unpack();
+    auto [dq, dk, dv] = fmha_bwd(dout, q.unpack(), k.unpack(), v.unpack(), ot, lse.unpack(), m, scale, is_causal, p_drop,
+                                 seed, offset, n);
+    torch::autograd::variable_list out(3); // (all three come out of the same two launches)
+    if (task_should_compute_output(0)) out[0] = std::move(dq);
+    if (task_should_compute_output(1)) out[1] = std::move(dk);
+    if (task_should_compute_output(2)) out[2] = std::move(dv);
+    return out;
   }
 };
 
@@ -544,8 +543,39 @@ std::tuple<at::Tensor, at::Tensor> fmha_fwd_autograd(const at::Tensor &q, const 
                                                      const c10::optional<at::Tensor> &mask, double scale,
                                                      bool is_causal, double p_drop, int64_t seed, int64_t offset,
                                                      const c10::optional<at::Tensor> &kv_len) {
-  auto r = FmhaFunction::apply(q, k, v, mask, scale, is_causal, p_drop, seed, offset, kv_len);
-  return std::make_tuple(r[0], r[1]);
+  TORCH_CHECK(!(torch::autograd::isFwGradDefined(q) || torch::autograd::isFwGradDefined(k) || torch::autograd::isFwGradDefined(v)),
+              "mha_manual: fmha_fwd has no forward-mode derivative");
+  std::shared_ptr<FmhaBackward> node;
+  if (torch::autograd::compute_requires_grad(q, k, v)) {
+    node = std::shared_ptr<FmhaBackward>(new FmhaBackward(), torch::autograd::deleteNode);
+    node->set_next_edges(torch::autograd::collect_next_edges(q, k, v));
+    node->q = torch::autograd::SavedVariable(q, false);
+    node->k = torch::autograd::SavedVariable(k, false);
+    node->v = torch::autograd::SavedVariable(v, false);
+    if (mask.has_value() && mask->defined()) {
+      node->has_mask = true;
+      node->mask = torch::autograd::SavedVariable(*mask, false);
+    }
+    if (kv_len.has_value() && kv_len->defined()) {
+      node->has_len = true;
+      node->kv_len = torch::autograd::SavedVariable(*kv_len, false);
+    }
+    node->scale = scale;
+    node->is_causal = is_causal;
+    node->p_drop = p_drop;
+    node->seed = seed;
+    node->offset = offset;
+  }
+  auto [o, lse] = [&] {
+    at::AutoDispatchBelowADInplaceOrView below;
+    return fmha_fwd(q, k, v, mask, scale, is_causal, p_drop, seed, offset, kv_len);
+  }();
+  if (node) {
+    torch::autograd::set_history(o, node);
+    node->o = torch::autograd::SavedVariable(o, true);
+    node->lse = torch::autograd::SavedVariable(lse, false);
+  }
+  return std::make_tuple(o, lse);
 }
 
 TORCH_LIBRARY(mha_manual, m) {

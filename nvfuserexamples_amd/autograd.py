@@ -3,10 +3,12 @@
 The reference registers its operators without an autograd formula (reference
 fmha/fmha_manual.cpp:1240-1250: no Autograd key, its perf runs are under ``no_grad``).  Here
 ``fmha_fwd`` carries one, registered in C++ under the Autograd dispatch key (fmha/fmha_manual.cpp,
-``FmhaFunction``): its backward calls ``fmha_bwd`` with the saved q, k, v, O and row log-sum-exp.
+``FmhaBackward``): its backward calls ``fmha_bwd`` with the saved q, k, v, O and row log-sum-exp.
 Dropout decisions are never stored: the backward regenerates them from the same ``(seed, offset)``.
 """
 from . import load_ops
+
+_fwd = None  # the operator, looked up once
 
 
 def attention(q, k, v, mask=None, scale=0.0, is_causal=False, p_drop=0.0, seed=0, offset=0, kv_len=None):
@@ -18,5 +20,7 @@ def attention(q, k, v, mask=None, scale=0.0, is_causal=False, p_drop=0.0, seed=0
     ``[B,1,1,Sk]``; ``scale <= 0`` means ``1/sqrt(D)``.
     ``kv_len``: optional int32 GPU vector of B valid key counts (B divides B*H): keys at or past a
     head's count are excluded and their key tiles skipped.  Masks and counts receive no gradient."""
-    return load_ops().fmha_fwd(q, k, v, mask, float(scale), bool(is_causal), float(p_drop), int(seed), int(offset),
-                               kv_len)[0]
+    global _fwd
+    if _fwd is None:
+        _fwd = load_ops().fmha_fwd
+    return _fwd(q, k, v, mask, float(scale), bool(is_causal), float(p_drop), int(seed), int(offset), kv_len)[0]
