@@ -558,12 +558,16 @@ int fmha_fwd_launch(const fmha_fwd_params *caller, void *hip_stream) {
   v.causal = p->causal != 0;
   v.drop = (p->drop_kind == FMHA_DROP_TENSOR || saving) ? 2 : (p->drop_kind == FMHA_DROP_PHILOX ? 1 : 0);
   v.saving = saving;
-  // Short key ranges under a full mask tensor run in one pass with whole-row accesses to the
-  // [.., sq, sk] tensors, which must then start on 16-byte boundaries row by row.
-  v.short_keys = !strided && p->d == 64 && p->sk <= 128 && (p->sk % 8) == 0 && v.mask == kMaskFull && !v.causal &&
-                 v.drop != 1 && !p->kv_len && aligned16(a.mask) && (a.mask_sb % 8) == 0 && (a.mask_sq % 8) == 0 &&
-                 (!a.drop_mask || aligned16(a.drop_mask)) && (!a.save_softmax || aligned16(a.save_softmax)) &&
-                 (!a.save_dropout || aligned16(a.save_dropout)) && (!saving || a.drop_mask) &&
+  // Full mask tensors in the operators' own use (every key visible, no dropout or a dropout tensor, head dims 64 and
+  // 128): the kernels below move the [.., sq, sk] tensors as whole rows.  Rows may have any length from 8 keys on
+  // and start at any element: a row's last request starts 8 keys before its end.  (The plain kernel, which reads such
+  // a tensor element by element, keeps shorter rows, causal masks, valid key counts and the Philox rule.  For the
+  // three operators it took 45 / 77 / 311 us at BH 48, S 483 where these take 14 / 19 / 35, 15 / 21 / 68 at BH 256,
+  // S 127 against 7.5 / 9.3 / 14, and 83 / 184 / 380 at head dim 128, BH 256, S 512 against 71 / 91 / 212.)
+  const bool rows = !strided && (p->d == 64 || p->d == 128) && p->sk >= 8 && v.mask == kMaskFull && !v.causal &&
+                    v.drop != 1 && (v.drop != 2 || a.drop_mask);
+  // Up to 128 keys at head dim 64: one pass.
+  v.short_keys = rows && p->d == 64 && p->sk <= 128 && !p->kv_len &&
                  (long long)p->sq * (a.mask_sq > 128 ? a.mask_sq : 128) < (1LL << 30) && // (the kernel forms 32-bit byte offsets within a head: mask rows, and [.., sq, sk] rows of up to 128 keys)
                  overrides().fwd_short != 0;
   // The same one-pass kernel without a full mask tensor: no mask, a per-key mask or valid key counts, no dropout or
@@ -581,26 +585,17 @@ int fmha_fwd_launch(const fmha_fwd_params *caller, void *hip_stream) {
   }
   // Longer key ranges: where the caller provides an LSE buffer, the save-intermediates operator is the forward
   // launch followed by a streaming kernel that derives both saved outputs from that LSE (instead of a second
-  // sweep inside a slower forward).  Same alignment needs as above.
-  v.save_split = saving && !v.short_keys && !strided && p->d == 64 && p->lse && (p->sk % 8) == 0 &&
-                 v.mask == kMaskFull && !v.causal && a.drop_mask && aligned16(a.mask) && (a.mask_sb % 8) == 0 &&
-                 (a.mask_sq % 8) == 0 && aligned16(a.drop_mask) && (!a.save_softmax || aligned16(a.save_softmax)) &&
-                 (!a.save_dropout || aligned16(a.save_dropout)) && overrides().fwd_save_split != 0;
-  // Up to 512 keys one launch does it all: a wave keeps its probabilities and dropout rows in registers until the
-  // row's log-sum-exp is known, so the mask and the dropout tensor are read once (no LSE buffer needed).
-  v.save_once = saving && !v.short_keys && !strided && p->d == 64 && p->sk <= 512 && (p->sk % 8) == 0 &&
-                v.mask == kMaskFull && !v.causal && !p->kv_len && a.drop_mask && aligned16(a.mask) &&
-                (a.mask_sb % 8) == 0 && (a.mask_sq % 8) == 0 && aligned16(a.drop_mask) &&
-                (!a.save_softmax || aligned16(a.save_softmax)) && (!a.save_dropout || aligned16(a.save_dropout)) &&
-                overrides().fwd_save_once != 0 && overrides().fwd_stream != 0; // (it is the streaming forward's arithmetic)
+  // sweep inside a slower forward).
+  v.save_split = rows && saving && !v.short_keys && p->lse && overrides().fwd_save_split != 0;
+  // Up to 512 keys (448 at head dim 128) one launch does it all: a wave keeps what the saved outputs are made of in registers
+  // until the row's log-sum-exp is known, so the mask and the dropout tensor are read once (no LSE buffer needed).
+  v.save_once = rows && saving && !v.short_keys && p->sk <= (p->d == 64 ? 512 : 448) && overrides().fwd_save_once != 0 &&
+                overrides().fwd_stream != 0; // (it is the streaming forward's arithmetic)
   if (v.save_once) v.save_split = false;
   if (v.save_split || v.save_once) v.saving = false; // (save_split: the forward launch itself saves nothing)
-  // Other forwards under an aligned full mask tensor (with or without a dropout tensor) are memory time at
-  // head dim 64: the streaming kernel.
-  v.stream = !v.short_keys && !v.saving && !strided && p->d == 64 && (p->sk % 8) == 0 && v.mask == kMaskFull &&
-             !v.causal && v.drop != 1 && !p->kv_len && aligned16(a.mask) && (a.mask_sb % 8) == 0 &&
-             (a.mask_sq % 8) == 0 && (v.drop != 2 || (a.drop_mask && aligned16(a.drop_mask))) &&
-             overrides().fwd_stream != 0;
+  // Other forwards under a full mask tensor (with or without a dropout tensor) are memory time: the streaming kernel.
+  v.stream = rows && !v.short_keys && !v.saving && !p->kv_len && overrides().fwd_stream != 0;
+  v.many = v.stream && (long long)p->bh * ((p->sq + 127) / 128) > 2LL * cu_count();
   // Two 32-query blocks per wave (on tiles of 32 keys) halve the LDS operand traffic per
   // flop.  That pays (4-6 % measured) for the unmasked variant at head dim 64 on long key
   // ranges when there is enough work for every resident workgroup to get several 256-query

@@ -373,6 +373,10 @@ FMHA_DEV void store_acc_rows(char *scratch, const f32x16 (&acc)[D / 32], float s
 // (row pitch = row + 16 bytes) is written in one layout and read in the other.  The scratch belongs
 // to one wave, whose LDS accesses execute in order: turn() only keeps the compiler from moving
 // accesses across the change of layout.
+// (accesses of 16, 8 and 4 bytes at element addresses: the hardware takes any)
+typedef u32x4 u32x4_any __attribute__((aligned(2)));
+typedef u32x2 u32x2_any __attribute__((aligned(2)));
+typedef uint32_t u32_any __attribute__((aligned(2)));
 template <int KEYS> struct RowScratch {
   static constexpr int LPR = KEYS / 8;    // lanes per row
   static constexpr int RPI = 64 / LPR;    // rows per instruction
@@ -395,6 +399,73 @@ template <int KEYS> struct RowScratch {
   FMHA_DEV void rows_in(const u32x4 (&r)[NI]) const {
 #pragma unroll
     for (int i = 0; i < NI; ++i) *(u32x4 *)(row + RPI * i * PITCH) = r[i];
+  }
+  // Rows of any length and alignment.  A request is 16 bytes at any element address; the last one of a row whose
+  // length is no multiple of 8 starts 8 keys before the row's end, so it never leaves the row (sk >= 8), and
+  // place_tail moves its keys to where the tile has them (for such rows only: TAIL in the kernels; built into one
+  // kernel for all rows it cost rows of whole chunks 2 to 6 %).  Lanes past the row's end re-read its last 8 keys.
+  template <bool TAIL> FMHA_DEV int first_key(int k0, int sk) const {
+    const int k = k0 + chunk * 8;
+    if (!TAIL) return k < sk ? k : 0; // (rows of whole chunks: past the end any chunk will do)
+    return k < sk - 8 ? k : sk - 8;
+  }
+  FMHA_DEV void place_tail(u32x4 (&r)[NI], int k0, int sk) const {
+    if (k0 + KEYS <= sk) return;   // (workgroup-uniform)
+    const int past = 8 - (sk & 7); // keys of the last request that the chunk before already holds
+    const bool last = k0 + chunk * 8 == (sk & ~7);
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      uint64_t lo = r[i].x | (uint64_t)r[i].y << 32, hi = r[i].z | (uint64_t)r[i].w << 32;
+      if (past >= 4) {
+        lo = hi;
+        hi = 0;
+      }
+      const int b = (past & 3) * 16;
+      if (b) {
+        lo = lo >> b | hi << (64 - b);
+        hi >>= b;
+      }
+      if (last) r[i] = u32x4{(uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32)};
+    }
+  }
+  // The scratch's rows leave as rows q0 .. q0 + 31 and keys k0 .. k0 + KEYS - 1 of a [sq][sk] tensor, as far as those
+  // exist; at(q) is the address of this lane's chunk of row q.  (All pieces are read before the first is stored: the
+  // compiler otherwise moves each read behind the condition of its store, and each store then waits for its own.)
+  template <bool TAIL, typename At> FMHA_DEV void rows_out(const At &at, int q0, int sq, int k0, int sk) const {
+    u32x4 t[NI];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) t[i] = row_out(i);
+#pragma unroll
+    for (int i = 0; i < NI; ++i) asm volatile("" : "+v"(t[i]));
+    if (q0 + 32 <= sq && k0 + KEYS <= sk) { // (wave-uniform)
+#pragma unroll
+      for (int i = 0; i < NI; ++i) *(u32x4_any *)at(q0 + RPI * i + rsub) = t[i];
+      return;
+    }
+    const int n = sk - (k0 + chunk * 8);
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int q = q0 + RPI * i + rsub;
+      if (q >= sq || n <= 0) continue;
+      char *p = at(q);
+      if (!TAIL || n >= 8) {
+        *(u32x4_any *)p = t[i];
+        continue;
+      }
+      const uint64_t lo = t[i].x | (uint64_t)t[i].y << 32, hi = t[i].z | (uint64_t)t[i].w << 32;
+      uint64_t rest = lo;
+      if (n & 4) {
+        *(u32x2_any *)p = u32x2{t[i].x, t[i].y};
+        p += 8;
+        rest = hi;
+      }
+      if (n & 2) {
+        *(u32_any *)p = (uint32_t)rest;
+        p += 4;
+        rest >>= 32;
+      }
+      if (n & 1) *(uint16_t *)p = (uint16_t)rest;
+    }
   }
   FMHA_DEV u32x4 row_out(int i) const { return *(const u32x4 *)(row + RPI * i * PITCH); }
   FMHA_DEV u32x2 piece(int sb, int g) const { return *(const u32x2 *)(frag + sb * 64 + g * 16); }

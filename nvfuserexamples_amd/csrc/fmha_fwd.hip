@@ -5,12 +5,17 @@
 #ifndef FMHA_TU_STRIDED
 #define FMHA_TU_STRIDED 0
 #endif
-#if FMHA_TU_D == 64 && !FMHA_TU_STRIDED
-#define FMHA_TU_SHORT 1
-#include "fmha_fwd_short.h"
+#if FMHA_TU_D != 256 && !FMHA_TU_STRIDED
+#define FMHA_TU_ROWS 1 // the kernels that move [.., sq, sk] tensors as whole rows
 #include "fmha_fwd_save.h"
 #include "fmha_fwd_stream.h"
 #include "fmha_fwd_stream_save.h"
+#else
+#define FMHA_TU_ROWS 0
+#endif
+#if FMHA_TU_D == 64 && !FMHA_TU_STRIDED
+#define FMHA_TU_SHORT 1
+#include "fmha_fwd_short.h"
 #include "fmha_fwd_head.h"
 #else
 #define FMHA_TU_SHORT 0
@@ -98,10 +103,11 @@ template <int QB, int MASK, bool CAUSAL, int DROP, bool kPipe = (DROP != 2)> int
 #if FMHA_TU_D == 64
 // short key ranges in one pass: under a full mask tensor (the reference's operators at their own shape), and under
 // no mask / a per-key mask / valid key counts, without dropout or with the Philox rule
-template <int MASK, int DROP, bool SAVE, bool FULL> int launch_short_as(FwdArgs &a, hipStream_t s) {
+template <int MASK, int DROP, bool SAVE, bool FULL, bool TAIL = false> int launch_short_as(FwdArgs &a, hipStream_t s) {
   static_assert(MASK != kMaskFull || !kStrided, "full mask tensors: folded layout only");
   auto kern = [] {
-    if constexpr (MASK == kMaskFull) return fmha_fwd_short_kernel<FMHA_TU_T, DROP, SAVE, FULL>;
+    if constexpr (MASK == kMaskFull && TAIL) return fmha_fwd_short_tail_kernel<FMHA_TU_T, DROP, SAVE, FULL>;
+    else if constexpr (MASK == kMaskFull) return fmha_fwd_short_kernel<FMHA_TU_T, DROP, SAVE, FULL>;
     else return fmha_fwd_short_kernel_keymask<FMHA_TU_T, MASK, DROP, FULL, kStrided>;
   }();
   constexpr int kLds = MASK == kMaskFull ? ShortCfg::LDS_BYTES : ShortCfg::LDS_BYTES_KEYMASK;
@@ -116,45 +122,71 @@ template <int MASK, int DROP, bool SAVE, bool FULL> int launch_short_as(FwdArgs 
 }
 // (more than 96 keys: every 32-key block exists, and the kernel is built without the conditions around them)
 template <int MASK, int DROP, bool SAVE> int launch_short(FwdArgs &a, hipStream_t s) {
+  if constexpr (MASK == kMaskFull)
+    if (a.sk & 7) // rows that end within a 16-byte piece
+      return a.sk > ShortCfg::SKMAX - 32 ? launch_short_as<MASK, DROP, SAVE, true, true>(a, s)
+                                         : launch_short_as<MASK, DROP, SAVE, false, true>(a, s);
   return a.sk > ShortCfg::SKMAX - 32 ? launch_short_as<MASK, DROP, SAVE, true>(a, s)
                                      : launch_short_as<MASK, DROP, SAVE, false>(a, s);
 }
 #endif
 
-#if FMHA_TU_SHORT
+#if FMHA_TU_ROWS
 // the saved outputs of the save-intermediates operator, from the row log-sum-exp of a forward launch
-int launch_save(FwdArgs &a, hipStream_t s) {
-  auto kern = fmha_fwd_save_kernel<FMHA_TU_T>;
+template <bool TAIL> int launch_save_as(FwdArgs &a, hipStream_t s) {
+  using SaveCfg = fmha::SaveCfg<FMHA_TU_D>;
+  auto kern = fmha_fwd_save_kernel<FMHA_TU_T, FMHA_TU_D, TAIL>;
+  static const bool ready = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
+                                                hipFuncAttributeMaxDynamicSharedMemorySize, SaveCfg::LDS_BYTES) == hipSuccess;
+  if (!ready) return 2;
   a.nqt = (a.sq + SaveCfg::QT - 1) / SaveCfg::QT;
   const long long nblk = (long long)a.bh * a.nqt;
   if (nblk > 0x7fffffffLL) return 2;
   hipLaunchKernelGGL(kern, dim3((unsigned)nblk), dim3(SaveCfg::NW * 64), SaveCfg::LDS_BYTES, s, a);
   return hipGetLastError() == hipSuccess ? 0 : 2;
 }
-#endif
 
-#if FMHA_TU_SHORT
+int launch_save(FwdArgs &a, hipStream_t s) { return a.sk & 7 ? launch_save_as<true>(a, s) : launch_save_as<false>(a, s); }
+
 // long key ranges under a full mask tensor (and a dropout tensor): the streaming forward
-template <bool DROPT> int launch_stream(FwdArgs &a, hipStream_t s) {
-  auto kern = fmha_fwd_stream_kernel<FMHA_TU_T, DROPT>;
+template <bool DROPT, bool TAIL, bool MANY> int launch_stream_as(FwdArgs &a, hipStream_t s) {
+  using StreamCfg = fmha::StreamCfg<FMHA_TU_D, MANY>;
+  auto kern = fmha_fwd_stream_kernel<FMHA_TU_T, FMHA_TU_D, DROPT, TAIL, MANY>;
+  constexpr int kLds = StreamCfg::lds_bytes(DROPT);
+  static const bool ready = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
+                                                hipFuncAttributeMaxDynamicSharedMemorySize, kLds) == hipSuccess;
+  if (!ready) return 2;
   a.nqt = (a.sq + StreamCfg::QT - 1) / StreamCfg::QT;
   const long long nblk = (long long)a.bh * a.nqt;
   if (nblk > 0x7fffffffLL) return 2;
-  hipLaunchKernelGGL(kern, dim3((unsigned)nblk), dim3(StreamCfg::NW * 64), StreamCfg::LDS_BYTES, s, a);
+  hipLaunchKernelGGL(kern, dim3((unsigned)nblk), dim3(StreamCfg::NW * 64), kLds, s, a);
   return hipGetLastError() == hipSuccess ? 0 : 2;
 }
-#endif
 
-#if FMHA_TU_SHORT
-// the save-intermediates operator for 129 to 512 keys in one launch (one wave per SIMD: the whole register file)
-int launch_stream_save(FwdArgs &a, hipStream_t s) {
-  auto kern = fmha_fwd_stream_save_kernel<FMHA_TU_T>;
+// TAIL: rows that end within a 16-byte piece; MANY: more than two workgroups per compute unit
+template <bool DROPT> int launch_stream(FwdArgs &a, const FwdVariant &v, hipStream_t s) {
+  if constexpr (FMHA_TU_D == 64 && !DROPT)
+    if (v.many) return a.sk & 7 ? launch_stream_as<false, true, true>(a, s) : launch_stream_as<false, false, true>(a, s);
+  return a.sk & 7 ? launch_stream_as<DROPT, true, false>(a, s) : launch_stream_as<DROPT, false, false>(a, s);
+}
+
+// the save-intermediates operator for up to 512 keys in one launch (one wave per SIMD: the whole register file)
+template <bool TAIL> int launch_stream_save_as(FwdArgs &a, hipStream_t s) {
+  using StreamSaveCfg = fmha::StreamSaveCfg<FMHA_TU_D>;
+  auto kern = fmha_fwd_stream_save_kernel<FMHA_TU_T, FMHA_TU_D, TAIL>;
+  constexpr int kLds = StreamSaveCfg::lds_bytes(TAIL || FMHA_TU_D != 64);
+  static const bool ready = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
+                                                hipFuncAttributeMaxDynamicSharedMemorySize, kLds) == hipSuccess;
+  if (!ready) return 2;
   if (a.sk > StreamSaveCfg::SKMAX) return 1;
   a.nqt = (a.sq + StreamSaveCfg::QT - 1) / StreamSaveCfg::QT;
   const long long nblk = (long long)a.bh * a.nqt;
   if (nblk > 0x7fffffffLL) return 2;
-  hipLaunchKernelGGL(kern, dim3((unsigned)nblk), dim3(StreamSaveCfg::NW * 64), StreamSaveCfg::LDS_BYTES, s, a);
+  hipLaunchKernelGGL(kern, dim3((unsigned)nblk), dim3(StreamSaveCfg::NW * 64), kLds, s, a);
   return hipGetLastError() == hipSuccess ? 0 : 2;
+}
+int launch_stream_save(FwdArgs &a, hipStream_t s) {
+  return a.sk & 7 ? launch_stream_save_as<true>(a, s) : launch_stream_save_as<false>(a, s);
 }
 #endif
 
@@ -266,19 +298,23 @@ int FMHA_NAME(FMHA_TU_TNAME, FMHA_TU_D)(FwdArgs &a, const FwdVariant &v, hipStre
       return v.drop == 1 ? launch_short<kMaskPerKey, 1, false>(a, s) : launch_short<kMaskPerKey, 0, false>(a, s);
     return v.drop == 1 ? launch_short<kMaskNone, 1, false>(a, s) : launch_short<kMaskNone, 0, false>(a, s);
   }
-  if (v.save_once) return launch_stream_save(a, s);
-  if (v.save_split) { // forward with LSE, then the saved outputs from that LSE
-    const int rc = v.stream ? launch_stream<true>(a, s) : launch<1, kMaskFull, false, 2, true>(a, s);
-    return rc ? rc : launch_save(a, s);
-  }
-  if (v.stream) return v.drop == 2 ? launch_stream<true>(a, s) : launch_stream<false>(a, s);
   if (v.head) {
     if (v.causal || v.drop == 2 || v.mask == kMaskFull) return 1;
     if (v.mask == kMaskPerKey) return v.drop ? launch_head<kMaskPerKey, 1>(a, s) : launch_head<kMaskPerKey, 0>(a, s);
     return v.drop ? launch_head<kMaskNone, 1>(a, s) : launch_head<kMaskNone, 0>(a, s);
   }
 #else
-  if (v.short_keys || v.save_split || v.save_once || v.stream || v.head) return 1;
+  if (v.short_keys || v.head) return 1;
+#endif
+#if FMHA_TU_ROWS
+  if (v.save_once) return launch_stream_save(a, s);
+  if (v.save_split) { // forward with LSE, then the saved outputs from that LSE
+    const int rc = v.stream ? launch_stream<true>(a, v, s) : launch<1, kMaskFull, false, 2, FMHA_TU_D == 64>(a, s);
+    return rc ? rc : launch_save(a, s);
+  }
+  if (v.stream) return v.drop == 2 ? launch_stream<true>(a, v, s) : launch_stream<false>(a, v, s);
+#else
+  if (v.save_split || v.save_once || v.stream) return 1;
 #endif
   if (v.drop == 2) { // tensor dropout / save-intermediates: the legacy ops' shape class
     if (v.causal) return 1;

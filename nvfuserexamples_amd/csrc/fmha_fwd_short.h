@@ -45,7 +45,8 @@ struct ShortCfg {
 // merged with their "block skipped" values afterwards, 32 register copies per block of the second product.
 // MASK: kMaskFull (the operators' [.., sq, sk] tensor), kMaskPerKey or kMaskNone.  DROP: 0 none, 1 the Philox
 // rule, 2 a [.., sq, sk] dropout tensor (kMaskFull only).  SAVE: kMaskFull with a dropout tensor only.
-template <typename T, int MASK, int DROP, bool SAVE, bool FULL, bool STRIDED = false> FMHA_DEV void fwd_short_body(const FwdArgs &a) {
+template <typename T, int MASK, int DROP, bool SAVE, bool FULL, bool STRIDED = false, bool TAIL = false>
+FMHA_DEV void fwd_short_body(const FwdArgs &a) {
   constexpr bool DROPT = DROP == 2;
   static_assert(!STRIDED || MASK != kMaskFull, "run-time row layouts: the builds without a full mask tensor only");
   constexpr bool ROWS = MASK == kMaskFull; // [.., sq, sk] tensors move through the row scratch
@@ -115,13 +116,12 @@ template <typename T, int MASK, int DROP, bool SAVE, bool FULL, bool STRIDED = f
   typename C::Scratch scr;
   scr.init(lds + 4 * TILEB + w * C::Scratch::BYTES, l);
   const int rsub = scr.rsub, chunk = scr.chunk;
-  const bool cvalid = chunk * 8 < a.sk;
   u32x4 mreg[8], dreg[8];
   if (ROWS) {
-    // Lanes whose chunk lies past sk read chunk 0 instead (their values are never used: those keys'
+    // Lanes whose chunk lies past sk re-read the row's last 8 keys instead (their values are never used: those keys'
     // scores are forced to -inf).  Unconditional loads matter: a load under a lane condition is merged
     // with its "else" value right behind it, which makes the compiler wait for it on the spot.
-    const int ch8 = cvalid ? chunk * 8 : 0;
+    const int ch8 = scr.template first_key<TAIL>(0, a.sk);
     const int mhead = a.mask_div == 1 ? bh : bh / a.mask_div;
     const char *mb = (const char *)((const T *)a.mask + (size_t)mhead * a.mask_sb);
     const char *db_ = DROPT ? (const char *)((const T *)a.drop_mask + (size_t)bh * a.sq * a.sk) : nullptr;
@@ -132,10 +132,10 @@ template <typename T, int MASK, int DROP, bool SAVE, bool FULL, bool STRIDED = f
       qrow[i] = q < a.sq ? q : a.sq - 1;
     }
 #pragma unroll
-    for (int i = 0; i < 8; ++i) mreg[i] = *(const u32x4 *)(mb + (uint32_t)(qrow[i] * (int)a.mask_sq + ch8) * 2u);
+    for (int i = 0; i < 8; ++i) mreg[i] = *(const u32x4_any *)(mb + (uint32_t)(qrow[i] * (int)a.mask_sq + ch8) * 2u);
     if (DROPT) {
 #pragma unroll
-      for (int i = 0; i < 8; ++i) dreg[i] = *(const u32x4 *)(db_ + (uint32_t)(qrow[i] * a.sk + ch8) * 2u);
+      for (int i = 0; i < 8; ++i) dreg[i] = *(const u32x4_any *)(db_ + (uint32_t)(qrow[i] * a.sk + ch8) * 2u);
     }
   }
   // Loads complete in the order they were requested.  The K and V copies went out first: once at most
@@ -167,6 +167,7 @@ template <typename T, int MASK, int DROP, bool SAVE, bool FULL, bool STRIDED = f
 
   // ---- scale and mask (log2 units); keys past the end drop out
   if (ROWS) {
+    if (TAIL) scr.place_tail(mreg, 0, a.sk);
     scr.rows_in(mreg);
     scr.turn();
   }
@@ -219,17 +220,13 @@ template <typename T, int MASK, int DROP, bool SAVE, bool FULL, bool STRIDED = f
   // rows of the scratch leave as whole rows of a [.., sq, sk] output
   auto store_rows = [&](void *out) {
     char *ob = (char *)((T *)out + (size_t)bh * a.sq * a.sk);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int q = q0w + 4 * i + rsub;
-      const u32x4 t = scr.row_out(i);
-      if (cvalid && q < a.sq) *(u32x4 *)(ob + (uint32_t)(q * a.sk + chunk * 8) * 2u) = t;
-    }
+    scr.template rows_out<TAIL>([&](int q) { return ob + (uint32_t)(q * a.sk + chunk * 8) * 2u; }, q0w, a.sq, 0, a.sk);
   };
   // ---- dropped, normalised probabilities in the element type: second operand and saved output.
   // (The dropout rows are the last loads to arrive; nothing is stored before they are consumed, so
   // that waiting for them never waits for a store.)
   if (DROPT) {
+    if (TAIL) scr.place_tail(dreg, 0, a.sk);
     scr.rows_in(dreg);
     scr.turn();
   }
@@ -330,6 +327,12 @@ template <typename T, int DROP, bool SAVE, bool FULL>
 __global__ __launch_bounds__(ShortCfg::NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void fmha_fwd_short_kernel(const FwdArgs a) {
   fwd_short_body<T, kMaskFull, DROP, SAVE, FULL>(a);
+}
+// ... and rows whose length is no multiple of 8 keys.
+template <typename T, int DROP, bool SAVE, bool FULL>
+__global__ __launch_bounds__(ShortCfg::NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void fmha_fwd_short_tail_kernel(const FwdArgs a) {
+  fwd_short_body<T, kMaskFull, DROP, SAVE, FULL, false, true>(a);
 }
 // Without one: four workgroups per compute unit (33 KB of LDS, at most 128 registers), which is what keeps launches
 // of more heads than the device holds at once level with the persistent pipelined kernel.

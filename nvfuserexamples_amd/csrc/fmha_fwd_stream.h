@@ -4,9 +4,11 @@
 // With such tensors the forward is memory time at head dim 64 (BH 512, S 512: 34 GFLOP against
 // 402 MB with the mask, 671 MB with mask and dropout tensor), so the kernel is built for streaming,
 // like the kernel that writes the saved outputs: [.., sq, sk] rows arrive as whole 128-byte row
-// segments (16 bytes per lane, 8 lanes per row), one tile ahead, and a wave-private LDS scratch
-// turns them into the accumulator layout; K and V tiles are staged through registers with them, so
-// every request of an iteration is in flight for a whole iteration.  The softmax is the textbook
+// segments (16 bytes per lane, 8 lanes per row; the last one of a row of any other length: TAIL), one
+// tile ahead, and a wave-private LDS scratch per tensor turns them into the accumulator layout; K and V
+// tiles are staged through registers with them, so every request of an iteration is in flight for a
+// whole iteration.  (Two tiles ahead, with exact waits, measured 2 to 5 % slower with every compute unit
+// busy: 91.1 -> 93.0 us at BH 512, S 512, 127.2 -> 134 with the dropout tensor.)  The softmax is the textbook
 // online one (running row maximum, rescale on every tile, fp32 row sum): at two waves per SIMD the
 // vector work hides under the memory time, which the lazily re-based, matrix-pipe-assisted softmax
 // of the pipelined kernel is not needed for.
@@ -15,29 +17,38 @@
 
 namespace fmha {
 
-struct StreamCfg {
-  static constexpr int D = 64;
+// MANY: the build for launches of more than two workgroups per compute unit, under the mask alone at head dim 64: one
+// K / V stage instead of two, written between two barriers, which lets three workgroups share a compute unit.  BH 512,
+// S 512: 87.5 -> 84.9 us, S 229: 28.4 -> 27.5; with fewer workgroups the second barrier only costs (BH 48, S 483: 13.7
+// -> 14.7 us).  (With the dropout tensor three would need 54.6 KB of LDS each; the two scratches make it 55.3.)
+// Head dim 128 has the one stage in any case: two would leave one workgroup per compute unit.
+template <int D_, bool MANY> struct StreamCfg {
+  static constexpr int D = D_;
   static constexpr int NW = 4;
   static constexpr int QT = NW * 32;
   static constexpr int BK = 64;
   static constexpr int ROWB = D * 2 + 16;          // padded K / V rows: conflict-free 16-byte and transpose reads
   static constexpr int TILEB = BK * ROWB;
   using Scratch = RowScratch<BK>;                  // wave-private: rows of a [.., sq, sk] tensor <-> accumulator layout
-  static constexpr int LDS_BYTES = 4 * TILEB + NW * Scratch::BYTES; // {K, V} x 2 stages + one scratch per wave
+  static constexpr int NST = D == 64 && !MANY ? 2 : 1;
+  static constexpr int OCC = MANY ? 3 : 2;
+  static constexpr int nscr(bool dropt) { return dropt ? 2 : 1; }
+  static constexpr int lds_bytes(bool dropt) { return NST * 2 * TILEB + NW * nscr(dropt) * Scratch::BYTES; } // {K, V} per stage + a wave's scratch
 };
 
-template <typename T, bool DROPT>
-__global__ __launch_bounds__(StreamCfg::NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
+template <typename T, int D, bool DROPT, bool TAIL, bool MANY>
+__global__ __launch_bounds__((StreamCfg<D, MANY>::NW * 64))
+__attribute__((amdgpu_waves_per_eu(StreamCfg<D, MANY>::OCC, StreamCfg<D, MANY>::OCC)))
 void fmha_fwd_stream_kernel(const FwdArgs a) {
   using E = Elem<T>;
   using v8 = typename E::v8;
   using v4 = typename E::v4;
-  using C = StreamCfg;
-  constexpr int D = C::D, KS = D / 16, DB = D / 32, BK = C::BK, NSB = BK / 32, NT = C::NW * 64, ROWB = C::ROWB;
+  using C = StreamCfg<D, MANY>;
+  static_assert(!MANY || (D == 64 && !DROPT), "three workgroups per compute unit: the mask alone at head dim 64");
+  constexpr int KS = D / 16, DB = D / 32, BK = C::BK, NSB = BK / 32, NT = C::NW * 64, ROWB = C::ROWB;
   constexpr int TILEB = C::TILEB;
   constexpr int CPR = D / 8, CPT = BK * CPR / NT;
   constexpr float NEG_INF = -__builtin_inff();
-  constexpr bool PF2 = !DROPT; // mask rows two tiles ahead
 
   extern __shared__ __attribute__((aligned(16))) char lds[];
 
@@ -68,8 +79,9 @@ void fmha_fwd_stream_kernel(const FwdArgs a) {
 
   // ---- staging.  K, V: global -> registers -> LDS (two stages).  [.., sq, sk] rows: instruction i covers
   // rows 8i .. 8i+7 of the wave's 32, eight lanes per row, 8 keys (16 bytes) per lane.
-  typename C::Scratch scr;
-  scr.init(lds + 4 * TILEB + w * C::Scratch::BYTES, l);
+  typename C::Scratch scr, scrd; // mask rows, dropout rows
+  scr.init(lds + C::NST * 2 * TILEB + w * C::nscr(DROPT) * C::Scratch::BYTES, l);
+  scrd.init(lds + C::NST * 2 * TILEB + (w * C::nscr(DROPT) + C::nscr(DROPT) - 1) * C::Scratch::BYTES, l);
   const int rsub = scr.rsub, chunk = scr.chunk;
   int qrow[4];
 #pragma unroll
@@ -83,7 +95,7 @@ void fmha_fwd_stream_kernel(const FwdArgs a) {
     u32x4 k[CPT], v[CPT], m[4], d[4];
   };
   // Every load is unconditional (a load under a lane condition makes the compiler wait for it on the
-  // spot): key rows past the end re-read the last row, chunks past sk re-read the row's first chunk;
+  // spot): key rows past the end re-read the last row, chunks past sk re-read the row's last 8 keys;
   // those keys' scores are forced to -inf, so P = 0 meets finite values of V.
   auto gload = [&](int k0, Stage &st) {
 #pragma unroll
@@ -94,19 +106,13 @@ void fmha_fwd_stream_kernel(const FwdArgs a) {
       st.k[i] = *(const u32x4 *)(Kb + (size_t)kr * D + (c % CPR) * 8);
       st.v[i] = *(const u32x4 *)(Vb + (size_t)kr * D + (c % CPR) * 8);
     }
-    const int koff = k0 + chunk * 8 < a.sk ? k0 + chunk * 8 : 0;
+    const int koff = scr.template first_key<TAIL>(k0, a.sk);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      if (!PF2) st.m[i] = *(const u32x4 *)(mb + (size_t)qrow[i] * a.mask_sq + koff);
-      if (DROPT) st.d[i] = *(const u32x4 *)(db_ + (size_t)qrow[i] * a.sk + koff);
+    for (int i = 0; i < 4; ++i) st.m[i] = *(const u32x4_any *)(mb + (size_t)qrow[i] * a.mask_sq + koff);
+    if (DROPT) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) st.d[i] = *(const u32x4_any *)(db_ + (size_t)qrow[i] * a.sk + koff);
     }
-  };
-  // Without a dropout tensor the registers allow the mask rows -- the larger half of an iteration's bytes -- to be
-  // requested two tiles ahead (BH 512, S 512: 99.6 -> 93.0 us; with the dropout tensor it measured level).
-  auto gload_mask = [&](int k0, u32x4 (&mm)[4]) {
-    const int koff = k0 + chunk * 8 < a.sk ? k0 + chunk * 8 : 0;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) mm[i] = *(const u32x4 *)(mb + (size_t)qrow[i] * a.mask_sq + koff);
   };
   auto lstore = [&](int stage, const Stage &st) {
 #pragma unroll
@@ -115,6 +121,16 @@ void fmha_fwd_stream_kernel(const FwdArgs a) {
       *(u32x4 *)(lds + stage * 2 * TILEB + (c / CPR) * ROWB + (c % CPR) * 16) = st.k[i];
       *(u32x4 *)(lds + stage * 2 * TILEB + TILEB + (c / CPR) * ROWB + (c % CPR) * 16) = st.v[i];
     }
+  };
+
+  auto rows_in = [&](int k0, Stage &st) {
+    if (TAIL) scr.place_tail(st.m, k0, a.sk);
+    scr.rows_in(st.m);
+    if (DROPT) {
+      if (TAIL) scrd.place_tail(st.d, k0, a.sk);
+      scrd.rows_in(st.d);
+    }
+    scr.turn();
   };
 
   // ---- running state: row maximum m (log2 units), this lane's part of the row sum, unnormalised O^T
@@ -126,25 +142,23 @@ void fmha_fwd_stream_kernel(const FwdArgs a) {
     for (int r = 0; r < 16; ++r) o[db][r] = 0.f;
 
   const int nkt = (a.sk + BK - 1) / BK;
-  Stage cur;
-  gload(0, cur);
-  u32x4 m_next[4];
-  if (PF2) {
-    gload_mask(0, cur.m);
-    gload_mask(nkt > 1 ? BK : 0, m_next);
-  }
-  lstore(0, cur);
+  Stage st;
+  __builtin_amdgcn_sched_barrier(0);
+  gload(0, st);
+  lstore(0, st);
+  rows_in(0, st);
+  // (The compiler would wait for Q at its first use inside the loop, on every iteration, and with it for the
+  // requests behind it.)
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(qreg[ks]));
   __syncthreads();
 
   for (int t = 0; t < nkt; ++t) {
     const int k0 = t * BK;
-    const char *ldsK = lds + (t & 1) * 2 * TILEB;
+    const char *ldsK = lds + (C::NST == 2 ? t & 1 : 0) * 2 * TILEB;
     const char *ldsV = ldsK + TILEB;
-    Stage nxt;
     const bool more = t + 1 < nkt; // workgroup-uniform
-    if (more) gload(k0 + BK, nxt);
-    u32x4 m_after[4];
-    if (PF2) gload_mask(t + 2 < nkt ? k0 + 2 * BK : k0, m_after); // (unconditional: past the last tile it re-reads this one)
+    if (more) gload(k0 + BK, st);
 
     // ---- scores in log2 units: x * scale + mask
     f32x16 x[NSB];
@@ -156,8 +170,6 @@ void fmha_fwd_stream_kernel(const FwdArgs a) {
       for (int ks = 0; ks < KS; ++ks)
         x[sb] = E::mfma(as_v8<T>(*(const u32x4 *)(ldsK + (sb * 32 + ql) * ROWB + ks * 32 + h * 16)), qreg[ks], x[sb]);
     }
-    scr.rows_in(cur.m);
-    scr.turn();
 #pragma unroll
     for (int sb = 0; sb < NSB; ++sb)
 #pragma unroll
@@ -210,10 +222,6 @@ void fmha_fwd_stream_kernel(const FwdArgs a) {
     }
 
     // ---- (dropped) probabilities in the element type: B operand of the second product
-    if (DROPT) {
-      scr.rows_in(cur.d);
-      scr.turn();
-    }
     v8 pfrag[NSB][2];
 #pragma unroll
     for (int sb = 0; sb < NSB; ++sb)
@@ -221,7 +229,7 @@ void fmha_fwd_stream_kernel(const FwdArgs a) {
       for (int g = 0; g < 4; ++g) {
         float keep[4] = {1.f, 1.f, 1.f, 1.f};
         if (DROPT) {
-          const v4 dm = as_v4<T>(scr.piece(sb, g));
+          const v4 dm = as_v4<T>(scrd.piece(sb, g));
 #pragma unroll
           for (int i = 0; i < 4; ++i) keep[i] = (float)dm[i];
         }
@@ -239,16 +247,10 @@ void fmha_fwd_stream_kernel(const FwdArgs a) {
         for (int db = 0; db < DB; ++db)
           o[db] = E::mfma(lds_load_a_transposed<T, ROWB>(ldsV, sb * 32, db * 32, c, l), pfrag[sb][c], o[db]);
 
+    if (C::NST == 1) __syncthreads(); // every wave is done with this tile
     if (more) {
-      lstore((t + 1) & 1, nxt);
-      cur = nxt;
-      if (PF2) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          cur.m[i] = m_next[i];
-          m_next[i] = m_after[i];
-        }
-      }
+      lstore(C::NST == 2 ? (t + 1) & 1 : 0, st);
+      rows_in(k0 + BK, st);
     }
     __syncthreads();
   }

@@ -16,27 +16,37 @@
 // Rounding: the saved softmax is rounded twice (p_t to the element type, then the product), at most
 // 2^-10 relative for fp16 instead of 2^-11; the second product O += P V takes exactly the operands
 // of the streaming forward, so the context is bit-identical to that kernel's.
+//
+// AGAIN (rows that end within a 16-byte piece, head dim 128) rounds once: the tile's mask rows are kept
+// in place of its probabilities, K stays in LDS, which the workgroup has to itself, and the second phase
+// forms the scores again, P = exp2(s - L).  That phase then is no longer free behind its stores: 92
+// instead of 82 us at BH 512, S 229 (forward and a second launch take 117).
 #pragma once
 #include "fmha_fwd_stream.h"
 
 namespace fmha {
 
-struct StreamSaveCfg : StreamCfg {
-  static constexpr int MAXT = 8;                   // 64-key tiles whose probabilities a wave can hold
-  static constexpr int SKMAX = MAXT * BK;
+template <int D_> struct StreamSaveCfg : StreamCfg<D_, false> {
+  using B = StreamCfg<D_, false>;
+  static constexpr int MAXT = D_ == 64 ? 8 : 7;    // 64-key tiles whose rows a wave, and whose K the workgroup, can hold
+  static constexpr int SKMAX = MAXT * B::BK;
+  static constexpr int nkst(bool again) { return again ? MAXT : 2; } // K stages
+  static constexpr int lds_bytes(bool again) { return (nkst(again) + B::NST) * B::TILEB + B::NW * B::Scratch::BYTES; } // K, V, a wave's scratch
 };
 
-template <typename T>
-__global__ __launch_bounds__(StreamSaveCfg::NW * 64) __attribute__((amdgpu_waves_per_eu(1, 1)))
+template <typename T, int D, bool TAIL>
+__global__ __launch_bounds__(StreamSaveCfg<D>::NW * 64) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void fmha_fwd_stream_save_kernel(const FwdArgs a) {
   using E = Elem<T>;
   using v8 = typename E::v8;
   using v4 = typename E::v4;
-  using C = StreamSaveCfg;
-  constexpr int D = C::D, KS = D / 16, DB = D / 32, BK = C::BK, NSB = BK / 32, NT = C::NW * 64, ROWB = C::ROWB;
+  using C = StreamSaveCfg<D>;
+  constexpr int KS = D / 16, DB = D / 32, BK = C::BK, NSB = BK / 32, NT = C::NW * 64, ROWB = C::ROWB;
   constexpr int TILEB = C::TILEB, MAXT = C::MAXT;
   constexpr int CPR = D / 8, CPT = BK * CPR / NT;
   constexpr float NEG_INF = -__builtin_inff();
+  constexpr bool AGAIN = TAIL || D != 64;
+  constexpr int NKST = C::nkst(AGAIN);
 
   extern __shared__ __attribute__((aligned(16))) char lds[];
 
@@ -68,7 +78,7 @@ void fmha_fwd_stream_save_kernel(const FwdArgs a) {
   // ---- staging, as in the streaming forward.  K, V: global -> registers -> LDS (two stages).  [.., sq, sk]
   // rows: instruction i covers rows 8i .. 8i+7 of the wave's 32, eight lanes per row, 8 keys per lane.
   typename C::Scratch scr;
-  scr.init(lds + 4 * TILEB + w * C::Scratch::BYTES, l);
+  scr.init(lds + (NKST + C::NST) * TILEB + w * C::Scratch::BYTES, l);
   const int rsub = scr.rsub, chunk = scr.chunk;
   int qrow[4];
 #pragma unroll
@@ -81,8 +91,8 @@ void fmha_fwd_stream_save_kernel(const FwdArgs a) {
   struct Stage {
     u32x4 k[CPT], v[CPT], m[4], d[4];
   };
-  // every load is unconditional: key rows past the end re-read the last row, chunks past sk the row's first
-  // chunk; those keys' scores are forced to -inf and their columns are never stored
+  // every load is unconditional: key rows past the end re-read the last row, chunks past sk the row's last
+  // 8 keys; those keys' scores are forced to -inf and their columns are never stored
   auto gload = [&](int k0, Stage &st) {
 #pragma unroll
     for (int i = 0; i < CPT; ++i) {
@@ -92,19 +102,60 @@ void fmha_fwd_stream_save_kernel(const FwdArgs a) {
       st.k[i] = *(const u32x4 *)(Kb + (size_t)kr * D + (c % CPR) * 8);
       st.v[i] = *(const u32x4 *)(Vb + (size_t)kr * D + (c % CPR) * 8);
     }
-    const int koff = k0 + chunk * 8 < a.sk ? k0 + chunk * 8 : 0;
+    const int koff = scr.template first_key<TAIL>(k0, a.sk);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      st.m[i] = *(const u32x4 *)(mb + (size_t)qrow[i] * a.mask_sq + koff);
-      st.d[i] = *(const u32x4 *)(db_ + (size_t)qrow[i] * a.sk + koff);
+      st.m[i] = *(const u32x4_any *)(mb + (size_t)qrow[i] * a.mask_sq + koff);
+      st.d[i] = *(const u32x4_any *)(db_ + (size_t)qrow[i] * a.sk + koff);
     }
   };
-  auto lstore = [&](int stage, const Stage &st) {
+  // (Everything that was requested is waited for here: the next tile's requests are made under a condition, and a wait
+  // behind them could not tell how many there are and would wait for them all.)
+  auto lstore = [&](int t, Stage &st) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      asm volatile("" : "+v"(st.m[i]));
+      asm volatile("" : "+v"(st.d[i]));
+    }
 #pragma unroll
     for (int i = 0; i < CPT; ++i) {
       const int c = tid + i * NT;
-      *(u32x4 *)(lds + stage * 2 * TILEB + (c / CPR) * ROWB + (c % CPR) * 16) = st.k[i];
-      *(u32x4 *)(lds + stage * 2 * TILEB + TILEB + (c / CPR) * ROWB + (c % CPR) * 16) = st.v[i];
+      *(u32x4 *)(lds + (AGAIN ? t : t & 1) * TILEB + (c / CPR) * ROWB + (c % CPR) * 16) = st.k[i];
+      *(u32x4 *)(lds + (NKST + (C::NST == 2 ? t & 1 : 0)) * TILEB + (c / CPR) * ROWB + (c % CPR) * 16) = st.v[i];
+    }
+  };
+  // scores of tile t in log2 units, x * scale + mask, with the tile's mask rows in registers
+  auto scores = [&](int t, const u32x4 (&mr)[4], f32x16 (&x)[NSB]) __attribute__((always_inline)) {
+    const int k0 = t * BK;
+    const char *ldsK = lds + (AGAIN ? t : t & 1) * TILEB;
+#pragma unroll
+    for (int sb = 0; sb < NSB; ++sb) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) x[sb][r] = 0.f;
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+        x[sb] = E::mfma(as_v8<T>(*(const u32x4 *)(ldsK + (sb * 32 + ql) * ROWB + ks * 32 + h * 16)), qreg[ks], x[sb]);
+    }
+    scr.rows_in(mr);
+    scr.turn();
+#pragma unroll
+    for (int sb = 0; sb < NSB; ++sb)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const v4 mv = as_v4<T>(scr.piece(sb, g));
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          x[sb][4 * g + i] = fmaf(x[sb][4 * g + i], a.scale_l2, fmaf((float)mv[i], a.mask_a, a.mask_b));
+      }
+    scr.turn();
+    if (k0 + BK > a.sk) { // only a partly filled last tile has keys to switch off (workgroup-uniform)
+#pragma unroll
+      for (int sb = 0; sb < NSB; ++sb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int kk = k0 + sb * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
+          x[sb][r] = kk < a.sk ? x[sb][r] : NEG_INF;
+        }
     }
   };
 
@@ -115,8 +166,8 @@ void fmha_fwd_stream_save_kernel(const FwdArgs a) {
   for (int db = 0; db < DB; ++db)
 #pragma unroll
     for (int r = 0; r < 16; ++r) o[db][r] = 0.f;
-  v8 psave[MAXT][NSB][2];
-  u32x4 dsave[MAXT][4];
+  u32x4 rsave[MAXT][4], dsave[MAXT][4]; // mask rows (AGAIN), dropout rows
+  v8 psave[MAXT][NSB][2];               // the tile's probabilities and the maximum they were formed under (!AGAIN)
   float msave[MAXT];
 
   // (Requests run one tile ahead of their use.  Two tiles ahead -- the registers would allow it -- measured
@@ -126,49 +177,27 @@ void fmha_fwd_stream_save_kernel(const FwdArgs a) {
   Stage cur;
   gload(0, cur);
   lstore(0, cur);
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(qreg[ks])); // (and for Q)
   __syncthreads();
 
 #pragma unroll
   for (int t = 0; t < MAXT; ++t) {
     if (t < nkt) { // workgroup-uniform
       const int k0 = t * BK;
-      const char *ldsK = lds + (t & 1) * 2 * TILEB;
-      const char *ldsV = ldsK + TILEB;
+      const char *ldsV = lds + (NKST + (C::NST == 2 ? t & 1 : 0)) * TILEB;
       Stage nxt;
       const bool more = t + 1 < nkt;
       if (more) gload(k0 + BK, nxt);
-
-      // ---- scores in log2 units: x * scale + mask
+      if (TAIL) scr.place_tail(cur.m, k0, a.sk);
+      if (TAIL) scr.place_tail(cur.d, k0, a.sk);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if (AGAIN) rsave[t][i] = cur.m[i];
+        dsave[t][i] = cur.d[i];
+      }
       f32x16 x[NSB];
-#pragma unroll
-      for (int sb = 0; sb < NSB; ++sb) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) x[sb][r] = 0.f;
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks)
-          x[sb] = E::mfma(as_v8<T>(*(const u32x4 *)(ldsK + (sb * 32 + ql) * ROWB + ks * 32 + h * 16)), qreg[ks], x[sb]);
-      }
-      scr.rows_in(cur.m);
-      scr.turn();
-#pragma unroll
-      for (int sb = 0; sb < NSB; ++sb)
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const v4 mv = as_v4<T>(scr.piece(sb, g));
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            x[sb][4 * g + i] = fmaf(x[sb][4 * g + i], a.scale_l2, fmaf((float)mv[i], a.mask_a, a.mask_b));
-        }
-      scr.turn();
-      if (k0 + BK > a.sk) { // only a partly filled last tile has keys to switch off (workgroup-uniform)
-#pragma unroll
-        for (int sb = 0; sb < NSB; ++sb)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const int kk = k0 + sb * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
-            x[sb][r] = kk < a.sk ? x[sb][r] : NEG_INF;
-          }
-      }
+      scores(t, cur.m, x);
       float tmax = NEG_INF;
 #pragma unroll
       for (int sb = 0; sb < NSB; ++sb)
@@ -181,7 +210,7 @@ void fmha_fwd_stream_save_kernel(const FwdArgs a) {
       const float muse = mnew == NEG_INF ? 0.f : mnew;
       const float alpha = m == NEG_INF ? 0.f : fast_exp2(m - mnew);
       m = mnew;
-      msave[t] = mnew; // -inf while the row has seen no key: the tile's probabilities are zeros and stay zeros
+      if (!AGAIN) msave[t] = mnew; // -inf while the row has seen no key: the tile's probabilities are zeros and stay zeros
       float rs = 0.f;
 #pragma unroll
       for (int sb = 0; sb < NSB; ++sb)
@@ -200,7 +229,7 @@ void fmha_fwd_stream_save_kernel(const FwdArgs a) {
       }
 
       // ---- dropped probabilities in the element type (B operand of the second product); undropped ones kept
-      scr.rows_in(cur.d);
+      scr.rows_in(dsave[t]);
       scr.turn();
       v8 pfrag[NSB][2];
 #pragma unroll
@@ -211,12 +240,10 @@ void fmha_fwd_stream_save_kernel(const FwdArgs a) {
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
             pfrag[sb][g >> 1][4 * (g & 1) + i] = (T)(x[sb][4 * g + i] * (float)dm[i]);
-            psave[t][sb][g >> 1][4 * (g & 1) + i] = (T)x[sb][4 * g + i];
+            if (!AGAIN) psave[t][sb][g >> 1][4 * (g & 1) + i] = (T)x[sb][4 * g + i];
           }
         }
       scr.turn();
-#pragma unroll
-      for (int i = 0; i < 4; ++i) dsave[t][i] = cur.d[i];
 
       // ---- O^T += V^T . P^T
 #pragma unroll
@@ -227,8 +254,9 @@ void fmha_fwd_stream_save_kernel(const FwdArgs a) {
           for (int db = 0; db < DB; ++db)
             o[db] = E::mfma(lds_load_a_transposed<T, ROWB>(ldsV, sb * 32, db * 32, c, l), pfrag[sb][c], o[db]);
 
+      if (C::NST == 1) __syncthreads(); // every wave is done with this tile
       if (more) {
-        lstore((t + 1) & 1, nxt);
+        lstore(t + 1, nxt);
         cur = nxt;
       }
       __syncthreads();
@@ -250,25 +278,27 @@ void fmha_fwd_stream_save_kernel(const FwdArgs a) {
   // row entered with no key seen (m_t = -inf) and a row that never saw one (L = +big) give factor zero.
   const float L = lt > 0.f ? m + fast_log2(lt) : 3.0e38f;
   auto rows_out = [&](void *out, int k0) {
-    const bool cvalid = k0 + chunk * 8 < a.sk;
     T *ob = (T *)out + (size_t)bh * a.sq * a.sk + k0 + chunk * 8;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int qq = q0w + 8 * i + rsub;
-      const u32x4 tt = scr.row_out(i);
-      if (cvalid && qq < a.sq) *(u32x4 *)(ob + (size_t)qq * a.sk) = tt;
-    }
+    scr.template rows_out<TAIL>([&](int q) { return (char *)(ob + (size_t)q * a.sk); }, q0w, a.sq, k0, a.sk);
   };
 #pragma unroll
   for (int t = 0; t < MAXT; ++t) {
     if (t < nkt) {
       const int k0 = t * BK;
-      const float f = fast_exp2(msave[t] - L);
-      float x[NSB][16];
+      f32x16 x[NSB];
+      if constexpr (AGAIN) {
+        scores(t, rsave[t], x);
 #pragma unroll
-      for (int sb = 0; sb < NSB; ++sb)
+        for (int sb = 0; sb < NSB; ++sb)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) x[sb][r] = (float)psave[t][sb][r >> 3][r & 7] * f;
+          for (int r = 0; r < 16; ++r) x[sb][r] = fast_exp2(x[sb][r] - L);
+      } else {
+        const float f = fast_exp2(msave[t] - L);
+#pragma unroll
+        for (int sb = 0; sb < NSB; ++sb)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) x[sb][r] = (float)psave[t][sb][r >> 3][r & 7] * f;
+      }
       if (a.save_softmax) {
 #pragma unroll
         for (int sb = 0; sb < NSB; ++sb)
