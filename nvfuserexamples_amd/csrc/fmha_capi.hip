@@ -762,6 +762,8 @@ int fmha_fwd_fp8_launch(const fmha_fwd_fp8_params *caller, void *hip_stream) {
   a.score_scale_l2 = p->scale * p->descale_q * p->descale_k * FMHA_LOG2E;
   a.inv_score_scale_l2 = 1.f / a.score_scale_l2;
   a.out_scale = p->descale_v;
+  a.trim = p->mask && overrides().mask_trim != 0 &&
+           448.0 * 448.0 * p->d * p->scale * p->descale_q * p->descale_k <= kFp8TrimScore;
   const int rc = fwd_fp8_dispatch(a, p->d, p->out_dtype == FMHA_DTYPE_BF16, p->causal != 0, (hipStream_t)hip_stream);
   return rc == 0 ? FMHA_OK : (rc == 1 ? FMHA_E_UNSUPPORTED : FMHA_E_LAUNCH);
 }

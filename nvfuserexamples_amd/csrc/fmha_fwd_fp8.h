@@ -13,13 +13,19 @@
 // of key block 1; register r of a lane (q, h) is key 8 (r / 4) + 4h + r % 4 of its block, so contraction byte
 // j = 16 b + r of half-wave h stands for key 32 b + 8 (r / 4) + 4 h + r % 4, and the V^T operand is fetched in
 // that order: transpose read (b, gp) covers the rows 32 b + 16 gp + 4 h + {0,1,2,3, 8,9,10,11}.
-// As in the 16-bit kernels the per-element vector work is what bounds the kernel (the fp8 products take a
-// quarter of its time), so everything that is a rank-one term rides in the matrix pipe: after the fp8 product
-// one bf16 32x32x16 step adds  (mask[key] - M[q]) / s  to the raw scores, with
-//   A row of a key   (1, 1, 1, mk_hi, mk_mid, mk_lo, 0, 0)      mk = mask term / s, "-inf" for keys past the end
-//   B col of a query (-Mr_hi, -Mr_mid, -Mr_lo, 1, 1, 1, 0, 0)   Mr = M / s
-// (three bf16 pieces each: exact to fp32), s = scale * descale_q * descale_k * log2(e).  Then P = exp2(s x): one
-// multiply, one exponential and half a conversion per element.  The row sums come out of the matrix pipe too:
+// The per-element vector work is what bounds the kernel: P = exp2(s x - M), s = scale * descale_q * descale_k *
+// log2(e), is one fused multiply-add, one exponential and half a conversion per element (and an add for the LSE).
+// A mask term or the end of the keys costs a tile that has one a bf16 32x32x16 step after the fp8 product,
+//   A row of a key   (mk_hi, mk_mid, mk_lo, 0 ..)   mk = mask term / s, "-inf" for keys past the end
+//   B col of a query (1, 1, 1, 0 ..)
+// (three bf16 pieces: exact to fp32); tiles whose keys are all there and unmasked -- most of a padded batch --
+// go without.  Key tiles of nothing but hard-masked keys at the end of a mask row are not visited where their
+// weights are zero whatever the inputs (Fp8Args::trim).
+// BH 512 S 512 D 64 with masks whose lengths are spread over [256, 512]: 47.7 -> 36.2 us; without a mask 43.2 -> 37.9 us;
+// BH 32 S 4096 D 128 causal 220 -> 112 us, BH 32 S 2048 D 64 causal 50.4 -> 30.4 us (the key-after-query test of the
+// diagonal tiles used to cost every tile two instructions per element; waves leave out the tiles past their own rows).
+// The registers are held to four waves per SIMD at head dim 64, three where causal.
+// The row sums come out of the matrix pipe too:
 // one more fp8 product of the rounded tile with an operand of ones gives every lane the sum of ITS row's
 // rounded probabilities, so O = sum P~ v / sum P~ is a convex combination of the values (a row with one
 // dominant key reproduces that key's value exactly, whatever the rounding did to its probability).  The row
@@ -48,7 +54,13 @@ struct Fp8Args {
   float score_scale_l2;     // s = scale * descale_q * descale_k * log2(e)
   float inv_score_scale_l2; // 1 / s
   float out_scale;          // descale_v
+  // Leave out the key tiles behind the last key whose mask term is above kFp8Hard, in rows that have a key at or above
+  // kFp8Live.  The launch code sets it where  |score| <= 448^2 d scale descale_q descale_k <= kFp8TrimScore  for any
+  // inputs: a hard-masked key's exponent is then at least 200 (288 in log2 units) below the row's reference, less the 8
+  // that the reference may sit below the maximum, so its probability is 0 in fp32 and leaving it out changes nothing.
+  int32_t trim;
 };
+constexpr float kFp8Hard = -9000.f, kFp8Live = -1000.f, kFp8TrimScore = 3900.f;
 
 typedef int i32x8 __attribute__((ext_vector_type(8)));
 typedef int i32x2v __attribute__((ext_vector_type(2)));
@@ -58,8 +70,10 @@ template <int D> struct Fp8Cfg {
   static constexpr int PITCH = D + 16;              // bytes per key row of the K and V tiles (16 rows, 16 bank groups)
   static constexpr int TILEB = BK * PITCH;
   static constexpr int XROWB = 32;                   // extra-step row of a key: 16 bf16
-  static constexpr int STAGEB = 2 * TILEB + BK * XROWB; // K tile, V tile, extra-step rows of the tile
-  static constexpr int LDS_BYTES = 2 * STAGEB;
+  static constexpr int LDS_FLAG = 2 * TILEB + BK * XROWB; // (in a stage) whether the tile takes the extra step
+  static constexpr int STAGEB = LDS_FLAG + 16;       // K tile, V tile, extra-step rows of the tile, flag
+  static constexpr int LDS_TRIM = 2 * STAGEB;        // per wave: keys up to its last live one, whether it saw a visible one
+  static constexpr int LDS_BYTES = LDS_TRIM + 2 * NW * 4;
 };
 
 // 32x32 += (32 x 64 e4m3) . (64 x 32 e4m3); format selectors 0 = e4m3 for both operands, no block scaling
@@ -88,7 +102,7 @@ FMHA_DEV void split3_bf16(float v, __bf16 &hi, __bf16 &mid, __bf16 &lo) {
 }
 
 template <typename TO, int D, bool CAUSAL, bool MASK>
-__global__ __launch_bounds__(Fp8Cfg<D>::NT) void fmha_fwd_fp8_kernel(const Fp8Args a) {
+__global__ __launch_bounds__(Fp8Cfg<D>::NT, D == 64 ? (CAUSAL ? 3 : 4) : 2) void fmha_fwd_fp8_kernel(const Fp8Args a) {
   using C = Fp8Cfg<D>;
   constexpr int NT = C::NT, QT = C::QT, BK = C::BK, DS = D / 64, DB = D / 32, PITCH = C::PITCH, XROWB = C::XROWB;
   constexpr int CPR = D / 16;            // 16-byte chunks per row
@@ -100,9 +114,20 @@ __global__ __launch_bounds__(Fp8Cfg<D>::NT) void fmha_fwd_fp8_kernel(const Fp8Ar
   extern __shared__ __attribute__((aligned(16))) char lds[];
 
   const int tid = threadIdx.x;
-  const int w = tid >> 6, l = tid & 63, ql = l & 31, h = l >> 5;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63, ql = l & 31, h = l >> 5;
   const int nqt = (a.sq + QT - 1) / QT;
-  const int bh = blockIdx.x / nqt, qt = blockIdx.x % nqt;
+  // Workgroups are dealt round-robin to the 8 XCDs: of every 8 heads each XCD gets one with all its query tiles, so a
+  // head's keys go through one L2, and heads of different lengths stay spread evenly.  Causal: the heads that an XCD
+  // gets from 32 workgroups on (one per compute unit) have the opposite order of tiles, so that a compute unit's
+  // workgroups add up alike, and the last ones go from long to short (all heads long to short: 1.46x the time of the
+  // plain order at BH 32 S 2048 D 64).
+  const int b = blockIdx.x, grouped = (a.bh & ~7) * nqt;
+  const int bh = b < grouped ? b / (8 * nqt) * 8 + (b & 7) : b / nqt;
+  int qt = b < grouped ? (b >> 3) % nqt : b % nqt;
+  if (CAUSAL) {
+    const int after = b < grouped ? (a.bh >> 3) - 1 - (b >> 3) / nqt : 0; // heads this XCD gets after this one
+    if (!((nqt >= 32 ? after : after * nqt / 32) & 1)) qt = nqt - 1 - qt;
+  }
   const int q = qt * QT + w * 32 + ql;
   const int qc = q < a.sq ? q : a.sq - 1;
   const float s = a.score_scale_l2, inv_s = a.inv_score_scale_l2;
@@ -133,7 +158,7 @@ __global__ __launch_bounds__(Fp8Cfg<D>::NT) void fmha_fwd_fp8_kernel(const Fp8Ar
 
   // tile staging: global -> registers -> LDS, both tiles as they are in memory; two LDS stages
   u32x4 kst[CPT], vst[CPT];
-  float mst = 0.f; // mask term of this thread's key in raw score units
+  TO mraw = (TO)0.f; // this thread's key's mask value, as it is in memory: whatever is made of it here would wait for it here
   auto gload = [&](int k0) {
 #pragma unroll
     for (int i = 0; i < CPT; ++i) {
@@ -143,39 +168,28 @@ __global__ __launch_bounds__(Fp8Cfg<D>::NT) void fmha_fwd_fp8_kernel(const Fp8Ar
       kst[i] = *(const u32x4 *)(Kb + (size_t)kr * D + col * 16);
       vst[i] = *(const u32x4 *)(Vb + (size_t)kr * D + col * 16);
     }
-    if (tid < BK) {
-      const int kr = k0 + tid;
-      mst = kr < a.sk ? 0.f : BIGNEG_RAW;
-      if (MASK && kr < a.sk) {
-        const float mk = (float)mkey[kr];
-        mst = mk == NEG_INF ? BIGNEG_RAW : fmaxf(mk * (FMHA_LOG2E * inv_s), BIGNEG_RAW);
-      }
-    }
+    if (MASK && tid < BK) mraw = mkey[k0 + tid < a.sk ? k0 + tid : a.sk - 1];
   };
-  auto lstore = [&](int stage) {
-    char *kd = lds + stage * C::STAGEB;
+  auto lstore = [&](int kt) {
+    char *kd = lds + (kt & 1) * C::STAGEB;
 #pragma unroll
     for (int i = 0; i < CPT; ++i) {
       const int c = tid + i * NT, row = c / CPR, col = c % CPR;
       *(u32x4 *)(kd + row * PITCH + col * 16) = kst[i];
       *(u32x4 *)(kd + C::TILEB + row * PITCH + col * 16) = vst[i];
     }
-    if (tid < BK) { // (1, 1, 1, mk_hi, mk_mid, mk_lo, 0 ...)
-      bf16x8 r0, z;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        r0[j] = (__bf16)0.f;
-        z[j] = (__bf16)0.f;
+    if (tid < BK) { // (wave 0) (mk_hi, mk_mid, mk_lo, 0 ...), the term in raw score units
+      const float mk = (float)mraw;
+      float mst = MASK ? (mk == NEG_INF ? BIGNEG_RAW : fmaxf(mk * (FMHA_LOG2E * inv_s), BIGNEG_RAW)) : 0.f;
+      if (kt * BK + tid >= a.sk) mst = BIGNEG_RAW;
+      const bool any = __builtin_amdgcn_ballot_w64(mst != 0.f) != 0;
+      if (any) {
+        __bf16 hi, mid, lo;
+        split3_bf16(mst, hi, mid, lo);
+        const uint32_t b0 = __builtin_bit_cast(uint16_t, hi), b1 = __builtin_bit_cast(uint16_t, mid), b2 = __builtin_bit_cast(uint16_t, lo);
+        *(u32x2 *)(kd + 2 * C::TILEB + tid * XROWB) = u32x2{b0 | b1 << 16, b2}; // (the rest of the row stays zero)
       }
-      r0[0] = r0[1] = r0[2] = (__bf16)1.f;
-      __bf16 hi, mid, lo;
-      split3_bf16(mst, hi, mid, lo);
-      r0[3] = hi;
-      r0[4] = mid;
-      r0[5] = lo;
-      bf16x8 *dst = (bf16x8 *)(kd + 2 * C::TILEB + tid * XROWB);
-      dst[0] = r0;
-      dst[1] = z;
+      if (tid == 0) *(int *)(kd + C::LDS_FLAG) = any;
     }
   };
 
@@ -191,33 +205,65 @@ __global__ __launch_bounds__(Fp8Cfg<D>::NT) void fmha_fwd_fp8_kernel(const Fp8Ar
     for (int r = 0; r < 16; ++r) oacc[db][r] = 0.f;
   float M = 0.f, l_run = 0.f, l_true = 0.f; // reference exponent (an integer); sums of the rounded / unrounded probabilities relative to it
   bool seen = false;          // M has been set from a tile with a live key
-  bf16x8 bx;                  // extra-step column of this lane's query
-  auto set_bx = [&]() {
-#pragma unroll
-    for (int j = 0; j < 8; ++j) bx[j] = (__bf16)0.f;
-    if (h == 0) {
-      __bf16 hi, mid, lo;
-      split3_bf16(-M * inv_s, hi, mid, lo);
-      bx[0] = hi;
-      bx[1] = mid;
-      bx[2] = lo;
-      bx[3] = bx[4] = bx[5] = (__bf16)1.f;
-    }
-  };
-  set_bx();
+  const uint32_t bx0 = h == 0 ? 0x3f803f80u : 0u, bx1 = h == 0 ? 0x3f80u : 0u; // extra-step column of a query: bf16 (1, 1, 1, 0 ..)
+  // the columns of the extra-step rows that stay zero
+  if (tid < 2 * BK) {
+    u32x4 *row = (u32x4 *)(lds + (tid / BK) * C::STAGEB + 2 * C::TILEB + (tid % BK) * XROWB);
+    row[0] = row[1] = u32x4{0, 0, 0, 0};
+  }
+  __syncthreads();
 
   gload(0);
+  const bool trim = MASK && !CAUSAL && a.trim && nkt > 1;
+  if (trim) {
+    int last = 0, seen_live = 0;
+    for (int j = w * 64; j < a.sk; j += NT) {
+      const float mk = j + l < a.sk ? (float)mkey[j + l] : NEG_INF;
+      const unsigned long long up = __builtin_amdgcn_ballot_w64(mk > kFp8Hard);
+      if (up) last = j + 64 - (int)__builtin_clzll(up);
+      seen_live |= __builtin_amdgcn_ballot_w64(mk >= kFp8Live) != 0;
+    }
+    if (l == 0) {
+      ((int *)(lds + C::LDS_TRIM))[2 * w] = last;
+      ((int *)(lds + C::LDS_TRIM))[2 * w + 1] = seen_live;
+    }
+  }
   lstore(0);
   if (nkt > 1) gload(BK);
   __syncthreads();
+  if (trim) {
+    int last = 0, seen_live = 0;
+#pragma unroll
+    for (int i = 0; i < C::NW; ++i) {
+      const int n = ((const int *)(lds + C::LDS_TRIM))[2 * i];
+      last = n > last ? n : last;
+      seen_live |= ((const int *)(lds + C::LDS_TRIM))[2 * i + 1];
+    }
+    last = __builtin_amdgcn_readfirstlane(last);
+    if (__builtin_amdgcn_readfirstlane(seen_live)) nkt = (last + BK - 1) / BK;
+  }
 
-  for (int kt = 0; kt < nkt; ++kt) {
+  auto stage_next = [&](int kt) { // the next tile goes to the other stage (its last readers passed the barrier that ended the previous iteration)
+    if (kt + 1 < nkt) {
+      lstore(kt + 1);
+      if (kt + 2 < nkt) gload((kt + 2) * BK);
+    }
+  };
+  // causal: the tiles that hold nothing up to this wave's own rows are left to the waves behind it
+  int nktw = nkt;
+  if (CAUSAL) {
+    const int own = (qt * QT + w * 32 + 31) / BK + 1;
+    nktw = own < nkt ? own : nkt;
+  }
+  for (int kt = 0; kt < nktw; ++kt) {
     const int k0 = kt * BK;
     const char *ldsK = lds + (kt & 1) * C::STAGEB;
     const char *ldsV = ldsK + C::TILEB;
     const char *ldsX = ldsK + 2 * C::TILEB;
 
-    // x = K.Q^T + (mask[key] - M[q]) / s  for the two 32-key blocks of the tile
+    const bool extra = MASK ? __builtin_amdgcn_readfirstlane(*(const int *)(ldsK + C::LDS_FLAG)) != 0 : k0 + BK > a.sk;
+
+    // x = K.Q^T + mask[key] / s  for the two 32-key blocks of the tile
     f32x16 x[2];
 #pragma unroll
     for (int sb = 0; sb < 2; ++sb) {
@@ -230,27 +276,34 @@ __global__ __launch_bounds__(Fp8Cfg<D>::NT) void fmha_fwd_fp8_kernel(const Fp8Ar
         const i32x8 ka = {(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
         x[sb] = mfma_fp8_k64(ka, qreg[ds], x[sb]);
       }
-      const bf16x8 xa = as_v8<__bf16>(*(const u32x4 *)(ldsX + (sb * 32 + ql) * XROWB + h * 16));
-      x[sb] = Elem<__bf16>::mfma(xa, bx, x[sb]);
     }
-    // the next tile goes to the other stage while this one is worked on (its last readers passed the barrier
-    // that ended the previous iteration)
-    if (kt + 1 < nkt) {
-      lstore((kt + 1) & 1);
-      if (kt + 2 < nkt) gload(k0 + 2 * BK);
+    if (extra) {
+#pragma unroll
+      for (int sb = 0; sb < 2; ++sb) {
+        const bf16x8 xa = as_v8<__bf16>(*(const u32x4 *)(ldsX + (sb * 32 + ql) * XROWB + h * 16));
+        x[sb] = Elem<__bf16>::mfma(xa, as_v8<__bf16>(u32x4{bx0, bx1, 0, 0}), x[sb]);
+      }
     }
+    stage_next(kt); // while this one is worked on
     // register r of block sb is key k0 + 32 sb + 8 (r / 4) + 4 h + r % 4
     const bool diag = CAUSAL && (k0 + BK - 1 > qt * QT + w * 32);
     const bool want_lse = a.lse != nullptr;
     float psum = 0.f; // unrounded row sum of the tile, only where the LSE is wanted
+    const int own = q - k0 - 4 * h; // causal: the lane's last visible key, in its own order
+    auto hide_later_keys = [&](f32x16 (&v)[2]) {
+#pragma unroll
+      for (int sb = 0; sb < 2; ++sb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          v[sb][r] = sb * 32 + 8 * (r / 4) + r % 4 <= own ? v[sb][r] : NEG_INF;
+          asm volatile("" : "+v"(v[sb][r])); // (a branch: as selects every tile would pay two instructions per element)
+        }
+    };
+    if (diag) hide_later_keys(x);
 #pragma unroll
     for (int sb = 0; sb < 2; ++sb)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        float p = fast_exp2(x[sb][r] * s);
-        if (diag) p = (k0 + sb * 32 + 8 * (r / 4) + 4 * h + r % 4 <= q) ? p : 0.f;
-        x[sb][r] = p;
-      }
+      for (int r = 0; r < 16; ++r) x[sb][r] = fast_exp2(fmaf(x[sb][r], s, -M));
     if (want_lse) {
 #pragma unroll
       for (int sb = 0; sb < 2; ++sb)
@@ -290,17 +343,17 @@ __global__ __launch_bounds__(Fp8Cfg<D>::NT) void fmha_fwd_fp8_kernel(const Fp8Ar
           const i32x8 ka = {(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
           y[sb] = mfma_fp8_k64(ka, qreg[ds], y[sb]);
         }
-        const bf16x8 xa = as_v8<__bf16>(*(const u32x4 *)(ldsX + (sb * 32 + ql) * XROWB + h * 16));
-        y[sb] = Elem<__bf16>::mfma(xa, bx, y[sb]);
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          float v = fmaf(y[sb][r], s, M); // the score in log2 units (plus mask term)
-          if (diag) v = (k0 + sb * 32 + 8 * (r / 4) + 4 * h + r % 4 <= q) ? v : NEG_INF;
-          y[sb][r] = v;
-          mx = fmaxf(mx, v);
+        if (extra) {
+          const bf16x8 xa = as_v8<__bf16>(*(const u32x4 *)(ldsX + (sb * 32 + ql) * XROWB + h * 16));
+          y[sb] = Elem<__bf16>::mfma(xa, as_v8<__bf16>(u32x4{bx0, bx1, 0, 0}), y[sb]);
         }
       }
-      mx = xhalf_max(mx);
+      if (diag) hide_later_keys(y);
+#pragma unroll
+      for (int sb = 0; sb < 2; ++sb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) mx = fmaxf(mx, y[sb][r]);
+      mx = xhalf_max(mx) * s; // the largest score of the tile in log2 units, mask term included
       const bool live = mx > -1e20f; // this tile shows the row a key that is not masked out
       float Mn = M;
       if (need && live) Mn = seen ? fmaxf(M, __builtin_ceilf(mx)) : __builtin_ceilf(mx);
@@ -310,7 +363,7 @@ __global__ __launch_bounds__(Fp8Cfg<D>::NT) void fmha_fwd_fp8_kernel(const Fp8Ar
       for (int sb = 0; sb < 2; ++sb)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          const float p = live ? fast_exp2(y[sb][r] - Mn) : 0.f;
+          const float p = live ? fast_exp2(fmaf(y[sb][r], s, -Mn)) : 0.f;
           y[sb][r] = p;
           psum_new += p;
         }
@@ -331,7 +384,6 @@ __global__ __launch_bounds__(Fp8Cfg<D>::NT) void fmha_fwd_fp8_kernel(const Fp8Ar
         for (int r = 0; r < 16; ++r) oacc[db][r] *= alpha;
       M = Mn;
       seen = seen || (need && live);
-      set_bx();
     }
     l_run += tsum;
     if (want_lse) l_true += xhalf_sum(psum);
@@ -350,6 +402,10 @@ __global__ __launch_bounds__(Fp8Cfg<D>::NT) void fmha_fwd_fp8_kernel(const Fp8Ar
       oacc[db] = mfma_fp8_k64(va, pb, oacc[db]);
     }
     __syncthreads(); // this stage is free again, the next one is complete
+  }
+  for (int kt = nktw; kt < nkt; ++kt) {
+    stage_next(kt);
+    __syncthreads();
   }
 
   // normalise and store: in the accumulator layout lane (q, h) holds head-dim columns 8g + 4h .. +3 of each 32-block
