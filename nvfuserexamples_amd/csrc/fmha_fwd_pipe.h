@@ -235,9 +235,10 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu((QB == 
     }
     // Causal items grow with the query tile.  A workgroup's items are G apart, which is often a
     // multiple of the tiles per head, so the order of the tiles is reversed in every other
-    // round: long and short items then alternate within each workgroup.  (Within a round the
-    // map stays one-to-one, so every item is still visited exactly once.)
-    if (CAUSAL && ((idx / G) & 1) == 0) it.qt = a.nqt - 1 - it.qt;
+    // round: long and short items then alternate within each workgroup.  (The round of the head's
+    // FIRST item decides for all of its tiles: where G is no multiple of the tiles per head some heads
+    // lie in two rounds, and by the item's own round they would get some tiles twice and others never.)
+    if (CAUSAL && ((it.bh * a.nqt / G) & 1) == 0) it.qt = a.nqt - 1 - it.qt;
     // keys this head may see at all: [0, sk) or its valid count (possibly 0: then every key is
     // treated as past the end, which yields O = 0 and LSE = -inf)
     int piece;
