@@ -53,12 +53,12 @@ template <typename K> int set_lds(K kern, int bytes) {
 // arithmetic (BH 256 S 1024: 335 against 343; causal 462 against 429, with dropout 197 against 169 the other way round).
 template <int MASK, bool CAUSAL, int DROP> constexpr bool pipe_built() { return FMHA_TU_D != 256 && MASK != kMaskFull; }
 template <bool CAUSAL> bool pipe_wanted(const BwdArgs &a) { return FMHA_TU_D == 64 || a.sq >= (CAUSAL ? 384 : 128); }
-// dQ of causal heads at head dim 128 where workgroups take pairs of tiles: each of the two passes pays the prologue with all
-// compute units in step, and the pipelined kernel is ahead from about 900 queries on (us, pipelined against phase by phase, at
-// 512 or 768 heads: S 384 153 / 129, S 512 134 / 123, with dropout 143 / 129, S 640 168 / 153, S 768 195 / 186, S 1024
-// 259 / 289; few heads, one tile a workgroup: BH 64 S 512 23.3 / 25.8).
+// dQ of causal heads at head dim 128: a pass pays the prologue with all compute units in step, and the pipelined kernel is
+// ahead from about 900 queries on (us, pipelined against phase by phase, at 512 or 768 heads: S 384 153 / 129, S 512
+// 134 / 123, with dropout 143 / 129, S 640 168 / 153, S 768 195 / 186, S 1024 259 / 289; at few heads the other way round,
+// BH 64 S 512 23.3 / 25.8, but a head's gradients do not depend on how many others there are).
 template <bool CAUSAL> bool pipe_wanted_dq(const BwdArgs &a) {
-  return pipe_wanted<CAUSAL>(a) && !(FMHA_TU_D == 128 && CAUSAL && a.pair && a.sq < 896);
+  return pipe_wanted<CAUSAL>(a) && !(FMHA_TU_D == 128 && CAUSAL && a.sq < 896);
 }
 
 template <typename K> int launch_one(K kern, BwdArgs &a, long long nblk, int threads, int lds, hipStream_t s) {

@@ -53,8 +53,8 @@ def test_pipelined_backward_at_its_edges(bh, sq, sk, d, dtype, pad, causal, p):
 @pytest.mark.parametrize("bh,sq,sk,dtype,pad,p", [(2, 384, 384, "fp16", False, 0.0), (2, 400, 333, "bf16", True, 0.1),
                                                   (1, 895, 900, "fp16", False, 0.1), (1, 896, 896, "fp16", True, 0.0)])
 def test_causal_pairs_at_head_dim_128_in_either_dq_kernel(bh, sq, sk, dtype, pad, p, monkeypatch):
-    """Workgroups with pairs of tiles (as launches of many heads have them) change their dQ kernel at 896 queries; the
-    dK / dV kernel and the delta it reads are the same on both sides."""
+    """The dQ kernel changes at 896 queries (here with pairs of tiles, as launches of many heads have them); the dK / dV
+    kernel and the delta it reads are the same on both sides."""
     monkeypatch.setenv("FMHA_BWD_PAIR", "1")
     capi.lib().fmha_reload_overrides()
     try:
