@@ -24,7 +24,7 @@
 // BH 512 S 512 D 64 with masks whose lengths are spread over [256, 512]: 47.7 -> 36.2 us; without a mask 43.2 -> 37.9 us;
 // BH 32 S 4096 D 128 causal 220 -> 112 us, BH 32 S 2048 D 64 causal 50.4 -> 30.4 us (the key-after-query test of the
 // diagonal tiles used to cost every tile two instructions per element; waves leave out the tiles past their own rows).
-// The registers are held to four waves per SIMD at head dim 64, three where causal.
+// The registers are held to four waves per SIMD at head dim 64, three where causal (a tighter budget spills in the loop).
 // The row sums come out of the matrix pipe too:
 // one more fp8 product of the rounded tile with an operand of ones gives every lane the sum of ITS row's
 // rounded probabilities, so O = sum P~ v / sum P~ is a convex combination of the values (a row with one
