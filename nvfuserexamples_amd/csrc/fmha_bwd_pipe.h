@@ -14,7 +14,8 @@
 //   * Causal: a wave leaves out the tiles on the masked side of its own diagonal, and only the tile on it compares indexes.
 //   * The per-key mask terms (dQ) and the rows (-LSE, -delta) (dK / dV) of the whole head are staged in LDS once, in
 //     segments of 4096 keys / 1024 queries, instead of per tile through registers: a load that the compiler waits for
-//     would also wait for every copy issued ahead of it.
+//     would also wait for every copy issued ahead of it.  (Where there is more than one segment, the second tile of a
+//     causal pair stages its first one again: the other tile's pass has overwritten it.)
 //   * Gradients leave as whole rows (store_acc_rows).
 //
 // Measured against the two-stage, phase-by-phase kernels (us, dQ / dK+dV): BH 64 S 2048 D 64 without dropout
@@ -206,7 +207,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
         to[ks] = *(const u32x4 *)(Ob + (size_t)qc * RW::ss(a.mo) + col);
       }
       const float lse_q = a.lse[(size_t)bh * a.sq + qc];
-      if (MASK == kMaskPerKey && pass == 0) {
+      if (MASK == kMaskPerKey && (pass == 0 || a.sk > C::MSEG)) { // (with more than one segment the first pass leaves a later one)
         const int n = stage_mask(0); // (its loads share the trip to memory)
         const bool trim = a.sk > 128 && a.sk <= C::MSEG && !(a.flags & kBwdFlagNoTrim);
         if (trim && n > 0 && n < skv) skv = n; // a row without any live key keeps all its keys

@@ -62,3 +62,45 @@ def test_causal_pairs_at_head_dim_128_in_either_dq_kernel(bh, sq, sk, dtype, pad
     finally:
         monkeypatch.delenv("FMHA_BWD_PAIR")
         capi.lib().fmha_reload_overrides()
+
+
+@pytest.mark.parametrize("sq,sk,d,dtype,live,p", [
+    (4097, 4097, 64, "fp16", 4097, 0.1),    # the smallest: one key and one query in the second segment
+    (4480, 4480, 64, "fp16", 3000, 0.0),    # every live key in the first segment, the second all hard-masked
+    (4480, 4480, 64, "bf16", 4300, 0.1),
+    (4300, 4128, 96, "fp16", 4128, 0.0),    # run-time rows with columns that do not exist
+    (4224, 4480, 128, "fp16", 2500, 0.1),
+    (4480, 4480, 128, "bf16", 4400, 0.0),
+    (8320, 8320, 64, "fp16", 8200, 0.0),    # three segments (both forms of the launch against each other only)
+])
+def test_causal_pairs_read_the_mask_terms_of_their_own_segment(sq, sk, d, dtype, live, p, monkeypatch):
+    """Pairs of causal query tiles under a per-key mask of more than 4096 keys: the first tile of a pair leaves the mask
+    terms of its last segment behind, the second one starts at key 0 again.  Distinct terms for every key and a hard-masked
+    tail; gradients against the oracle, and the same bits as without pairs (a tile's arithmetic does not depend on them)."""
+    q, k, v, do = make_qkv(1, sq, sk, d, seed=sq + sk, std=0.7, dtype=dtype, with_dout=True)
+    m = -2.0 * torch.rand(1, 1, 1, sk, generator=torch.Generator().manual_seed(3))
+    m[..., live:] = -10000.0
+    m = m.to(TDT[dtype])
+    kw, okw = dict(causal=True), dict(causal=True)
+    if p > 0:
+        kw.update(drop_kind=capi.DROP_PHILOX, p_drop=p, seed=99, offset=12)
+        okw.update(philox=True, p_drop=p, seed=99, offset=12)
+    dev = [t.cuda() for t in (q, k, v, do, m)]
+    o, lse, _, _ = capi.fwd(*dev[:3], mask=dev[4], want_lse=True, **kw)
+    got = {}
+    try:
+        for pair in ("0", "1"):
+            monkeypatch.setenv("FMHA_BWD_PAIR", pair)
+            capi.lib().fmha_reload_overrides()
+            got[pair] = capi.bwd(dev[3], *dev[:3], o, lse, mask=dev[4], **kw)
+            torch.cuda.synchronize()
+    finally:
+        monkeypatch.delenv("FMHA_BWD_PAIR")
+        capi.lib().fmha_reload_overrides()
+    for name, a, b in zip(("dq", "dk", "dv"), got["0"], got["1"]):
+        assert torch.equal(a, b), name
+    if sk > 8192:
+        return
+    ref = oracle.attention(f32(q), f32(k), f32(v), mask=f32(m), dout=f32(do), want=("dq", "dk", "dv"), **okw)
+    for name, t in zip(("dq", "dk", "dv"), got["1"]):
+        assert rel_to_max(f32(t.cpu()), ref[name], floor=1e-2) <= TOL[dtype], name
