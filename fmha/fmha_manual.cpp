@@ -505,8 +505,9 @@ at::Tensor philox_keep_mask_op(const at::Tensor &like, int64_t bh, int64_t sq, i
 }
 
 // Autograd formula of fmha_fwd (the reference registers none: fmha/fmha_manual.cpp:1240-1250, its perf runs
-// are under no_grad): O is differentiable in q, k and v; the row log-sum-exp, the mask and the key counts
-// are not.  Nothing of size S x S is kept for the backward: it recomputes P from the saved LSE and
+// are under no_grad): O is differentiable in q, k and v; the row log-sum-exp is not, and the key counts and the mask receive
+// no gradient (a mask that asks for one still makes O part of the graph, so that a caller may send O backward whichever
+// inputs are frozen).  Nothing of size S x S is kept for the backward: it recomputes P from the saved LSE and
 // regenerates the dropout decisions from the same (seed, offset).
 //
 // A plain graph node with typed members: the generic custom-function wrapper keeps its scalars in a dictionary and looks
@@ -531,7 +532,7 @@ struct FmhaBackward : public torch::autograd::Node {
     if (has_len) n = kv_len.unpack();
     auto [dq, dk, dv] = fmha_bwd(dout, q.unpack(), k.unpack(), v.unpack(), ot, lse.unpack(), m, scale, is_causal, p_drop,
                                  seed, offset, n);
-    torch::autograd::variable_list out(3); // (all three come out of the same two launches)
+    torch::autograd::variable_list out(4); // q, k, v (all three come out of the same two launches), mask (none)
     if (task_should_compute_output(0)) out[0] = std::move(dq);
     if (task_should_compute_output(1)) out[1] = std::move(dk);
     if (task_should_compute_output(2)) out[2] = std::move(dv);
@@ -543,18 +544,20 @@ std::tuple<at::Tensor, at::Tensor> fmha_fwd_autograd(const at::Tensor &q, const 
                                                      const c10::optional<at::Tensor> &mask, double scale,
                                                      bool is_causal, double p_drop, int64_t seed, int64_t offset,
                                                      const c10::optional<at::Tensor> &kv_len) {
-  TORCH_CHECK(!(torch::autograd::isFwGradDefined(q) || torch::autograd::isFwGradDefined(k) || torch::autograd::isFwGradDefined(v)),
+  const at::Tensor amask = mask.has_value() ? *mask : at::Tensor();
+  TORCH_CHECK(!(torch::autograd::isFwGradDefined(q) || torch::autograd::isFwGradDefined(k) || torch::autograd::isFwGradDefined(v) ||
+                torch::autograd::isFwGradDefined(amask)),
               "mha_manual: fmha_fwd has no forward-mode derivative");
   std::shared_ptr<FmhaBackward> node;
-  if (torch::autograd::compute_requires_grad(q, k, v)) {
+  if (torch::autograd::compute_requires_grad(q, k, v, amask)) {
     node = std::shared_ptr<FmhaBackward>(new FmhaBackward(), torch::autograd::deleteNode);
-    node->set_next_edges(torch::autograd::collect_next_edges(q, k, v));
+    node->set_next_edges(torch::autograd::collect_next_edges(q, k, v, amask));
     node->q = torch::autograd::SavedVariable(q, false);
     node->k = torch::autograd::SavedVariable(k, false);
     node->v = torch::autograd::SavedVariable(v, false);
-    if (mask.has_value() && mask->defined()) {
+    if (amask.defined()) {
       node->has_mask = true;
-      node->mask = torch::autograd::SavedVariable(*mask, false);
+      node->mask = torch::autograd::SavedVariable(amask, false);
     }
     if (kv_len.has_value() && kv_len->defined()) {
       node->has_len = true;

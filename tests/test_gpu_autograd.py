@@ -57,3 +57,30 @@ def test_the_operator_itself_is_differentiable():
     with torch.no_grad():
         o2, _ = ops.fmha_fwd(qa, ka, va, None, 0.0, True, 0.1, 3, 1)
     assert not o2.requires_grad and torch.equal(o2, o.detach())
+
+
+def test_a_mask_that_asks_for_a_gradient_joins_the_graph_and_receives_none():
+    """Whichever of q, k, v and the mask ask for a gradient, O may be sent backward; the mask's stays None.  A forward-mode
+    tangent on any of the four is refused."""
+    import torch.autograd.forward_ad as fwad
+    from nvfuserexamples_amd import load_ops
+    ops = load_ops()
+    bh, s, d = 4, 160, 64
+    q, k, v, do = (t.cuda() for t in make_qkv(bh, s, s, d, seed=9, with_dout=True))
+    m = pad_mask(2, s, s // 2, s).half().cuda()
+    ref = [t.clone().requires_grad_(True) for t in (q, k, v)]
+    ops.fmha_fwd(*ref, m, 0.0, False, 0.0, 0, 0)[0].backward(do)
+    for want in ((0, 0, 0, 1), (1, 0, 0, 1), (0, 1, 1, 1), (0, 0, 1, 0)):
+        a = [t.clone().requires_grad_(bool(w)) for t, w in zip((q, k, v, m), want)]
+        o, lse = ops.fmha_fwd(*a, 0.0, False, 0.0, 0, 0)
+        assert o.requires_grad and not lse.requires_grad
+        o.backward(do)
+        for t, w, r in zip(a[:3], want, ref):
+            assert torch.equal(t.grad, r.grad) if w else t.grad is None
+        assert a[3].grad is None
+    for i in range(4):
+        with fwad.dual_level():
+            a = [q, k, v, m]
+            a[i] = fwad.make_dual(a[i], torch.ones_like(a[i]))
+            with pytest.raises(RuntimeError):
+                ops.fmha_fwd(*a, 0.0, False, 0.0, 0, 0)
