@@ -413,15 +413,17 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
       }
     };
     // top of the iteration of tile kt: tile kt + 1 has landed, tile kt + 3 goes on its way
-    auto turn = [&](int kt) -> uint32_t {
+    // (`No`: for a wave's last tile, behind which nothing is read: the head may have no mask terms there, nor LDS for them)
+    auto turn = [&](auto next_tag, int kt) -> uint32_t {
       if (MASK == kMaskPerKey && ((kt + 1) * BT & (C::MSEG - 1)) == 0 && kt + 1 < nkt) stage_mask((kt + 1) * BT); // (4096 keys on)
-      const uint32_t hl = hl_of(kt + 1);
+      uint32_t hl = 0u;
+      if constexpr (decltype(next_tag)::value) hl = hl_of(kt + 1);
       bwd_vm_wait<(NST - 3) * VPT>();
       bwd_lds_barrier(); // ... everybody's part of it, and tile kt - 1 is no longer read
       return hl;
     };
     auto mid = [&](int kt, const f32x16 &xc, const f32x16 &gc, const uint32_t (&wc)[4], f32x16 &xn, f32x16 &gn, uint32_t (&wn)[4]) {
-      const uint32_t hl = turn(kt);
+      const uint32_t hl = turn(Yes{}, kt);
       step(Yes{}, No{}, kt, hl, xc, gc, wc, xn, gn, wn);
     };
     int kt = 0;
@@ -440,10 +442,10 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
       mid(kt + 1, xB, gB, wdB, xA, gA, wdA);
     }
     {
-      turn(kt);
+      turn(No{}, kt);
       step(No{}, std::integral_constant<bool, CAUSAL || !XS>{}, kt, 0u, xA, gA, wdA, xB, gB, wdB);
       for (++kt; kt < nkt; ++kt) {
-        turn(kt);
+        turn(No{}, kt);
         dma_kv(kt + NST - 1);
       } // (causal: tiles that only later waves of the workgroup need)
     }
