@@ -46,17 +46,26 @@ template <typename K> int set_lds(K kern, int bytes) {
 }
 
 // The pipelined kernels (fmha_bwd_pipe.hip) take everything but full mask tensors and head dim 256 -- at head dim 128 from
-// a number of queries on: their prologue costs more, and a causal head's streams are cut short by its diagonal (us,
-// pipelined against phase by phase, causal: S 128 110 / 95, S 256 121 / 116, S 384 130 / 129, S 512 153 / 163;
-// dropout: S 61 116 / 110, S 128 99 / 101, S 256 121 / 130).  And one exception: dK / dV at head dim 128 without causal
-// mask and dropout, where 32-row tiles at two waves per SIMD overlap one workgroup's start and stores with another's
-// arithmetic (BH 256 S 1024: 335 against 343; causal 462 against 429, with dropout 197 against 169 the other way round).
+// a number of queries on, because their prologue costs more and a causal head's streams are cut short by its diagonal.
+// Kernel times, us, pipelined / phase by phase, 512 heads, D 128, fp16, S queries and keys:
+//   dQ, no causal mask     S 61 13 / 11, S 128 20 / 21, S 256 58 / 62, S 512 131 / 131, S 1024 402 / 418
+//     with dropout         S 61 15 / 13, S 128 22 / 22, S 256 59 / 59, S 512 147 / 152, S 1024 455 / 471
+//   dK+dV with dropout     S 61 19 / 18, S 128 32 / 31, S 192 60 / 67, S 256 75 / 84, S 1024 774 / 846   (line at 128)
+//   dK+dV, causal          S 128 33 / 30, S 256 73 / 74, S 384 127 / 127, S 512 163 / 166, S 1024 441 / 494
+//     with dropout         S 128 36 / 33, S 256 82 / 86, S 384 144 / 153, S 512 174 / 192, S 1024 488 / 569
+// (causal: without dropout level from 256 to 384, behind below and ahead above; the line of both is 384).
+// One exception: dK / dV at head dim 128 without causal mask and dropout stays on 32-row tiles at two waves per SIMD, which
+// overlap one workgroup's start and stores with another's arithmetic.  The two differ by what a box does to either: BH 256
+// S 1024 343 / 335 on one, 347 / 359-369 on another, there also S 512 206 / 211-215 and BH 64 S 2048 278 / 281-285.
 template <int MASK, bool CAUSAL, int DROP> constexpr bool pipe_built() { return FMHA_TU_D != 256 && MASK != kMaskFull; }
 template <bool CAUSAL> bool pipe_wanted(const BwdArgs &a) { return FMHA_TU_D == 64 || a.sq >= (CAUSAL ? 384 : 128); }
-// dQ of causal heads at head dim 128: a pass pays the prologue with all compute units in step, and the pipelined kernel is
-// ahead from about 900 queries on (us, pipelined against phase by phase, at 512 or 768 heads: S 384 153 / 129, S 512
-// 134 / 123, with dropout 143 / 129, S 640 168 / 153, S 768 195 / 186, S 1024 259 / 289; at few heads the other way round,
-// BH 64 S 512 23.3 / 25.8, but a head's gradients do not depend on how many others there are).
+// dQ of causal heads at head dim 128 has a line of its own: a pass pays the prologue with all compute units in step, and
+// workgroups take pairs of short streams.  Same measurement (us, pipelined / phase by phase, 512 heads, fp16, in brackets
+// bf16): S 384 107 / 93, S 512 134 / 126 (144 / 117), S 640 170 / 161, S 768 198 / 198 (204 / 195), S 896 257 / 256
+// (265 / 254), S 1024 292 / 303 (293 / 289), S 1536 534 / 571 (529 / 558); with dropout S 512 142 / 129, S 768 230 / 216,
+// S 896 300 / 292, S 1024 336 / 335; BH 256 S 2048 438 / 484, with dropout BH 128 S 2048 271 / 281: level to 4 % either way
+// from 896 to 1024, ahead beyond.  (At few heads ahead earlier, BH 64 S 512 23 / 25, but a head's gradients do not depend
+// on how many others there are.)
 template <bool CAUSAL> bool pipe_wanted_dq(const BwdArgs &a) {
   return pipe_wanted<CAUSAL>(a) && !(FMHA_TU_D == 128 && CAUSAL && a.sq < 896);
 }
