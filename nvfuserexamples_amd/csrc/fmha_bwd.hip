@@ -55,7 +55,7 @@ template <typename K> int set_lds(K kern, int bytes) {
 //     with dropout         S 128 36 / 33, S 256 82 / 86, S 384 144 / 153, S 512 174 / 192, S 1024 488 / 569
 // (causal: without dropout level from 256 to 384, behind below and ahead above; the line of both is 384).
 // One exception: dK / dV at head dim 128 without causal mask and dropout stays on 32-row tiles at two waves per SIMD, which
-// overlap one workgroup's start and stores with another's arithmetic.  The two differ by what a box does to either: BH 256
+// overlap one workgroup's start and stores with another's arithmetic.  The two differ by what a card makes of either: BH 256
 // S 1024 343 / 335 on one, 347 / 359-369 on another, there also S 512 206 / 211-215 and BH 64 S 2048 278 / 281-285.
 template <int MASK, bool CAUSAL, int DROP> constexpr bool pipe_built() { return FMHA_TU_D != 256 && MASK != kMaskFull; }
 template <bool CAUSAL> bool pipe_wanted(const BwdArgs &a) { return FMHA_TU_D == 64 || a.sq >= (CAUSAL ? 384 : 128); }

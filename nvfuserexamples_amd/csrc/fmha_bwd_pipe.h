@@ -18,7 +18,7 @@
 //     causal pair stages its first one again: the other tile's pass has overwritten it.)
 //   * Gradients leave as whole rows (store_acc_rows).
 //
-// Measured against the two-stage, phase-by-phase kernels on one box (kernel times, us, dQ / dK+dV, fp16 unless said): BH 64
+// Measured against the two-stage, phase-by-phase kernels on one card (kernel times, us, dQ / dK+dV, fp16 unless said): BH 64
 // S 2048 D 64 without dropout 126.9 / 159.3 -> 116.6 / 153.1, with dropout 140.0 / 194.5 -> 135.9 / 174.7; BH 192 S 1024 D 64
 // causal 84.3 / 98.2 -> 66.4 / 81.9; BH 32 S 4096 D 128 causal 280 / 335 -> 225 / 304 (bf16 272 / 329 -> 214 / 275); BH 512
 // S 1024 D 128 causal bf16 285 / 455 -> 293 / 413 (the lines between the two at head dim 128: fmha_bwd.hip).

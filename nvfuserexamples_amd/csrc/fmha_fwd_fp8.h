@@ -21,8 +21,8 @@
 // (three bf16 pieces: exact to fp32); tiles whose keys are all there and unmasked -- most of a padded batch --
 // go without.  Key tiles of nothing but hard-masked keys at the end of a mask row are not visited where their
 // weights are zero whatever the inputs (Fp8Args::trim).
-// BH 512 S 512 D 64, before and now on one box: with masks whose lengths are spread over [256, 512] 45.5 -> 35.2 us, without a
-// mask 39.9 -> 34.1 us (other boxes: 47.7-48.8 -> 36.2-38.1 and 43.2 -> 37.9);
+// BH 512 S 512 D 64, before and now on one card: with masks whose lengths are spread over [256, 512] 45.5 -> 35.2 us, without a
+// mask 39.9 -> 34.1 us (other cards: 47.7-48.8 -> 36.2-38.1 and 43.2 -> 37.9);
 // BH 32 S 4096 D 128 causal 211 -> 108 us, BH 32 S 2048 D 64 causal 48.1 -> 28.5 us (the key-after-query test of the
 // diagonal tiles used to cost every tile two instructions per element; waves leave out the tiles past their own rows).
 // The registers are held to four waves per SIMD at head dim 64, three where causal (a tighter budget spills in the loop).
