@@ -46,19 +46,17 @@ template <typename K> int set_lds(K kern, int bytes) {
 }
 
 // The pipelined kernels (fmha_bwd_pipe.hip) take everything but full mask tensors and head dim 256 -- at head dim 128 from
-// a number of queries on, because their prologue costs more and a causal head's streams are cut short by its diagonal.
+// a number of queries on, because their prologue costs more and a causal head's dQ streams are cut short by its diagonal.
 // Kernel times, us, pipelined / phase by phase, 512 heads, D 128, fp16, S queries and keys:
 //   dQ, no causal mask     S 61 13 / 11, S 128 20 / 21, S 256 58 / 62, S 512 131 / 131, S 1024 402 / 418
 //     with dropout         S 61 15 / 13, S 128 22 / 22, S 256 59 / 59, S 512 147 / 152, S 1024 455 / 471
-//   dK+dV with dropout     S 61 19 / 18, S 128 32 / 31, S 192 60 / 67, S 256 75 / 84, S 1024 774 / 846   (line at 128)
-//   dK+dV, causal          S 128 33 / 30, S 256 73 / 74, S 384 127 / 127, S 512 163 / 166, S 1024 441 / 494
-//     with dropout         S 128 36 / 33, S 256 82 / 86, S 384 144 / 153, S 512 174 / 192, S 1024 488 / 569
-// (causal: without dropout level from 256 to 384, behind below and ahead above; the line of both is 384).
-// One exception: dK / dV at head dim 128 without causal mask and dropout stays on 32-row tiles at two waves per SIMD, which
-// overlap one workgroup's start and stores with another's arithmetic.  The two differ by what a card makes of either: BH 256
-// S 1024 343 / 335 on one, 347 / 359-369 on another, there also S 512 206 / 211-215 and BH 64 S 2048 278 / 281-285.
+//   dK+dV (persistent)     S 61 16 / 13, S 128 23 / 23, S 192 44 / 48, S 256 56 / 62, 2048 heads S 128 80 / 104
+//     with dropout         S 61 19 / 17, S 128 27 / 31
+//   dK+dV, causal          S 128 27 / 30, S 192 43 / 56, S 256 55 / 71, 2048 heads S 128 with dropout 101 / 126
+//   dK+dV of few heads (one round of workgroups, the plain pipelined kernel): 64 heads S 200 12 / 17, causal 14 / 16
+// The line is 128 queries.
 template <int MASK, bool CAUSAL, int DROP> constexpr bool pipe_built() { return FMHA_TU_D != 256 && MASK != kMaskFull; }
-template <bool CAUSAL> bool pipe_wanted(const BwdArgs &a) { return FMHA_TU_D == 64 || a.sq >= (CAUSAL ? 384 : 128); }
+static inline bool pipe_wanted(const BwdArgs &a) { return FMHA_TU_D == 64 || a.sq >= 128; }
 // dQ of causal heads at head dim 128 has a line of its own: a pass pays the prologue with all compute units in step, and
 // workgroups take pairs of short streams.  Same measurement (us, pipelined / phase by phase, 512 heads, fp16, in brackets
 // bf16): S 384 107 / 93, S 512 134 / 126 (144 / 117), S 640 170 / 161, S 768 198 / 198 (204 / 195), S 896 257 / 256
@@ -67,7 +65,7 @@ template <bool CAUSAL> bool pipe_wanted(const BwdArgs &a) { return FMHA_TU_D == 
 // from 896 to 1024, ahead beyond.  (At few heads ahead earlier, BH 64 S 512 23 / 25, but a head's gradients do not depend
 // on how many others there are.)
 template <bool CAUSAL> bool pipe_wanted_dq(const BwdArgs &a) {
-  return pipe_wanted<CAUSAL>(a) && !(FMHA_TU_D == 128 && CAUSAL && a.sq < 896);
+  return pipe_wanted(a) && !(FMHA_TU_D == 128 && CAUSAL && a.sq < 896);
 }
 
 template <typename K> int launch_one(K kern, BwdArgs &a, long long nblk, int threads, int lds, hipStream_t s) {
@@ -102,9 +100,9 @@ template <int MASK, bool CAUSAL, int DROP> int launch_dkdv(BwdArgs &a, const Bwd
   static const int attr = set_lds(kern, Cfg::LDS_BYTES);
   return attr ? 2 : launch_one(kern, a, nblk, Cfg::NW * 64, Cfg::LDS_BYTES, s);
 #else
-  constexpr bool kPipe = pipe_built<MASK, CAUSAL, DROP>() && !bwd_dkdv_small_tiles<FMHA_TU_D, CAUSAL, DROP>();
+  constexpr bool kPipe = pipe_built<MASK, CAUSAL, DROP>();
   if constexpr (kPipe) {
-    if (pipe_wanted<CAUSAL>(a)) return FMHA_PIPE_NAME(FMHA_TU_TNAME, FMHA_TU_D)(a, v, true, nblk, s);
+    if (pipe_wanted(a)) return FMHA_PIPE_NAME(FMHA_TU_TNAME, FMHA_TU_D)(a, v, true, nblk, s);
   }
   if constexpr (!(kPipe && FMHA_TU_D == 64)) {
     using Cfg = BwdCfg<FMHA_TU_D, bwd_dkdv_tile_rows<FMHA_TU_D, CAUSAL, DROP>()>;
