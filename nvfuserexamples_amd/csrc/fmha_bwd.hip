@@ -101,8 +101,12 @@ template <int MASK, bool CAUSAL, int DROP> int launch_dkdv(BwdArgs &a, const Bwd
   return attr ? 2 : launch_one(kern, a, nblk, Cfg::NW * 64, Cfg::LDS_BYTES, s);
 #else
   constexpr bool kPipe = pipe_built<MASK, CAUSAL, DROP>();
+  // One exception: under a mask or key counts, without causal mask and dropout, dK / dV at head dim 128 stays on 32-row tiles at
+  // two waves per SIMD, which overlap one workgroup's start and stores with another's arithmetic as the persistent kernel
+  // does where there is neither (plain pipelined kernel / this: BH 256 S 1024 343 / 335 us on one card, 347 / 359-369 on another).
+  constexpr bool kTwoWaves = bwd_dkdv_small_tiles<FMHA_TU_D, CAUSAL, DROP>();
   if constexpr (kPipe) {
-    if (pipe_wanted(a)) return FMHA_PIPE_NAME(FMHA_TU_TNAME, FMHA_TU_D)(a, v, true, nblk, s);
+    if (pipe_wanted(a) && !(kTwoWaves && (MASK != kMaskNone || a.kv_len))) return FMHA_PIPE_NAME(FMHA_TU_TNAME, FMHA_TU_D)(a, v, true, nblk, s);
   }
   if constexpr (!(kPipe && FMHA_TU_D == 64)) {
     using Cfg = BwdCfg<FMHA_TU_D, bwd_dkdv_tile_rows<FMHA_TU_D, CAUSAL, DROP>()>;

@@ -1,4 +1,4 @@
-// Persistent dK / dV kernel for head dim 128 (no mask or a per-key mask; full mask tensors stay on fmha_bwd_kernel.h).
+// Persistent dK / dV kernel for head dim 128 without mask and key counts (with either: fmha_bwd_pipe.h and fmha_bwd_kernel.h).
 // Mathematics, register layouts and the hand-ordered stream of an iteration are those of fmha_bwd_dkdv_pipe_kernel
 // (fmha_bwd_pipe.h).  At head dim 128 a wave's accumulators and operands take both halves of the register file, so there is one
 // wave per SIMD and one workgroup per compute unit: nothing ran while a workgroup fetched its K and V rows and first tiles, nor
@@ -8,13 +8,14 @@
 //   * The stream of query tiles runs on into the next item; its K and V rows and its rows (LSE, delta) are copied into LDS of
 //     their own while this item is computed.  Between two items a wave turns what has landed into registers and hands the last
 //     item's gradients, whole rows through its own part of that LDS, to stores that nobody waits for before two tiles later.
-//   * Items without work (hidden by a mask's tail or the key counts) get their zeros on the way and take no turn in the list.
+//   * The list is dealt in advance and evens out causal tiles.  A mask's hidden tiles it cannot know: with masks it measured 2 to
+//     6 % behind the plain kernels, whose workgroups come and go as there is work.
 //   * At head dim 64 there are two workgroups per compute unit, and one's start and stores run under the other's products
 //     already; the same kernel there measured level (BH 512 S 512) to 8 % behind (causal), so it is built for 128 only.
 //
 // Kernel times on one card, us, plain pipelined kernel (without causal mask and dropout: phase by phase) -> this one: BH 512
-// S 1024 causal bf16 406 -> 374, BH 300 S 400 causal 91 -> 65, BH 64 S 1500 causal 110 -> 94, BH 256 S 1024 341 -> 293, BH 32
-// S 4096 507 -> 466, causal 262 -> 256.  What bounds it now: at long sequences the board's power (BH 32 S 4096 causal on
+// S 1024 causal bf16 415 -> 369, BH 300 S 400 causal 91 -> 62, BH 64 S 1500 causal 110 -> 91, BH 256 S 1024 341 -> 291, BH 32
+// S 4096 507 -> 466, causal 265 -> 253.  What bounds it now: at long sequences the board's power (BH 32 S 4096 causal on
 // zeros 231); at short ones the turn from item to item, about 5 us of which 2 are the gradients' way through LDS and 1.5 the
 // issue of the next item's copies behind their stores.  (Spread over the first turns those copies cost more than they hid:
 // 291 -> 303 us at BH 256 S 1024.)
@@ -45,7 +46,7 @@ FMHA_DEV void dma_global_to_lds_b32(const void *uniform_base, uint32_t lane_offs
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds_wave_base), "v"(lane_offset), "s"(ub) : "memory");
 }
 
-template <typename T, int D, int NW, int MASK, bool CAUSAL, int DROP, bool STRIDED>
+template <typename T, int D, int NW, bool CAUSAL, int DROP, bool STRIDED>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(1, 1))) void fmha_bwd_dkdv_persist_kernel(const BwdArgs a) {
   using RW = Rows<STRIDED, D>;
   using E = Elem<T>;
@@ -55,7 +56,6 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(1, 1)))
   constexpr int NT = NW * 64, KT = NW * 32;
   constexpr float NEG_INF = -__builtin_inff();
   constexpr float BIGNEG = -60000.f;
-  static_assert(MASK != kMaskFull, "full mask tensors: fmha_bwd_dkdv_kernel");
   static_assert(NW == C::NW && RowStore<D>::BYTES <= 2 * TILEB, "a wave's K and V rows share their LDS with its output rows");
   static_assert(KT / BT == 4 && NST == 4, "the counts of copies in flight below");
 
@@ -64,7 +64,6 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(1, 1)))
   u32x4 *ldsX = (u32x4 *)(lds + C::OFF_Q); // per query of the segment: (-L_hi, -L_lo, 1, 1, -delta_hi, -delta_lo, 0, 0)
   float *ldsRaw = (float *)(ldsX + nseg);  // LSE, then delta of the segment that comes next
   float *ldsD = ldsRaw + 2 * nseg;         // -delta (dropout)
-  int *ldsR = (int *)ldsX;                 // (between two items only, when no extra-step row is live)
 
   const int tid = threadIdx.x;
   const int w = tid >> 6, l = tid & 63, kl = l & 31, h = l >> 5;
@@ -72,49 +71,29 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(1, 1)))
   char *ldsKV = lds + C::OFF_KV + ws * 2 * TILEB; // this wave's own part
 
   // ---- schedule: in round r this workgroup takes unit r * G + lb, a key tile or a causal pair of them.  Workgroups of one XCD
-  // work on a contiguous run of units at a time, so a head's Q and dO rows are read by neighbours.
+  // (every eighth one) work on neighbouring units, so a head's Q and dO rows are read through one L2.
   const int G = gridDim.x;
+  const bool paired = CAUSAL && a.pair, by_length = CAUSAL && !paired;
   int lb = blockIdx.x;
-  if ((G & 7) == 0) lb = (lb & 7) * (G >> 3) + (lb >> 3);
-  const bool paired = CAUSAL && a.pair;
+  if (!by_length && (G & 7) == 0) lb = (lb & 7) * (G >> 3) + (lb >> 3);
   const int npair = paired ? (a.ntile + 1) / 2 : a.ntile;
   const int nunit = a.bh * npair;
   const int nqt = (a.sq + BT - 1) / BT;
   int base = 0, pass = 0; // of the item that is looked at next: its round's first unit, and which tile of a pair
-  auto unit_of = [&]() -> int { // causal without pairs: the order turns from round to round, see locate
-    return base + (CAUSAL && !paired && (base / G & 1) ? G - 1 - lb : lb);
-  };
+  // Causal without pairs (few heads): the longest tiles of all heads come first, and the order of the workgroups turns from
+  // round to round, so that who had a long one gets a short one next.  (With a multiple of eight heads the tiles of one stay
+  // on its XCD.)
+  auto unit_of = [&]() -> int { return base + (by_length && (base / G & 1) ? G - 1 - lb : lb); };
   auto locate = [&](int &bh, int &kt) {
-    const int unit = unit_of();
-    if (CAUSAL && !paired) {
-      // few heads: the longest tiles of all heads first, and who had a long one gets a short one next; as many tiles of a head
-      // side by side as a round has room for
-      const int n = a.bh * 2 <= G ? (G / a.bh < a.ntile ? G / a.bh : a.ntile) : 1;
-      const int g = unit / (a.bh * n), r = unit - g * (a.bh * n);
-      const int wd = n < a.ntile - g * n ? n : a.ntile - g * n;
-      bh = r / wd;
-      kt = g * n + r - bh * wd;
-    } else {
-      bh = unit / npair;
-      kt = unit - bh * npair;
-      if (paired) {
-        if (pass) kt = a.ntile - 1 - kt;
-      } else {
-        // A workgroup's units are G apart, often a multiple of the tiles per head: without a turn it would get the same tile of
-        // every head, the hidden last one of a padded batch for one.  (The round of the head's first unit decides for all
-        // of its tiles.)
-        kt += bh * npair / G % a.ntile;
-        if (kt >= a.ntile) kt -= a.ntile;
-      }
-    }
+    const int unit = unit_of(), n = by_length ? a.bh : npair, hi = unit / n, lo = unit - hi * n;
+    bh = by_length ? lo : hi;
+    kt = by_length ? hi : lo;
+    if (paired && pass) kt = a.ntile - 1 - kt;
   };
 
-  MaskTail<T, NT> tail;
-  int live_keys = a.sk, tail_row = -1; // keys up to the last one that mask row tail_row does not hide
   int nbh = 0, nkt = 0;                // the next item
   bool more = false;
-  // -> (nbh, nkt, more).  Key tiles without any work (hidden by the mask's tail or the key counts, or behind every query)
-  // get their zeros on the way.  Uses ldsR where there is a per-key mask (barriers inside).
+  // -> (nbh, nkt, more).  Causal key tiles behind every query get their zeros on the way.
   auto seek = [&]() {
     more = false;
     for (; base < nunit;) {
@@ -128,16 +107,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(1, 1)))
         pass = 0;
         base += G;
       }
-      const int skv = bwd_valid_keys(a, nbh);
-      if (MASK == kMaskPerKey) {
-        const int row = nbh / a.mask_div;
-        if (row != tail_row) {
-          tail.issue(a, (const T *)a.mask + (size_t)row * a.mask_sb, tid);
-          live_keys = tail.finish(a, ldsR, tid);
-          tail_row = row;
-        }
-      }
-      if (nkt * KT < (live_keys < skv ? live_keys : skv) && !(CAUSAL && nkt * KT >= nqt * BT)) {
+      if (!CAUSAL || nkt * KT < nqt * BT) {
         more = true;
         return;
       }
@@ -236,21 +206,9 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(1, 1)))
     copy_raw(bh, first_seg(kt));
   };
 
-  if (unit_of() < nunit) { // the first item's copies run while its mask row is looked at
-    int bh0, kt0;
-    locate(bh0, kt0);
-    start_item(bh0, kt0);
-    seek();
-    if (more && (nbh != bh0 || nkt != kt0)) {
-      bwd_vm_wait<0>();
-      bwd_lds_barrier();
-      start_item(nbh, nkt);
-    }
-  }
-  if (!more) {
-    bwd_vm_wait<0>();
-    return;
-  }
+  seek();
+  if (!more) return;
+  start_item(nbh, nkt);
 
   f32x16 dk[DB], dv[DB];
 #pragma unroll
@@ -279,9 +237,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(1, 1)))
     const int qt0 = first_tile(ktile);
     const int nj = nqt - qt0;             // query tiles it walks
     const int ntl = nj < 3 ? 3 : nj;      // turns it takes: at least three, so that the stream looks one item ahead at most
-    T mraw = (T)0.f;
-    if (MASK == kMaskPerKey) mraw = ((const T *)a.mask)[(size_t)(bh / a.mask_div) * a.mask_sb + (key < a.sk ? key : a.sk - 1)];
-    if (MASK != kMaskPerKey) seek();
+    seek();
     bwd_vm_wait<0>();
     bwd_lds_barrier(); // tiles 0 .. 2, the K and V rows and the raw rows are there, and nobody reads the last item's any more
 
@@ -299,9 +255,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(1, 1)))
           vreg[ks][j] = DROP == 1 ? (T)((float)vraw[j] * a.drop_scale) : vraw[j];
         }
       }
-      float mk = 0.f;
-      if (MASK == kMaskPerKey) mk = fmaf((float)mraw, a.mask_a, a.mask_b);
-      if (key >= bwd_valid_keys(a, bh)) mk = BIGNEG; // keys past the valid ones: their dK, dV rows are zero
+      const float mk = key < a.sk ? 0.f : BIGNEG;
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         bxs[j] = (T)0.f;
@@ -318,7 +272,6 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(1, 1)))
         bxd[5] = (T)1.f;
       }
     }
-    if (MASK == kMaskPerKey) seek(); // (reads the next item's mask row through ldsR)
     stage_rows(first_seg(ktile));
     if (pbh >= 0) { // the previous item's gradients leave under this one's products
       store_item();
@@ -377,6 +330,8 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(1, 1)))
       next_copy();
       const uint32_t dst = dst_of(tj + NST - 1);
       const int q0 = (qt0 + tj) * BT;
+      DropCtx dctx = a.drop; // (the ten rounds' keys are formed where they are used: kept for the whole kernel they would not fit)
+      if (DROP == 1) asm volatile("" : "+s"(dctx.seed_lo), "+s"(dctx.seed_hi));
       auto fetch = [&](int j) -> v8 {
         if (j < NA) return panel_read_rows<T, BT>(ldsN + (j & 1) * TILEB, pl, 0, j >> 1);
         const int i = j - NA; // dO^T and Q^T alternate
@@ -415,8 +370,8 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(1, 1)))
         }
       };
       auto philox = [&](int s) {
-        if (s == 0) ph.start(a.drop, (uint32_t)bh, (uint32_t)((q0 + BT) >> 2) + (uint32_t)h + 2u * ((uint32_t)l & 3u), (uint32_t)key >> 2);
-        else if (s <= 10) ph.round(a.drop, s - 1);
+        if (s == 0) ph.start(dctx, (uint32_t)bh, (uint32_t)((q0 + BT) >> 2) + (uint32_t)h + 2u * ((uint32_t)l & 3u), (uint32_t)key >> 2);
+        else if (s <= 10) ph.round(dctx, s - 1);
         else {
           const int t = s - 11;
           const uint32_t a1 = __builtin_amdgcn_perm(quad_perm<0xB1>(ph.c[t]), ph.c[t], sel1);

@@ -31,25 +31,28 @@ template <int MASK, bool CAUSAL, int DROP> int launch(const BwdArgs &a, bool dkd
   if (nblk > 0x7fffffffLL) return 2;
   if (dkdv) {
 #if FMHA_TU_D == 128
-    // More than one round of workgroups: persistent ones, as many as the device keeps resident (by the current device at the
-    // first call).  A single round has nothing to run ahead of, and the plain kernel starts sooner: 16 heads, S 1024 causal
-    // 33.6 us persistent, 31.7 plain, with dropout instead of the causal mask 38.4 / 36.4.
-    using PCfg = BwdPersistCfg<FMHA_TU_D>;
-    static_assert(PCfg::MAX_LDS <= 160 * 1024, "does not fit the LDS of a compute unit");
-    auto persist = fmha_bwd_dkdv_persist_kernel<FMHA_TU_T, FMHA_TU_D, kNW, MASK, CAUSAL, DROP, kStrided>;
-    static const int resident = [&]() -> int {
-      const void *f = reinterpret_cast<const void *>(persist);
-      int dev = 0, cus = 0, per_cu = 0;
-      if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, PCfg::MAX_LDS) != hipSuccess || hipGetDevice(&dev) != hipSuccess ||
-          hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-          hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, f, kNW * 64, PCfg::MAX_LDS) != hipSuccess || cus < 1 || per_cu < 1)
-        return -1;
-      return cus * per_cu;
-    }();
-    if (resident < 0) return 2;
-    if (nblk > resident) {
-      hipLaunchKernelGGL(persist, dim3((unsigned)resident), dim3(kNW * 64), PCfg::lds_bytes(DROP, a.sq), s, a);
-      return hipGetLastError() == hipSuccess ? 0 : 2;
+    if constexpr (MASK == kMaskNone) {
+      // From one and a half rounds of workgroups on: persistent ones, as many as the device keeps resident (by the current
+      // device at the first call).  A single round has nothing to run ahead of, and the plain kernel starts sooner: 16 heads,
+      // S 1024 causal 33.6 us persistent, 31.7 plain, with dropout instead of the causal mask 38.4 / 36.4; 1.2 rounds, the few
+      // second ones short (12 heads, S 3232 causal, head dim 80) 94 / 87; 2.3 rounds (32 heads, S 1921 causal) 77 / 97.
+      using PCfg = BwdPersistCfg<FMHA_TU_D>;
+      static_assert(PCfg::MAX_LDS <= 160 * 1024, "does not fit the LDS of a compute unit");
+      auto persist = fmha_bwd_dkdv_persist_kernel<FMHA_TU_T, FMHA_TU_D, kNW, CAUSAL, DROP, kStrided>;
+      static const int resident = [&]() -> int {
+        const void *f = reinterpret_cast<const void *>(persist);
+        int dev = 0, cus = 0, per_cu = 0;
+        if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, PCfg::MAX_LDS) != hipSuccess || hipGetDevice(&dev) != hipSuccess ||
+            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+            hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, f, kNW * 64, PCfg::MAX_LDS) != hipSuccess || cus < 1 || per_cu < 1)
+          return -1;
+        return cus * per_cu;
+      }();
+      if (resident < 0) return 2;
+      if (2 * nblk >= 3LL * resident && !a.kv_len) {
+        hipLaunchKernelGGL(persist, dim3((unsigned)resident), dim3(kNW * 64), PCfg::lds_bytes(DROP, a.sq), s, a);
+        return hipGetLastError() == hipSuccess ? 0 : 2;
+      }
     }
 #endif
     auto kern = fmha_bwd_dkdv_pipe_kernel<FMHA_TU_T, FMHA_TU_D, kNW, MASK, CAUSAL, DROP, kStrided>;
