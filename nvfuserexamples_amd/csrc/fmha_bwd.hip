@@ -31,6 +31,7 @@
 #endif
 #define FMHA_NAME(t, d) FMHA_CAT3(bwd_dispatch_, t, d)
 #define FMHA_PIPE_NAME(t, d) FMHA_CAT3(bwd_pipe_launch_, t, d)
+#define FMHA_ONE_NAME(t, d) FMHA_CAT3(bwd_one_launch_, t, d)
 
 namespace fmha {
 namespace {
@@ -170,7 +171,16 @@ template <int MASK, bool CAUSAL> int by_drop(BwdArgs &a, const BwdVariant &v, hi
 int FMHA_NAME(FMHA_TU_TNAME, FMHA_TU_D)(BwdArgs &a, const BwdVariant &v, hipStream_t s) {
 #if FMHA_TU_SHORT
   if (v.short_seq) {
+    // Beyond 128 rows a launch of more heads than the device holds at once goes to the one-pass kernel, which forms the scores
+    // once and has the next head's rows on their way (us, one-pass / this kernel, S 256 BH 300 38.1 / 41.5, S 130 BH 300 with
+    // dropout 28.1 / 31.3, S 200 BH 257 causal 29.4 / 31.3; more in fmha_bwd_one.h).  Where every head has a compute unit to
+    // itself there is no next head, and its longer start shows: S 130 BH 256 15.2 / 14.3, S 200 BH 100 17.2 / 16.5, S 256
+    // BH 64 18.7 / 18.2, though S 256 BH 256 25.4 / 27.0.
     const bool small = a.sq <= 128 && a.sk <= 128;
+    if (!small) {
+      const int rc = FMHA_ONE_NAME(FMHA_TU_TNAME, FMHA_TU_D)(a, v, s);
+      if (rc != kBwdNotHere) return rc;
+    }
     if (v.causal) {
       if (small) return v.drop == 1 ? launch_short<1, 128, true>(a, s) : launch_short<0, 128, true>(a, s);
       return v.drop == 1 ? launch_short<1, 256, true>(a, s) : launch_short<0, 256, true>(a, s);

@@ -1,6 +1,5 @@
-// Backward kernel for short sequences (sq and sk <= 128, or <= 256; head dim 64; no mask, a per-key mask
-// and / or the causal mask): one workgroup per
-// head, one launch, every tensor crosses HBM once.
+// Backward kernel for short sequences (sq and sk <= 128, or, while there is a compute unit for every head, <= 256; head dim 64;
+// no mask, a per-key mask and / or the causal mask): one workgroup per head, one launch, every tensor crosses HBM once.
 //
 // At these shapes the backward is mostly memory time (BH 512, S 128: 5.4 GFLOP against 67 MB), and a head's
 // Q, K, V and dO fit in LDS together (64 KB; 128 KB at 256 rows).  The general path launches two kernels that each

@@ -43,7 +43,7 @@ struct BwdVariant {
   bool causal;
   int drop; // 0 none, 1 Philox
   int pair; // causal tile pairing: -1 decide from the amount of work, 0 off, 1 on
-  bool short_seq; // sq, sk <= 256 without a full mask tensor: the one-launch kernel (head dim 64)
+  bool short_seq; // sq, sk <= 256 without a full mask tensor: the one-launch kernels (head dim 64)
 };
 
 int bwd_dispatch_f16_d64(BwdArgs &a, const BwdVariant &v, hipStream_t s);
@@ -69,6 +69,14 @@ int bwd_pipe_launch_f16_d64_strided(const BwdArgs &a, const BwdVariant &v, bool 
 int bwd_pipe_launch_f16_d128_strided(const BwdArgs &a, const BwdVariant &v, bool dkdv, long long nblk, hipStream_t s);
 int bwd_pipe_launch_bf16_d64_strided(const BwdArgs &a, const BwdVariant &v, bool dkdv, long long nblk, hipStream_t s);
 int bwd_pipe_launch_bf16_d128_strided(const BwdArgs &a, const BwdVariant &v, bool dkdv, long long nblk, hipStream_t s);
+
+// The one-pass backward for heads of up to 256 queries and keys at head dim 64 (fmha_bwd_one.hip).  kBwdNotHere: nothing was
+// launched, the call belongs to the kernel for short heads.
+constexpr int kBwdNotHere = 3;
+int bwd_one_launch_f16_d64(const BwdArgs &a, const BwdVariant &v, hipStream_t s);
+int bwd_one_launch_bf16_d64(const BwdArgs &a, const BwdVariant &v, hipStream_t s);
+int bwd_one_launch_f16_d64_strided(const BwdArgs &a, const BwdVariant &v, hipStream_t s);
+int bwd_one_launch_bf16_d64_strided(const BwdArgs &a, const BwdVariant &v, hipStream_t s);
 
 // e4m3 forward (fmha_fwd_fp8.hip): 0 ok, 1 not built, 2 launch failed
 struct Fp8Args;
