@@ -55,7 +55,7 @@ template <typename K> int set_lds(K kern, int bytes) {
 //     with dropout         S 61 19 / 17, S 128 27 / 31
 //   dK+dV, causal          S 128 27 / 30, S 192 43 / 56, S 256 55 / 71, 2048 heads S 128 with dropout 101 / 126
 //   dK+dV of few heads (one round of workgroups, the plain pipelined kernel): 64 heads S 200 12 / 17, causal 14 / 16
-// The line is 128 queries.
+// The line is 128 queries (192 for causal dK / dV that is not persistent, see fmha_bwd_pipe.hip).
 template <int MASK, bool CAUSAL, int DROP> constexpr bool pipe_built() { return FMHA_TU_D != 256 && MASK != kMaskFull; }
 static inline bool pipe_wanted(const BwdArgs &a) { return FMHA_TU_D == 64 || a.sq >= 128; }
 // dQ of causal heads at head dim 128 has a line of its own: a pass pays the prologue with all compute units in step, and
@@ -107,7 +107,10 @@ template <int MASK, bool CAUSAL, int DROP> int launch_dkdv(BwdArgs &a, const Bwd
   // does where there is neither (plain pipelined kernel / this: BH 256 S 1024 343 / 335 us on one card, 347 / 359-369 on another).
   constexpr bool kTwoWaves = bwd_dkdv_small_tiles<FMHA_TU_D, CAUSAL, DROP>();
   if constexpr (kPipe) {
-    if (pipe_wanted(a) && !(kTwoWaves && (MASK != kMaskNone || a.kv_len))) return FMHA_PIPE_NAME(FMHA_TU_TNAME, FMHA_TU_D)(a, v, true, nblk, s);
+    if (pipe_wanted(a) && !(kTwoWaves && (MASK != kMaskNone || a.kv_len))) {
+      const int rc = FMHA_PIPE_NAME(FMHA_TU_TNAME, FMHA_TU_D)(a, v, true, nblk, s);
+      if (FMHA_TU_D == 64 || rc != kBwdNotHere) return rc;
+    }
   }
   if constexpr (!(kPipe && FMHA_TU_D == 64)) {
     using Cfg = BwdCfg<FMHA_TU_D, bwd_dkdv_tile_rows<FMHA_TU_D, CAUSAL, DROP>()>;

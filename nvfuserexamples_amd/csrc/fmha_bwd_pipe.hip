@@ -54,6 +54,9 @@ template <int MASK, bool CAUSAL, int DROP> int launch(const BwdArgs &a, bool dkd
         return hipGetLastError() == hipSuccess ? 0 : 2;
       }
     }
+    // Short causal heads that the persistent kernel does not take: phase by phase (backward, us, this kernel / that one: S 128
+    // BH 350 43.4 / 40.6; under a padding mask BH 512 S 128 54.2 / 51.2, S 176 95.1 / 91.3, S 160 level; S 200 103.4 / 105.5).
+    if (CAUSAL && a.sq < 192) return kBwdNotHere;
 #endif
     auto kern = fmha_bwd_dkdv_pipe_kernel<FMHA_TU_T, FMHA_TU_D, kNW, MASK, CAUSAL, DROP, kStrided>;
     static const bool ready = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,

@@ -59,6 +59,8 @@ int bwd_dispatch_f16_d128_strided(BwdArgs &a, const BwdVariant &v, hipStream_t s
 int bwd_dispatch_bf16_d64_strided(BwdArgs &a, const BwdVariant &v, hipStream_t s);
 int bwd_dispatch_bf16_d128_strided(BwdArgs &a, const BwdVariant &v, hipStream_t s);
 
+// (kBwdNotHere of the launchers below: nothing was launched, the call belongs to an older kernel)
+constexpr int kBwdNotHere = 3;
 // One launch of the software-pipelined backward (fmha_bwd_pipe.hip): the dQ kernel, or the dK / dV kernel; a.ntile and
 // a.pair as for the general kernels.
 int bwd_pipe_launch_f16_d64(const BwdArgs &a, const BwdVariant &v, bool dkdv, long long nblk, hipStream_t s);
@@ -70,9 +72,8 @@ int bwd_pipe_launch_f16_d128_strided(const BwdArgs &a, const BwdVariant &v, bool
 int bwd_pipe_launch_bf16_d64_strided(const BwdArgs &a, const BwdVariant &v, bool dkdv, long long nblk, hipStream_t s);
 int bwd_pipe_launch_bf16_d128_strided(const BwdArgs &a, const BwdVariant &v, bool dkdv, long long nblk, hipStream_t s);
 
-// The one-pass backward for heads of up to 256 queries and keys at head dim 64 (fmha_bwd_one.hip).  kBwdNotHere: nothing was
-// launched, the call belongs to the kernel for short heads.
-constexpr int kBwdNotHere = 3;
+// The one-pass backward for heads of up to 256 queries and keys at head dim 64 (fmha_bwd_one.hip); kBwdNotHere: for the kernel
+// for short heads.
 int bwd_one_launch_f16_d64(const BwdArgs &a, const BwdVariant &v, hipStream_t s);
 int bwd_one_launch_bf16_d64(const BwdArgs &a, const BwdVariant &v, hipStream_t s);
 int bwd_one_launch_f16_d64_strided(const BwdArgs &a, const BwdVariant &v, hipStream_t s);

@@ -1,7 +1,11 @@
 """The persistent dK / dV kernel (head dim 128, no mask, from one and a half rounds of workgroups on): what a workgroup hands from
 item to item.  A head's gradients do not depend on the heads beside it, so a launch of many heads has to give the bits of
 launches of few heads, which run on the plain pipelined kernel (compared with the oracle in test_gpu_bwd_pipe.py).  The cases
-with a mask or key counts are those whose launches stay on the plain kernels."""
+with a mask or key counts are those whose launches stay on the plain kernels.
+
+Few causal heads of fewer than 192 queries run phase by phase, with other roundings of the scaled operands: scores
+are off by u of themselves (u = 2^-11, bf16 2^-8; |score| < 6 for nearly all of P), and roundings of P, dS and the result may
+fall the other way: errors of either sign that add up like the gradient's own terms do, 8 u max|gradient|."""
 import pytest
 import torch
 
@@ -11,6 +15,7 @@ from conftest import make_qkv, tail_mask
 pytestmark = pytest.mark.gpu
 
 TDT = {"fp16": torch.float16, "bf16": torch.bfloat16}
+U = {"fp16": 2.0 ** -11, "bf16": 2.0 ** -8}
 HPR = 10  # heads per mask row / key count
 
 CASES = [
@@ -22,6 +27,7 @@ CASES = [
     (260, 130, 300, 128, "fp16", "tail", False, 0.1, None),
     (100, 160, 700, 128, "fp16", "len", False, 0.0, None),       # key counts, among them 0
     (200, 130, 260, 128, "fp16", None, True, 0.1, "0"),          # items of one query tile; key tiles behind every query
+    (200, 288, 420, 128, "fp16", None, True, 0.1, "0"),          # ... to the bit
     (400, 420, 420, 128, "bf16", None, True, 0.0, "1"),          # pairs, an even and (next) an odd number of tiles
     (400, 300, 300, 128, "fp16", None, True, 0.1, "1"),
     (200, 420, 420, 128, "bf16", None, True, 0.1, "0"),          # rounds in turned order
@@ -70,7 +76,11 @@ def test_many_heads_give_the_bits_of_few(bh, sq, sk, d, dtype, mask, causal, p, 
             few = capi.bwd(do[h0:h1], q[h0:h1], k[h0:h1], v[h0:h1], o[h0:h1], lse[h0:h1].contiguous(), **args(h0, h1))
             torch.cuda.synchronize()
             for name, a, b in zip(("dq", "dk", "dv"), got, few):
-                assert torch.equal(a[h0:h1], b), (name, h0)
+                if causal and sq < 192:
+                    b = b.float()
+                    assert (a[h0:h1].float() - b).abs().max().item() <= 8 * U[dtype] * b.abs().max().item(), (name, h0)
+                else:
+                    assert torch.equal(a[h0:h1], b), (name, h0)
     finally:
         if pair is not None:
             monkeypatch.delenv("FMHA_BWD_PAIR")
