@@ -52,7 +52,7 @@ DropCtx make_drop_ctx(uint64_t seed, uint64_t offset, float p, int sq, int sk) {
 // FMHA_FWD_SAVE_SPLIT=0 keep the save-intermediates operator beyond 128 keys off its one-launch kernel / off the
 // forward-then-save pair of launches,
 // FMHA_FWD_SHORT=0 / FMHA_BWD_SHORT=0 keep short key ranges / short sequences off their
-// one-pass kernels (FMHA_FWD_SHORT=2: only the forwards without a full mask tensor) (FMHA_BWD_SHORT=128 limits the backward one to 128 rows), FMHA_BWD_PAIR=0|1 sets the
+// one-pass kernels (FMHA_FWD_SHORT=2: only the forwards without a full mask tensor; both keep 129 to 256 keys on the pipelined kernel) (FMHA_BWD_SHORT=128 limits the backward one to 128 rows), FMHA_BWD_PAIR=0|1 sets the
 // pairing of causal tiles in the backward, FMHA_MASK_TRIM=0 makes forward and backward visit the key tiles
 // that a per-key mask hard-masks (as FMHA_FLAG_NO_MASK_TRIM does per call), FMHA_FWD_SPLIT=0 never cuts a
 // forward's key range into pieces, FMHA_FWD_SPLIT=n (2..64) cuts it into about n wherever pieces are possible,
@@ -434,6 +434,7 @@ static int fwd_split_launch(const fmha_fwd_params *p, const FwdArgs &a, const Sp
   v.causal = false;
   v.drop = 0;
   v.saving = v.save_split = v.save_once = v.stream = v.short_keys = v.head = false;
+  v.mid = 0;
   const int rc = fwd_dispatch_strided(b, v, p->dtype, D, s);
   if (rc != 0) return rc == 1 ? FMHA_E_UNSUPPORTED : FMHA_E_LAUNCH;
   {
@@ -627,6 +628,23 @@ int fmha_fwd_launch(const fmha_fwd_params *caller, void *hip_stream) {
     const bool full = chunks * 512 - p->sq <= 128; // at most two of the eight waves of a head's last item idle
     const bool even = cus > 0 && (items % cus == 0 || items >= 4LL * cus);
     v.head = overrides().fwd_head == 1 || (p->sk > 256 && full && even);
+  }
+  // Key ranges of 129 to 256 keys at head dim 64, from 129 queries on: K and V of a head in LDS, whole blocks of 32 keys and
+  // queries instead of tiles of 64 and 128 (fmha_fwd_mid.h); four waves a workgroup while each has a compute unit to itself.
+  // It saves padding, and work beside the products that grows with it.  Where there is neither -- eight blocks of keys, no
+  // dropout -- the pipelined kernel's finer overlap counts for more (us, this / pipelined: BH 512 S 256 20.0 / 17.1, S 230 21.2 /
+  // 18.0, causal BH 512 18.1 / 17.4, BH 1024 30.8 / 29.6) until workgroups are many (BH 2048 S 256 57.3 / 61.4, BH 1024 S 230
+  // 29.7 / 32.3; causal with a mask or key counts BH 1024 S 256 30.3 / 34.7), and on few heads from seven blocks on (BH 24 S 200
+  // 6.4 / 6.2, BH 64 512 x 256 7.5 / 7.1; S 160 5.4 / 6.1).
+  v.mid = 0;
+  if (p->d == 64 && p->sk > 128 && p->sk <= 256 && p->sq > 128 && v.mask != kMaskFull && v.drop != 2 && !saving && !v.head &&
+      overrides().fwd_short == 1) {
+    const int cus = cu_count();
+    const bool plain = v.mask == kMaskNone && v.drop == 0;
+    if ((long long)p->bh * ((p->sq + 127) / 128) <= cus) v.mid = plain && !v.causal && p->sk > 192 ? 0 : 4;
+    else if (v.drop != 0 || p->sk <= 224) v.mid = 8;
+    else if (v.causal) v.mid = plain && !p->kv_len ? 0 : 8;
+    else v.mid = (long long)p->bh * ((p->sq + 255) / 256) >= 4LL * cus ? 8 : 0;
   }
 
   int rc;

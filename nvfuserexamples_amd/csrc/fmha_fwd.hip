@@ -17,11 +17,13 @@
 #define FMHA_TU_SHORT 1
 #include "fmha_fwd_short.h"
 #include "fmha_fwd_head.h"
+#include "fmha_fwd_mid.h"
 #else
 #define FMHA_TU_SHORT 0
 #if FMHA_TU_D == 64
 #include "fmha_fwd_short.h" // run-time row layouts: its builds without a full mask tensor
-#include "fmha_fwd_head.h"  // and the whole-head kernel
+#include "fmha_fwd_head.h"  // the whole-head kernel
+#include "fmha_fwd_mid.h"   // and the one for 129 to 256 keys
 #endif
 #endif
 
@@ -128,6 +130,27 @@ template <int MASK, int DROP, bool SAVE> int launch_short(FwdArgs &a, hipStream_
                                          : launch_short_as<MASK, DROP, SAVE, false, true>(a, s);
   return a.sk > ShortCfg::SKMAX - 32 ? launch_short_as<MASK, DROP, SAVE, true>(a, s)
                                      : launch_short_as<MASK, DROP, SAVE, false>(a, s);
+}
+#endif
+
+#if FMHA_TU_D == 64
+// 129 to 256 keys
+template <int NW, int MASK, bool CAUSAL, int DROP> int launch_mid_as(FwdArgs &a, hipStream_t s) {
+  using MidCfg = fmha::MidCfg<NW>;
+  auto kern = fmha_fwd_mid_kernel<FMHA_TU_T, NW, MASK, CAUSAL, DROP, kStrided>;
+  static const bool ready = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
+                                                hipFuncAttributeMaxDynamicSharedMemorySize, MidCfg::LDS_BYTES) == hipSuccess;
+  if (!ready) return 2;
+  if (a.sk > MidCfg::SKMAX) return 1;
+  a.nqt = (a.sq + MidCfg::QT - 1) / MidCfg::QT;
+  const long long nblk = (long long)a.bh * a.nqt;
+  if (nblk > 0x7fffffffLL) return 2;
+  hipLaunchKernelGGL(kern, dim3((unsigned)nblk), dim3(MidCfg::NT), MidCfg::LDS_BYTES, s, a);
+  return hipGetLastError() == hipSuccess ? 0 : 2;
+}
+template <int NW, int MASK> int launch_mid(FwdArgs &a, const FwdVariant &v, hipStream_t s) {
+  if (v.causal) return v.drop == 1 ? launch_mid_as<NW, MASK, true, 1>(a, s) : launch_mid_as<NW, MASK, true, 0>(a, s);
+  return v.drop == 1 ? launch_mid_as<NW, MASK, false, 1>(a, s) : launch_mid_as<NW, MASK, false, 0>(a, s);
 }
 #endif
 
@@ -271,6 +294,13 @@ int FMHA_NAME(FMHA_TU_TNAME, FMHA_TU_D)(FwdArgs &a, const FwdVariant &v, hipStre
 int FMHA_NAME(FMHA_TU_TNAME, FMHA_TU_D)(FwdArgs &a, const FwdVariant &v, hipStream_t s) {
 #if defined(FMHA_DEV_MINIMAL) || FMHA_TU_STRIDED
   if (v.drop == 2 || v.qb == 2) return 1; // folded layout only
+#endif
+#if FMHA_TU_D == 64
+  if (v.mid) {
+    if (v.drop == 2 || v.mask == kMaskFull) return 1;
+    if (v.mid == 4) return v.mask == kMaskPerKey ? launch_mid<4, kMaskPerKey>(a, v, s) : launch_mid<4, kMaskNone>(a, v, s);
+    return v.mask == kMaskPerKey ? launch_mid<8, kMaskPerKey>(a, v, s) : launch_mid<8, kMaskNone>(a, v, s);
+  }
 #endif
 #if FMHA_TU_D == 64 && FMHA_TU_STRIDED
   if (v.head && !v.short_keys) { // run-time row layouts: the whole-head kernel

@@ -22,6 +22,7 @@ struct FwdVariant {
   bool many;       // stream: more workgroups than two per compute unit
   bool head;       // up to 512 keys, no / per-key mask, no causal mask: the whole-head kernel (head dim 64, folded layout)
   bool short_keys; // sk <= 128: the one-pass kernel (head dim 64, folded layout)
+  int mid;         // 129 to 256 keys, no full mask tensor: waves per workgroup of the kernel that has a head's K and V in LDS, 0: not that (head dim 64)
 };
 
 // Return 0 on success, 1 if the variant is not built, 2 if the launch failed.
