@@ -54,8 +54,8 @@ def _tus():
                 defs = [f"-DFMHA_TU_BF16={bf}", f"-DFMHA_TU_D={d}", f"-DFMHA_TU_STRIDED={strided}"]
                 tus.append(("fmha_fwd.hip", f"fmha_fwd_{tag}.o", defs))
                 tus.append(("fmha_bwd.hip", f"fmha_bwd_{tag}.o", defs))
-                if d == 64: # (operands and accumulators in one file, as below)
-                    tus.append(("fmha_bwd_one.hip", f"fmha_bwd_one_{tag}.o", defs + [FREE_MFMA_FORM]))
+                if d == 64:
+                    tus.append(("fmha_bwd_one.hip", f"fmha_bwd_one_{tag}.o", defs))
                 if d != 256:
                     # At head dim 128 the dK / dV kernel runs one wave per SIMD on both halves of the register file and
                     # wants its accumulators in the accumulation half; the compiler finds that split by itself only
