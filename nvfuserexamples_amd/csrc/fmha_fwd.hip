@@ -271,10 +271,16 @@ template <int QB> int by_mask(FwdArgs &a, const FwdVariant &v, hipStream_t s) {
 } // namespace
 
 #if FMHA_TU_D == 256
-// Head dim 256: built for coverage, not tuned.  Every variant runs on the plain (not software-pipelined)
-// loop at one wave per SIMD: the output accumulators alone take 128 registers per lane.
+// Head dim 256, one wave per SIMD: the output accumulators alone take 128 registers per lane, all in all about 400 of the 512 that
+// a wave then has.  The pipelined loop (132 KB of LDS) takes what needs no [.., sq, sk] tensor and has more than one key tile;
+// us, pipelined / plain loop: BH 128 S 2048 646 / 909, causal 382 / 623; BH 72 S 1408 bf16 189 / 300; BH 300 S 512 causal with
+// dropout 106 / 193; BH 512 S 256 padding mask 70 / 97; BH 512 S 100 24.2 / 33.5; BH 12 S 500 21.5 / 31.6; rows of 200 elements
+// BH 64 S 2048 262 / 405.  One tile has nothing to overlap: BH 1900 S 31 60.4 / 58.8, 64 keys level.
 namespace { // (per translation unit: the element type differs between units of the same name)
-template <int MASK, bool CAUSAL> int plain_by_drop(FwdArgs &a, int drop, hipStream_t s) {
+template <int MASK, bool CAUSAL> int d256_by_drop(FwdArgs &a, int drop, hipStream_t s) {
+  if constexpr (MASK != kMaskFull) {
+    if (a.sk > 64 && drop < 2) return drop == 1 ? launch<1, MASK, CAUSAL, 1>(a, s) : launch<1, MASK, CAUSAL, 0>(a, s);
+  }
   if (drop == 0) return launch<1, MASK, CAUSAL, 0, false>(a, s);
   if (drop == 1) return launch<1, MASK, CAUSAL, 1, false>(a, s);
   if (drop == 2 && !CAUSAL) return launch<1, MASK, false, 2, false>(a, s);
@@ -285,10 +291,10 @@ template <int MASK, bool CAUSAL> int plain_by_drop(FwdArgs &a, int drop, hipStre
 int FMHA_NAME(FMHA_TU_TNAME, FMHA_TU_D)(FwdArgs &a, const FwdVariant &v, hipStream_t s) {
   if (v.qb == 2 || v.short_keys || v.save_split || v.save_once || v.stream || v.head || (kStrided && v.drop == 2)) return 1;
   if (v.mask == kMaskPerKey)
-    return v.causal ? plain_by_drop<kMaskPerKey, true>(a, v.drop, s) : plain_by_drop<kMaskPerKey, false>(a, v.drop, s);
+    return v.causal ? d256_by_drop<kMaskPerKey, true>(a, v.drop, s) : d256_by_drop<kMaskPerKey, false>(a, v.drop, s);
   if (v.mask == kMaskFull)
-    return v.causal ? plain_by_drop<kMaskFull, true>(a, v.drop, s) : plain_by_drop<kMaskFull, false>(a, v.drop, s);
-  return v.causal ? plain_by_drop<kMaskNone, true>(a, v.drop, s) : plain_by_drop<kMaskNone, false>(a, v.drop, s);
+    return v.causal ? d256_by_drop<kMaskFull, true>(a, v.drop, s) : d256_by_drop<kMaskFull, false>(a, v.drop, s);
+  return v.causal ? d256_by_drop<kMaskNone, true>(a, v.drop, s) : d256_by_drop<kMaskNone, false>(a, v.drop, s);
 }
 #else
 int FMHA_NAME(FMHA_TU_TNAME, FMHA_TU_D)(FwdArgs &a, const FwdVariant &v, hipStream_t s) {

@@ -60,7 +60,7 @@ template <int D, int QB> struct PipeCfg {
 // matrix pipe (about twice the issue interval).
 struct FwdOperandList {
   int n;
-  int kind[48], a0[48], a1[48], a2[48];
+  int kind[72], a0[72], a1[72], a2[72]; // (66 at head dim 256)
 };
 template <int NSB, int KS, int DB, bool WITH_FIRST_PRODUCT> constexpr FwdOperandList fwd_operand_list() {
   FwdOperandList L{};
