@@ -33,6 +33,7 @@ HIP_FLAGS = [
     "-fno-honor-nans",
     "-Wno-unused-command-line-argument",
 ]
+UNROLL_FREE = ["-mllvm", "-pragma-unroll-threshold=200000"]
 FREE_MFMA_FORM = object()  # marks a translation unit that is compiled without -amdgpu-mfma-vgpr-form
 
 
@@ -61,6 +62,9 @@ def _tus():
                     # wants its accumulators in the accumulation half; the compiler finds that split by itself only
                     # where it is free to choose the form of every matrix instruction.
                     tus.append(("fmha_bwd_pipe.hip", f"fmha_bwd_pipe_{tag}.o", defs + [FREE_MFMA_FORM]))
+                else:
+                    # (the stream of a tile is longer than the compiler unrolls by itself: its operands would land in memory)
+                    tus.append(("fmha_bwd_pipe.hip", f"fmha_bwd_pipe_{tag}.o", defs + UNROLL_FREE))
     return tus
 
 

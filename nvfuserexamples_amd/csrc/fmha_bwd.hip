@@ -65,6 +65,9 @@ static inline bool pipe_wanted(const BwdArgs &a) { return FMHA_TU_D == 64 || a.s
 // S 896 300 / 292, S 1024 336 / 335; BH 256 S 2048 438 / 484, with dropout BH 128 S 2048 271 / 281: level to 4 % either way
 // from 896 to 1024, ahead beyond.  (At few heads ahead earlier, BH 64 S 512 23 / 25, but a head's gradients do not depend
 // on how many others there are.)
+// dQ at head dim 256, one wave per SIMD: from 128 queries on as well (us, pipelined / phase by phase: BH 128 S 2048 750 / 1041,
+// causal 440 / 616; BH 64 S 1000 with dropout 118 / 140; BH 300 S 512 bf16 causal with dropout 174 / 244; BH 512 S 256 119 / 126,
+// causal 113 / 126, S 128 42.6 / 43.7; BH 1000 S 129 causal 164 / 174; BH 8 S 1750 59 / 102).
 template <bool CAUSAL> bool pipe_wanted_dq(const BwdArgs &a) {
   return pipe_wanted(a) && !(FMHA_TU_D == 128 && CAUSAL && a.sq < 896);
 }
@@ -76,11 +79,9 @@ template <typename K> int launch_one(K kern, BwdArgs &a, long long nblk, int thr
 }
 
 template <int MASK, bool CAUSAL, int DROP> int launch_dq(BwdArgs &a, const BwdVariant &v, long long nblk, hipStream_t s) {
-#if FMHA_TU_D != 256
-  if constexpr (pipe_built<MASK, CAUSAL, DROP>()) {
+  if constexpr (MASK != kMaskFull) { // (pipe_built, or head dim 256, where it is built for dQ only)
     if (pipe_wanted_dq<CAUSAL>(a)) return FMHA_PIPE_NAME(FMHA_TU_TNAME, FMHA_TU_D)(a, v, false, nblk, s);
   }
-#endif
   if constexpr (!(pipe_built<MASK, CAUSAL, DROP>() && FMHA_TU_D == 64)) { // (there the pipelined kernel takes all)
     constexpr int kLds = BwdCfg<FMHA_TU_D, bwd_dq_tile_rows<FMHA_TU_D>()>::LDS_BYTES;
     static_assert(kLds <= 160 * 1024, "tiles do not fit the LDS of a compute unit");

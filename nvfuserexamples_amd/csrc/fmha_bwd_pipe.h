@@ -1,4 +1,4 @@
-// Software-pipelined backward kernels for head dims 64 and 128 (no mask or a per-key mask; full mask tensors stay on
+// Software-pipelined backward kernels for head dims 64 and 128, and dQ at 256 (no mask or a per-key mask; full mask tensors stay on
 // fmha_bwd_kernel.h).  Mathematics, register layouts and the extra contraction step are those of fmha_bwd_kernel.h, whose
 // header describes them; what changes is the order of work and how tiles arrive:
 //
@@ -98,8 +98,10 @@ struct PhiloxSlices {
 };
 
 // ------------------------------------------------------------------------------ dQ
+// (waves per SIMD: at head dim 256 a wave needs about 400 registers, and the tiles leave room for one workgroup)
+template <int D> constexpr int bwd_dq_pipe_occ() { return D == 256 ? 1 : 2; }
 template <typename T, int D, int NW, int MASK, bool CAUSAL, int DROP, bool STRIDED>
-__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void fmha_bwd_dq_pipe_kernel(const BwdArgs a) {
+__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(bwd_dq_pipe_occ<D>(), bwd_dq_pipe_occ<D>()))) void fmha_bwd_dq_pipe_kernel(const BwdArgs a) {
   using RW = Rows<STRIDED, D>;
   using E = Elem<T>;
   using v8 = typename E::v8;

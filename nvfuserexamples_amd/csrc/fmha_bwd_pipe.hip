@@ -29,6 +29,9 @@ using Cfg = BwdPipeCfg<FMHA_TU_D>;
 
 template <int MASK, bool CAUSAL, int DROP> int launch(const BwdArgs &a, bool dkdv, long long nblk, hipStream_t s) {
   if (nblk > 0x7fffffffLL) return 2;
+#if FMHA_TU_D == 256 // (dQ only)
+  if (dkdv) return 1;
+#else
   if (dkdv) {
 #if FMHA_TU_D == 128
     if constexpr (MASK == kMaskNone) {
@@ -63,7 +66,9 @@ template <int MASK, bool CAUSAL, int DROP> int launch(const BwdArgs &a, bool dkd
                                                   Cfg::dkdv_lds_bytes(DROP, Cfg::QSEG)) == hipSuccess;
     if (!ready) return 2;
     hipLaunchKernelGGL(kern, dim3((unsigned)nblk), dim3(kNW * 64), Cfg::dkdv_lds_bytes(DROP, a.sq), s, a);
-  } else {
+  } else
+#endif
+  {
     static const bool ready = hipFuncSetAttribute(reinterpret_cast<const void *>(fmha_bwd_dq_pipe_kernel<FMHA_TU_T, FMHA_TU_D, kNW, MASK, CAUSAL, DROP, kStrided>),
                                                   hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::dq_lds_bytes(MASK, Cfg::MSEG)) == hipSuccess;
     if (!ready) return 2;

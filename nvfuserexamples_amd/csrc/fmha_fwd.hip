@@ -273,7 +273,7 @@ template <int QB> int by_mask(FwdArgs &a, const FwdVariant &v, hipStream_t s) {
 #if FMHA_TU_D == 256
 // Head dim 256, one wave per SIMD: the output accumulators alone take 128 registers per lane, all in all about 400 of the 512 that
 // a wave then has.  The pipelined loop (132 KB of LDS) takes what needs no [.., sq, sk] tensor and has more than one key tile;
-// us, pipelined / plain loop: BH 128 S 2048 646 / 909, causal 382 / 623; BH 72 S 1408 bf16 189 / 300; BH 300 S 512 causal with
+// us, pipelined / plain loop: BH 128 S 2048 631 / 911, causal 372 / 624; BH 72 S 1408 bf16 188 / 299; BH 300 S 512 causal with
 // dropout 106 / 193; BH 512 S 256 padding mask 70 / 97; BH 512 S 100 24.2 / 33.5; BH 12 S 500 21.5 / 31.6; rows of 200 elements
 // BH 64 S 2048 262 / 405.  One tile has nothing to overlap: BH 1900 S 31 60.4 / 58.8, 64 keys level.
 namespace { // (per translation unit: the element type differs between units of the same name)

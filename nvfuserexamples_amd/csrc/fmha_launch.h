@@ -73,6 +73,11 @@ int bwd_pipe_launch_f16_d128_strided(const BwdArgs &a, const BwdVariant &v, bool
 int bwd_pipe_launch_bf16_d64_strided(const BwdArgs &a, const BwdVariant &v, bool dkdv, long long nblk, hipStream_t s);
 int bwd_pipe_launch_bf16_d128_strided(const BwdArgs &a, const BwdVariant &v, bool dkdv, long long nblk, hipStream_t s);
 
+int bwd_pipe_launch_f16_d256(const BwdArgs &a, const BwdVariant &v, bool dkdv, long long nblk, hipStream_t s);
+int bwd_pipe_launch_bf16_d256(const BwdArgs &a, const BwdVariant &v, bool dkdv, long long nblk, hipStream_t s);
+int bwd_pipe_launch_f16_d256_strided(const BwdArgs &a, const BwdVariant &v, bool dkdv, long long nblk, hipStream_t s);
+int bwd_pipe_launch_bf16_d256_strided(const BwdArgs &a, const BwdVariant &v, bool dkdv, long long nblk, hipStream_t s);
+
 // The one-pass backward for heads of up to 256 queries and keys at head dim 64 (fmha_bwd_one.hip); kBwdNotHere: for the kernel
 // for short heads.
 int bwd_one_launch_f16_d64(const BwdArgs &a, const BwdVariant &v, hipStream_t s);
