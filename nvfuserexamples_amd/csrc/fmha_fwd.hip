@@ -80,6 +80,21 @@ template <int QB, int MASK, bool CAUSAL, int DROP, bool kPipe = (DROP != 2)> int
   long long nblk = (long long)a.bh * a.nqt;
   if (nblk > 0x7fffffffLL) return 2;
   if (kPipe && nblk > resident) nblk = resident;
+  // Causal items, from half a round to four: by length, unless the rounds pair a head's tiles exactly anyway (whole heads in an
+  // even number of rounds).  A head's items in turn met as they came, and a workgroup with two long ones ended the launch (us,
+  // bf16, in turn / by length): D 64 16 heads S 5573 169 / 90, 84 heads S 1562 74 / 46, 88 heads S 2368 132 / 90, 300 heads S 512
+  // 31.8 / 26.8; D 128 32 heads S 4286 240 / 155, 48 heads S 2194 101 / 74, 12 heads S 3584 85 / 72, 40 heads S 1000 33.3 / 27.9.
+  // Exact pairs keep a head on fewer compute units at a time (32 heads S 4001), beyond four rounds little is left to gain.
+  a.deal = a.deal_heads = 0;
+  if (kPipe && CAUSAL && MASK == kMaskNone && a.sk_whole == 0) {
+    const long long items = (long long)a.bh * a.nqt, G = nblk;
+    if (2 * items > resident && items < 4 * G && !(G % a.nqt == 0 && items % (2 * G) == 0)) {
+      int lg = 0;
+      while (G % 8 == 0 && lg < 3 && a.bh % (2 << lg) == 0) ++lg;
+      a.deal = lg + 1;
+      a.deal_heads = a.bh >> lg;
+    }
+  }
   a.bal_rows = 0;
   if (kPipe && MASK == kMaskPerKey && !CAUSAL && a.mask_div > 0 && a.bh % a.mask_div == 0) {
     // shapes whose mask rows can be dealt to the workgroups by length (see FwdArgs::bal_rows): an
@@ -96,6 +111,16 @@ template <int QB, int MASK, bool CAUSAL, int DROP, bool kPipe = (DROP != 2)> int
       a.bal_ipr = (int32_t)ipr;
       a.bal_R = (int32_t)(nblk / ipr);
       a.bal_inv_ipr = 1.f / (float)ipr;
+    }
+  }
+  if constexpr (kPipe && CAUSAL && MASK == kMaskNone) {
+    if (a.deal) {
+      auto dealt = fmha_fwd_pipe_kernel<FMHA_TU_T, FMHA_TU_D, QB, kNW, MASK, CAUSAL, DROP, kStrided, true>;
+      static const bool ready = hipFuncSetAttribute(reinterpret_cast<const void *>(dealt), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                    kLds) == hipSuccess;
+      if (!ready) return 2;
+      hipLaunchKernelGGL(dealt, dim3((unsigned)nblk), dim3(kNW * 64), kLds, s, a);
+      return hipGetLastError() == hipSuccess ? 0 : 2;
     }
   }
   hipLaunchKernelGGL(kern, dim3((unsigned)nblk), dim3(kNW * 64), kLds, s, a);

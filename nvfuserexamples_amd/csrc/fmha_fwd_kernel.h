@@ -57,6 +57,10 @@ struct FwdArgs {
   float mask_a, mask_b; // mask term in log2 units = mask_value * mask_a + mask_b
   int32_t bh, sq, sk;
   int32_t nqt;       // query tiles per head
+  // Causal items dealt by length (pipelined kernel without a mask; set by its launch code, 0 = off): the heads fall into
+  // 2^(deal - 1) groups of deal_heads, each with its share of the XCDs, that are dealt separately.  (Beside nqt: a line of the
+  // arguments that every workgroup reads anyway.)
+  int32_t deal, deal_heads;
   float scale_l2;    // scale * log2(e)
   float inv_scale_l2; // 1 / scale_l2
   float drop_scale;

@@ -85,7 +85,8 @@ template <int NSB, int KS, int DB, bool WITH_FIRST_PRODUCT> constexpr FwdOperand
 // (Two query blocks per wave, head dim 128, and the staged values of a full mask tensor under a
 // causal mask need more than the 256 registers of a two-waves-per-SIMD budget by a few; the occupancy attribute makes the compiler spill those
 // few instead of settling for one wave per SIMD, which measures 8-30 % faster.)
-template <typename T, int D, int QB, int NW, int MASK, bool CAUSAL, int DROP, bool STRIDED>
+// DEAL: causal items dealt by length, see FwdArgs::deal (a build of its own: the choice at run time cost short launches 0.5 us).
+template <typename T, int D, int QB, int NW, int MASK, bool CAUSAL, int DROP, bool STRIDED, bool DEAL = false>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu((QB == 2 || D == 128 || MASK == kMaskFull || DROP == 2) ? 2 : 1, 2))) void fmha_fwd_pipe_kernel(const FwdArgs a) {
   using RW = Rows<STRIDED, D>;
   using E = Elem<T>;
@@ -212,6 +213,16 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu((QB == 
     }
   }
 
+  // Causal items dealt by length: the heads fall into up to eight groups, each with its XCDs; a group's items go out longest
+  // first, and every other round of its workgroups the other way round, so that a long item meets a short one whatever the
+  // tiles per head and whatever is left for the last round.
+  static_assert(!DEAL || (CAUSAL && MASK == kMaskNone), "");
+  constexpr bool deal = DEAL;
+  const int dlog = deal ? a.deal - 1 : 0, dgrp = (int)blockIdx.x & ((1 << dlog) - 1); // (workgroups go to XCDs by turns)
+  const int dwg = (int)blockIdx.x >> dlog, dG = G >> dlog, dheads = a.deal_heads;
+  auto dealt = [&](int ord) -> int { return ord * dG + ((ord & 1) ? dG - 1 - dwg : dwg); };
+  auto exists = [&](int ord) -> bool { return deal ? dealt(ord) < dheads * a.nqt : lb + ord * G < nitems; };
+
   // Everything that depends on the item.  Keys: tiles [0, nkt), keys [0, kend); the tile count
   // is padded to even (nkt2) with an all-masked phantom tile so that the two x / P buffers and
   // the two LDS stages alternate with fixed roles across items as well.
@@ -229,8 +240,10 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu((QB == 
       it.bh = mrow * a.mask_div + bal_h0;
       it.qt = bal_qt0;
     } else {
-      it.bh = idx / a.nqt;
-      it.qt = idx - it.bh * a.nqt;
+      // (one division for both orders: the code of a short launch is read from memory as it runs)
+      const int num = deal ? dealt(ord) : idx, den = deal ? dheads : a.nqt, quo = num / den, rem = num - quo * den;
+      it.bh = deal ? (rem << dlog) + dgrp : quo;
+      it.qt = deal ? a.nqt - 1 - quo : rem;
       mrow = MASK == kMaskPerKey ? it.bh / a.mask_div : 0;
     }
     // Causal items grow with the query tile.  A workgroup's items are G apart, which is often a
@@ -238,7 +251,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu((QB == 
     // round: long and short items then alternate within each workgroup.  (The round of the head's
     // FIRST item decides for all of its tiles: where G is no multiple of the tiles per head some heads
     // lie in two rounds, and by the item's own round they would get some tiles twice and others never.)
-    if (CAUSAL && ((it.bh * a.nqt / G) & 1) == 0) it.qt = a.nqt - 1 - it.qt;
+    if (CAUSAL && !deal && ((it.bh * a.nqt / G) & 1) == 0) it.qt = a.nqt - 1 - it.qt;
     // keys this head may see at all: [0, sk) or its valid count (possibly 0: then every key is
     // treated as past the end, which yields O = 0 and LSE = -inf)
     int piece;
@@ -283,7 +296,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu((QB == 
     for (int i = 0; i < kTrimSlots; ++i) bal_row[i] = grp + i * a.bal_R;
   }
   Item cur = make_item(lb, 0);
-  Item nxt = make_item(lb + G < nitems ? lb + G : lb, lb + G < nitems ? 1 : 0); // without a successor the streams harmlessly re-read the item
+  Item nxt = make_item(exists(1) ? lb + G : lb, exists(1) ? 1 : 0); // without a successor the streams harmlessly re-read the item
   int bh = cur.bh, q0w = cur.qt * QT + w * (QB * 32); // of the current item
 
   // ---- staging
@@ -334,7 +347,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu((QB == 
   int nn_kend = cur.kend;      // key range and per-key mask of the item after next
   const T *nn_mkey = cur.mkey;
   auto set_after_next = [&](int idx, int ord) {
-    const bool has = idx + 2 * G < nitems;
+    const bool has = exists(ord + 2);
     const Item it = trimmed(make_item(has ? idx + 2 * G : idx, has ? ord + 2 : ord), has ? ord + 2 : ord);
     nn_kend = it.kend;
     nn_mkey = it.mkey;
@@ -907,7 +920,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu((QB == 
 
   for (int idx = lb, ord = 0;;) {
     const int nidx = idx + G;
-    const bool more = nidx < nitems;
+    const bool more = exists(ord + 1);
     nxt = trimmed(make_item(more ? nidx : idx, more ? ord + 1 : ord), more ? ord + 1 : ord);
     set_after_next(idx, ord);
     bh = cur.bh;
