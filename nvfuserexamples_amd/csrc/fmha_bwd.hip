@@ -132,8 +132,10 @@ template <int MASK, bool CAUSAL, int DROP> int launch(BwdArgs &a, const BwdVaria
   constexpr int KT = kNW * kKB * 32;
 #endif
   constexpr int QT = kNW * kQB * 32;
-  // causal: workgroups take pairs of tiles (see the kernels) when that leaves at least two
-  // rounds of workgroups for the device
+  // causal: workgroups take pairs of tiles (see bwd_item) when that leaves at least two
+  // rounds of workgroups for the device -- but not of three tiles, where the middle one is left alone with half a pair's work
+  // (us, paired / one by one, longest first: D 64 BH 1000 S 300 dQ 70.7 / 63.6, dK / dV 74.3 / 63.8, BH 1500 S 380 with dropout
+  // 138 / 120 and 170 / 145; D 128 BH 600 S 380 109 / 93 and 128 / 105; five tiles, BH 600 S 600, 83.4 / 86.2 and 93.4 / 96.1)
   static const int cus = [] {
     int dev = 0, n = 0;
     if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
@@ -142,7 +144,7 @@ template <int MASK, bool CAUSAL, int DROP> int launch(BwdArgs &a, const BwdVaria
   }();
   auto blocks = [&](int ntile) -> long long {
     a.ntile = ntile;
-    a.pair = CAUSAL && (v.pair >= 0 ? v.pair != 0 : (long long)a.bh * ((ntile + 1) / 2) >= 4LL * cus);
+    a.pair = CAUSAL && (v.pair >= 0 ? v.pair != 0 : ntile != 3 && (long long)a.bh * ((ntile + 1) / 2) >= 4LL * cus);
     return (long long)a.bh * (a.pair ? (ntile + 1) / 2 : ntile);
   };
   // dQ first: it also writes delta, which the dK/dV kernel reads (same stream => ordered)

@@ -91,6 +91,31 @@ FMHA_DEV int bwd_valid_keys(const BwdArgs &a, int bh) {
   return n < 0 ? 0 : (n < a.sk ? n : a.sk);
 }
 
+// The workgroup's head and tile (pi: counted from the longest under a causal mask), and whether it takes one tile or two.
+// With a causal mask the work of a tile depends on its index, so a workgroup takes a pair of tiles (i, n-1-i), one after the
+// other: every workgroup then has the same amount of work (the host launches ceil(n/2) workgroups per head; it does so when
+// that still fills the device).  Otherwise one tile per workgroup, the longest of all heads first: what starts last is short, and
+// a compute unit's second workgroup is as short as its first is long (us, head by head / so, dQ and dK / dV: D 64 BH 88 S 1368
+// with dropout 62.0 / 53.9, 81.8 / 67.5, BH 40 S 1088 30.3 / 24.6, 38.1 / 31.7, BH 128 S 512 17.6 / 15.2, 21.0 / 17.1; D 128 BH 12
+// S 3584 101 / 83 and, persistent, 99; a single tile a compute unit, BH 16 S 2816, level).
+template <bool CAUSAL> FMHA_DEV void bwd_item(const BwdArgs &a, int &bh, int &pi, int &npass) {
+  int bid = blockIdx.x;
+  const int nb = gridDim.x;
+  const bool paired = CAUSAL && a.pair;
+  if (CAUSAL && !paired) { // (groups of heads that keep to their XCDs: workgroups go to XCDs by turns)
+    const int tz = __builtin_ctz((unsigned)a.bh), lg = tz < 3 ? tz : 3, m = bid >> lg, heads = a.bh >> lg;
+    pi = m / heads;
+    bh = ((m - pi * heads) << lg) + (bid & ((1 << lg) - 1));
+    npass = 1;
+    return;
+  }
+  if ((nb & 7) == 0) bid = (bid & 7) * (nb >> 3) + (bid >> 3);
+  const int npair = paired ? (a.ntile + 1) / 2 : a.ntile;
+  bh = bid / npair;
+  pi = bid - bh * npair;
+  npass = (paired && a.ntile - 1 - pi != pi) ? 2 : 1;
+}
+
 // BwdArgs::flags
 enum { kBwdFlagNoTrim = 1 }; // visit every key tile even where a per-key mask hard-masks the tail
 
@@ -173,18 +198,8 @@ __global__ __launch_bounds__(NW * 64)
   const int tid = threadIdx.x;
   const int w = tid >> 6, l = tid & 63, ql = l & 31, h = l >> 5;
 
-  int bid = blockIdx.x;
-  const int nb = gridDim.x;
-  if ((nb & 7) == 0) bid = (bid & 7) * (nb >> 3) + (bid >> 3);
-  // With a causal mask the work of a query tile grows with its index, so a workgroup takes a
-  // pair of tiles (i, n-1-i), one after the other: every workgroup then has the same amount of
-  // work (the host launches ceil(n/2) workgroups per head; it does so when that still fills the
-  // device, otherwise one tile per workgroup, longest first).
-  const bool paired = CAUSAL && a.pair;
-  const int npair = paired ? (a.ntile + 1) / 2 : a.ntile;
-  const int bh = bid / npair;
-  const int pi = bid - bh * npair;
-  const int npass = (paired && a.ntile - 1 - pi != pi) ? 2 : 1;
+  int bh, pi, npass;
+  bwd_item<CAUSAL>(a, bh, pi, npass);
   MaskTail<T, NT> tail;
   int live_keys = a.sk; // the mask's own count of keys worth visiting
   if (MASK == kMaskPerKey) tail.issue(a, (const T *)a.mask + (size_t)(bh / a.mask_div) * a.mask_sb, tid);
@@ -519,15 +534,8 @@ __global__ __launch_bounds__(NW * 64)
   if (a.ws != nullptr && l == 0) tl[0] = __builtin_amdgcn_s_memrealtime();
   stamp();
 #endif
-  int bid = blockIdx.x;
-  const int nb = gridDim.x;
-  if ((nb & 7) == 0) bid = (bid & 7) * (nb >> 3) + (bid >> 3);
-  // causal: a pair of key tiles (i, n-1-i) per workgroup, as in the dQ kernel
-  const bool paired = CAUSAL && a.pair;
-  const int npair = paired ? (a.ntile + 1) / 2 : a.ntile;
-  const int bh = bid / npair;
-  const int pi = bid - bh * npair;
-  const int npass = (paired && a.ntile - 1 - pi != pi) ? 2 : 1;
+  int bh, pi, npass;
+  bwd_item<CAUSAL>(a, bh, pi, npass);
   MaskTail<T, NT> tail;
   int live_keys = a.sk; // the mask's own count of keys worth visiting
   if (MASK == kMaskPerKey) tail.issue(a, (const T *)a.mask + (size_t)(bh / a.mask_div) * a.mask_sb, tid);

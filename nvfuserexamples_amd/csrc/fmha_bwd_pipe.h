@@ -122,14 +122,8 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(bwd_dq_
   const int tid = threadIdx.x;
   const int w = tid >> 6, l = tid & 63, ql = l & 31, h = l >> 5;
 
-  int bid = blockIdx.x;
-  const int nb = gridDim.x;
-  if ((nb & 7) == 0) bid = (bid & 7) * (nb >> 3) + (bid >> 3);
-  const bool paired = CAUSAL && a.pair;
-  const int npair = paired ? (a.ntile + 1) / 2 : a.ntile;
-  const int bh = bid / npair;
-  const int pi = bid - bh * npair;
-  const int npass = (paired && a.ntile - 1 - pi != pi) ? 2 : 1;
+  int bh, pi, npass;
+  bwd_item<CAUSAL>(a, bh, pi, npass);
 
   const T *Qb = (const T *)a.q + RW::head(a.mq, bh, a.sq);
   const T *Ob = (const T *)a.o + RW::head(a.mo, bh, a.sq);
@@ -487,14 +481,8 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(bwd_dkd
   const int tid = threadIdx.x;
   const int w = tid >> 6, l = tid & 63, kl = l & 31, h = l >> 5;
 
-  int bid = blockIdx.x;
-  const int nb = gridDim.x;
-  if ((nb & 7) == 0) bid = (bid & 7) * (nb >> 3) + (bid >> 3);
-  const bool paired = CAUSAL && a.pair;
-  const int npair = paired ? (a.ntile + 1) / 2 : a.ntile;
-  const int bh = bid / npair;
-  const int pi = bid - bh * npair;
-  const int npass = (paired && a.ntile - 1 - pi != pi) ? 2 : 1;
+  int bh, pi, npass;
+  bwd_item<CAUSAL>(a, bh, pi, npass);
 
   const T *Qb = (const T *)a.q + RW::head(a.mq, bh, a.sq);
   const T *dOb = (const T *)a.dout + RW::head(a.mdo, bh, a.sq);

@@ -60,14 +60,8 @@ __global__ __launch_bounds__(bwd_wide_threads<D>()) __attribute__((amdgpu_waves_
   const bool roleG = (w & 1) != 0; // wave-uniform
   u32x4 *exch = (u32x4 *)(lds + W::OFF_EXCH) + pairi * (NSB * 2 * 64) + l;
 
-  int bid = blockIdx.x;
-  const int nb = gridDim.x;
-  if ((nb & 7) == 0) bid = (bid & 7) * (nb >> 3) + (bid >> 3);
-  const bool paired = CAUSAL && a.pair;
-  const int npair = paired ? (a.ntile + 1) / 2 : a.ntile;
-  const int bh = bid / npair;
-  const int pi = bid - bh * npair;
-  const int npass = (paired && a.ntile - 1 - pi != pi) ? 2 : 1;
+  int bh, pi, npass;
+  bwd_item<CAUSAL>(a, bh, pi, npass);
   MaskTail<T, NT> tail;
   int live_keys = a.sk;
   if (MASK == kMaskPerKey) tail.issue(a, (const T *)a.mask + (size_t)(bh / a.mask_div) * a.mask_sb, tid);
