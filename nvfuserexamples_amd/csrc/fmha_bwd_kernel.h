@@ -98,12 +98,13 @@ FMHA_DEV int bwd_valid_keys(const BwdArgs &a, int bh) {
 // a compute unit's second workgroup is as short as its first is long (us, head by head / so, dQ and dK / dV: D 64 BH 88 S 1368
 // with dropout 62.0 / 53.9, 81.8 / 67.5, BH 40 S 1088 30.3 / 24.6, 38.1 / 31.7, BH 128 S 512 17.6 / 15.2, 21.0 / 17.1; D 128 BH 12
 // S 3584 101 / 83 and, persistent, 99; a single tile a compute unit, BH 16 S 2816, level).
-template <bool CAUSAL> FMHA_DEV void bwd_item(const BwdArgs &a, int &bh, int &pi, int &npass) {
+// TWO: two workgroups share a compute unit.
+template <bool CAUSAL, bool TWO> FMHA_DEV void bwd_item(const BwdArgs &a, int &bh, int &pi, int &npass) {
   int bid = blockIdx.x;
   const int nb = gridDim.x;
   const bool paired = CAUSAL && a.pair;
-  if (CAUSAL && !paired) { // (groups of heads that keep to their XCDs: workgroups go to XCDs by turns)
-    const int tz = __builtin_ctz((unsigned)a.bh), lg = tz < 3 ? tz : 3, m = bid >> lg, heads = a.bh >> lg;
+  if (CAUSAL && !paired) {
+    const int lg = head_groups_log2(a.bh), m = TWO ? by_length(bid, nb, lg) : bid >> lg, heads = a.bh >> lg;
     pi = m / heads;
     bh = ((m - pi * heads) << lg) + (bid & ((1 << lg) - 1));
     npass = 1;
@@ -199,7 +200,7 @@ __global__ __launch_bounds__(NW * 64)
   const int w = tid >> 6, l = tid & 63, ql = l & 31, h = l >> 5;
 
   int bh, pi, npass;
-  bwd_item<CAUSAL>(a, bh, pi, npass);
+  bwd_item<CAUSAL, D != 256>(a, bh, pi, npass);
   MaskTail<T, NT> tail;
   int live_keys = a.sk; // the mask's own count of keys worth visiting
   if (MASK == kMaskPerKey) tail.issue(a, (const T *)a.mask + (size_t)(bh / a.mask_div) * a.mask_sb, tid);
@@ -535,7 +536,7 @@ __global__ __launch_bounds__(NW * 64)
   stamp();
 #endif
   int bh, pi, npass;
-  bwd_item<CAUSAL>(a, bh, pi, npass);
+  bwd_item<CAUSAL, D != 256>(a, bh, pi, npass);
   MaskTail<T, NT> tail;
   int live_keys = a.sk; // the mask's own count of keys worth visiting
   if (MASK == kMaskPerKey) tail.issue(a, (const T *)a.mask + (size_t)(bh / a.mask_div) * a.mask_sb, tid);

@@ -219,7 +219,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu((QB == 
   static_assert(!DEAL || (CAUSAL && MASK == kMaskNone), "");
   constexpr bool deal = DEAL;
   const int dlog = deal ? a.deal - 1 : 0, dgrp = (int)blockIdx.x & ((1 << dlog) - 1); // (workgroups go to XCDs by turns)
-  const int dwg = (int)blockIdx.x >> dlog, dG = G >> dlog, dheads = a.deal_heads;
+  const int dwg = by_length((int)blockIdx.x, G, dlog), dG = G >> dlog, dheads = a.deal_heads;
   auto dealt = [&](int ord) -> int { return ord * dG + ((ord & 1) ? dG - 1 - dwg : dwg); };
   auto exists = [&](int ord) -> bool { return deal ? dealt(ord) < dheads * a.nqt : lb + ord * G < nitems; };
 
