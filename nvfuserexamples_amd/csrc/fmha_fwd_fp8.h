@@ -118,16 +118,18 @@ __global__ __launch_bounds__(Fp8Cfg<D>::NT, D == 64 ? (CAUSAL ? 3 : 4) : 2) void
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63, ql = l & 31, h = l >> 5;
   const int nqt = (a.sq + QT - 1) / QT;
   // Workgroups are dealt round-robin to the 8 XCDs: of every 8 heads each XCD gets one with all its query tiles, so a
-  // head's keys go through one L2, and heads of different lengths stay spread evenly.  Causal: the heads that an XCD
-  // gets from 32 workgroups on (one per compute unit) have the opposite order of tiles, so that a compute unit's
-  // workgroups add up alike, and the last ones go from long to short (all heads long to short: 1.46x the time of the
-  // plain order at BH 32 S 2048 D 64).
+  // head's keys go through one L2, and heads of different lengths stay spread evenly.  Causal: the longest tiles of all heads
+  // first (us, against heads in turn with the order of tiles reversed from 32 workgroups of an XCD to the next: D 64 BH 20 S 4000
+  // 65.9 / 48.6, BH 128 S 2048 76.9 / 62.0, BH 512 S 1024 79.2 / 71.3, BH 240 S 552 24.2 / 20.0; D 128 BH 64 S 1524 49.4 / 40.0, BH
+  // 32 S 3616 97.1 / 81.9, BH 304 S 400 31.7 / 27.4, BH 8 S 8000 122 / 123).
   const int b = blockIdx.x, grouped = (a.bh & ~7) * nqt;
-  const int bh = b < grouped ? b / (8 * nqt) * 8 + (b & 7) : b / nqt;
+  int bh = b < grouped ? b / (8 * nqt) * 8 + (b & 7) : b / nqt;
   int qt = b < grouped ? (b >> 3) % nqt : b % nqt;
   if (CAUSAL) {
-    const int after = b < grouped ? (a.bh >> 3) - 1 - (b >> 3) / nqt : 0; // heads this XCD gets after this one
-    if (!((nqt >= 32 ? after : after * nqt / 32) & 1)) qt = nqt - 1 - qt;
+    const int lg = head_groups_log2(a.bh), m = by_length(b, (int)gridDim.x, lg), heads = a.bh >> lg;
+    qt = m / heads;
+    bh = ((m - qt * heads) << lg) + (b & ((1 << lg) - 1));
+    qt = nqt - 1 - qt;
   }
   const int q = qt * QT + w * 32 + ql;
   const int qc = q < a.sq ? q : a.sq - 1;
