@@ -635,16 +635,22 @@ int fmha_fwd_launch(const fmha_fwd_params *caller, void *hip_stream) {
   // dropout -- the pipelined kernel's finer overlap counts for more (us, this / pipelined: BH 512 S 256 20.0 / 17.1, S 230 21.2 /
   // 18.0, causal BH 512 18.1 / 17.4, BH 1024 30.8 / 29.6) until workgroups are many (BH 2048 S 256 57.3 / 61.4, BH 1024 S 230
   // 29.7 / 32.3; causal with a mask or key counts BH 1024 S 256 30.3 / 34.7), and on few heads from seven blocks on (BH 24 S 200
-  // 6.4 / 6.2, BH 64 512 x 256 7.5 / 7.1; S 160 5.4 / 6.1).
+  // 6.4 / 6.2, BH 64 512 x 256 7.5 / 7.1; S 160 5.4 / 6.1).  Dropout without a mask or key counts follows that line too (S 256 BH 300
+  // 20.5 / 20.3, BH 512 23.9 / 21.3, BH 768 33.3 / 32.6, BH 1280 52.3 / 53.3, BH 2048 80.8 / 83.2; S 230 BH 512 22.5 / 21.0, BH 1024 40.3 /
+  // 41.8), under the causal mask from three workgroups a compute unit on (S 256 BH 300 17.2 / 15.9, BH 512 20.4 / 19.6, BH 640 26.9 /
+  // 25.3, BH 768 28.6 / 29.8, BH 1280 43.7 / 48.5); with a mask or key counts this one is ahead (S 256 BH 300 21.2 / 24.3, causal 18.1 /
+  // 23.3, BH 1024 40.6 / 44.4, with key counts 41.0 / 42.6, but BH 512 23.6 / 22.1).
   v.mid = 0;
   if (p->d == 64 && p->sk > 128 && p->sk <= 256 && p->sq > 128 && v.mask != kMaskFull && v.drop != 2 && !saving && !v.head &&
       overrides().fwd_short == 1) {
     const int cus = cu_count();
-    const bool plain = v.mask == kMaskNone && v.drop == 0;
+    const bool plain = v.mask == kMaskNone && v.drop == 0, open = v.mask == kMaskNone && !p->kv_len;
+    const long long groups = (long long)p->bh * ((p->sq + 255) / 256);
     if ((long long)p->bh * ((p->sq + 127) / 128) <= cus) v.mid = plain && !v.causal && p->sk > 192 ? 0 : 4;
-    else if (v.drop != 0 || p->sk <= 224) v.mid = 8;
-    else if (v.causal) v.mid = plain && !p->kv_len ? 0 : 8;
-    else v.mid = (long long)p->bh * ((p->sq + 255) / 256) >= 4LL * cus ? 8 : 0;
+    else if (p->sk <= 224) v.mid = 8;
+    else if (v.drop != 0) v.mid = !open || groups >= (v.causal ? 3LL : 4LL) * cus ? 8 : 0;
+    else if (v.causal) v.mid = open ? 0 : 8;
+    else v.mid = groups >= 4LL * cus ? 8 : 0;
   }
 
   int rc;
