@@ -64,6 +64,7 @@ struct Fp8Args {
 constexpr float kFp8Hard = -9000.f, kFp8Live = -1000.f, kFp8TrimScore = 3900.f;
 
 typedef int i32x8 __attribute__((ext_vector_type(8)));
+typedef int i32x4v __attribute__((ext_vector_type(4)));
 typedef int i32x2v __attribute__((ext_vector_type(2)));
 
 template <int D> struct Fp8Cfg {
@@ -81,6 +82,10 @@ template <int D> struct Fp8Cfg {
 FMHA_DEV f32x16 mfma_fp8_k64(i32x8 a, i32x8 b, f32x16 c) {
   return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, c, 0, 0, 0, 0, 0, 0);
 }
+// 16x16 = (16 x 128 e2m1) . (128 x 16 e4m3); the 4-bit operand takes the first half of its registers
+FMHA_DEV f32x4 mfma_fp4_fp8_k128(i32x4v a, i32x8 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(i32x8{a.x, a.y, a.z, a.w, 0, 0, 0, 0}, b, c, 4, 0, 0, 0, 0, 0);
+}
 FMHA_DEV i32x2v lds_read_tr8(const char *lds_ptr) {
   typedef __attribute__((address_space(3))) i32x2v lds_vec;
   return __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_vec *)(lds_ptr));
@@ -88,7 +93,8 @@ FMHA_DEV i32x2v lds_read_tr8(const char *lds_ptr) {
 
 // Four floats to four e4m3 bytes (round to nearest even), element 0 in the lowest byte.
 FMHA_DEV int pack4_e4m3(float a, float b, float c, float d) {
-  int w = 0;
+  int w;
+  asm("" : "=v"(w) : "v"(a)); // (any register: both halves are written, nothing has to be cleared first)
   w = __builtin_amdgcn_cvt_pk_fp8_f32(a, b, w, false);
   w = __builtin_amdgcn_cvt_pk_fp8_f32(c, d, w, true);
   return w;
@@ -208,6 +214,13 @@ __global__ __launch_bounds__(Fp8Cfg<D>::NT, D == 64 ? (CAUSAL ? 3 : 4) : 2) void
     for (int r = 0; r < 16; ++r) oacc[db][r] = 0.f;
   float M = 0.f, l_run = 0.f, l_true = 0.f; // reference exponent (an integer); sums of the rounded / unrounded probabilities relative to it
   bool seen = false;          // M has been set from a tile with a live key
+  // Row sums: the rounded tile's registers, read as the 128 x 16 operand of the 16x16 product, hold in column c and
+  // lane group j (lane 16 j + c) the probabilities of query c + 16 (j & 1).  Rows 4 i .. 4 i + 3 of the other operand are ones
+  // in the contraction indices of groups of i's parity, and come out in the lanes 16 i + c: every lane gets the whole sum of
+  // its own row.  (As measured: index k belongs to group k / 16 % 4 in an 8-bit operand, to register k / 8 % 4 of group
+  // k / 32 in a 4-bit one.)
+  const int one0 = (l >> 2) & 1 ? 0 : 0x22222222, one1 = 0x22222222 - one0; // (1.0 in e2m1)
+  const i32x4v ones = {one0, one0, one1, one1};
   const uint32_t bx0 = h == 0 ? 0x3f803f80u : 0u, bx1 = h == 0 ? 0x3f80u : 0u; // extra-step column of a query: bf16 (1, 1, 1, 0 ..)
   // the columns of the extra-step rows that stay zero
   if (tid < 2 * BK) {
@@ -291,7 +304,6 @@ __global__ __launch_bounds__(Fp8Cfg<D>::NT, D == 64 ? (CAUSAL ? 3 : 4) : 2) void
     // register r of block sb is key k0 + 32 sb + 8 (r / 4) + 4 h + r % 4
     const bool diag = CAUSAL && (k0 + BK - 1 > qt * QT + w * 32);
     const bool want_lse = a.lse != nullptr;
-    float psum = 0.f; // unrounded row sum of the tile, only where the LSE is wanted
     const int own = q - k0 - 4 * h; // causal: the lane's last visible key, in its own order
     auto hide_later_keys = [&](f32x16 (&v)[2]) {
 #pragma unroll
@@ -302,39 +314,56 @@ __global__ __launch_bounds__(Fp8Cfg<D>::NT, D == 64 ? (CAUSAL ? 3 : 4) : 2) void
           asm volatile("" : "+v"(v[sb][r])); // (a branch: as selects every tile would pay two instructions per element)
         }
     };
+    // the largest score of the tile in log2 units, mask term included
+    auto row_max = [&](const f32x16 (&v)[2]) {
+      float m0 = NEG_INF, m1 = NEG_INF;
+#pragma unroll
+      for (int r = 0; r < 16; r += 2) {
+        m0 = max3(m0, v[0][r], v[0][r + 1]);
+        m1 = max3(m1, v[1][r], v[1][r + 1]);
+      }
+      return xhalf_max(fmaxf(m0, m1)) * s;
+    };
+    // unrounded row sum (this half-wave's share), on four accumulators
+    auto add_up = [&](const f32x16 (&v)[2]) {
+      float t[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int sb = 0; sb < 2; ++sb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) t[r & 3] += v[sb][r];
+      return (t[0] + t[1]) + (t[2] + t[3]);
+    };
     if (diag) hide_later_keys(x);
+    // a row's first tile with a key that is not masked out sets its reference (wave-uniform branch: as a rule the first tile's only)
+    if (__builtin_amdgcn_ballot_w64(!seen)) {
+      const float mx = row_max(x);
+      if (!seen && mx > -1e20f) {
+        M = __builtin_ceilf(mx); // (nothing has been accumulated before)
+        seen = true;
+      }
+    }
 #pragma unroll
     for (int sb = 0; sb < 2; ++sb)
 #pragma unroll
       for (int r = 0; r < 16; ++r) x[sb][r] = fast_exp2(fmaf(x[sb][r], s, -M));
-    if (want_lse) {
-#pragma unroll
-      for (int sb = 0; sb < 2; ++sb)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) psum += x[sb][r];
-    }
+    float psum = 0.f;
+    if (want_lse) psum = add_up(x);
     i32x8 pb;
 #pragma unroll
     for (int sb = 0; sb < 2; ++sb)
 #pragma unroll
       for (int g = 0; g < 4; ++g) pb[sb * 4 + g] = pack4_e4m3(x[sb][4 * g], x[sb][4 * g + 1], x[sb][4 * g + 2], x[sb][4 * g + 3]);
-    // sum of the rounded probabilities of this lane's row over the tile: ones . P~ (every row of the result alike)
-    const i32x8 ones = {0x38383838, 0x38383838, 0x38383838, 0x38383838, 0x38383838, 0x38383838, 0x38383838, 0x38383838};
-    f32x16 zero;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) zero[r] = 0.f;
-    float tsum = mfma_fp8_k64(ones, pb, zero)[0];
-    // Slow path, wave-uniform: the first tile of a row (no reference yet), or a row sum beyond the range that
-    // guarantees representable probabilities (compared as bit patterns: the sum is never negative, and a NaN
-    // from a saturated conversion must take this path although the build tells the compiler that NaNs do not
-    // occur).  The scores are recomputed from the operands (the fast path has
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    float tsum = mfma_fp4_fp8_k128(ones, pb, zero)[0]; // of the rounded probabilities of this lane's row
+    // Slow path, wave-uniform: a row sum beyond the range that guarantees representable probabilities (compared as
+    // bit patterns: the sum is never negative, and a NaN from a saturated conversion must take this path although the
+    // build tells the compiler that NaNs do not occur).  The scores are recomputed from the operands (the fast path has
     // overwritten them), the reference becomes ceil(max), everything is rescaled by the exact power of two.
     // Only the rows that need it change their reference (and take the recomputed probabilities): a row's result
     // depends on that row alone, whatever rows share its wave.
-    const bool need = !seen || __float_as_uint(tsum) > __float_as_uint(SUM_LIMIT);
+    const bool need = __float_as_uint(tsum) > __float_as_uint(SUM_LIMIT);
     if (__builtin_amdgcn_ballot_w64(need)) {
       f32x16 y[2];
-      float mx = NEG_INF;
 #pragma unroll
       for (int sb = 0; sb < 2; ++sb) {
 #pragma unroll
@@ -352,24 +381,13 @@ __global__ __launch_bounds__(Fp8Cfg<D>::NT, D == 64 ? (CAUSAL ? 3 : 4) : 2) void
         }
       }
       if (diag) hide_later_keys(y);
+      const float mx = row_max(y), Mn = need ? fmaxf(M, __builtin_ceilf(mx)) : M;
+      const float alpha = fast_exp2(M - Mn); // (1 where the reference stays)
 #pragma unroll
       for (int sb = 0; sb < 2; ++sb)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) mx = fmaxf(mx, y[sb][r]);
-      mx = xhalf_max(mx) * s; // the largest score of the tile in log2 units, mask term included
-      const bool live = mx > -1e20f; // this tile shows the row a key that is not masked out
-      float Mn = M;
-      if (need && live) Mn = seen ? fmaxf(M, __builtin_ceilf(mx)) : __builtin_ceilf(mx);
-      const float alpha = seen ? fast_exp2(M - Mn) : 1.f; // (nothing has been accumulated before the first live tile; 1 where the reference stays)
-      float psum_new = 0.f;
-#pragma unroll
-      for (int sb = 0; sb < 2; ++sb)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const float p = live ? fast_exp2(fmaf(y[sb][r], s, -Mn)) : 0.f;
-          y[sb][r] = p;
-          psum_new += p;
-        }
+        for (int r = 0; r < 16; ++r) y[sb][r] = fast_exp2(fmaf(y[sb][r], s, -Mn));
+      const float psum_new = add_up(y);
       psum = need ? psum_new : psum;
 #pragma unroll
       for (int sb = 0; sb < 2; ++sb)
@@ -378,7 +396,7 @@ __global__ __launch_bounds__(Fp8Cfg<D>::NT, D == 64 ? (CAUSAL ? 3 : 4) : 2) void
           const int pn = pack4_e4m3(y[sb][4 * g], y[sb][4 * g + 1], y[sb][4 * g + 2], y[sb][4 * g + 3]);
           pb[sb * 4 + g] = need ? pn : pb[sb * 4 + g]; // (both half-waves of a row decide alike: the sums they test are the row's)
         }
-      tsum = mfma_fp8_k64(ones, pb, zero)[0];
+      tsum = mfma_fp4_fp8_k128(ones, pb, zero)[0];
       l_run *= alpha;
       l_true *= alpha;
 #pragma unroll
@@ -386,10 +404,9 @@ __global__ __launch_bounds__(Fp8Cfg<D>::NT, D == 64 ? (CAUSAL ? 3 : 4) : 2) void
 #pragma unroll
         for (int r = 0; r < 16; ++r) oacc[db][r] *= alpha;
       M = Mn;
-      seen = seen || (need && live);
     }
     l_run += tsum;
-    if (want_lse) l_true += xhalf_sum(psum);
+    if (want_lse) l_true += psum;
     // O^T += V^T.P^T: one K = 64 product per 32 head-dim columns
 #pragma unroll
     for (int db = 0; db < DB; ++db) {
@@ -411,6 +428,7 @@ __global__ __launch_bounds__(Fp8Cfg<D>::NT, D == 64 ? (CAUSAL ? 3 : 4) : 2) void
     __syncthreads();
   }
 
+  l_true = xhalf_sum(l_true);
   // normalise and store: in the accumulator layout lane (q, h) holds head-dim columns 8g + 4h .. +3 of each 32-block
   if (q < a.sq) {
     const float inv = l_run > 0.f ? a.out_scale / l_run : 0.f;
