@@ -21,10 +21,12 @@
 // (three bf16 pieces: exact to fp32); tiles whose keys are all there and unmasked -- most of a padded batch --
 // go without.  Key tiles of nothing but hard-masked keys at the end of a mask row are not visited where their
 // weights are zero whatever the inputs (Fp8Args::trim).
-// BH 512 S 512 D 64, before and now on one card: with masks whose lengths are spread over [256, 512] 45.5 -> 35.2 us, without a
-// mask 39.9 -> 34.1 us (other cards: 47.7-48.8 -> 36.2-38.1 and 43.2 -> 37.9);
-// BH 32 S 4096 D 128 causal 211 -> 108 us, BH 32 S 2048 D 64 causal 48.1 -> 28.5 us (the key-after-query test of the
-// diagonal tiles used to cost every tile two instructions per element; waves leave out the tiles past their own rows).
+// Counted at BH 156 S 2432 D 64: 163 vector instructions a tile and wave, 112 of them those above (an exponential and a
+// packed conversion take the pipe about nine cycles, the others four), the vector pipe busy 74 % of the launch, the matrix
+// pipe 25 %; clearing the conversions' registers, copies of the operand of ones and the first tile's second computation
+// were the rest.  Without them 167 -> 154 us; BH 512 S 512 with masks whose lengths are spread over [256, 512] 38.0 -> 34.0,
+// without a mask 38.4 -> 33.3.  (A loop that skews the products of the tiles before and after against a tile's exponentials
+// inside a wave, at two waves a SIMD for its registers, lost: 154 -> 167, D 128 BH 384 S 960 138 -> 154.)
 // The registers are held to four waves per SIMD at head dim 64, three where causal (a tighter budget spills in the loop).
 // The row sums come out of the matrix pipe too:
 // one more fp8 product of the rounded tile with an operand of ones gives every lane the sum of ITS row's
@@ -60,6 +62,7 @@ struct Fp8Args {
   // inputs: a hard-masked key's exponent is then at least 200 (288 in log2 units) below the row's reference, less the 8
   // that the reference may sit below the maximum, so its probability is 0 in fp32 and leaving it out changes nothing.
   int32_t trim;
+  int32_t split; // the waves of a workgroup share 32 queries and take their key tiles in turn
 };
 constexpr float kFp8Hard = -9000.f, kFp8Live = -1000.f, kFp8TrimScore = 3900.f;
 
@@ -67,14 +70,23 @@ typedef int i32x8 __attribute__((ext_vector_type(8)));
 typedef int i32x4v __attribute__((ext_vector_type(4)));
 typedef int i32x2v __attribute__((ext_vector_type(2)));
 
-template <int D> struct Fp8Cfg {
-  static constexpr int NW = 4, NT = NW * 64, QT = NW * 32, BK = 64;
+// SPLIT: the four waves of a workgroup take the key tiles of the same 32 queries in turn instead of 32 queries each, every
+// wave with an LDS stage of its own (no barrier), and their partial rows meet in LDS at the end.  A tile takes a wave
+// that has its SIMD to itself 0.8 us from end to end, so a launch of few workgroups lasts as long as its longest row of
+// tiles: four times the workgroups of a quarter of the tiles each use the idle units.  Large launches keep the other
+// form (K and V are staged once per 128 queries there, not per 32; D 64 BH 512 S 512 34.5 / 52.8 us).  The line between them: fp8_split in
+// fmha_capi.hip.  Before / now, us: BH 8 S 3712 D 64 causal 44.2 / 20.2, BH 16 S 2013 25.3 / 22.8, S 600 causal 10.0 / 6.8.
+template <int D, bool SPLIT> struct Fp8Cfg {
+  static constexpr int NW = 4, NT = NW * 64, QT = SPLIT ? 32 : NW * 32, BK = 64;
   static constexpr int PITCH = D + 16;              // bytes per key row of the K and V tiles (16 rows, 16 bank groups)
   static constexpr int TILEB = BK * PITCH;
-  static constexpr int XROWB = 32;                   // extra-step row of a key: 16 bf16
+  static constexpr int XROWB = 16;                  // extra-step row of a key: 8 bf16
   static constexpr int LDS_FLAG = 2 * TILEB + BK * XROWB; // (in a stage) whether the tile takes the extra step
-  static constexpr int STAGEB = LDS_FLAG + 16;       // K tile, V tile, extra-step rows of the tile, flag
-  static constexpr int LDS_TRIM = 2 * STAGEB;        // per wave: keys up to its last live one, whether it saw a visible one
+  static constexpr int STAGEB = LDS_FLAG + 16;      // K tile, V tile, extra-step rows of the tile, flag
+  static constexpr int NSTAGE = SPLIT ? NW : 2;     // one for each wave / two that all waves share
+  static constexpr int LDS_MERGE = NW * 32 * D * 4; // SPLIT, over the stages: the waves' outputs, then their rows' sums
+  static constexpr int LDS_TILES = SPLIT && NSTAGE * STAGEB < LDS_MERGE + NW * 3 * 32 * 4 ? LDS_MERGE + NW * 3 * 32 * 4 : NSTAGE * STAGEB;
+  static constexpr int LDS_TRIM = LDS_TILES;        // per wave: keys up to its last live one, whether it saw a visible one
   static constexpr int LDS_BYTES = LDS_TRIM + 2 * NW * 4;
 };
 
@@ -108,12 +120,14 @@ FMHA_DEV void split3_bf16(float v, __bf16 &hi, __bf16 &mid, __bf16 &lo) {
   lo = (__bf16)(r - (float)mid);
 }
 
-template <typename TO, int D, bool CAUSAL, bool MASK>
-__global__ __launch_bounds__(Fp8Cfg<D>::NT, D == 64 ? (CAUSAL ? 3 : 4) : 2) void fmha_fwd_fp8_kernel(const Fp8Args a) {
-  using C = Fp8Cfg<D>;
+template <typename TO, int D, bool CAUSAL, bool MASK, bool SPLIT>
+__global__ __launch_bounds__((Fp8Cfg<D, SPLIT>::NT), D == 64 ? (SPLIT || CAUSAL ? 3 : 4) : 2) void fmha_fwd_fp8_kernel(const Fp8Args a) {
+  using C = Fp8Cfg<D, SPLIT>;
   constexpr int NT = C::NT, QT = C::QT, BK = C::BK, DS = D / 64, DB = D / 32, PITCH = C::PITCH, XROWB = C::XROWB;
   constexpr int CPR = D / 16;            // 16-byte chunks per row
-  constexpr int CPT = BK * CPR / NT;     // chunks per thread and tile
+  constexpr int TT = SPLIT ? 64 : NT;    // threads that stage a tile
+  constexpr int CPT = BK * CPR / TT;     // chunks per thread and tile
+  constexpr int STEP = SPLIT ? C::NW : 1; // a wave's tiles are this far apart
   static_assert(CPT >= 1, "tile must cover the workgroup");
   constexpr float NEG_INF = -__builtin_inff();
   constexpr float SUM_LIMIT = 256.f;     // a row sum up to here: every probability fits e4m3 (maximum 448)
@@ -122,6 +136,7 @@ __global__ __launch_bounds__(Fp8Cfg<D>::NT, D == 64 ? (CAUSAL ? 3 : 4) : 2) void
 
   const int tid = threadIdx.x;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63, ql = l & 31, h = l >> 5;
+  const int ts = SPLIT ? l : tid; // among the threads that stage a tile
   const int nqt = (a.sq + QT - 1) / QT;
   // Workgroups are dealt round-robin to the 8 XCDs: of every 8 heads each XCD gets one with all its query tiles, so a
   // head's keys go through one L2, and heads of different lengths stay spread evenly.  Causal: the longest tiles of all heads
@@ -137,7 +152,7 @@ __global__ __launch_bounds__(Fp8Cfg<D>::NT, D == 64 ? (CAUSAL ? 3 : 4) : 2) void
     bh = ((m - qt * heads) << lg) + (b & ((1 << lg) - 1));
     qt = nqt - 1 - qt;
   }
-  const int q = qt * QT + w * 32 + ql;
+  const int q0 = qt * QT + (SPLIT ? 0 : w * 32), q = q0 + ql;
   const int qc = q < a.sq ? q : a.sq - 1;
   const float s = a.score_scale_l2, inv_s = a.inv_score_scale_l2;
   // a masked key's term in raw score units: -1e25 in log2 units whatever the scale (kept inside the bf16 range)
@@ -165,40 +180,42 @@ __global__ __launch_bounds__(Fp8Cfg<D>::NT, D == 64 ? (CAUSAL ? 3 : 4) : 2) void
     if (need < nkt) nkt = need;
   }
 
-  // tile staging: global -> registers -> LDS, both tiles as they are in memory; two LDS stages
+  // tile staging: global -> registers -> LDS, both tiles as they are in memory; two LDS stages, or one of the wave's own
   u32x4 kst[CPT], vst[CPT];
   TO mraw = (TO)0.f; // this thread's key's mask value, as it is in memory: whatever is made of it here would wait for it here
+  auto stage_of = [&](int kt) { return lds + (SPLIT ? w : kt & 1) * C::STAGEB; };
   auto gload = [&](int k0) {
 #pragma unroll
     for (int i = 0; i < CPT; ++i) {
-      const int c = tid + i * NT, row = c / CPR, col = c % CPR;
+      const int c = ts + i * TT, row = c / CPR, col = c % CPR;
       int kr = k0 + row;
       kr = kr < a.sk ? kr : a.sk - 1; // keys past the end re-read the last row; their mask term is "-inf"
-      kst[i] = *(const u32x4 *)(Kb + (size_t)kr * D + col * 16);
-      vst[i] = *(const u32x4 *)(Vb + (size_t)kr * D + col * 16);
+      const uint32_t at = (uint32_t)(kr * D + col * 16);
+      kst[i] = *(const u32x4 *)(Kb + at);
+      vst[i] = *(const u32x4 *)(Vb + at);
     }
-    if (MASK && tid < BK) mraw = mkey[k0 + tid < a.sk ? k0 + tid : a.sk - 1];
+    if (MASK && ts < BK) mraw = mkey[k0 + ts < a.sk ? k0 + ts : a.sk - 1];
   };
   auto lstore = [&](int kt) {
-    char *kd = lds + (kt & 1) * C::STAGEB;
+    char *kd = stage_of(kt);
 #pragma unroll
     for (int i = 0; i < CPT; ++i) {
-      const int c = tid + i * NT, row = c / CPR, col = c % CPR;
+      const int c = ts + i * TT, row = c / CPR, col = c % CPR;
       *(u32x4 *)(kd + row * PITCH + col * 16) = kst[i];
       *(u32x4 *)(kd + C::TILEB + row * PITCH + col * 16) = vst[i];
     }
-    if (tid < BK) { // (wave 0) (mk_hi, mk_mid, mk_lo, 0 ...), the term in raw score units
+    if (ts < BK) { // (one wave) (mk_hi, mk_mid, mk_lo, 0 ...), the term in raw score units
       const float mk = (float)mraw;
       float mst = MASK ? (mk == NEG_INF ? BIGNEG_RAW : fmaxf(mk * (FMHA_LOG2E * inv_s), BIGNEG_RAW)) : 0.f;
-      if (kt * BK + tid >= a.sk) mst = BIGNEG_RAW;
+      if (kt * BK + ts >= a.sk) mst = BIGNEG_RAW;
       const bool any = __builtin_amdgcn_ballot_w64(mst != 0.f) != 0;
       if (any) {
         __bf16 hi, mid, lo;
         split3_bf16(mst, hi, mid, lo);
         const uint32_t b0 = __builtin_bit_cast(uint16_t, hi), b1 = __builtin_bit_cast(uint16_t, mid), b2 = __builtin_bit_cast(uint16_t, lo);
-        *(u32x2 *)(kd + 2 * C::TILEB + tid * XROWB) = u32x2{b0 | b1 << 16, b2}; // (the rest of the row stays zero)
+        *(u32x4 *)(kd + 2 * C::TILEB + ts * XROWB) = u32x4{b0 | b1 << 16, b2, 0, 0};
       }
-      if (tid == 0) *(int *)(kd + C::LDS_FLAG) = any;
+      if (ts == 0) *(int *)(kd + C::LDS_FLAG) = any;
     }
   };
 
@@ -221,15 +238,11 @@ __global__ __launch_bounds__(Fp8Cfg<D>::NT, D == 64 ? (CAUSAL ? 3 : 4) : 2) void
   // k / 32 in a 4-bit one.)
   const int one0 = (l >> 2) & 1 ? 0 : 0x22222222, one1 = 0x22222222 - one0; // (1.0 in e2m1)
   const i32x4v ones = {one0, one0, one1, one1};
-  const uint32_t bx0 = h == 0 ? 0x3f803f80u : 0u, bx1 = h == 0 ? 0x3f80u : 0u; // extra-step column of a query: bf16 (1, 1, 1, 0 ..)
-  // the columns of the extra-step rows that stay zero
-  if (tid < 2 * BK) {
-    u32x4 *row = (u32x4 *)(lds + (tid / BK) * C::STAGEB + 2 * C::TILEB + (tid % BK) * XROWB);
-    row[0] = row[1] = u32x4{0, 0, 0, 0};
-  }
-  __syncthreads();
+  // extra-step column of a query: bf16 (1, 1, 1, 0 ..); the other half-wave, which reads the same rows, takes zeros
+  const uint32_t bx0 = h == 0 ? 0x3f803f80u : 0u, bx1 = h == 0 ? 0x3f80u : 0u;
 
-  gload(0);
+  const int first = SPLIT ? w : 0; // this wave's first tile
+  gload(first * BK);
   const bool trim = MASK && !CAUSAL && a.trim && nkt > 1;
   if (trim) {
     int last = 0, seen_live = 0;
@@ -244,9 +257,9 @@ __global__ __launch_bounds__(Fp8Cfg<D>::NT, D == 64 ? (CAUSAL ? 3 : 4) : 2) void
       ((int *)(lds + C::LDS_TRIM))[2 * w + 1] = seen_live;
     }
   }
-  lstore(0);
-  if (nkt > 1) gload(BK);
-  __syncthreads();
+  lstore(first);
+  if (first + STEP < nkt) gload((first + STEP) * BK);
+  if (trim || !SPLIT) __syncthreads();
   if (trim) {
     int last = 0, seen_live = 0;
 #pragma unroll
@@ -259,21 +272,23 @@ __global__ __launch_bounds__(Fp8Cfg<D>::NT, D == 64 ? (CAUSAL ? 3 : 4) : 2) void
     if (__builtin_amdgcn_readfirstlane(seen_live)) nkt = (last + BK - 1) / BK;
   }
 
-  auto stage_next = [&](int kt) { // the next tile goes to the other stage (its last readers passed the barrier that ended the previous iteration)
-    if (kt + 1 < nkt) {
-      lstore(kt + 1);
-      if (kt + 2 < nkt) gload((kt + 2) * BK);
+  // The next tile goes to the other stage, whose last readers passed the barrier that ended the previous iteration; a wave
+  // with a stage of its own overwrites it when it has read it (LDS serves a wave's requests in order).
+  auto stage_next = [&](int kt) {
+    if (kt + STEP < nkt) {
+      lstore(kt + STEP);
+      if (kt + 2 * STEP < nkt) gload((kt + 2 * STEP) * BK);
     }
   };
   // causal: the tiles that hold nothing up to this wave's own rows are left to the waves behind it
   int nktw = nkt;
-  if (CAUSAL) {
-    const int own = (qt * QT + w * 32 + 31) / BK + 1;
+  if (CAUSAL && !SPLIT) {
+    const int own = (q0 + 31) / BK + 1;
     nktw = own < nkt ? own : nkt;
   }
-  for (int kt = 0; kt < nktw; ++kt) {
+  for (int kt = first; kt < nktw; kt += STEP) {
     const int k0 = kt * BK;
-    const char *ldsK = lds + (kt & 1) * C::STAGEB;
+    const char *ldsK = stage_of(kt);
     const char *ldsV = ldsK + C::TILEB;
     const char *ldsX = ldsK + 2 * C::TILEB;
 
@@ -296,13 +311,13 @@ __global__ __launch_bounds__(Fp8Cfg<D>::NT, D == 64 ? (CAUSAL ? 3 : 4) : 2) void
     if (extra) {
 #pragma unroll
       for (int sb = 0; sb < 2; ++sb) {
-        const bf16x8 xa = as_v8<__bf16>(*(const u32x4 *)(ldsX + (sb * 32 + ql) * XROWB + h * 16));
+        const bf16x8 xa = as_v8<__bf16>(*(const u32x4 *)(ldsX + (sb * 32 + ql) * XROWB));
         x[sb] = Elem<__bf16>::mfma(xa, as_v8<__bf16>(u32x4{bx0, bx1, 0, 0}), x[sb]);
       }
     }
-    stage_next(kt); // while this one is worked on
+    if (!SPLIT) stage_next(kt); // while this one is worked on
     // register r of block sb is key k0 + 32 sb + 8 (r / 4) + 4 h + r % 4
-    const bool diag = CAUSAL && (k0 + BK - 1 > qt * QT + w * 32);
+    const bool diag = CAUSAL && (k0 + BK - 1 > q0);
     const bool want_lse = a.lse != nullptr;
     const int own = q - k0 - 4 * h; // causal: the lane's last visible key, in its own order
     auto hide_later_keys = [&](f32x16 (&v)[2]) {
@@ -376,7 +391,7 @@ __global__ __launch_bounds__(Fp8Cfg<D>::NT, D == 64 ? (CAUSAL ? 3 : 4) : 2) void
           y[sb] = mfma_fp8_k64(ka, qreg[ds], y[sb]);
         }
         if (extra) {
-          const bf16x8 xa = as_v8<__bf16>(*(const u32x4 *)(ldsX + (sb * 32 + ql) * XROWB + h * 16));
+          const bf16x8 xa = as_v8<__bf16>(*(const u32x4 *)(ldsX + (sb * 32 + ql) * XROWB));
           y[sb] = Elem<__bf16>::mfma(xa, as_v8<__bf16>(u32x4{bx0, bx1, 0, 0}), y[sb]);
         }
       }
@@ -421,18 +436,68 @@ __global__ __launch_bounds__(Fp8Cfg<D>::NT, D == 64 ? (CAUSAL ? 3 : 4) : 2) void
         }
       oacc[db] = mfma_fp8_k64(va, pb, oacc[db]);
     }
-    __syncthreads(); // this stage is free again, the next one is complete
+    if (SPLIT) {
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      stage_next(kt);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    } else {
+      __syncthreads(); // this stage is free again, the next one is complete
+    }
   }
-  for (int kt = nktw; kt < nkt; ++kt) {
+  if (!SPLIT) for (int kt = nktw; kt < nkt; ++kt) {
     stage_next(kt);
     __syncthreads();
   }
 
   l_true = xhalf_sum(l_true);
+  TO *Or = (TO *)a.o + ((size_t)bh * a.sq + q) * D;
+  if (SPLIT) {
+    // The waves' partial rows meet in LDS: references are integers, so bringing them to the largest is exact.
+    __syncthreads();
+    f32x4 *part = (f32x4 *)lds;
+    float *rows = (float *)(lds + C::LDS_MERGE);
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        part[((w * DB + db) * 4 + g) * 64 + l] = f32x4{oacc[db][4 * g], oacc[db][4 * g + 1], oacc[db][4 * g + 2], oacc[db][4 * g + 3]};
+    if (h == 0) {
+      rows[(w * 3 + 0) * 32 + ql] = seen ? M : NEG_INF;
+      rows[(w * 3 + 1) * 32 + ql] = l_run;
+      rows[(w * 3 + 2) * 32 + ql] = l_true;
+    }
+    __syncthreads();
+    if (w >= DB) return; // a wave for each 32 columns
+    float top = NEG_INF, alpha[C::NW];
+#pragma unroll
+    for (int j = 0; j < C::NW; ++j) top = fmaxf(top, rows[j * 3 * 32 + ql]);
+    M = top == NEG_INF ? 0.f : top;
+    l_run = l_true = 0.f;
+    f32x16 acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+#pragma unroll
+    for (int j = 0; j < C::NW; ++j) {
+      alpha[j] = fast_exp2(rows[j * 3 * 32 + ql] - M);
+      l_run += alpha[j] * rows[(j * 3 + 1) * 32 + ql];
+      l_true += alpha[j] * rows[(j * 3 + 2) * 32 + ql];
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const f32x4 v = part[((j * DB + w) * 4 + g) * 64 + l];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[4 * g + i] += alpha[j] * v[i];
+      }
+    }
+    if (q < a.sq) {
+      const float inv = l_run > 0.f ? a.out_scale / l_run : 0.f;
+      store_acc_block_row<TO>(Or + w * 32, acc, inv, h);
+      if (a.lse && h == 0 && w == 0) a.lse[(size_t)bh * a.sq + q] = l_true > 0.f ? (M + fast_log2(l_true)) * FMHA_LN2 : NEG_INF;
+    }
+    return;
+  }
   // normalise and store: in the accumulator layout lane (q, h) holds head-dim columns 8g + 4h .. +3 of each 32-block
   if (q < a.sq) {
     const float inv = l_run > 0.f ? a.out_scale / l_run : 0.f;
-    TO *Or = (TO *)a.o + ((size_t)bh * a.sq + q) * D;
 #pragma unroll
     for (int db = 0; db < DB; ++db) store_acc_block_row<TO>(Or + db * 32, oacc[db], inv, h);
     if (a.lse && h == 0) a.lse[(size_t)bh * a.sq + q] = l_true > 0.f ? (M + fast_log2(l_true)) * FMHA_LN2 : NEG_INF;

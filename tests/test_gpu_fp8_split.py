@@ -1,0 +1,58 @@
+"""The e4m3 forward whose four waves take the key tiles of 32 queries in turn: waves without a tile, with one, with tiles the
+end of the keys / the diagonal / the masks pass through, rows whose keys are all hidden in some waves' tiles.  Against
+the oracle with the same rounding (bounds as in test_gpu_fp8_tiles.py) and against the form without the split."""
+import numpy as np
+import pytest
+import torch
+
+from nvfuserexamples_amd import capi
+from conftest import f32
+from test_gpu_fp8_tiles import _check, _inputs
+
+pytestmark = pytest.mark.gpu
+
+
+def _both(monkeypatch, *args, **kw):
+    got = []
+    for split in ("1", "0"):
+        monkeypatch.setenv("FMHA_FP8_SPLIT", split)
+        got.append(capi.fwd_fp8(*args, want_lse=True, **kw))
+        torch.cuda.synchronize()
+    monkeypatch.delenv("FMHA_FP8_SPLIT")
+    return got
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("sq,sk,causal", [(1, 1, False), (5, 64, False), (33, 65, False), (32, 256, False), (31, 257, True),
+                                          (70, 193, True), (200, 300, False), (129, 577, True), (40, 1100, False), (300, 40, True)])
+def test_waves_that_split_the_keys(sq, sk, causal, d, monkeypatch):
+    monkeypatch.setenv("FMHA_FWD_DECODE", "0")
+    bh = 3
+    q8, dq, k8, dk, v8, dv = _inputs(bh, sq, sk, d, sq + sk)
+    (o, lse), (o0, lse0) = _both(monkeypatch, q8.cuda(), k8.cuda(), v8.cuda(), dq, dk, dv, causal=causal)
+    monkeypatch.delenv("FMHA_FWD_DECODE")
+    _check(o, lse, q8, dq, k8, dk, v8, dv, d, None, causal)
+    # Partial sums of up to 1 100 fp32 terms in another order (2^-24 sqrt(n) each way, under 1e-5 relative); where a wave's reference lies below the row's,
+    # probabilities that rounded to 2^-9 steps there keep their three mantissa bits: half a step of a weight under 2^-6.
+    vmax = float(v8.float().abs().max()) * dv
+    assert (o.float() - o0.float()).abs().max().item() <= 2.0 ** -10 * vmax + 2.0 ** -10 * o0.float().abs().max().item()
+    assert (lse - lse0).abs().max().item() <= 1e-5 * max(1.0, lse0.abs().max().item())
+
+
+@pytest.mark.parametrize("d,sk", [(64, 300), (128, 577)])
+def test_masked_tiles_of_some_waves(d, sk, monkeypatch):
+    """Rows whose live keys lie in one wave's tiles only, at the start or the end, under -inf and -10000, and rows without any."""
+    spans = [(0, 1), (0, 64), (64, 65), (128, 200), (sk - 1, sk), (sk - 70, sk), (0, sk), (0, 0)]
+    b, sq = len(spans), 45
+    q8, dq, k8, dk, v8, dv = _inputs(b, sq, sk, d, sk)
+    for hidden in (-10000.0, float("-inf")):
+        m = torch.full((b, 1, sk), hidden)
+        for i, (lo, hi) in enumerate(spans):
+            m[i, :, lo:hi] = 0.0
+        m = m.half()
+        (o, lse), (o0, lse0) = _both(monkeypatch, q8.cuda(), k8.cuda(), v8.cuda(), dq, dk, dv, mask=m.cuda())
+        n = b if hidden > float("-inf") else b - 1      # (a row hidden by -inf throughout: zeros and -inf, below)
+        _check(o[:n], lse[:n], q8[:n], dq, k8[:n], dk, v8[:n], dv, d, np.broadcast_to(f32(m[:n]), (n, sq, sk)).copy(), False)
+        if n < b:
+            assert torch.equal(o[n:], torch.zeros_like(o[n:])) and bool(torch.isneginf(lse[n:]).all())
+            assert torch.equal(o0[n:], o[n:]) and torch.equal(lse0[n:], lse[n:])
