@@ -349,6 +349,7 @@ std::tuple<at::Tensor, at::Tensor> fmha_fwd(const at::Tensor &q_, const at::Tens
   set_stride(p.v_stride, v);
   set_stride(p.o_stride, orow);
   p.lse = lse.data_ptr<float>();
+  p.flags = FMHA_FLAG_SPLIT_KEYS; // few heads, not so few query rows
   p.causal = is_causal ? 1 : 0;
   MaskLayout m;
   set_mask_and_dropout(p, m, mask, q, k.s, p_drop, seed, offset);

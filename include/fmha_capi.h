@@ -55,7 +55,11 @@ enum {
  * exceeds every visible key's by more than 8800.  FMHA_FLAG_NO_MASK_TRIM makes them visit every tile
  * regardless. */
 enum {
-  FMHA_FLAG_NO_MASK_TRIM = 1
+  FMHA_FLAG_NO_MASK_TRIM = 1,
+  /* Forward only: a launch of few workgroups may share the keys of 32 queries out to the waves of a workgroup, which
+   * merge their partial sums in fp32.  Up to twice as fast there; without it the bits of a head's result do not depend on
+   * how many heads the launch has (the operators set it). */
+  FMHA_FLAG_SPLIT_KEYS = 4
   /* (value 2 asked for a one-pass backward kernel in earlier versions; it never beat the default and was
    * removed: the bit is accepted and ignored) */
 };
@@ -123,7 +127,7 @@ typedef struct fmha_fwd_params {
   int32_t bh, sq, sk, d;
   int32_t dtype;
   float scale; /* > 0; 1/8 in the reference (fmha_manual.cpp:68) */
-  int32_t flags; /* 0 or FMHA_FLAG_NO_MASK_TRIM */
+  int32_t flags; /* 0 or FMHA_FLAG_NO_MASK_TRIM | FMHA_FLAG_SPLIT_KEYS */
 
   /* Optional valid key counts (the "padded version" the reference leaves as a TODO,
    * fmha_manual.cpp:110,178): head b attends keys [0, kv_len[b / kv_len_bh_div]) only, exactly
@@ -309,7 +313,7 @@ float fmha_drop_scale(float p_drop);
 const char *fmha_strerror(int code);
 
 /* The FMHA_* environment variables -- tuning and test overrides of the variant selection: FMHA_MASK_TRIM,
- * FMHA_FWD_QB, FMHA_FWD_SHORT, FMHA_FWD_STREAM, FMHA_FWD_SAVE_ONCE, FMHA_FWD_SAVE_SPLIT, FMHA_FWD_SPLIT, FMHA_FWD_DECODE, FMHA_FWD_HEAD, FMHA_FP8_SPLIT, FMHA_BWD_SHORT, FMHA_BWD_PAIR
+ * FMHA_FWD_QB, FMHA_FWD_SHORT, FMHA_FWD_STREAM, FMHA_FWD_SAVE_ONCE, FMHA_FWD_SAVE_SPLIT, FMHA_FWD_SPLIT, FMHA_FWD_DECODE, FMHA_FWD_HEAD, FMHA_FWD_FEW, FMHA_FP8_SPLIT, FMHA_BWD_SHORT, FMHA_BWD_PAIR
  * -- are read once per process, on the first launch.  This reads them again; not to be
  * called while another thread is launching.  (No counterpart in the reference.) */
 void fmha_reload_overrides(void);

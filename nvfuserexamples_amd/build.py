@@ -54,6 +54,7 @@ def _tus():
                 tag = f"{'bf16' if bf else 'f16'}_d{d}" + ("_strided" if strided else "")
                 defs = [f"-DFMHA_TU_BF16={bf}", f"-DFMHA_TU_D={d}", f"-DFMHA_TU_STRIDED={strided}"]
                 tus.append(("fmha_fwd.hip", f"fmha_fwd_{tag}.o", defs))
+                tus.append(("fmha_fwd_few.hip", f"fmha_fwd_few_{tag}.o", defs))
                 tus.append(("fmha_bwd.hip", f"fmha_bwd_{tag}.o", defs))
                 if d == 64:
                     tus.append(("fmha_bwd_one.hip", f"fmha_bwd_one_{tag}.o", defs))

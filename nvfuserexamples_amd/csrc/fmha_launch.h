@@ -22,6 +22,7 @@ struct FwdVariant {
   bool many;       // stream: more workgroups than two per compute unit
   bool head;       // up to 512 keys, no / per-key mask, no causal mask: the whole-head kernel (head dim 64, folded layout)
   bool short_keys; // sk <= 128: the one-pass kernel (head dim 64, folded layout)
+  int few;         // few workgroups: waves per workgroup of the kernel whose waves share 32 queries, 0: not that (no full mask tensor, no dropout tensor)
   int mid;         // 129 to 256 keys, no full mask tensor: waves per workgroup of the kernel that has a head's K and V in LDS, 0: not that (head dim 64)
 };
 
@@ -38,6 +39,20 @@ int fwd_dispatch_f16_d64_strided(FwdArgs &a, const FwdVariant &v, hipStream_t s)
 int fwd_dispatch_f16_d128_strided(FwdArgs &a, const FwdVariant &v, hipStream_t s);
 int fwd_dispatch_bf16_d64_strided(FwdArgs &a, const FwdVariant &v, hipStream_t s);
 int fwd_dispatch_bf16_d128_strided(FwdArgs &a, const FwdVariant &v, hipStream_t s);
+
+// The forward whose waves share 32 queries (fmha_fwd_few.hip).
+int fwd_few_launch_f16_d64(FwdArgs &a, const FwdVariant &v, hipStream_t s);
+int fwd_few_launch_f16_d64_strided(FwdArgs &a, const FwdVariant &v, hipStream_t s);
+int fwd_few_launch_bf16_d64(FwdArgs &a, const FwdVariant &v, hipStream_t s);
+int fwd_few_launch_bf16_d64_strided(FwdArgs &a, const FwdVariant &v, hipStream_t s);
+int fwd_few_launch_f16_d128(FwdArgs &a, const FwdVariant &v, hipStream_t s);
+int fwd_few_launch_f16_d128_strided(FwdArgs &a, const FwdVariant &v, hipStream_t s);
+int fwd_few_launch_bf16_d128(FwdArgs &a, const FwdVariant &v, hipStream_t s);
+int fwd_few_launch_bf16_d128_strided(FwdArgs &a, const FwdVariant &v, hipStream_t s);
+int fwd_few_launch_f16_d256(FwdArgs &a, const FwdVariant &v, hipStream_t s);
+int fwd_few_launch_f16_d256_strided(FwdArgs &a, const FwdVariant &v, hipStream_t s);
+int fwd_few_launch_bf16_d256(FwdArgs &a, const FwdVariant &v, hipStream_t s);
+int fwd_few_launch_bf16_d256_strided(FwdArgs &a, const FwdVariant &v, hipStream_t s);
 
 struct BwdVariant {
   int mask;  // kMaskNone / kMaskPerKey / kMaskFull
