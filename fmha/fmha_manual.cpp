@@ -292,7 +292,7 @@ void set_mask_and_dropout(P &p, MaskLayout &m, const c10::optional<at::Tensor> &
 
 
 // The C ABI takes any head dim that is a multiple of 8 up to 256 as it is (rows of whole 16-byte pieces:
-// the kernels run at the next built size, 64 / 128 / 256, and neither read nor write the missing columns).
+// the kernels run at the next built size, 32 / 64 / 96 / 128 / 256, and neither read nor write the missing columns).
 // Only head dims that are not multiples of 8 are zero-padded here, to the next multiple: zero columns add
 // nothing to Q.K^T, the padded columns of V give zero columns of O (and zero columns of dO leave the other
 // gradients untouched), so results are those of the original head dim, at the cost of a copy of every operand.

@@ -86,7 +86,7 @@ enum {
  * so [bh,sq,sk] is (div 1, stride_b sq*sk, stride_q sk), a [B,1,1,sk] padding mask
  * over bh = B*H is (div H, stride_b sk, stride_q 0).
  * Head dim d: 64 in the reference (fmha_manual.cpp:24-29); here any multiple of 8 up to 256.  The kernels
- * are built for 64, 128 and 256; other head dims run at the next of those and neither read nor write
+ * are built for 64, 128 and 256 (without a full mask tensor also for 32 and 96); other head dims run at the next of those and neither read nor write
  * the columns a row does not have (no padded copies), on the run-time-layout code path.  Tensor dropout
  * and the saved outputs exist at d = 64, 128 and 256 only.
  * Computes  O = (dropout(softmax(scale * q k^T + mask_term [+ causal]))) v

@@ -49,8 +49,9 @@ def _tus():
     tus = [("fmha_capi.hip", "fmha_capi.o", []), ("fmha_fwd_fp8.hip", "fmha_fwd_fp8.o", []),
            ("fmha_fwd_decode.hip", "fmha_fwd_decode.o", []), ("fmha_probe.hip", "fmha_probe.o", [])]
     for bf in (0, 1):
-        for d in (64, 128, 256):
-            for strided in (0, 1):  # folded contiguous tensors / row layouts given at run time
+        for d in (32, 64, 96, 128, 256):
+            # folded contiguous tensors / row layouts given at run time (the widths between whole panels: only these)
+            for strided in (0, 1) if d % 64 == 0 else (1,):
                 tag = f"{'bf16' if bf else 'f16'}_d{d}" + ("_strided" if strided else "")
                 defs = [f"-DFMHA_TU_BF16={bf}", f"-DFMHA_TU_D={d}", f"-DFMHA_TU_STRIDED={strided}"]
                 tus.append(("fmha_fwd.hip", f"fmha_fwd_{tag}.o", defs))

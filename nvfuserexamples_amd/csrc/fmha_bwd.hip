@@ -1,5 +1,5 @@
 // Instantiates the backward kernels for one (element type, head dim, row layout kind) triple, chosen
-// with -DFMHA_TU_BF16={0,1} -DFMHA_TU_D={64,128,256} -DFMHA_TU_STRIDED={0,1}, and exports their dispatcher.
+// with -DFMHA_TU_BF16={0,1} -DFMHA_TU_D={32,64,96,128,256} -DFMHA_TU_STRIDED={0,1}, and exports their dispatcher.
 #include "fmha_launch.h"
 #ifndef FMHA_TU_STRIDED
 #define FMHA_TU_STRIDED 0
@@ -56,8 +56,12 @@ template <typename K> int set_lds(K kern, int bytes) {
 //   dK+dV, causal          S 128 27 / 30, S 192 43 / 56, S 256 55 / 71, 2048 heads S 128 with dropout 101 / 126
 //   dK+dV of few heads (one round of workgroups, the plain pipelined kernel): 64 heads S 200 12 / 17, causal 14 / 16
 // The line is 128 queries (192 for causal dK / dV that is not persistent, see fmha_bwd_pipe.hip).
+// At head dim 96 dQ has no line of its own for causal heads, and dK / dV is never pipelined: phase by phase on 32-row tiles it has the
+// registers for two waves per SIMD, pipelined it does not (backward, us, persistent or pipelined / so: BH 512 S 512 padding mask and
+// dropout 316 / 270, without either 265 / 245; causal BH 608 S 365 181 / 158, BH 128 S 1024 with dropout 171 / 154, BH 32 S 3000 232 /
+// 228; BH 576 S 120 56 / 49).
 template <int MASK, bool CAUSAL, int DROP> constexpr bool pipe_built() { return FMHA_TU_D != 256 && MASK != kMaskFull; }
-static inline bool pipe_wanted(const BwdArgs &a) { return FMHA_TU_D == 64 || a.sq >= 128; }
+static inline bool pipe_wanted(const BwdArgs &a) { return FMHA_TU_D <= 64 || a.sq >= 128; }
 // dQ of causal heads at head dim 128 has a line of its own: a pass pays the prologue with all compute units in step, and
 // workgroups take pairs of short streams.  Same measurement (us, pipelined / phase by phase, 512 heads, fp16, in brackets
 // bf16): S 384 107 / 93, S 512 134 / 126 (144 / 117), S 640 170 / 161, S 768 198 / 198 (204 / 195), S 896 257 / 256
@@ -82,7 +86,7 @@ template <int MASK, bool CAUSAL, int DROP> int launch_dq(BwdArgs &a, const BwdVa
   if constexpr (MASK != kMaskFull) { // (pipe_built, or head dim 256, where it is built for dQ only)
     if (pipe_wanted_dq<CAUSAL>(a)) return FMHA_PIPE_NAME(FMHA_TU_TNAME, FMHA_TU_D)(a, v, false, nblk, s);
   }
-  if constexpr (!(pipe_built<MASK, CAUSAL, DROP>() && FMHA_TU_D == 64)) { // (there the pipelined kernel takes all)
+  if constexpr (!(pipe_built<MASK, CAUSAL, DROP>() && FMHA_TU_D <= 64)) { // (there the pipelined kernel takes all)
     constexpr int kLds = BwdCfg<FMHA_TU_D, bwd_dq_tile_rows<FMHA_TU_D>()>::LDS_BYTES;
     static_assert(kLds <= 160 * 1024, "tiles do not fit the LDS of a compute unit");
     auto kern = fmha_bwd_dq_kernel<FMHA_TU_T, FMHA_TU_D, kQB, kNW, MASK, CAUSAL, DROP, kStrided>;
@@ -107,13 +111,13 @@ template <int MASK, bool CAUSAL, int DROP> int launch_dkdv(BwdArgs &a, const Bwd
   // two waves per SIMD, which overlap one workgroup's start and stores with another's arithmetic as the persistent kernel
   // does where there is neither (plain pipelined kernel / this: BH 256 S 1024 343 / 335 us on one card, 347 / 359-369 on another).
   constexpr bool kTwoWaves = bwd_dkdv_small_tiles<FMHA_TU_D, CAUSAL, DROP>();
-  if constexpr (kPipe) {
+  if constexpr (kPipe && FMHA_TU_D != 96) { // (see pipe_wanted)
     if (pipe_wanted(a) && !(kTwoWaves && (MASK != kMaskNone || a.kv_len))) {
       const int rc = FMHA_PIPE_NAME(FMHA_TU_TNAME, FMHA_TU_D)(a, v, true, nblk, s);
-      if (FMHA_TU_D == 64 || rc != kBwdNotHere) return rc;
+      if (FMHA_TU_D <= 64 || rc != kBwdNotHere) return rc;
     }
   }
-  if constexpr (!(kPipe && FMHA_TU_D == 64)) {
+  if constexpr (!(kPipe && FMHA_TU_D <= 64)) {
     using Cfg = BwdCfg<FMHA_TU_D, bwd_dkdv_tile_rows<FMHA_TU_D, CAUSAL, DROP>()>;
     constexpr int kLds = Cfg::LDS_BYTES + (MASK == kMaskFull ? Cfg::MASK_BYTES : 0);
     static_assert(kLds <= 160 * 1024, "tiles do not fit the LDS of a compute unit");
@@ -148,7 +152,7 @@ template <int MASK, bool CAUSAL, int DROP> int launch(BwdArgs &a, const BwdVaria
   }();
   auto blocks = [&](int ntile, bool dq) -> long long {
     const long long tiles = (long long)a.bh * ntile, pairs = (long long)a.bh * ((ntile + 1) / 2), over = tiles - 2LL * cus;
-    const bool by_head = (ntile == 3 || ntile == 5) && ((tiles >= (ntile + 1LL) * cus && (dq || DROP == 0)) || (FMHA_TU_D == 64 && over > 0 && 16 * over <= cus));
+    const bool by_head = (ntile == 3 || ntile == 5) && ((tiles >= (ntile + 1LL) * cus && (dq || DROP == 0)) || (FMHA_TU_D <= 64 && over > 0 && 16 * over <= cus));
     a.ntile = ntile;
     a.pair = kTilesByLength;
     if (CAUSAL && v.pair >= 0) a.pair = v.pair;
@@ -210,8 +214,12 @@ int FMHA_NAME(FMHA_TU_TNAME, FMHA_TU_D)(BwdArgs &a, const BwdVariant &v, hipStre
 #endif
   if (v.mask == kMaskPerKey)
     return v.causal ? by_drop<kMaskPerKey, true>(a, v, s) : by_drop<kMaskPerKey, false>(a, v, s);
+#if FMHA_TU_D % 64 == 0
   if (v.mask == kMaskFull)
     return v.causal ? by_drop<kMaskFull, true>(a, v, s) : by_drop<kMaskFull, false>(a, v, s);
+#else // (full mask tensors: the next whole panel's kernels)
+  if (v.mask == kMaskFull) return 1;
+#endif
   return v.causal ? by_drop<kMaskNone, true>(a, v, s) : by_drop<kMaskNone, false>(a, v, s);
 }
 

@@ -71,7 +71,7 @@ struct BwdArgs {
 // too much, so those keep 64-row tiles at one wave per SIMD.
 template <int D> constexpr int bwd_dq_tile_rows() { return 64; }
 // (Head dim 256 has a dK/dV kernel of its own, fmha_bwd_wide.h.)
-template <int D, bool CAUSAL, int DROP> constexpr bool bwd_dkdv_small_tiles() { return D == 128 && !CAUSAL && DROP == 0; }
+template <int D, bool CAUSAL, int DROP> constexpr bool bwd_dkdv_small_tiles() { return D == 96 || (D == 128 && !CAUSAL && DROP == 0); }
 template <int D, bool CAUSAL, int DROP> constexpr int bwd_dkdv_tile_rows() {
   return bwd_dkdv_small_tiles<D, CAUSAL, DROP>() ? 32 : 64;
 }
@@ -81,7 +81,7 @@ template <int D, int BT_> struct BwdCfg {
   static constexpr int NSB = BT / 32;
   static constexpr int KS = D / 16;
   static constexpr int DB = D / 32;
-  static constexpr int TILEB = BT * D * 2; // swizzled panel layout of fmha_common.h, no padding
+  static constexpr int TILEB = BT * tile_cols(D) * 2; // swizzled panel layout of fmha_common.h, no padding
   static constexpr int XROWB = 32;        // extra-step rows: 16 elements
   // two tiles x 2 stages + two sets of extra rows x 2 stages + {delta} x 2 stages
   static constexpr int LDS_BYTES = 4 * TILEB + 2 * 2 * BT * XROWB + 2 * BT * 4;
@@ -184,7 +184,7 @@ template <typename T> FMHA_DEV void split_hi_lo(float v, T &hi, T &lo) {
 // wave per SIMD, +10 % measured.)
 template <typename T, int D, int QB, int NW, int MASK, bool CAUSAL, int DROP, bool STRIDED>
 __global__ __launch_bounds__(NW * 64)
-    __attribute__((amdgpu_waves_per_eu((D == 128 || MASK == kMaskFull) ? 2 : 1, 2))) void fmha_bwd_dq_kernel(const BwdArgs a) {
+    __attribute__((amdgpu_waves_per_eu((D == 96 || D == 128 || MASK == kMaskFull) ? 2 : 1, 2))) void fmha_bwd_dq_kernel(const BwdArgs a) {
   using RW = Rows<STRIDED, D>;
   using E = Elem<T>;
   using v8 = typename E::v8;
@@ -308,7 +308,7 @@ __global__ __launch_bounds__(NW * 64)
   PanelLane pl;
   pl.init(l);
   TileCopy<T, D, BK, NT> tcopy;
-  tcopy.init(tid, RW::ss(a.mk)); // K and V rows are equally far apart
+  tcopy.init(tid, RW::ss(a.mk), RW::cols(a)); // K and V rows are equally far apart
   auto dma_kv = [&](int kt) {
     const uint32_t dst = lds_base + (uint32_t)(kt & 1) * 2 * TILEB;
     tcopy.issue(Kb, kt * BK, kclamp, dst, tid, RW::cols(a));
@@ -635,8 +635,8 @@ __global__ __launch_bounds__(NW * 64)
   PanelLane pl;
   pl.init(l);
   TileCopy<T, D, BQ, NT> tcopy, tcopy_do; // Q and dO rows need not be equally far apart
-  tcopy.init(tid, RW::ss(a.mq));
-  tcopy_do.init(tid, RW::ss(a.mdo));
+  tcopy.init(tid, RW::ss(a.mq), RW::cols(a));
+  tcopy_do.init(tid, RW::ss(a.mdo), RW::cols(a));
   auto dma_qdo = [&](int qt) {
     const uint32_t dst = lds_base + (uint32_t)(qt & 1) * 2 * TILEB;
     tcopy.issue(Qb, qt * BQ, a.sq, dst, tid, RW::cols(a));

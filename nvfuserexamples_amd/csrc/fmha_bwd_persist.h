@@ -28,7 +28,7 @@ template <int D> struct BwdPersistCfg {
   static constexpr int NW = 4;
   static constexpr int BT = 32, NST = 4; // rows per tile, tiles resident per operand
   static constexpr int KS = D / 16, DB = D / 32;
-  static constexpr int TILEB = BT * D * 2, STAGEB = 2 * TILEB;
+  static constexpr int TILEB = BT * tile_cols(D) * 2, STAGEB = 2 * TILEB;
   static constexpr int QSEG = 1024;                 // queries whose extra-step rows are staged at once
   // tiles, then the K and V rows of the next item (a wave's 32 of each), then the extra-step rows, the raw (LSE, delta) of the
   // segment that comes next, and -delta (dropout; with more than one segment of two, see stage_rows)
@@ -128,7 +128,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(1, 1)))
   qcopy.init(tid, RW::ss(a.mq), a.sq, RW::cols(a));
   dcopy.init(tid, RW::ss(a.mdo), a.sq, RW::cols(a));
   constexpr int VPT = 2 * PipeCopy<T, D, NT>::CPT; // copies per tile pair and wave
-  constexpr int VKV = 2 * (32 * D / 8 / 64);       // copies of a wave's K and V rows
+  constexpr int VKV = 2 * (32 * tile_cols(D) / 8 / 64);       // copies of a wave's K and V rows
   // the stream of tiles: the one that is copied next; behind an item's last turn come the next item's first tiles
   struct {
     const T *q, *d;

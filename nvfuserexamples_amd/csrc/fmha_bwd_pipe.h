@@ -37,7 +37,7 @@ template <int N> FMHA_DEV void bwd_vm_wait() { asm volatile("s_waitcnt vmcnt(%0)
 template <int D> struct BwdPipeCfg {
   static constexpr int BT = 32, NST = 4; // rows per tile, tiles resident per operand
   static constexpr int KS = D / 16, DB = D / 32;
-  static constexpr int TILEB = BT * D * 2, STAGEB = 2 * TILEB;
+  static constexpr int TILEB = BT * tile_cols(D) * 2, STAGEB = 2 * TILEB;
   static constexpr int OFF_X = NST * STAGEB;
   static_assert(4 * RowStore<D>::BYTES <= OFF_X, "the output rows are turned in the tiles' LDS");
   static constexpr int MSEG = 4096;             // per-key mask terms staged at once
@@ -52,8 +52,8 @@ template <int D> struct BwdPipeCfg {
 // row does not have are filled with its first ones: they meet zeros in the register operand, or land in output columns
 // that are not stored.
 template <typename T, int D, int NT> struct PipeCopy {
-  static constexpr int BT = 32, CPT = BT * D / 8 / NT;
-  static_assert(CPT * NT * 8 == BT * D, "tile must divide evenly over the workgroup");
+  static constexpr int BT = 32, CPT = BT * tile_cols(D) / 8 / NT;
+  static_assert(CPT * NT * 8 == BT * tile_cols(D), "tile must divide evenly over the workgroup");
   uint32_t voff[CPT], lim[CPT], dst;
   uint32_t tile_step; // bytes between the first rows of consecutive tiles
   FMHA_DEV void init(int tid, int64_t row_stride, int rend, int dv) {
@@ -98,10 +98,11 @@ struct PhiloxSlices {
 };
 
 // ------------------------------------------------------------------------------ dQ
-// (waves per SIMD: at head dim 256 a wave needs about 400 registers, and the tiles leave room for one workgroup)
-template <int D> constexpr int bwd_dq_pipe_occ() { return D == 256 ? 1 : 2; }
+// (waves per SIMD: at head dim 256 a wave needs about 400 registers, and the tiles leave room for one workgroup; at 32 without a
+// causal mask three waves have the 150 it needs: with dK / dV at three as well BH 512 S 512 backward 96 -> 89 us, BH 1760 S 64 under a padding mask 35 -> 29)
+template <int D, bool CAUSAL> constexpr int bwd_dq_pipe_occ() { return D == 256 ? 1 : D == 32 && !CAUSAL ? 3 : 2; }
 template <typename T, int D, int NW, int MASK, bool CAUSAL, int DROP, bool STRIDED>
-__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(bwd_dq_pipe_occ<D>(), bwd_dq_pipe_occ<D>()))) void fmha_bwd_dq_pipe_kernel(const BwdArgs a) {
+__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(bwd_dq_pipe_occ<D, CAUSAL>(), bwd_dq_pipe_occ<D, CAUSAL>()))) void fmha_bwd_dq_pipe_kernel(const BwdArgs a) {
   using RW = Rows<STRIDED, D>;
   using E = Elem<T>;
   using v8 = typename E::v8;
@@ -113,7 +114,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(bwd_dq_
   static_assert(MASK != kMaskFull, "full mask tensors: fmha_bwd_dq_kernel");
   // Rank-one terms: at head dim 64 the vector pipe is the busier one and they ride in an extra contraction step (XS, GS);
   // at head dim 128 it is the matrix pipe, and a subtraction per element costs less: there only a per-key mask does.
-  constexpr bool XS = D == 64 || MASK == kMaskPerKey, GS = D == 64, LS = D == 64; // (LS: the LSE rides in the extra step)
+  constexpr bool XS = D <= 64 || MASK == kMaskPerKey, GS = D <= 64, LS = D <= 64; // (LS: the LSE rides in the extra step)
 
   extern __shared__ __attribute__((aligned(16))) char lds[];
   uint32_t *ldsM = (uint32_t *)(lds + C::OFF_X + 64); // (mask_hi, mask_lo) per key of the current segment
@@ -123,7 +124,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(bwd_dq_
   const int w = tid >> 6, l = tid & 63, ql = l & 31, h = l >> 5;
 
   int bh, pi, npass;
-  bwd_item<CAUSAL, bwd_dq_pipe_occ<D>() == 2>(a, bh, pi, npass);
+  bwd_item<CAUSAL, bwd_dq_pipe_occ<D, CAUSAL>() == 2>(a, bh, pi, npass);
 
   const T *Qb = (const T *)a.q + RW::head(a.mq, bh, a.sq);
   const T *Ob = (const T *)a.o + RW::head(a.mo, bh, a.sq);
@@ -458,10 +459,11 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(bwd_dq_
 }
 
 // --------------------------------------------------------------------------- dK, dV
-template <int D> constexpr int bwd_dkdv_pipe_occ() { return D == 64 ? 2 : 1; }
+// (with dropout three waves would spill 16 registers: head dim 32 BH 208 S 1602 487 -> 554 us)
+template <int D, bool CAUSAL, int DROP> constexpr int bwd_dkdv_pipe_occ() { return D == 32 && !CAUSAL && DROP == 0 ? 3 : D <= 64 ? 2 : 1; }
 
 template <typename T, int D, int NW, int MASK, bool CAUSAL, int DROP, bool STRIDED>
-__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(bwd_dkdv_pipe_occ<D>(), bwd_dkdv_pipe_occ<D>()))) void fmha_bwd_dkdv_pipe_kernel(const BwdArgs a) {
+__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(bwd_dkdv_pipe_occ<D, CAUSAL, DROP>(), bwd_dkdv_pipe_occ<D, CAUSAL, DROP>()))) void fmha_bwd_dkdv_pipe_kernel(const BwdArgs a) {
   using RW = Rows<STRIDED, D>;
   using E = Elem<T>;
   using v8 = typename E::v8;
@@ -482,7 +484,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(bwd_dkd
   const int w = tid >> 6, l = tid & 63, kl = l & 31, h = l >> 5;
 
   int bh, pi, npass;
-  bwd_item<CAUSAL, bwd_dkdv_pipe_occ<D>() == 2>(a, bh, pi, npass);
+  bwd_item<CAUSAL, bwd_dkdv_pipe_occ<D, CAUSAL, DROP>() == 2>(a, bh, pi, npass);
 
   const T *Qb = (const T *)a.q + RW::head(a.mq, bh, a.sq);
   const T *dOb = (const T *)a.dout + RW::head(a.mdo, bh, a.sq);
@@ -617,8 +619,8 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(bwd_dkd
                     f32x16 &xn, f32x16 &gn, uint32_t (&rn)[4]) {
       constexpr bool NEXT = decltype(next_tag)::value, GUARD = decltype(guard_tag)::value;
       constexpr int NX = NEXT ? 2 : 0, NA = NEXT ? 2 * KS : 0, NC = 4 * DB, NO = NA + NC, NM = NX + NO;
-      constexpr int AHEAD = D == 128 ? 4 : 3;
-      constexpr bool SWAP = D == 128;
+      constexpr int AHEAD = D > 64 ? 4 : 3;
+      constexpr bool SWAP = D > 64;
       constexpr int NS = 10;
       constexpr int NP = DROP == 1 && NEXT ? 15 : 0;
       constexpr int JS = NEXT ? NX + NA : 0;

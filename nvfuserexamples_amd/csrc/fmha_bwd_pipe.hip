@@ -1,5 +1,5 @@
 // Instantiates the software-pipelined backward kernels for one (element type, head dim, row layout kind) triple, chosen
-// with -DFMHA_TU_BF16={0,1} -DFMHA_TU_D={64,128,256} -DFMHA_TU_STRIDED={0,1}, and exports their launcher.
+// with -DFMHA_TU_BF16={0,1} -DFMHA_TU_D={32,64,96,128,256} -DFMHA_TU_STRIDED={0,1}, and exports their launcher.
 #include "fmha_launch.h"
 #include "fmha_bwd_persist.h"
 #ifndef FMHA_TU_STRIDED
@@ -45,7 +45,7 @@ int persist_half_rounds(const BwdArgs &a, bool causal, bool drop) {
 
 template <int MASK, bool CAUSAL, int DROP> int launch(const BwdArgs &a, bool dkdv, long long nblk, hipStream_t s) {
   if (nblk > 0x7fffffffLL) return 2;
-#if FMHA_TU_D == 256 // (dQ only)
+#if FMHA_TU_D == 96 || FMHA_TU_D == 256 // (dQ only)
   if (dkdv) return 1;
 #else
   if (dkdv) {

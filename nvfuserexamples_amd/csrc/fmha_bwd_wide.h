@@ -132,8 +132,8 @@ __global__ __launch_bounds__(bwd_wide_threads<D>()) __attribute__((amdgpu_waves_
     PanelLane pl;
     pl.init(l);
     TileCopy<T, D, BQ, NT> tcopy, tcopy_do;
-    tcopy.init(tid, RW::ss(a.mq));
-    tcopy_do.init(tid, RW::ss(a.mdo));
+    tcopy.init(tid, RW::ss(a.mq), RW::cols(a));
+    tcopy_do.init(tid, RW::ss(a.mdo), RW::cols(a));
     auto dma_qdo = [&](int qt) {
       const uint32_t dst = lds_base + (uint32_t)(qt & 1) * 2 * TILEB;
       tcopy.issue(Qb, qt * BQ, a.sq, dst, tid, RW::cols(a));

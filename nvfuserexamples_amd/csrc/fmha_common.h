@@ -126,6 +126,8 @@ FMHA_DEV int by_length(int bid, int blocks, int lg) {
 // one logical chunk over all sixteen 16-byte bank groups, which is what a conflict-free
 // ds_read_b128 needs.  The copying lane simply fetches the chunk that belongs at its slot.
 constexpr int kPanelRowB = 128;
+// Columns of an LDS tile for head dim d: whole panels (at 32 and 96 half of the last one is never read).
+constexpr int tile_cols(int d) { return (d + 63) / 64 * 64; }
 
 // One wave-wide 16-byte-per-lane copy from global memory into LDS: lane i's chunk lands at
 // LDS byte address lds_wave_base + 16*i.  Written as inline assembly with hand-placed waits
@@ -180,6 +182,9 @@ struct RowMap {
 // Kernels are built twice: for the folded contiguous layout, whose strides are compile-time
 // constants (the row map is not read at all), and for row maps given at run time, which cost a
 // few per cent in scalar address arithmetic and registers.
+// Head dims 32 and 96 are built on tiles of whole panels (tile_cols): contraction steps and output blocks past them are left out, which on
+// the next whole panel's kernels were multiplied as zeros (BH 512 S 512, padding mask and dropout, forward / backward us: 96 columns
+// 107 / 345 -> 88 / 270, 80 columns 99 / 320 -> 84 / 257, 32 columns 66 / 158 -> 58 / 125).
 // Head dims between the built ones: a tensor's rows hold `dcols` < D elements (a multiple of 8: whole 16-byte
 // chunks) and the kernels behave as if the rows were padded with zeros up to D -- chunks past dcols are
 // never read (register loads fetch chunk 0 instead and are zeroed afterwards; direct copies to LDS take
@@ -207,9 +212,9 @@ template <bool STRIDED, int D> struct Rows {
 };
 
 template <typename T, int D, int BT, int NT> struct TileCopy {
-  static constexpr int CHUNKS = BT * D / 8;
+  static constexpr int CHUNKS = BT * tile_cols(D) / 8;
   static constexpr int CPT = CHUNKS / NT;
-  static_assert(D % 64 == 0 && CHUNKS % NT == 0, "tile must divide evenly over the workgroup");
+  static_assert(D % 32 == 0 && CHUNKS % NT == 0, "tile must divide evenly over the workgroup");
   uint32_t voff[CPT];
   uint32_t ss; // elements between rows of the source tensor
 
@@ -220,20 +225,53 @@ template <typename T, int D, int BT, int NT> struct TileCopy {
     row = (c / 8) % BT;
     col = panel * 8 + (pos ^ ((row >> 1) & 7));
   }
-  FMHA_DEV void init(int tid, int64_t row_stride) {
+  // dv: elements a row really has.  At head dims 32 and 96 slots past them fetch the row's first chunk (of a full tile, see issue).
+  FMHA_DEV void init(int tid, int64_t row_stride, int dv = D) {
     ss = (uint32_t)row_stride;
 #pragma unroll
     for (int i = 0; i < CPT; ++i) {
       int row, col;
       slot(tid + i * NT, row, col);
-      voff[i] = (uint32_t)row * ss * 2u + (uint32_t)(col * 16);
+      voff[i] = (uint32_t)row * ss * 2u + (D % 64 == 0 || col * 8 < dv ? (uint32_t)(col * 16) : 0u);
     }
   }
   // base: row 0 of the head; lds_tile: LDS byte address of the destination tile; tid: the caller's
   // index among the NT threads
-  // dv: elements a row really has (chunks past them come from g_zero_chunk)
-  FMHA_DEV void issue(const T *base, int row0, int rend, uint32_t lds_tile, int tid, int dv = D) const {
+  // dv: as for init.  Chunks between them and column D come from g_zero_chunk: they meet zeros, and an infinity repeated there
+  // would make a NaN.  At head dims 32 and 96 nobody reads the chunks past column D, so full tiles of whole rows are copied from
+  // a uniform base plus the lane's offset, and tiles that only make columns nobody stores there (any_past) as well; other full tiles choose
+  // between that address and the zeros, which costs four instructions a copy where the address from the row's index costs ten
+  // (80 columns, BH 608 S 365 causal forward 47.3 -> 45.8 us; at 128, with registers to the limit, the same made 112 columns slower).
+  FMHA_DEV void issue(const T *base, int row0, int rend, uint32_t lds_tile, int tid, int dv = D, bool any_past = false) const {
     const uint32_t wave_dst = lds_tile + (uint32_t)(tid >> 6) * 1024u;
+    if constexpr (D % 64 != 0) { // (all conditions are wave-uniform)
+      const T *tb = base + (uint32_t)row0 * ss;
+      if (row0 + BT > rend) {
+#pragma unroll
+        for (int i = 0; i < CPT; ++i) {
+          int row, col;
+          slot(tid + i * NT, row, col);
+          int r = row0 + row;
+          r = r < rend ? r : rend - 1;
+          const T *src = col * 8 < dv ? base + ((uint32_t)r * ss + (uint32_t)(col * 8)) : (const T *)g_zero_chunk;
+          dma_global_to_lds_b128(src, wave_dst + (uint32_t)(i * NT * 16));
+        }
+        return;
+      }
+      if (dv == D || any_past) {
+#pragma unroll
+        for (int i = 0; i < CPT; ++i) dma_global_to_lds_b128(tb, voff[i], wave_dst + (uint32_t)(i * NT * 16));
+        return;
+      }
+#pragma unroll
+      for (int i = 0; i < CPT; ++i) {
+        int row, col;
+        slot(tid + i * NT, row, col);
+        const char *src = (const char *)tb + voff[i];
+        dma_global_to_lds_b128(col * 8 < dv ? src : (const char *)g_zero_chunk, wave_dst + (uint32_t)(i * NT * 16));
+      }
+      return;
+    }
     if (dv < D) { // wave-uniform
 #pragma unroll
       for (int i = 0; i < CPT; ++i) {
@@ -347,8 +385,8 @@ template <typename T> FMHA_DEV void store_acc_block_row(T *dst_row, const f32x16
 // 32 different rows per instruction; here the block is turned in a wave-private LDS scratch first (its accesses execute
 // in order, no barrier) and leaves as 16 bytes per lane along the rows: every instruction writes complete cache lines.
 template <int D> struct RowStore {
-  static constexpr int PITCH = D * 2 + 16, BYTES = 32 * PITCH; // of LDS per wave, 16-byte aligned
-  static constexpr int LPR = D / 8, RPI = 64 / LPR;             // lanes per row, rows per instruction
+  static constexpr int PITCH = tile_cols(D) * 2 + 16, BYTES = 32 * PITCH; // of LDS per wave, 16-byte aligned
+  static constexpr int LPR = tile_cols(D) / 8, RPI = 64 / LPR;             // lanes per row, rows per instruction
 };
 // base: row 0 of the block; rows [0, nrows) and columns [0, ncol) exist (ncol a multiple of 8)
 template <typename T, int D>

@@ -1,5 +1,5 @@
 // Instantiates the forward kernel for one (element type, head dim, row layout kind) triple, chosen
-// with -DFMHA_TU_BF16={0,1} -DFMHA_TU_D={64,128,256} -DFMHA_TU_STRIDED={0,1}, and exports its dispatcher.
+// with -DFMHA_TU_BF16={0,1} -DFMHA_TU_D={32,64,96,128,256} -DFMHA_TU_STRIDED={0,1}, and exports its dispatcher.
 #include "fmha_launch.h"
 #include "fmha_fwd_pipe.h"
 #ifndef FMHA_TU_STRIDED
@@ -91,7 +91,7 @@ template <int QB, int MASK, bool CAUSAL, int DROP, bool kPipe = (DROP != 2)> int
   a.deal = a.deal_heads = 0;
   if (kPipe && CAUSAL && MASK == kMaskNone && a.sk_whole == 0) {
     const long long items = (long long)a.bh * a.nqt, G = nblk;
-    constexpr bool kWhole = FMHA_TU_D != 128 || (DROP != 0 && kStrided);
+    constexpr bool kWhole = (FMHA_TU_D != 96 && FMHA_TU_D != 128) || (DROP != 0 && kStrided);
     const int quarters = kWhole ? 16 : DROP == 0 && a.nqt <= 3 ? 9 : 13;
     if (2 * items > resident && 4 * items < quarters * G && !(G % a.nqt == 0 && items % (2 * G) == 0)) {
       int lg = 0;
@@ -293,7 +293,11 @@ template <int QB> int by_mask(FwdArgs &a, const FwdVariant &v, hipStream_t s) {
 #else
 template <int QB> int by_mask(FwdArgs &a, const FwdVariant &v, hipStream_t s) {
   if (v.mask == kMaskPerKey) return by_causal<QB, kMaskPerKey>(a, v, s);
+#if FMHA_TU_D % 64 == 0
   if (v.mask == kMaskFull) return by_causal<QB, kMaskFull>(a, v, s);
+#else // (full mask tensors: the next whole panel's kernels)
+  if (v.mask == kMaskFull) return 1;
+#endif
   return by_causal<QB, kMaskNone>(a, v, s);
 }
 #endif
@@ -394,6 +398,7 @@ int FMHA_NAME(FMHA_TU_TNAME, FMHA_TU_D)(FwdArgs &a, const FwdVariant &v, hipStre
 #else
   if (v.save_split || v.save_once || v.stream) return 1;
 #endif
+#if !FMHA_TU_STRIDED
   if (v.drop == 2) { // tensor dropout / save-intermediates: the legacy ops' shape class
     if (v.causal) return 1;
 #if FMHA_TU_D == 64
@@ -407,6 +412,7 @@ int FMHA_NAME(FMHA_TU_TNAME, FMHA_TU_D)(FwdArgs &a, const FwdVariant &v, hipStre
     if (v.mask == kMaskFull) return launch<1, kMaskFull, false, 2>(a, s);
     return launch<1, kMaskNone, false, 2>(a, s);
   }
+#endif
 #if FMHA_TU_D == 64
   // two query blocks per wave: only where their accumulators fit the register file and only
   // for the variants the host ever selects them for

@@ -18,9 +18,9 @@
 namespace fmha {
 
 template <int D, int NW_> struct FewCfg {
-  static constexpr int BK = D == 64 ? 64 : 32; // keys per block: what a lane holds of the next one fits beside the rest in 256 registers
+  static constexpr int BK = D <= 64 ? 64 : 32; // keys per block: what a lane holds of the next one fits beside the rest in 256 registers
   static constexpr int NW = NW_, NT = NW * 64, QT = 32;
-  static constexpr int TILEB = BK * D * 2;
+  static constexpr int TILEB = BK * tile_cols(D) * 2;
   static constexpr int LDS_M = 2 * TILEB;            // (in a wave's stage) mask terms of the block's keys
   static constexpr int STAGEB = LDS_M + BK * 4;
   static constexpr int LDS_MERGE = NW * 32 * D * 4;  // over the stages: the waves' outputs
@@ -36,7 +36,7 @@ __global__ __launch_bounds__((FewCfg<D, NW>::NT), D == 256 ? 1 : 2) void fmha_fw
   using v8 = typename E::v8;
   using RW = Rows<STRIDED, D>;
   constexpr int KS = D / 16, DB = D / 32, BK = C::BK, NSB = BK / 32;
-  constexpr int CPT = BK * D / 8 / 64; // 16-byte chunks per lane and block of K (of V)
+  constexpr int CPT = BK * tile_cols(D) / 8 / 64; // 16-byte chunks per lane and block of K (of V)
   constexpr float NEG_INF = -__builtin_inff();
 
   extern __shared__ __attribute__((aligned(16))) char lds[];

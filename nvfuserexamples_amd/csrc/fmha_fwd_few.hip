@@ -1,5 +1,5 @@
 // The forward whose waves share 32 queries (fmha_fwd_few.h) for one (element type, head dim, row layout kind) triple, chosen with
-// -DFMHA_TU_BF16={0,1} -DFMHA_TU_D={64,128,256} -DFMHA_TU_STRIDED={0,1}, and its dispatcher.
+// -DFMHA_TU_BF16={0,1} -DFMHA_TU_D={32,64,96,128,256} -DFMHA_TU_STRIDED={0,1}, and its dispatcher.
 #include "fmha_launch.h"
 
 #if FMHA_TU_BF16

@@ -43,11 +43,11 @@ template <int D, int QB> struct PipeCfg {
   static constexpr int NSB = BK / 32; // 32-key sub-blocks per tile
   static constexpr int KS = D / 16;   // contraction steps of K.Q^T
   static constexpr int DB = D / 32;   // 32-row blocks of O^T
-  static constexpr int TILEB = BK * D * 2; // swizzled panel layout, no padding
+  static constexpr int TILEB = BK * tile_cols(D) * 2; // swizzled panel layout, no padding
   static constexpr int XROWB = 32;    // pitch of the extra-contraction-step rows (16 elements)
   // The next item's Q rows are prefetched into LDS where that still leaves room for two
   // workgroups per CU; otherwise Q is loaded from global memory when the item starts.
-  static constexpr bool QLDS = (D == 64);
+  static constexpr bool QLDS = (D <= 64);
   static constexpr int LDS_BYTES = 4 * TILEB + 2 * BK * XROWB; // {K,V} x 2 stages + extra rows x 2 stages
   static constexpr int TRIM_BYTES = 256; // per-item key counts derived from a per-key mask, at the very end
   static constexpr int lds_bytes(int nw) { return LDS_BYTES + (QLDS ? nw * QB * 32 * D * 2 : 0) + TRIM_BYTES; }
@@ -87,7 +87,7 @@ template <int NSB, int KS, int DB, bool WITH_FIRST_PRODUCT> constexpr FwdOperand
 // few instead of settling for one wave per SIMD, which measures 8-30 % faster.)
 // DEAL: causal items dealt by length, see FwdArgs::deal (a build of its own: the choice at run time cost short launches 0.5 us).
 template <typename T, int D, int QB, int NW, int MASK, bool CAUSAL, int DROP, bool STRIDED, bool DEAL = false>
-__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu((QB == 2 || D == 128 || MASK == kMaskFull || DROP == 2) ? 2 : 1, 2))) void fmha_fwd_pipe_kernel(const FwdArgs a) {
+__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu((QB == 2 || D == 96 || D == 128 || MASK == kMaskFull || DROP == 2) ? 2 : 1, 2))) void fmha_fwd_pipe_kernel(const FwdArgs a) {
   using RW = Rows<STRIDED, D>;
   using E = Elem<T>;
   using v8 = typename E::v8;
@@ -100,7 +100,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu((QB == 
   static_assert(NT >= BK, "the extra rows are staged by the first BK threads");
   static_assert(DROP == 0 || DROP == 1 || (DROP == 2 && D == 64 && !CAUSAL),
                 "the save pass, and tensor dropout at head dim 128, use fmha_fwd_kernel");
-  static_assert(D % 64 == 0, "tiles are stored as panels of 64 columns");
+  static_assert(D % 32 == 0, "whole blocks of 32 output columns");
   constexpr float NEG_INF = -__builtin_inff();
   constexpr float WINDOW = 16384.f;
 
@@ -306,17 +306,17 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu((QB == 
   // offset area_off.  Rows past kend re-read the last valid row: their scores get -inf through
   // the extra step, and finite garbage in V is multiplied by P = 0.
   TileCopy<T, D, BK, NT> tcopy;
-  tcopy.init(tid, RW::ss(a.mk)); // K and V rows are equally far apart
-  auto dma_tile = [&](const T *base, int kend, int tile, uint32_t area_off) {
-    tcopy.issue(base, tile * BK, kend > 0 ? kend : 1, lds_base + area_off + (uint32_t)(tile & 1) * TILEB, tid, RW::cols(a));
+  tcopy.init(tid, RW::ss(a.mk), RW::cols(a)); // K and V rows are equally far apart
+  auto dma_tile = [&](const T *base, int kend, int tile, uint32_t area_off, bool any_past) {
+    tcopy.issue(base, tile * BK, kend > 0 ? kend : 1, lds_base + area_off + (uint32_t)(tile & 1) * TILEB, tid, RW::cols(a), any_past);
   };
   // K tile u of the stream that runs from the current item on into the next one (u may reach
   // past the current item's last tile; nkt2 is even, so the stage parity carries over)
   auto dmaK = [&](int u) {
     const bool here = u < cur.nkt2;
-    dma_tile(here ? cur.Kb : nxt.Kb, here ? cur.kend : nxt.kend, here ? u : u - cur.nkt2, 0u);
+    dma_tile(here ? cur.Kb : nxt.Kb, here ? cur.kend : nxt.kend, here ? u : u - cur.nkt2, 0u, false);
   };
-  auto dmaV = [&](int tile) { dma_tile(cur.Vb, cur.kend, tile, 2u * TILEB); };
+  auto dmaV = [&](int tile) { dma_tile(cur.Vb, cur.kend, tile, 2u * TILEB, true); };
 
   // Q rows of an item: lane (ql, h) of wave w owns chunks [16*ks + 8*h, +8) of row q0 + 32*qb + ql.
   // Each wave copies its own rows into its own part of the Q buffer, exactly where its lanes

@@ -1,6 +1,6 @@
 // Internal interface between the C-ABI translation unit and the per-(element type,
 // head dim) kernel translation units.  Each kernel TU is compiled once per
-// combination with -DFMHA_TU_BF16={0,1} -DFMHA_TU_D={64,128,256} -DFMHA_TU_STRIDED={0,1} and exports
+// combination with -DFMHA_TU_BF16={0,1} -DFMHA_TU_D={32,64,96,128,256} -DFMHA_TU_STRIDED={0,1} and exports
 // one dispatcher per pass (the _strided ones read the row maps of the argument block; the
 // others assume folded contiguous tensors).
 #pragma once
@@ -36,15 +36,23 @@ int fwd_dispatch_bf16_d256(FwdArgs &a, const FwdVariant &v, hipStream_t s);
 int fwd_dispatch_f16_d256_strided(FwdArgs &a, const FwdVariant &v, hipStream_t s);
 int fwd_dispatch_bf16_d256_strided(FwdArgs &a, const FwdVariant &v, hipStream_t s);
 int fwd_dispatch_f16_d64_strided(FwdArgs &a, const FwdVariant &v, hipStream_t s);
+int fwd_dispatch_f16_d32_strided(FwdArgs &a, const FwdVariant &v, hipStream_t s);
+int fwd_dispatch_f16_d96_strided(FwdArgs &a, const FwdVariant &v, hipStream_t s);
 int fwd_dispatch_f16_d128_strided(FwdArgs &a, const FwdVariant &v, hipStream_t s);
 int fwd_dispatch_bf16_d64_strided(FwdArgs &a, const FwdVariant &v, hipStream_t s);
+int fwd_dispatch_bf16_d32_strided(FwdArgs &a, const FwdVariant &v, hipStream_t s);
+int fwd_dispatch_bf16_d96_strided(FwdArgs &a, const FwdVariant &v, hipStream_t s);
 int fwd_dispatch_bf16_d128_strided(FwdArgs &a, const FwdVariant &v, hipStream_t s);
 
 // The forward whose waves share 32 queries (fmha_fwd_few.hip).
 int fwd_few_launch_f16_d64(FwdArgs &a, const FwdVariant &v, hipStream_t s);
 int fwd_few_launch_f16_d64_strided(FwdArgs &a, const FwdVariant &v, hipStream_t s);
+int fwd_few_launch_f16_d32_strided(FwdArgs &a, const FwdVariant &v, hipStream_t s);
+int fwd_few_launch_f16_d96_strided(FwdArgs &a, const FwdVariant &v, hipStream_t s);
 int fwd_few_launch_bf16_d64(FwdArgs &a, const FwdVariant &v, hipStream_t s);
 int fwd_few_launch_bf16_d64_strided(FwdArgs &a, const FwdVariant &v, hipStream_t s);
+int fwd_few_launch_bf16_d32_strided(FwdArgs &a, const FwdVariant &v, hipStream_t s);
+int fwd_few_launch_bf16_d96_strided(FwdArgs &a, const FwdVariant &v, hipStream_t s);
 int fwd_few_launch_f16_d128(FwdArgs &a, const FwdVariant &v, hipStream_t s);
 int fwd_few_launch_f16_d128_strided(FwdArgs &a, const FwdVariant &v, hipStream_t s);
 int fwd_few_launch_bf16_d128(FwdArgs &a, const FwdVariant &v, hipStream_t s);
@@ -71,8 +79,12 @@ int bwd_dispatch_bf16_d256(BwdArgs &a, const BwdVariant &v, hipStream_t s);
 int bwd_dispatch_f16_d256_strided(BwdArgs &a, const BwdVariant &v, hipStream_t s);
 int bwd_dispatch_bf16_d256_strided(BwdArgs &a, const BwdVariant &v, hipStream_t s);
 int bwd_dispatch_f16_d64_strided(BwdArgs &a, const BwdVariant &v, hipStream_t s);
+int bwd_dispatch_f16_d32_strided(BwdArgs &a, const BwdVariant &v, hipStream_t s);
+int bwd_dispatch_f16_d96_strided(BwdArgs &a, const BwdVariant &v, hipStream_t s);
 int bwd_dispatch_f16_d128_strided(BwdArgs &a, const BwdVariant &v, hipStream_t s);
 int bwd_dispatch_bf16_d64_strided(BwdArgs &a, const BwdVariant &v, hipStream_t s);
+int bwd_dispatch_bf16_d32_strided(BwdArgs &a, const BwdVariant &v, hipStream_t s);
+int bwd_dispatch_bf16_d96_strided(BwdArgs &a, const BwdVariant &v, hipStream_t s);
 int bwd_dispatch_bf16_d128_strided(BwdArgs &a, const BwdVariant &v, hipStream_t s);
 
 // (kBwdNotHere of the launchers below: nothing was launched, the call belongs to an older kernel)
@@ -84,8 +96,12 @@ int bwd_pipe_launch_f16_d128(const BwdArgs &a, const BwdVariant &v, bool dkdv, l
 int bwd_pipe_launch_bf16_d64(const BwdArgs &a, const BwdVariant &v, bool dkdv, long long nblk, hipStream_t s);
 int bwd_pipe_launch_bf16_d128(const BwdArgs &a, const BwdVariant &v, bool dkdv, long long nblk, hipStream_t s);
 int bwd_pipe_launch_f16_d64_strided(const BwdArgs &a, const BwdVariant &v, bool dkdv, long long nblk, hipStream_t s);
+int bwd_pipe_launch_f16_d32_strided(const BwdArgs &a, const BwdVariant &v, bool dkdv, long long nblk, hipStream_t s);
+int bwd_pipe_launch_f16_d96_strided(const BwdArgs &a, const BwdVariant &v, bool dkdv, long long nblk, hipStream_t s);
 int bwd_pipe_launch_f16_d128_strided(const BwdArgs &a, const BwdVariant &v, bool dkdv, long long nblk, hipStream_t s);
 int bwd_pipe_launch_bf16_d64_strided(const BwdArgs &a, const BwdVariant &v, bool dkdv, long long nblk, hipStream_t s);
+int bwd_pipe_launch_bf16_d32_strided(const BwdArgs &a, const BwdVariant &v, bool dkdv, long long nblk, hipStream_t s);
+int bwd_pipe_launch_bf16_d96_strided(const BwdArgs &a, const BwdVariant &v, bool dkdv, long long nblk, hipStream_t s);
 int bwd_pipe_launch_bf16_d128_strided(const BwdArgs &a, const BwdVariant &v, bool dkdv, long long nblk, hipStream_t s);
 
 int bwd_pipe_launch_f16_d256(const BwdArgs &a, const BwdVariant &v, bool dkdv, long long nblk, hipStream_t s);
