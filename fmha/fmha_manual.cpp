@@ -97,6 +97,7 @@ void fill_common(fmha_fwd_params &p, const at::Tensor &q, const at::Tensor &k, c
   p.d = static_cast<int32_t>(q.size(2));
   p.dtype = dtype_code(q);
   p.scale = static_cast<float>(scale);
+  p.flags = FMHA_FLAG_SPLIT_KEYS; // few heads
 }
 
 void launch_fwd(const fmha_fwd_params &p, const at::Tensor &q) {

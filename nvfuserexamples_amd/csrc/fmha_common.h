@@ -356,28 +356,33 @@ FMHA_DEV float xhalf_sum(float x) {
 // lane h = 0 the first half of a 32-byte group, lane h = 1 the second -- so the same data leaves
 // in half as many, twice as large, writes.  dst: the lane's row; the block starts at column 0.
 // ncol: columns of this block that exist in the destination row (a multiple of 8).
+// (The two pieces of a 32-byte group.)
+template <typename T, typename P> FMHA_DEV void store_acc_pieces(T *dst_row, const P &lo, const P &hi, float scale, int h, int ncol = 16) {
+  typename Elem<T>::v4 x, y;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    x[i] = (T)(lo[i] * scale);
+    y[i] = (T)(hi[i] * scale);
+  }
+  Pack8 px, py;
+  if constexpr (sizeof(T) == 2 && __is_same(T, _Float16)) {
+    px.h = x;
+    py.h = y;
+  } else {
+    px.b = x;
+    py.b = y;
+  }
+  // after the swaps: lanes h = 0 hold (own x, partner's x), lanes h = 1 hold (partner's y, own y)
+  auto r0 = __builtin_amdgcn_permlane32_swap((int)px.u.x, (int)py.u.x, false, false);
+  auto r1 = __builtin_amdgcn_permlane32_swap((int)px.u.y, (int)py.u.y, false, false);
+  const u32x4 both = {(uint32_t)r0[0], (uint32_t)r1[0], (uint32_t)r0[1], (uint32_t)r1[1]};
+  if (8 * h < ncol) *(u32x4 *)(dst_row + 8 * h) = both;
+}
 template <typename T> FMHA_DEV void store_acc_block_row(T *dst_row, const f32x16 &acc, float scale, int h, int ncol = 32) {
 #pragma unroll
-  for (int gp = 0; gp < 2; ++gp) {
-    typename Elem<T>::v4 x, y; // pieces g = 2gp and g = 2gp + 1
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      x[i] = (T)(acc[4 * (2 * gp) + i] * scale);
-      y[i] = (T)(acc[4 * (2 * gp + 1) + i] * scale);
-    }
-    Pack8 px, py;
-    if constexpr (sizeof(T) == 2 && __is_same(T, _Float16)) {
-      px.h = x;
-      py.h = y;
-    } else {
-      px.b = x;
-      py.b = y;
-    }
-    // after the swaps: lanes h = 0 hold (own x, partner's x), lanes h = 1 hold (partner's y, own y)
-    auto r0 = __builtin_amdgcn_permlane32_swap((int)px.u.x, (int)py.u.x, false, false);
-    auto r1 = __builtin_amdgcn_permlane32_swap((int)px.u.y, (int)py.u.y, false, false);
-    const u32x4 both = {(uint32_t)r0[0], (uint32_t)r1[0], (uint32_t)r0[1], (uint32_t)r1[1]};
-    if (16 * gp + 8 * h < ncol) *(u32x4 *)(dst_row + 16 * gp + 8 * h) = both;
+  for (int gp = 0; gp < 2; ++gp) { // pieces g = 2gp and g = 2gp + 1
+    const f32x4 x = {acc[8 * gp], acc[8 * gp + 1], acc[8 * gp + 2], acc[8 * gp + 3]}, y = {acc[8 * gp + 4], acc[8 * gp + 5], acc[8 * gp + 6], acc[8 * gp + 7]};
+    store_acc_pieces<T>(dst_row + 16 * gp, x, y, scale, h, ncol - 16 * gp);
   }
 }
 

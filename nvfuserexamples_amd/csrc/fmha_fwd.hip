@@ -10,6 +10,7 @@
 #include "fmha_fwd_save.h"
 #include "fmha_fwd_stream.h"
 #include "fmha_fwd_stream_save.h"
+#include "fmha_fwd_cols.h"
 #else
 #define FMHA_TU_ROWS 0
 #endif
@@ -243,6 +244,27 @@ int launch_stream_save(FwdArgs &a, hipStream_t s) {
 }
 #endif
 
+#if FMHA_TU_ROWS
+// 32 queries a workgroup, 64 keys a wave
+template <bool DROPT, bool SAVE, bool TAIL> int launch_cols_as(FwdArgs &a, hipStream_t s) {
+  using ColsCfg = fmha::ColsCfg<FMHA_TU_D>;
+  auto kern = fmha_fwd_cols_kernel<FMHA_TU_T, FMHA_TU_D, DROPT, SAVE, TAIL>;
+  static const bool ready = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                ColsCfg::lds_bytes(ColsCfg::MAXW)) == hipSuccess;
+  if (!ready) return 2;
+  if (a.sk > ColsCfg::SKMAX || (DROPT && !a.drop_mask)) return 1;
+  a.nqt = (a.sq + ColsCfg::QT - 1) / ColsCfg::QT;
+  const long long nblk = (long long)a.bh * a.nqt;
+  if (nblk > 0x7fffffffLL) return 2;
+  const int nw = (a.sk + ColsCfg::BK - 1) / ColsCfg::BK;
+  hipLaunchKernelGGL(kern, dim3((unsigned)nblk), dim3(nw * 64), ColsCfg::lds_bytes(nw), s, a);
+  return hipGetLastError() == hipSuccess ? 0 : 2;
+}
+template <bool DROPT, bool SAVE> int launch_cols(FwdArgs &a, hipStream_t s) {
+  return a.sk & 7 ? launch_cols_as<DROPT, SAVE, true>(a, s) : launch_cols_as<DROPT, SAVE, false>(a, s);
+}
+#endif
+
 #if FMHA_TU_D == 64
 // a whole head's K and V resident in LDS: one persistent workgroup per compute unit
 #ifndef FMHA_HEAD_QB
@@ -389,6 +411,7 @@ int FMHA_NAME(FMHA_TU_TNAME, FMHA_TU_D)(FwdArgs &a, const FwdVariant &v, hipStre
   if (v.short_keys || v.head) return 1;
 #endif
 #if FMHA_TU_ROWS
+  if (v.cols) return v.drop != 2 ? launch_cols<false, false>(a, s) : a.save_softmax || a.save_dropout ? launch_cols<true, true>(a, s) : launch_cols<true, false>(a, s);
   if (v.save_once) return launch_stream_save(a, s);
   if (v.save_split) { // forward with LSE, then the saved outputs from that LSE
     const int rc = v.stream ? launch_stream<true>(a, v, s) : launch<1, kMaskFull, false, 2, FMHA_TU_D == 64>(a, s);
@@ -396,7 +419,7 @@ int FMHA_NAME(FMHA_TU_TNAME, FMHA_TU_D)(FwdArgs &a, const FwdVariant &v, hipStre
   }
   if (v.stream) return v.drop == 2 ? launch_stream<true>(a, v, s) : launch_stream<false>(a, v, s);
 #else
-  if (v.save_split || v.save_once || v.stream) return 1;
+  if (v.save_split || v.save_once || v.stream || v.cols) return 1;
 #endif
 #if !FMHA_TU_STRIDED
   if (v.drop == 2) { // tensor dropout / save-intermediates: the legacy ops' shape class

@@ -19,6 +19,7 @@ struct FwdVariant {
   bool save_split; // saving beyond the one-pass kernel's range with a caller-provided LSE buffer: forward, then a save kernel
   bool save_once;  // saving for up to 512 keys: one launch that keeps a wave's probabilities in registers (folded layout)
   bool stream;     // full mask tensor beyond the one-pass range: the streaming forward (head dims 64 and 128, folded layout)
+  bool cols;       // full mask tensor: a workgroup per 32 queries, a wave per 64 keys (head dims 64 and 128, folded layout)
   bool many;       // stream: more workgroups than two per compute unit
   bool head;       // up to 512 keys, no / per-key mask, no causal mask: the whole-head kernel (head dim 64, folded layout)
   bool short_keys; // sk <= 128: the one-pass kernel (head dim 64, folded layout)
