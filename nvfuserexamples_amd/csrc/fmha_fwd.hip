@@ -225,9 +225,9 @@ template <bool DROPT> int launch_stream(FwdArgs &a, const FwdVariant &v, hipStre
 }
 
 // the save-intermediates operator for up to 512 keys in one launch (one wave per SIMD: the whole register file)
-template <bool TAIL> int launch_stream_save_as(FwdArgs &a, hipStream_t s) {
-  using StreamSaveCfg = fmha::StreamSaveCfg<FMHA_TU_D>;
-  auto kern = fmha_fwd_stream_save_kernel<FMHA_TU_T, FMHA_TU_D, TAIL>;
+template <bool TAIL, int NTILE> int launch_stream_save_as(FwdArgs &a, hipStream_t s) {
+  using StreamSaveCfg = fmha::StreamSaveCfg<FMHA_TU_D, NTILE>;
+  auto kern = fmha_fwd_stream_save_kernel<FMHA_TU_T, FMHA_TU_D, TAIL, NTILE>;
   constexpr int kLds = StreamSaveCfg::lds_bytes(TAIL || FMHA_TU_D != 64);
   static const bool ready = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
                                                 hipFuncAttributeMaxDynamicSharedMemorySize, kLds) == hipSuccess;
@@ -240,7 +240,17 @@ template <bool TAIL> int launch_stream_save_as(FwdArgs &a, hipStream_t s) {
   return hipGetLastError() == hipSuccess ? 0 : 2;
 }
 int launch_stream_save(FwdArgs &a, hipStream_t s) {
-  return a.sk & 7 ? launch_stream_save_as<true>(a, s) : launch_stream_save_as<false>(a, s);
+  // Few tiles leave the registers for two waves per SIMD (us, one wave / two): three at head dim 64 BH 352 S 173 52.4 / 41.0, BH 800 S 192
+  // 95.5 / 70.4, BH 96 S 144 13.9 / 12.7; one at 128 BH 504 S 40 16.3 / 10.7, BH 1500 S 64 51.5 / 34.7; two at 128 spill 50 registers
+  // and pay where workgroups share compute units: BH 504 S 72 28.9 / 25.3, BH 1500 S 128 104.7 / 103.0, but BH 150 S 100 15.4 / 17.2.
+  // (Four at 64 spill 45 and do not: BH 352 S 240 56.4 / 62.1.)
+  constexpr int kFew = FMHA_TU_D == 64 ? 3 : 1, kMost = FMHA_TU_D == 64 ? 8 : 7;
+  if (a.sk <= kFew * 64) return a.sk & 7 ? launch_stream_save_as<true, kFew>(a, s) : launch_stream_save_as<false, kFew>(a, s);
+#if FMHA_TU_D == 128
+  if (a.sk <= 128 && (long long)a.bh * ((a.sq + 127) / 128) > kCUs)
+    return a.sk & 7 ? launch_stream_save_as<true, 2>(a, s) : launch_stream_save_as<false, 2>(a, s);
+#endif
+  return a.sk & 7 ? launch_stream_save_as<true, kMost>(a, s) : launch_stream_save_as<false, kMost>(a, s);
 }
 #endif
 

@@ -8,7 +8,7 @@
 // tile the unnormalised probabilities exp2(s - m_t) of its 32 queries, rounded to the element type
 // (16 registers), the tile's dropout rows as loaded (16 registers) and the running maximum m_t they
 // were formed under.  Eight tiles make 264 registers, so the kernel runs one wave per SIMD with the
-// whole 512-entry register file (the key loop is unrolled: register arrays are indexed by constants).
+// whole 512-entry register file (builds for few tiles run two) (the key loop is unrolled: register arrays are indexed by constants).
 // After the last tile the row's log-sum-exp L is known and a second, store-only, phase writes
 //   softmax = round(p_t * exp2(m_t - L)),   dropout = round(p_t * exp2(m_t - L) * d * scale)
 // tile by tile through the wave's LDS scratch as whole 128-byte row segments.
@@ -26,21 +26,22 @@
 
 namespace fmha {
 
-template <int D_> struct StreamSaveCfg : StreamCfg<D_, false> {
+template <int D_, int MAXT_> struct StreamSaveCfg : StreamCfg<D_, false> {
   using B = StreamCfg<D_, false>;
-  static constexpr int MAXT = D_ == 64 ? 8 : 7;    // 64-key tiles whose rows a wave, and whose K the workgroup, can hold
+  static constexpr int MAXT = MAXT_;               // 64-key tiles whose rows a wave, and whose K the workgroup, holds
+  static constexpr int OCC = MAXT <= (D_ == 64 ? 3 : 2) ? 2 : 1;
   static constexpr int SKMAX = MAXT * B::BK;
   static constexpr int nkst(bool again) { return again ? MAXT : 2; } // K stages
   static constexpr int lds_bytes(bool again) { return (nkst(again) + B::NST) * B::TILEB + B::NW * B::Scratch::BYTES; } // K, V, a wave's scratch
 };
 
-template <typename T, int D, bool TAIL>
-__global__ __launch_bounds__(StreamSaveCfg<D>::NW * 64) __attribute__((amdgpu_waves_per_eu(1, 1)))
+template <typename T, int D, bool TAIL, int NTILE>
+__global__ __launch_bounds__((StreamSaveCfg<D, NTILE>::NW * 64)) __attribute__((amdgpu_waves_per_eu(StreamSaveCfg<D, NTILE>::OCC, StreamSaveCfg<D, NTILE>::OCC)))
 void fmha_fwd_stream_save_kernel(const FwdArgs a) {
   using E = Elem<T>;
   using v8 = typename E::v8;
   using v4 = typename E::v4;
-  using C = StreamSaveCfg<D>;
+  using C = StreamSaveCfg<D, NTILE>;
   constexpr int KS = D / 16, DB = D / 32, BK = C::BK, NSB = BK / 32, NT = C::NW * 64, ROWB = C::ROWB;
   constexpr int TILEB = C::TILEB, MAXT = C::MAXT;
   constexpr int CPR = D / 8, CPT = BK * CPR / NT;
@@ -187,7 +188,7 @@ void fmha_fwd_stream_save_kernel(const FwdArgs a) {
       const int k0 = t * BK;
       const char *ldsV = lds + (NKST + (C::NST == 2 ? t & 1 : 0)) * TILEB;
       Stage nxt;
-      const bool more = t + 1 < nkt;
+      const bool more = t + 1 < MAXT && t + 1 < nkt;
       if (more) gload(k0 + BK, nxt);
       if (TAIL) scr.place_tail(cur.m, k0, a.sk);
       if (TAIL) scr.place_tail(cur.d, k0, a.sk);
