@@ -1,5 +1,5 @@
 // Forward kernel for launches of few workgroups (no mask, a per-key mask and / or the causal mask, valid key counts; no dropout or
-// the Philox rule): the four waves of a workgroup share 32 queries and take their blocks of keys in turn.
+// the Philox rule): the four (eight, one) waves of a workgroup share 32 queries and take their blocks of keys in turn.
 //
 // The other forward kernels give a workgroup 128 queries or more and walk its keys one tile after the other.  Where that makes
 // fewer workgroups than the chip has room for, the launch lasts as long as one workgroup's row of tiles, about 1.5 us each for a
@@ -7,8 +7,12 @@
 // stages its own blocks (global -> registers -> LDS, one stage, so no barrier: LDS serves a wave's requests in order, and
 // the next block's rows are on their way in registers while one is worked on); at the end the four partial rows meet in LDS.
 // K and V are read once per 32 queries, which is what large launches cannot afford.  The rule and both sides' times are at few_waves in
-// fmha_capi.hip; us, before -> now: BH 12 821 x 856 d 96 26.2 -> 15.5, BH 64 S 448 d 128 padding mask packed 19.3 -> FILL1, BH 4 S 7937 d 128
-// causal 139.8 -> FILL2, BH 1 S 2304 d 32 key counts 29.9 -> 11.3.
+// fmha_capi.hip; us, before -> now: BH 12 821 x 856 d 96 26.2 -> 15.5, BH 4 S 7937 d 128
+// causal 139.4 -> 115.3, BH 1 S 2304 d 32 key counts 29.9 -> 11.3.
+//
+// A build with one wave per workgroup serves short key ranges of any number of heads: the other kernels' workgroups of 128 queries are mostly
+// padding there, and their pipelines have nothing to run ahead of (BH 2460 S 24 d 32 22.0 -> 8.1 us, BH 1690 17 x 24 d 96 with dropout
+// 34.0 -> 8.0, BH 3531 S 52 d 128 packed with dropout 87.6 -> 43.5, BH 3273 S 16 d 256 packed 96.1 -> 32.0).
 //
 // Softmax as in fmha_fwd_mid.h: scores are scaled in fp32, the reference follows the row's maximum only where that has run ahead
 // by more than 2^8, row sums are those of the rounded P.
@@ -217,6 +221,16 @@ __global__ __launch_bounds__((FewCfg<D, NW>::NT), D == 256 ? 1 : 2) void fmha_fw
     fence();
   }
 
+  if constexpr (NW == 1) {
+    sum = xhalf_sum(sum + sum2);
+    if (q >= a.sq) return;
+    const float out = sum > 0.f ? a.drop_scale / sum : 0.f;
+    T *Or = (T *)a.o + RW::head(a.mo, bh, a.sq) + (size_t)q * RW::ss(a.mo);
+#pragma unroll
+    for (int db = 0; db < DB; ++db) store_acc_block_row<T>(Or + db * 32, o[db], out, h, cols - db * 32);
+    if (a.lse && h == 0) a.lse[(size_t)bh * a.sq + q] = sum > 0.f ? (mref + fast_log2(sum)) * FMHA_LN2 : NEG_INF;
+    return;
+  }
   // ---- the waves' partial rows meet in LDS; wave i takes the columns 32 i .., 32 (i + 4) .. of the head
   sum = xhalf_sum(sum + sum2);
   __syncthreads();

@@ -37,6 +37,7 @@ template <int MASK, bool CAUSAL, int DROP> int launch(FwdArgs &a, int nw, hipStr
 #if FMHA_TU_D != 256
   if (nw == 8) return launch_as<8, MASK, CAUSAL, DROP>(a, s);
 #endif
+  if (nw == 1) return launch_as<1, MASK, CAUSAL, DROP>(a, s);
   return launch_as<4, MASK, CAUSAL, DROP>(a, s);
 }
 
