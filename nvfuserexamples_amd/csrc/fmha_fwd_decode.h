@@ -5,9 +5,16 @@
 // loads (D / 8 neighbouring lanes cover one row, so a load instruction fetches 64 / (D / 8) complete rows),
 // keeps eight K loads and eight V loads in flight (up to 16 KB per wave, 128 KB per compute unit),
 // and does the arithmetic on the vector pipe in fp32: dot products on v_dot2c_f32_f16 / _bf16 (exact products of
-// the packed elements, fp32 sums; multiply-adds on unpacked elements for e4m3 rows), summed over the lanes of a
-// row by three or four DPP additions, an online softmax per lane group, P.V by multiply-add.
+// the packed elements, fp32 sums; e4m3 rows as fp16, which holds every e4m3 value), summed over the lanes of a
+// row by DPP additions, an online softmax per lane group, P.V by multiply-add.
 // Nothing is staged in LDS and nothing is rounded on the way (scores, probabilities and sums are fp32).
+//
+// Several query rows, and short ranges of one, are bound by instructions, so no lane repeats another's: the 8 or 16 lanes of a row
+// form two or four banks of four lanes, the sum over the lanes leaves a different score (query row, or key where rows are fewer) in each
+// bank, and reference, exponential and sum are formed once a bank; P.V reads the probability of another bank through DPP.  Before, every
+// lane had every score, and e4m3 rows were multiplied unpacked: a workgroup alone on its compute unit took 15.5 ns a key for four rows at
+// D 128, now 13, 8.5 at D 64, now 6.3.  Whole steps of one, two and four rows at 724 drawn sizes are 1.10, 1.19 and 1.32 times as fast (with
+// the lengths of the pieces that follow from this).
 //
 // Work split: a workgroup of four waves owns one (head, piece of the key range); its waves take the piece's
 // blocks of keys in turn, and inside a wave the 64 / (D / 8) lane groups take every such-th key.  Each lane
@@ -44,16 +51,25 @@ struct DecodeArgs {
 
 constexpr int kDecodeWaves = 4;
 
-// A lane's eight elements of a row: one 16-byte load of 16-bit elements, one 8-byte load of e4m3 bytes; and how
-// many K (and V) loads a wave keeps in flight per block (the same bytes either way).
+// A lane's eight elements of a row: one 16-byte load of 16-bit elements, one 8-byte load of e4m3 bytes; how many K (and V) loads a
+// wave keeps in flight per block (the same bytes either way); and the 16-bit type of the dot products (every e4m3 value is an fp16 value).
 template <typename TI> struct DecodeIn {
   using Load = u32x4;
+  using Dot = TI;
   static constexpr int LOADS = 8;
 };
 template <> struct DecodeIn<uint8_t> {
   using Load = u32x2;
+  using Dot = _Float16;
   static constexpr int LOADS = 16;
 };
+FMHA_DEV u32x4 dot_form(u32x4 w) { return w; }
+FMHA_DEV u32x4 dot_form(u32x2 w) { // eight e4m3 bytes as fp16
+  return u32x4{__builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w[0], 1.f, false)),
+               __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w[0], 1.f, true)),
+               __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w[1], 1.f, false)),
+               __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w[1], 1.f, true))};
+}
 
 template <typename T> FMHA_DEV void unpack8(u32x4 w, float (&x)[8]) {
   if constexpr (__is_same(T, _Float16)) {
@@ -92,35 +108,77 @@ template <typename T> FMHA_DEV float dot2(uint32_t a, uint32_t b, float c) {
   }
 }
 
-// Sum over the LPR (8 or 16) neighbouring lanes that hold one row; every lane gets the total.
-template <int LPR> FMHA_DEV float row_sum(float x) {
-  x += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0xB1, 0xf, 0xf, true));  // quad_perm [1,0,3,2]
-  x += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x4E, 0xf, 0xf, true));  // quad_perm [2,3,0,1]
-  x += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x141, 0xf, 0xf, true)); // row_half_mirror
-  if constexpr (LPR == 16)
-    x += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x140, 0xf, 0xf, true)); // row_mirror
+template <int V> struct Int {
+  static constexpr int value = V;
+};
+template <int N, int I = 0, typename F> FMHA_DEV void static_for(const F &f) {
+  if constexpr (I < N) {
+    f(Int<I>{});
+    static_for<N, I + 1>(f);
+  }
+}
+
+// Among the LPR (8 or 16) neighbouring lanes that hold one row, the LPR / 4 fours of lanes are its banks.  score_banks sums LPR / 4
+// values over those lanes at once and leaves value b in bank b, in all four of its lanes: what follows a score (reference, exponential,
+// sum) is then done once per bank and not by every lane.
+template <int CTRL> FMHA_DEV float dpp(float x) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xf, 0xf, true));
+}
+constexpr int DPP_ROW_MIRROR = 0x140, DPP_HALF_MIRROR = 0x141, DPP_ROR8 = 0x128, DPP_BCAST = 0x150; // (BCAST + n: lane n of each 16)
+template <int LPR> FMHA_DEV float score_banks(const float (&v)[LPR / 4], bool odd_bank, bool upper) {
+  float x, y;
+  if constexpr (LPR == 16) {
+    const float a = v[0] + dpp<DPP_ROW_MIRROR>(v[0]), b = v[1] + dpp<DPP_ROW_MIRROR>(v[1]);
+    const float c = v[2] + dpp<DPP_ROW_MIRROR>(v[2]), d = v[3] + dpp<DPP_ROW_MIRROR>(v[3]);
+    x = upper ? c : a;
+    y = upper ? d : b;
+  } else {
+    x = v[0];
+    y = v[1];
+  }
+  x += dpp<DPP_HALF_MIRROR>(x);
+  y += dpp<DPP_HALF_MIRROR>(y);
+  x = odd_bank ? y : x;
+  x += dpp<0xB1>(x); // quad_perm [1,0,3,2]
+  x += dpp<0x4E>(x); // quad_perm [2,3,0,1]
   return x;
+}
+// Bank b's value in every lane of the row (x is the same in the four lanes of a bank).
+template <int LPR, int B> FMHA_DEV float from_bank(float x) {
+  if constexpr (LPR == 16) return dpp<DPP_BCAST + 4 * B>(x);
+  else {
+    const int i = __builtin_bit_cast(int, x);
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(i, i, DPP_HALF_MIRROR, 0xf, B == 0 ? 0xA : 0x5, false));
+  }
 }
 
 // TI: element type of q, k, v (fp16, bf16 or uint8_t = e4m3); TO: of o and the mask (= TI unless TI is e4m3).
 template <typename TI, typename TO, int D, int NQ, bool MASK>
-__global__ __launch_bounds__(kDecodeWaves * 64) void fmha_fwd_decode_kernel(const DecodeArgs a) {
+// Two waves per SIMD at most, though fewer registers than 170 are needed: with three workgroups on some compute units and fewer on others the
+// fullest one is waited for (e4m3, one row, BH 30 20 092 keys D 128: 33.4 us, with two 30.0; 700 drawn sizes 1.006 times as fast, 0.92 to 1.35).
+__global__ __launch_bounds__(kDecodeWaves * 64) __attribute__((amdgpu_waves_per_eu(1, 2))) void fmha_fwd_decode_kernel(const DecodeArgs a) {
   using T = TI;
   using Load = typename DecodeIn<TI>::Load;
   constexpr int LPR = D / 8;       // lanes per row
   constexpr int NG = 64 / LPR;     // lane groups per wave = rows per load instruction
+  using Dot = typename DecodeIn<TI>::Dot;
   constexpr int U = NQ >= 4 ? 8 : DecodeIn<TI>::LOADS; // (four query rows: fewer loads in flight, for the registers)
+  constexpr int BANKS = LPR / 4;
+  constexpr int RP = NQ < BANKS ? NQ : BANKS; // the banks' scores: RP query rows of
+  constexpr int KP = BANKS / RP;              // KP keys (bank b: row b % RP, key b / RP)
+  constexpr int RR = NQ / RP, JJ = U / KP;
   constexpr int BLK = U * NG;      // keys per wave and block
   constexpr int NS = kDecodeWaves * NG; // softmax states per workgroup
   constexpr float NEG_INF = -__builtin_inff();
   static_assert(D == 64 || D == 128, "rows of 8 or 16 lanes");
 
-  constexpr int RG = NQ < 4 ? NQ : 4; // query rows that meet in LDS at a time
-  __shared__ float s_m[NS][RG], s_l[NS][RG];
-  __shared__ float s_acc[NS][RG][D];
+  __shared__ float s_m[NS][NQ], s_l[NS][NQ];
+  __shared__ float s_acc[NS][NQ][D];
 
   const int tid = threadIdx.x, w = tid >> 6, l = tid & 63;
   const int g = l / LPR, c8 = l % LPR; // the lane's group and its 8 columns
+  const bool odd_bank = l & 4, upper = l & 8;
+  const int bank = c8 >> 2, koff = bank / RP;
   const int head = blockIdx.x / a.pieces, piece = blockIdx.x - head * a.pieces;
 
   // keys of this piece: [k0, k1)
@@ -138,29 +196,23 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void fmha_fwd_decode_kernel(cons
   const size_t kss = (size_t)a.mk.ss, vss = (size_t)a.mv.ss;
   const TO *mrow = MASK ? (const TO *)a.mask + (size_t)(head / a.mask_div) * (size_t)a.mask_sb : nullptr;
 
-  // the lane's 8 columns of every query row: 16-bit rows stay packed (the dot products run on v_dot2c_f32_*, exact
-  // products summed in fp32, and the score is scaled afterwards); e4m3 rows are unpacked and scaled here
-  constexpr bool DOT2 = sizeof(TI) == 2;
-  Load qp[DOT2 ? NQ : 1];
-  float qf[DOT2 ? 1 : NQ][8];
+  // the lane's 8 columns of every query row, packed (the dot products run on v_dot2c_f32_*: exact products summed in fp32, and the
+  // score is scaled afterwards)
+  u32x4 qp[NQ];
 #pragma unroll
   for (int r = 0; r < NQ; ++r) {
     const int qr = r < a.sq ? r : a.sq - 1;
-    const Load t = *(const Load *)((const T *)a.q + a.mq.head(head) + (size_t)qr * (size_t)a.mq.ss + c8 * 8);
-    if constexpr (DOT2) {
-      qp[r] = t;
-    } else {
-      unpack8<T>(t, qf[r]);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) qf[r][e] *= a.scale_l2;
-    }
+    qp[r] = dot_form(*(const Load *)((const T *)a.q + a.mq.head(head) + (size_t)qr * (size_t)a.mq.ss + c8 * 8));
   }
 
-  float m_run[NQ], l_run[NQ], acc[NQ][8];
+  float m_run[RR], l_run[RR], acc[NQ][8];
+#pragma unroll
+  for (int rr = 0; rr < RR; ++rr) {
+    m_run[rr] = NEG_INF;
+    l_run[rr] = 0.f;
+  }
 #pragma unroll
   for (int r = 0; r < NQ; ++r) {
-    m_run[r] = NEG_INF;
-    l_run[r] = 0.f;
 #pragma unroll
     for (int e = 0; e < 8; ++e) acc[r][e] = 0.f;
   }
@@ -171,7 +223,7 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void fmha_fwd_decode_kernel(cons
   // scores are formed, its V loads as soon as this block's P.V is done, so that 8-16 loads per wave (and the other
   // waves of the SIMD) cover the trip to memory.
   Load kc[U], vc[U];
-  float mc[U];
+  float mc[JJ]; // (of the lane's bank)
   auto key_of = [&](int b, int j) {
     const int key = k0 + b * BLK + j * NG + g;
     return key < k1 ? key : k1 - 1; // keys past the end repeat the last one (their scores are set to -inf)
@@ -181,7 +233,10 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void fmha_fwd_decode_kernel(cons
     for (int j = 0; j < U; ++j) {
       const int key = key_of(b, j);
       kc[j] = *(const Load *)(Kb + (size_t)key * kss);
-      if constexpr (MASK) mc[j] = (float)mrow[key];
+    }
+    if constexpr (MASK) {
+#pragma unroll
+      for (int jj = 0; jj < JJ; ++jj) mc[jj] = (float)mrow[key_of(b, jj * KP + koff)];
     }
   };
   auto issue_v = [&](int b) {
@@ -196,112 +251,131 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void fmha_fwd_decode_kernel(cons
     const bool more = b + kDecodeWaves < nblk;
     const int kb = k0 + b * BLK;
     // scores of the group's U keys, all query rows
-    float s[NQ][U];
+    float s[RR][JJ];
 #pragma unroll
-    for (int j = 0; j < U; ++j) {
-      const bool live = kb + j * NG + g < k1;
-      float x[8];
-      if constexpr (!DOT2) unpack8<T>(kc[j], x);
+    for (int jj = 0; jj < JJ; ++jj) {
+      u32x4 x[KP];
 #pragma unroll
-      for (int r = 0; r < NQ; ++r) {
-        float d = 0.f;
-        if constexpr (DOT2) {
+      for (int kk = 0; kk < KP; ++kk) x[kk] = dot_form(kc[jj * KP + kk]);
+      const bool live = kb + (jj * KP + koff) * NG + g < k1;
 #pragma unroll
-          for (int i = 0; i < 4; ++i) d = dot2<T>(qp[r][i], kc[j][i], d);
-          d = row_sum<LPR>(d) * a.scale_l2;
-        } else {
+      for (int rr = 0; rr < RR; ++rr) {
+        float v[BANKS];
 #pragma unroll
-          for (int e = 0; e < 8; ++e) d = fmaf(qf[r][e], x[e], d);
-          d = row_sum<LPR>(d);
+        for (int bk = 0; bk < BANKS; ++bk) {
+          float d = 0.f;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) d = dot2<Dot>(qp[rr * RP + bk % RP][i], x[bk / RP][i], d);
+          v[bk] = d;
         }
-        if constexpr (MASK) d += fmaf(mc[j], a.mask_a, a.mask_b);
-        s[r][j] = live ? d : NEG_INF;
+        float d = score_banks<LPR>(v, odd_bank, upper) * a.scale_l2;
+        if constexpr (MASK) d += fmaf(mc[jj], a.mask_a, a.mask_b);
+        s[rr][jj] = live ? d : NEG_INF;
       }
     }
     if (more) issue_k(b + kDecodeWaves);
     // online softmax: raise the reference, rescale, turn the scores into probabilities
+    float alpha[RR];
 #pragma unroll
-    for (int r = 0; r < NQ; ++r) {
-      float bm = s[r][0];
+    for (int rr = 0; rr < RR; ++rr) {
+      float bm = s[rr][0];
 #pragma unroll
-      for (int j = 1; j < U; ++j) bm = fmaxf(bm, s[r][j]);
-      const float m_new = fmaxf(m_run[r], bm);
+      for (int jj = 1; jj < JJ; ++jj) bm = fmaxf(bm, s[rr][jj]);
+      if constexpr (KP == 4 || (KP == 2 && LPR == 8)) bm = fmaxf(bm, dpp<DPP_HALF_MIRROR>(bm)); // one reference for the keys' banks
+      if constexpr (KP > 1 && LPR == 16) bm = fmaxf(bm, dpp<DPP_ROR8>(bm));
+      const float m_new = fmaxf(m_run[rr], bm);
       const float m_use = m_new == NEG_INF ? 0.f : m_new; // nothing visible yet: every probability is 0
-      const float alpha = fast_exp2(m_run[r] - m_use);    // (2^-inf = 0 at the start)
-      m_run[r] = m_new;
+      alpha[rr] = fast_exp2(m_run[rr] - m_use);           // (2^-inf = 0 at the start)
+      m_run[rr] = m_new;
       float ps = 0.f;
 #pragma unroll
-      for (int j = 0; j < U; ++j) {
-        s[r][j] = fast_exp2(s[r][j] - m_use);
-        ps += s[r][j];
+      for (int jj = 0; jj < JJ; ++jj) {
+        s[rr][jj] = fast_exp2(s[rr][jj] - m_use);
+        ps += s[rr][jj];
       }
-      l_run[r] = l_run[r] * alpha + ps;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) acc[r][e] *= alpha;
+      l_run[rr] = l_run[rr] * alpha[rr] + ps; // (of the bank's keys)
     }
+    static_for<RP>([&](auto rp) {
+      constexpr int RI = decltype(rp)::value;
 #pragma unroll
-    for (int j = 0; j < U; ++j) {
-      float x[8];
-      unpack8<T>(vc[j], x);
+      for (int rr = 0; rr < RR; ++rr) {
+        const float al = from_bank<LPR, RI>(alpha[rr]);
 #pragma unroll
-      for (int r = 0; r < NQ; ++r) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) acc[r][e] = fmaf(s[r][j], x[e], acc[r][e]);
+        for (int e = 0; e < 8; ++e) acc[rr * RP + RI][e] *= al;
       }
+    });
+#pragma unroll
+    for (int jj = 0; jj < JJ; ++jj) {
+      static_for<KP>([&](auto kk) {
+        constexpr int KI = decltype(kk)::value;
+        float x[8];
+        unpack8<T>(vc[jj * KP + KI], x);
+        static_for<RP>([&](auto rp) {
+          constexpr int RI = decltype(rp)::value;
+#pragma unroll
+          for (int rr = 0; rr < RR; ++rr) {
+            const float p = from_bank<LPR, RI + RP * KI>(s[rr][jj]);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) acc[rr * RP + RI][e] = fmaf(p, x[e], acc[rr * RP + RI][e]);
+          }
+        });
+      });
     }
     if (more) issue_v(b + kDecodeWaves);
   }
 
-  // ---- the workgroup's NS partial softmaxes meet in LDS (up to four query rows at a time: RG)
+  // ---- the workgroup's NS partial softmaxes meet in LDS
   const int st = w * NG + g;
 #pragma unroll
-  for (int r0 = 0; r0 < NQ; r0 += RG) {
-    if (r0 > 0) __syncthreads(); // the previous rows have been read
-#pragma unroll
-    for (int rr = 0; rr < RG; ++rr) {
-      if (c8 == 0) {
-        s_m[st][rr] = m_run[r0 + rr];
-        s_l[st][rr] = l_run[r0 + rr];
-      }
-#pragma unroll
-      for (int e = 0; e < 8; ++e) s_acc[st][rr][c8 * 8 + e] = acc[r0 + rr][e];
+  for (int rr = 0; rr < RR; ++rr) {
+    float tot = l_run[rr];
+    if constexpr (KP == 4 || (KP == 2 && LPR == 8)) tot += dpp<DPP_HALF_MIRROR>(tot);
+    if constexpr (KP > 1 && LPR == 16) tot += dpp<DPP_ROR8>(tot);
+    if ((c8 & 3) == 0 && koff == 0) {
+      s_m[st][rr * RP + bank] = m_run[rr];
+      s_l[st][rr * RP + bank] = tot;
     }
-    __syncthreads();
-    // thread t: query row r0 + t / LPR, columns 8 * (t % LPR) .. +7
-    const int rr = tid / LPR, r = r0 + rr;
-    if (rr < RG && r < a.sq) {
-      float M = NEG_INF;
+  }
 #pragma unroll
-      for (int i = 0; i < NS; ++i) M = fmaxf(M, s_m[i][rr]);
-      float tot = 0.f, out[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-      if (M != NEG_INF) {
+  for (int r = 0; r < NQ; ++r) {
 #pragma unroll
-        for (int i = 0; i < NS; ++i) {
-          const float f = fast_exp2(s_m[i][rr] - M); // (an empty state: 2^-inf = 0)
-          tot = fmaf(s_l[i][rr], f, tot);
+    for (int e = 0; e < 8; ++e) s_acc[st][r][c8 * 8 + e] = acc[r][e];
+  }
+  __syncthreads();
+  // thread t: query row t / LPR, columns 8 * (t % LPR) .. +7
+  const int r = tid / LPR;
+  if (r < NQ && r < a.sq) {
+    float M = NEG_INF;
 #pragma unroll
-          for (int e = 0; e < 8; ++e) out[e] = fmaf(s_acc[i][rr][c8 * 8 + e], f, out[e]);
-        }
+    for (int i = 0; i < NS; ++i) M = fmaxf(M, s_m[i][r]);
+    float tot = 0.f, out[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    if (M != NEG_INF) {
+#pragma unroll
+      for (int i = 0; i < NS; ++i) {
+        const float f = fast_exp2(s_m[i][r] - M); // (an empty state: 2^-inf = 0)
+        tot = fmaf(s_l[i][r], f, tot);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) out[e] = fmaf(s_acc[i][r][c8 * 8 + e], f, out[e]);
       }
-      const float inv = tot > 0.f ? a.out_scale / tot : 0.f; // no visible key: O = 0, LSE = -inf
-      const float lse = tot > 0.f ? (M + fast_log2(tot)) * FMHA_LN2 : NEG_INF;
-      if (a.pieces > 1) {
-        float *dst = a.o_part + ((size_t)blockIdx.x * a.sq + r) * D + c8 * 8;
-        f32x4 lo = {out[0] * inv, out[1] * inv, out[2] * inv, out[3] * inv};
-        f32x4 hi = {out[4] * inv, out[5] * inv, out[6] * inv, out[7] * inv};
-        *(f32x4 *)dst = lo;
-        *(f32x4 *)(dst + 4) = hi;
-        if (c8 == 0) a.lse_part[(size_t)blockIdx.x * a.sq + r] = lse;
-      } else {
-        Pack16 y;
+    }
+    const float inv = tot > 0.f ? a.out_scale / tot : 0.f; // no visible key: O = 0, LSE = -inf
+    const float lse = tot > 0.f ? (M + fast_log2(tot)) * FMHA_LN2 : NEG_INF;
+    if (a.pieces > 1) {
+      float *dst = a.o_part + ((size_t)blockIdx.x * a.sq + r) * D + c8 * 8;
+      f32x4 lo = {out[0] * inv, out[1] * inv, out[2] * inv, out[3] * inv};
+      f32x4 hi = {out[4] * inv, out[5] * inv, out[6] * inv, out[7] * inv};
+      *(f32x4 *)dst = lo;
+      *(f32x4 *)(dst + 4) = hi;
+      if (c8 == 0) a.lse_part[(size_t)blockIdx.x * a.sq + r] = lse;
+    } else {
+      Pack16 y;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          if constexpr (__is_same(TO, _Float16)) y.h[e] = (_Float16)(out[e] * inv);
-          else y.b[e] = (__bf16)(out[e] * inv);
-        }
-        *(u32x4 *)((TO *)a.o + a.mo.head(head) + (size_t)r * (size_t)a.mo.ss + c8 * 8) = y.u;
-        if (a.lse && c8 == 0) a.lse[(size_t)head * a.sq + r] = lse;
+      for (int e = 0; e < 8; ++e) {
+        if constexpr (__is_same(TO, _Float16)) y.h[e] = (_Float16)(out[e] * inv);
+        else y.b[e] = (__bf16)(out[e] * inv);
       }
+      *(u32x4 *)((TO *)a.o + a.mo.head(head) + (size_t)r * (size_t)a.mo.ss + c8 * 8) = y.u;
+      if (a.lse && c8 == 0) a.lse[(size_t)head * a.sq + r] = lse;
     }
   }
 }

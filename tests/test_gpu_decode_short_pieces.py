@@ -55,4 +55,5 @@ def test_a_workspace_for_the_longer_pieces_only():
 
 
 def test_ranges_that_stay_whole():
-    assert _need(8, 1, 789, 64) == 0 and _need(16, 1, 1100, 128) == 0 and _need(178, 1, 1660, 128) == 0 and _need(255, 4, 1500, 128) == 0
+    """.. where the model of the two times has the merge cost more than the pieces save."""
+    assert _need(8, 1, 789, 64) == 0 and _need(16, 1, 700, 128) == 0 and _need(178, 1, 1660, 128) == 0 and _need(255, 4, 1500, 128) == 0
