@@ -57,8 +57,9 @@ enum {
 enum {
   FMHA_FLAG_NO_MASK_TRIM = 1,
   /* Forward only: a launch of few workgroups may share the keys of 32 queries out to the waves of a workgroup, which
-   * merge their partial sums in fp32.  Up to twice as fast there; without it the bits of a head's result do not depend on
-   * how many heads the launch has (the operators set it). */
+   * merge their partial sums in fp32, and with a workspace also cut the key range into pieces whose partial sums are fp32.  Up to
+   * four times as fast there; without it the bits of a head's result do not depend on how many heads the launch has (the
+   * operators set it). */
   FMHA_FLAG_SPLIT_KEYS = 4
   /* (value 2 asked for a one-pass backward kernel in earlier versions; it never beat the default and was
    * removed: the bit is accepted and ignored) */

@@ -14,6 +14,12 @@
 // padding there, and their pipelines have nothing to run ahead of (BH 2460 S 24 d 32 22.0 -> 8.1 us, BH 1690 17 x 24 d 96 with dropout
 // 34.0 -> 8.0, BH 3531 S 52 d 128 packed with dropout 87.6 -> 43.5, BH 3273 S 16 d 256 packed 96.1 -> 32.0).
 //
+// A build for pieces of the key range (few_chunk in fmha_capi.hip) serves launches whose 32-query groups leave most compute units idle, or
+// each with a long row: a head is a (head, piece), the mask and the key counts stay the whole range's, and the normalised rows go out
+// in fp32 with their log-sum-exps for a second launch to merge.  Bound by the piece's chain of blocks and the merge's 5 us; us, whole or in
+// plain pieces -> so: BH 17 19 x 1 698 d 256 54.7 -> 16.8, BH 1 12 x 1 568 d 80 38.1 -> 9.5, BH 2 613 x 2 785 d 128 55.3 -> 16.2; 743 drawn
+// launches (1 to 300 heads, 5 to 1 000 queries, 300 to 50 000 keys) 1.64 times as fast (least 0.92).
+//
 // Softmax as in fmha_fwd_mid.h: scores are scaled in fp32, the reference follows the row's maximum only where that has run ahead
 // by more than 2^8, row sums are those of the rounded P.
 #pragma once
@@ -33,7 +39,8 @@ template <int D, int NW_> struct FewCfg {
   static constexpr int LDS_BYTES = LDS_LAST + NW * 4;
 };
 
-template <typename T, int D, int NW, int MASK, bool CAUSAL, int DROP, bool STRIDED>
+// PIECES: a head is a piece of the key range (FwdArgs::pieces; the mask and the key counts are the whole range's); o gets fp32 rows [bh, sq, dcols].
+template <typename T, int D, int NW, int MASK, bool CAUSAL, int DROP, bool STRIDED, bool PIECES = false>
 __global__ __launch_bounds__((FewCfg<D, NW>::NT), D == 256 ? 1 : 2) void fmha_fwd_few_kernel(const FwdArgs a) {
   using C = FewCfg<D, NW>;
   using E = Elem<T>;
@@ -59,14 +66,17 @@ __global__ __launch_bounds__((FewCfg<D, NW>::NT), D == 256 ? 1 : 2) void fmha_fw
     qt = b0 < grouped ? (b0 >> 3) % a.nqt : b0 % a.nqt;
   }
   const int q0 = qt * C::QT, q = q0 + ql;
-  const T *Qr = (const T *)a.q + RW::head(a.mq, bh, a.sq) + (size_t)(q < a.sq ? q : a.sq - 1) * RW::ss(a.mq) + h * 8;
-  const T *Kb = (const T *)a.k + RW::head(a.mk, bh, a.sk);
-  const T *Vb = (const T *)a.v + RW::head(a.mv, bh, a.sk);
-  const T *mkey = MASK == kMaskPerKey ? (const T *)a.mask + (size_t)(bh / a.mask_div) * a.mask_sb : nullptr;
+  int piece = 0, head = bh;
+  if constexpr (PIECES) real_head<true>(a, bh, head, piece);
+  const T *Qr = (const T *)a.q + RW::head(a.mq, head, a.sq) + (size_t)(q < a.sq ? q : a.sq - 1) * RW::ss(a.mq) + h * 8;
+  const int sk = PIECES && a.sk_whole - piece * a.sk < a.sk ? a.sk_whole - piece * a.sk : a.sk; // rows that exist
+  const T *Kb = (const T *)a.k + RW::head(a.mk, head, a.sk) + (PIECES ? piece * a.piece_stride : 0);
+  const T *Vb = (const T *)a.v + RW::head(a.mv, head, a.sk) + (PIECES ? piece * a.piece_stride : 0);
+  const T *mkey = MASK == kMaskPerKey ? (const T *)a.mask + (size_t)(head / a.mask_div) * a.mask_sb + (PIECES ? piece * a.sk : 0) : nullptr;
   const uint32_t ss = RW::ss(a.mk);
   const int cols = RW::cols(a);
 
-  int kend = visible_keys<STRIDED>(a, bh, 0);
+  int kend = visible_keys<STRIDED>(a, head, piece);
   if (CAUSAL && kend > q0 + 32) kend = q0 + 32;
 
   // ---- a wave's block: its keys are b * BK .., chunk slot l + 64 i of the swizzled panel layout is this lane's
@@ -80,13 +90,13 @@ __global__ __launch_bounds__((FewCfg<D, NW>::NT), D == 256 ? 1 : 2) void fmha_fw
       int row, col;
       TileCopy<T, D, BK, 64>::slot(l + i * 64, row, col);
       int r = b * BK + row;
-      r = r < a.sk ? r : a.sk - 1; // rows past the end: their scores get -inf, and P = 0 meets finite values
+      r = r < sk ? r : sk - 1; // rows past the end: their scores get -inf, and P = 0 meets finite values
       const bool live = col * 8 < cols;
       const uint32_t at = (uint32_t)r * ss + (uint32_t)(live ? col * 8 : 0);
       kst[i] = *(const u32x4 *)(Kb + at);
       vst[i] = *(const u32x4 *)(Vb + at);
     }
-    if (MASK == kMaskPerKey) mraw = mkey[b * BK + (l & (BK - 1)) < a.sk ? b * BK + (l & (BK - 1)) : a.sk - 1];
+    if (MASK == kMaskPerKey) mraw = mkey[b * BK + (l & (BK - 1)) < sk ? b * BK + (l & (BK - 1)) : sk - 1];
   };
   auto store = [&](int b) {
 #pragma unroll
@@ -111,7 +121,7 @@ __global__ __launch_bounds__((FewCfg<D, NW>::NT), D == 256 ? 1 : 2) void fmha_fw
   if (MASK == kMaskPerKey && !(a.flags & kFwdFlagNoTrim)) { // hard-masked keys at the end need not be visited
     int *last = (int *)(lds + C::LDS_LAST), n = 0;
     for (int j = w * 64; j < kend; j += NW * 64) {
-      const float mk = fmaf((float)mkey[j + l < a.sk ? j + l : a.sk - 1], a.mask_a, a.mask_b);
+      const float mk = fmaf((float)mkey[j + l < sk ? j + l : sk - 1], a.mask_a, a.mask_b);
       const unsigned long long up = __builtin_amdgcn_ballot_w64(j + l < kend && mk > -9000.f * FMHA_LOG2E);
       if (up) n = j + 64 - (int)__builtin_clzll(up);
     }
@@ -272,7 +282,14 @@ __global__ __launch_bounds__((FewCfg<D, NW>::NT), D == 256 ? 1 : 2) void fmha_fw
 #pragma unroll
         for (int i = 0; i < 4; ++i) acc[4 * g + i] = fmaf(wt[j], v[i], acc[4 * g + i]);
       }
-    store_acc_block_row<T>(Or + db * 32, acc, out, h, cols - db * 32);
+    if constexpr (PIECES) {
+      float *dst = (float *)a.o + ((size_t)bh * a.sq + q) * cols + db * 32 + 4 * h;
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        if (db * 32 + 8 * g < cols) *(f32x4 *)(dst + 8 * g) = f32x4{acc[4 * g] * out, acc[4 * g + 1] * out, acc[4 * g + 2] * out, acc[4 * g + 3] * out};
+    } else {
+      store_acc_block_row<T>(Or + db * 32, acc, out, h, cols - db * 32);
+    }
   }
   if (a.lse && h == 0 && w == 0) a.lse[(size_t)bh * a.sq + q] = lt > 0.f ? (ref + fast_log2(lt)) * FMHA_LN2 : NEG_INF;
 }

@@ -20,9 +20,9 @@
 namespace fmha {
 namespace {
 
-template <int NW, int MASK, bool CAUSAL, int DROP> int launch_as(FwdArgs &a, hipStream_t s) {
+template <int NW, int MASK, bool CAUSAL, int DROP, bool PIECES = false> int launch_as(FwdArgs &a, hipStream_t s) {
   using C = FewCfg<FMHA_TU_D, NW>;
-  auto kern = fmha_fwd_few_kernel<FMHA_TU_T, FMHA_TU_D, NW, MASK, CAUSAL, DROP, FMHA_TU_STRIDED != 0>;
+  auto kern = fmha_fwd_few_kernel<FMHA_TU_T, FMHA_TU_D, NW, MASK, CAUSAL, DROP, FMHA_TU_STRIDED != 0, PIECES>;
   static const bool ready = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                                                 C::LDS_BYTES) == hipSuccess;
   if (!ready) return 2;
@@ -49,7 +49,13 @@ template <int MASK> int by_variant(FwdArgs &a, const FwdVariant &v, hipStream_t 
 } // namespace
 
 int FMHA_NAME(FMHA_TU_TNAME, FMHA_TU_D)(FwdArgs &a, const FwdVariant &v, hipStream_t s) {
-  if (v.mask == kMaskFull || v.drop == 2 || a.sk_whole != 0) return 1;
+  if (v.mask == kMaskFull || v.drop == 2) return 1;
+  if (a.sk_whole != 0) {
+#if FMHA_TU_STRIDED
+    if (!v.causal && !v.drop) return v.mask == kMaskPerKey ? launch_as<4, kMaskPerKey, false, 0, true>(a, s) : launch_as<4, kMaskNone, false, 0, true>(a, s);
+#endif
+    return 1;
+  }
   return v.mask == kMaskPerKey ? by_variant<kMaskPerKey>(a, v, s) : by_variant<kMaskNone>(a, v, s);
 }
 
