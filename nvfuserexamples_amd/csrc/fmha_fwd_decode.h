@@ -179,7 +179,9 @@ __global__ __launch_bounds__(kDecodeWaves * 64) __attribute__((amdgpu_waves_per_
   const int g = l / LPR, c8 = l % LPR; // the lane's group and its 8 columns
   const bool odd_bank = l & 4, upper = l & 8;
   const int bank = c8 >> 2, koff = bank / RP;
-  const int head = blockIdx.x / a.pieces, piece = blockIdx.x - head * a.pieces;
+  // The first pieces of all heads, then the second ones: with 8 pieces a head's would lie on one XCD each, and those of the last ones, which short
+  // heads don't have, idle; the full ones start first (724 drawn steps, half of them with key counts, 1.02 times as fast).
+  const int piece = blockIdx.x / a.bh, head = blockIdx.x - piece * a.bh, part = head * a.pieces + piece;
 
   // keys of this piece: [k0, k1)
   int n = a.sk;
@@ -361,12 +363,12 @@ __global__ __launch_bounds__(kDecodeWaves * 64) __attribute__((amdgpu_waves_per_
     const float inv = tot > 0.f ? a.out_scale / tot : 0.f; // no visible key: O = 0, LSE = -inf
     const float lse = tot > 0.f ? (M + fast_log2(tot)) * FMHA_LN2 : NEG_INF;
     if (a.pieces > 1) {
-      float *dst = a.o_part + ((size_t)blockIdx.x * a.sq + r) * D + c8 * 8;
+      float *dst = a.o_part + ((size_t)part * a.sq + r) * D + c8 * 8;
       f32x4 lo = {out[0] * inv, out[1] * inv, out[2] * inv, out[3] * inv};
       f32x4 hi = {out[4] * inv, out[5] * inv, out[6] * inv, out[7] * inv};
       *(f32x4 *)dst = lo;
       *(f32x4 *)(dst + 4) = hi;
-      if (c8 == 0) a.lse_part[(size_t)blockIdx.x * a.sq + r] = lse;
+      if (c8 == 0) a.lse_part[(size_t)part * a.sq + r] = lse;
     } else {
       Pack16 y;
 #pragma unroll

@@ -67,7 +67,12 @@ __global__ __launch_bounds__((FewCfg<D, NW>::NT), D == 256 ? 1 : 2) void fmha_fw
   }
   const int q0 = qt * C::QT, q = q0 + ql;
   int piece = 0, head = bh;
-  if constexpr (PIECES) real_head<true>(a, bh, head, piece);
+  if constexpr (PIECES) { // (the first pieces of all heads, then the second ones: the last ones of short heads are empty, and else lie on few XCDs)
+    const int heads = a.bh / a.pieces;
+    piece = bh / heads;
+    head = bh - piece * heads;
+    bh = head * a.pieces + piece;
+  }
   const T *Qr = (const T *)a.q + RW::head(a.mq, head, a.sq) + (size_t)(q < a.sq ? q : a.sq - 1) * RW::ss(a.mq) + h * 8;
   const int sk = PIECES && a.sk_whole - piece * a.sk < a.sk ? a.sk_whole - piece * a.sk : a.sk; // rows that exist
   const T *Kb = (const T *)a.k + RW::head(a.mk, head, a.sk) + (PIECES ? piece * a.piece_stride : 0);
