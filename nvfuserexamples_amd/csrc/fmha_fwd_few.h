@@ -74,14 +74,14 @@ __global__ __launch_bounds__((FewCfg<D, NW>::NT), D == 256 ? 1 : 2) void fmha_fw
     bh = head * a.pieces + piece;
   }
   const T *Qr = (const T *)a.q + RW::head(a.mq, head, a.sq) + (size_t)(q < a.sq ? q : a.sq - 1) * RW::ss(a.mq) + h * 8;
-  const int sk = PIECES && a.sk_whole - piece * a.sk < a.sk ? a.sk_whole - piece * a.sk : a.sk; // rows that exist
+  int kend = visible_keys<STRIDED>(a, head, piece);
+  const int sk = kend > 0 ? kend : 1; // rows that may be read: those behind the head's count hold anything (a piece behind it: its first row)
   const T *Kb = (const T *)a.k + RW::head(a.mk, head, a.sk) + (PIECES ? piece * a.piece_stride : 0);
   const T *Vb = (const T *)a.v + RW::head(a.mv, head, a.sk) + (PIECES ? piece * a.piece_stride : 0);
   const T *mkey = MASK == kMaskPerKey ? (const T *)a.mask + (size_t)(head / a.mask_div) * a.mask_sb + (PIECES ? piece * a.sk : 0) : nullptr;
   const uint32_t ss = RW::ss(a.mk);
   const int cols = RW::cols(a);
 
-  int kend = visible_keys<STRIDED>(a, head, piece);
   if (CAUSAL && kend > q0 + 32) kend = q0 + 32;
 
   // ---- a wave's block: its keys are b * BK .., chunk slot l + 64 i of the swizzled panel layout is this lane's
