@@ -132,7 +132,8 @@ typedef struct fmha_fwd_params {
 
   /* Optional valid key counts (the "padded version" the reference leaves as a TODO,
    * fmha_manual.cpp:110,178): head b attends keys [0, kv_len[b / kv_len_bh_div]) only, exactly
-   * as if the others carried a -inf mask, and whole key tiles past the count are never touched.
+   * as if the others carried a -inf mask.  k and v rows at or past the count may hold anything, NaN included (the unused
+   * part of a cache), but for the first row of a head whose count is 0.
    * Device pointer to int32, or NULL for all sk keys.  Not with FMHA_DROP_TENSOR / the save outputs. */
   const int32_t *kv_len;
   int32_t kv_len_bh_div;
@@ -258,7 +259,9 @@ typedef struct fmha_bwd_params {
   float scale;
   int32_t flags; /* 0 or FMHA_FLAG_NO_MASK_TRIM */
 
-  const int32_t *kv_len; /* as in fmha_fwd_params; dk and dv rows at or past the count are zero */
+  /* as in fmha_fwd_params; dk and dv rows at or past the count are zero.  (k and v rows there meet weights of zero in some
+   * kernels of the backward: finite values.) */
+  const int32_t *kv_len;
   int32_t kv_len_bh_div;
 
   /* Optional row layouts, as in fmha_fwd_params, of q, k, v, o, dout and of the outputs dq, dk, dv. */

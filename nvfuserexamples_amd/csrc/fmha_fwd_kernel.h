@@ -245,11 +245,9 @@ __global__ __launch_bounds__(NW * 64) void fmha_fwd_kernel(const FwdArgs a) {
     if (need < nkt) nkt = need;
   }
 
-  // rows of K and V that exist from Kb / Vb on: all sk, or what the whole key range leaves for this piece (>= 1)
-  int krows = a.sk;
-  if constexpr (STRIDED) {
-    if (a.pieces > 1 && a.sk_whole - piece * a.sk < krows) krows = a.sk_whole - piece * a.sk;
-  }
+  // rows of K and V that may be read from Kb / Vb on: those behind the head's count hold anything (a head or piece without a
+  // visible key: its first row)
+  const int krows = skv > 0 ? skv : 1;
 
   // ---- tile staging: global -> registers -> LDS
   u32x4 kst[CPT], vst[CPT];
@@ -260,7 +258,7 @@ __global__ __launch_bounds__(NW * 64) void fmha_fwd_kernel(const FwdArgs a) {
     for (int i = 0; i < CPT; ++i) {
       const int c = tid + i * NT;
       const int row = c / CPR, col = c % CPR;
-      // keys past the end re-read the last row: their scores get -inf through the extra step, so P = 0
+      // keys past the end re-read the last visible row: their scores get -inf through the extra step, so P = 0
       // meets finite values of V (unconditional loads do not stall on each other)
       int kr = k0 + row;
       kr = kr < krows ? kr : krows - 1;

@@ -66,9 +66,10 @@ __global__ __launch_bounds__(MidCfg<NW>::NT) __attribute__((amdgpu_waves_per_eu(
   TileCopy<T, D, C::BT, C::NT> tcopy;
   tcopy.init(tid, RW::ss(a.mk));
   const uint32_t lds0 = lds_address(lds);
-  const int nt = (a.sk + C::BT - 1) / C::BT;
-  for (int t = 0; t < nt; ++t) tcopy.issue(Kb, t * C::BT, a.sk, lds0 + (uint32_t)(t * C::TILEB), tid);
-  for (int t = 0; t < nt; ++t) tcopy.issue(Vb, t * C::BT, a.sk, lds0 + (uint32_t)(C::LDS_V + t * C::TILEB), tid);
+  const int rows = kend > 0 ? kend : 1; // rows behind the head's count hold anything
+  const int nt = (rows + C::BT - 1) / C::BT;
+  for (int t = 0; t < nt; ++t) tcopy.issue(Kb, t * C::BT, rows, lds0 + (uint32_t)(t * C::TILEB), tid);
+  for (int t = 0; t < nt; ++t) tcopy.issue(Vb, t * C::BT, rows, lds0 + (uint32_t)(C::LDS_V + t * C::TILEB), tid);
   const int q = q0w + ql;
   v8 qreg[KS];
 #pragma unroll

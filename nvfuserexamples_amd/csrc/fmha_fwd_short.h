@@ -94,10 +94,11 @@ FMHA_DEV void fwd_short_body(const FwdArgs &a) {
   tcopy.init(tid, RW::ss(a.mk));
   const uint32_t lds0 = lds_address(lds);
   const bool two_tiles = FULL || a.sk > C::BT;
-  tcopy.issue(Kb, 0, a.sk, lds0, tid);
-  if (two_tiles) tcopy.issue(Kb, C::BT, a.sk, lds0 + TILEB, tid);
-  tcopy.issue(Vb, 0, a.sk, lds0 + 2 * TILEB, tid);
-  if (two_tiles) tcopy.issue(Vb, C::BT, a.sk, lds0 + 3 * TILEB, tid);
+  const int rows = ROWS || kend > 0 ? kend : 1; // rows behind the head's count hold anything
+  tcopy.issue(Kb, 0, rows, lds0, tid);
+  if (two_tiles) tcopy.issue(Kb, C::BT, rows, lds0 + TILEB, tid);
+  tcopy.issue(Vb, 0, rows, lds0 + 2 * TILEB, tid);
+  if (two_tiles) tcopy.issue(Vb, C::BT, rows, lds0 + 3 * TILEB, tid);
 
   v8 qreg[KS];
   {
