@@ -470,6 +470,7 @@ std::tuple<at::Tensor, at::Tensor> fmha_fwd_fp8(const at::Tensor &q8, const at::
   p.descale_q = static_cast<float>(descale_q);
   p.descale_k = static_cast<float>(descale_k);
   p.descale_v = static_cast<float>(descale_v);
+  p.flags = FMHA_FLAG_SPLIT_KEYS; // few heads
   p.causal = is_causal ? 1 : 0;
   MaskLayout m;
   if (mask.has_value() && mask->defined()) {

@@ -219,6 +219,10 @@ typedef struct fmha_fwd_fp8_params {
   int32_t kv_len_bh_div;
   void *workspace;
   uint64_t workspace_bytes;
+  /* 0 or FMHA_FLAG_SPLIT_KEYS: a launch of few workgroups may share the keys of 32 queries out to the waves of a workgroup (up to twice
+   * as fast there).  Each wave has an M of its own, so probabilities deep below the row's maximum round differently there; without the flag, the
+   * bits of a head of more than four query rows (or a causal mask) do not depend on how many heads the launch has. */
+  int32_t flags;
 } fmha_fwd_fp8_params;
 
 int fmha_fwd_fp8_launch(const fmha_fwd_fp8_params *p, void *hip_stream);

@@ -13,6 +13,7 @@ LIB_PATH = os.path.join(_HERE, "lib", "libfmha_hip.so")
 F16, BF16 = 0, 1
 MASK_NONE, MASK_ADDITIVE, MASK_KEEP01 = 0, 1, 2
 FLAG_NO_MASK_TRIM = 1  # fwd(flags=...): visit every key tile even where a per-key mask hard-masks the tail
+FLAG_SPLIT_KEYS = 4    # fwd(flags=...), fwd_fp8(flags=...): launches of few workgroups may split their keys (the operators set it)
 DROP_NONE, DROP_PHILOX, DROP_TENSOR = 0, 1, 2
 
 EXPORTS = ("fmha_fwd_launch", "fmha_bwd_launch", "fmha_bwd_workspace_bytes", "fmha_philox_keep_mask",
@@ -95,6 +96,7 @@ class FwdFp8Params(_Params):
         ("causal", C.c_int32),
         ("kv_len", C.c_void_p), ("kv_len_bh_div", C.c_int32),
         ("workspace", C.c_void_p), ("workspace_bytes", C.c_uint64),
+        ("flags", C.c_int32),
     ]
 
 
@@ -372,11 +374,11 @@ def bwd(dout, q, k, v, o, lse, mask=None, mask_kind=MASK_ADDITIVE, mask_neg=-100
 
 
 def fwd_fp8(q8, k8, v8, descale_q=1.0, descale_k=1.0, descale_v=1.0, mask=None, causal=False, scale=None,
-            out_dtype=None, want_lse=False, kv_len=None, workspace=True):
+            out_dtype=None, want_lse=False, kv_len=None, workspace=True, flags=0):
     """Forward on e4m3 inputs (torch.float8_e4m3fn, contiguous [bh, s, d]) on the current stream.
     Returns (o, lse|None); o is float16 unless out_dtype says bfloat16.  mask: additive [bh|B, 1, sk] /
     [B,1,1,sk] in o's dtype.  kv_len (valid key counts, as in fwd) and workspace (as in fwd) apply to launches
-    of one to four query rows without a causal mask, which run on the streaming decode kernel."""
+    of one to four query rows without a causal mask, which run on the streaming decode kernel.  flags: 0 or FLAG_SPLIT_KEYS."""
     import torch
     out_dtype = out_dtype or torch.float16
     for t in (q8, k8, v8):
@@ -396,6 +398,7 @@ def fwd_fp8(q8, k8, v8, descale_q=1.0, descale_k=1.0, descale_v=1.0, mask=None, 
     P.scale = float(scale) if scale is not None else d ** -0.5
     P.descale_q, P.descale_k, P.descale_v = descale_q, descale_k, descale_v
     P.causal = int(bool(causal))
+    P.flags = flags
     if mask is not None:
         mask, div, sb, sqs = mask_layout(mask, bh, sq, sk)
         if mask.dtype != out_dtype or sqs != 0:

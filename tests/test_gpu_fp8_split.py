@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 import torch
 
-from nvfuserexamples_amd import capi
+from nvfuserexamples_amd import capi, load_ops
 from conftest import f32
 from test_gpu_fp8_tiles import _check, _inputs
 
@@ -56,3 +56,23 @@ def test_masked_tiles_of_some_waves(d, sk, monkeypatch):
         if n < b:
             assert torch.equal(o[n:], torch.zeros_like(o[n:])) and bool(torch.isneginf(lse[n:]).all())
             assert torch.equal(o0[n:], o[n:]) and torch.equal(lse0[n:], lse[n:])
+
+
+@pytest.mark.parametrize("sq,sk,d,causal", [(300, 600, 64, False), (600, 600, 64, True), (257, 700, 128, False), (700, 1100, 128, True)])
+def test_the_flag_decides(sq, sk, d, causal, monkeypatch):
+    """Without FMHA_FLAG_SPLIT_KEYS a head's bits are those it has in a launch of many heads; with it, as from the operator, few heads take the split
+    form."""
+    b, few = 200, 3
+    g = torch.Generator(device="cuda").manual_seed(sk)
+    q8, k8, v8 = (torch.randn(b, s, d, device="cuda", generator=g).to(torch.float8_e4m3fn) for s in (sq, sk, sk))
+    head = [x[:few].contiguous() for x in (q8, k8, v8)]
+    o, lse = capi.fwd_fp8(q8, k8, v8, causal=causal, want_lse=True)
+    o1, lse1 = capi.fwd_fp8(*head, causal=causal, want_lse=True)
+    assert torch.equal(o1, o[:few]) and torch.equal(lse1, lse[:few])
+    flagged = capi.fwd_fp8(*head, causal=causal, want_lse=True, flags=capi.FLAG_SPLIT_KEYS)
+    op = load_ops().fmha_fwd_fp8(*head, 1.0, 1.0, 1.0, None, 0.0, causal)
+    split, whole = _both(monkeypatch, *head, causal=causal)
+    assert not torch.equal(split[0], whole[0])
+    for got in (flagged, op):
+        assert torch.equal(got[0], split[0]) and torch.equal(got[1], split[1])
+    assert torch.equal(o1, whole[0]) and torch.equal(lse1, whole[1])
