@@ -238,6 +238,19 @@ __global__ __launch_bounds__((Fp8Cfg<D, SPLIT>::NT), D == 64 ? (SPLIT || CAUSAL 
   // k / 32 in a 4-bit one.)
   const int one0 = (l >> 2) & 1 ? 0 : 0x22222222, one1 = 0x22222222 - one0; // (1.0 in e2m1)
   const i32x4v ones = {one0, one0, one1, one1};
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  // A NaN of query c times 0 is a NaN in the sum of query c + 16.  So where there may be one, rows with a NaN are cleared before
+  // the product is formed; whether this lane's row was:
+  auto clear_nan_row = [&](i32x8 &p) {
+    int any = 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) any |= (p[i] & 0x7f7f7f7f) + 0x01010101; // (e4m3: all seven bits)
+    const auto both = __builtin_amdgcn_permlane32_swap(any, any, false, false);
+    const bool nan = ((both[0] | both[1]) & 0x80808080) != 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) p[i] = nan ? 0 : p[i];
+    return nan;
+  };
   // extra-step column of a query: bf16 (1, 1, 1, 0 ..); the other half-wave, which reads the same rows, takes zeros
   const uint32_t bx0 = h == 0 ? 0x3f803f80u : 0u, bx1 = h == 0 ? 0x3f80u : 0u;
 
@@ -368,7 +381,6 @@ __global__ __launch_bounds__((Fp8Cfg<D, SPLIT>::NT), D == 64 ? (SPLIT || CAUSAL 
     for (int sb = 0; sb < 2; ++sb)
 #pragma unroll
       for (int g = 0; g < 4; ++g) pb[sb * 4 + g] = pack4_e4m3(x[sb][4 * g], x[sb][4 * g + 1], x[sb][4 * g + 2], x[sb][4 * g + 3]);
-    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
     float tsum = mfma_fp4_fp8_k128(ones, pb, zero)[0]; // of the rounded probabilities of this lane's row
     // Slow path, wave-uniform: a row sum beyond the range that guarantees representable probabilities (compared as
     // bit patterns: the sum is never negative, and a NaN from a saturated conversion must take this path although the
@@ -376,8 +388,13 @@ __global__ __launch_bounds__((Fp8Cfg<D, SPLIT>::NT), D == 64 ? (SPLIT || CAUSAL 
     // overwritten them), the reference becomes ceil(max), everything is rescaled by the exact power of two.
     // Only the rows that need it change their reference (and take the recomputed probabilities): a row's result
     // depends on that row alone, whatever rows share its wave.
-    const bool need = __float_as_uint(tsum) > __float_as_uint(SUM_LIMIT);
-    if (__builtin_amdgcn_ballot_w64(need)) {
+    if (__builtin_amdgcn_ballot_w64(__float_as_uint(tsum) > __float_as_uint(SUM_LIMIT))) {
+      bool need = __float_as_uint(tsum) > __float_as_uint(SUM_LIMIT);
+      if (__builtin_amdgcn_ballot_w64(__float_as_uint(tsum) > 0x7f800000u)) { // (wave-uniform, as the product wants all lanes)
+        const bool over = clear_nan_row(pb);
+        tsum = mfma_fp4_fp8_k128(ones, pb, zero)[0];
+        need = over || tsum > SUM_LIMIT;
+      }
       f32x16 y[2];
 #pragma unroll
       for (int sb = 0; sb < 2; ++sb) {
@@ -411,7 +428,10 @@ __global__ __launch_bounds__((Fp8Cfg<D, SPLIT>::NT), D == 64 ? (SPLIT || CAUSAL 
           const int pn = pack4_e4m3(y[sb][4 * g], y[sb][4 * g + 1], y[sb][4 * g + 2], y[sb][4 * g + 3]);
           pb[sb * 4 + g] = need ? pn : pb[sb * 4 + g]; // (both half-waves of a row decide alike: the sums they test are the row's)
         }
+      const bool lost = clear_nan_row(pb); // (a NaN among the inputs: the row's output is one)
       tsum = mfma_fp4_fp8_k128(ones, pb, zero)[0];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) pb[i] = lost ? 0x7f7f7f7f : pb[i];
       l_run *= alpha;
       l_true *= alpha;
 #pragma unroll
