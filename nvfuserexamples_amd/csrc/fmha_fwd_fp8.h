@@ -273,6 +273,7 @@ __global__ __launch_bounds__((Fp8Cfg<D, SPLIT>::NT), D == 64 ? (SPLIT || CAUSAL 
   lstore(first);
   if (first + STEP < nkt) gload((first + STEP) * BK);
   if (trim || !SPLIT) __syncthreads();
+  else __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); // (as behind every later stage: other lanes read what this one wrote)
   if (trim) {
     int last = 0, seen_live = 0;
 #pragma unroll
