@@ -58,8 +58,9 @@ enum {
   FMHA_FLAG_NO_MASK_TRIM = 1,
   /* Forward only: a launch of few workgroups may share the keys of 32 queries out to the waves of a workgroup, which
    * merge their partial sums in fp32, and with a workspace also cut the key range into pieces whose partial sums are fp32.  Up to
-   * four times as fast there; without it the bits of a head's result do not depend on how many heads the launch has (the
-   * operators set it). */
+   * four times as fast there (the operators set it).  The number of heads then decides between forms that differ in the last
+   * bits.  Without the flag it still decides in some ranges of the 16-bit forward: how a workspace's pieces are cut and, at head dim 64,
+   * which kernel takes up to 512 keys, or 1024 and more. */
   FMHA_FLAG_SPLIT_KEYS = 4
   /* (value 2 asked for a one-pass backward kernel in earlier versions; it never beat the default and was
    * removed: the bit is accepted and ignored) */
@@ -132,7 +133,8 @@ typedef struct fmha_fwd_params {
 
   /* Optional valid key counts (the "padded version" the reference leaves as a TODO,
    * fmha_manual.cpp:110,178): head b attends keys [0, kv_len[b / kv_len_bh_div]) only, exactly
-   * as if the others carried a -inf mask.  k and v rows at or past the count may hold anything, NaN included (the unused
+   * as if the others carried a -inf mask (in the bits of a -10000 mask, wherever both forms take the same kernel: at head dim 64, 129 to 256 keys and
+   * 1024 keys and more, they have lines of their own).  k and v rows at or past the count may hold anything, NaN included (the unused
    * part of a cache), but for the first row of a head whose count is 0.
    * Device pointer to int32, or NULL for all sk keys.  Not with FMHA_DROP_TENSOR / the save outputs. */
   const int32_t *kv_len;
@@ -160,15 +162,17 @@ typedef struct fmha_fwd_params {
 
   /* Optional device memory for a forward whose key range is cut into pieces (no counterpart in the
    * reference, whose shapes are fixed at 128 x 128 per head, fmha_manual.cpp:24-29).  A decode step -- one
-   * or a few query rows per head against a long key range -- on fewer heads than the chip has compute units
-   * would leave most of them idle while each busy one streams a whole K and V.  Given a workspace of at
+   * or a few query rows per head against a long key range -- on few heads
+   * would leave most compute units idle, or some with twice the work of others, while each streams a whole K and V.  Given a workspace of at
    * least fmha_fwd_workspace_bytes(p) bytes (16-byte aligned), such a launch runs every piece of the key
    * range as a workgroup (or head) of its own, keeps the pieces' normalised outputs and log-sum-exps in the
    * workspace and merges them in a second launch:
    *   O = sum_c exp(LSE_c - LSE) O_c,   LSE = log sum_c exp(LSE_c).
    * Launches of one to four query rows at head dim 64 or 128 (which have a streaming kernel of their own,
-   * with or without pieces) keep their pieces in fp32; other shapes keep them in the element type, so their
-   * results differ from the plain launch by one more rounding to that type.  Pieces are used without a
+   * with or without pieces), and with FMHA_FLAG_SPLIT_KEYS those of few queries or few heads, keep their pieces in fp32; the others (many
+   * queries of long ranges, or without the flag, on fewer workgroups than compute units) keep them in the element type, so their
+   * results differ from the plain launch by one more rounding to that type.  A workspace smaller than asked for may still hold a plan of pieces of 1024 keys or more,
+   * which is then taken.  Pieces are used without a
    * causal mask, dropout or saved outputs, with no mask or a mask that is constant along the queries, with
    * or without kv_len; everything else, a NULL or too small workspace included, takes the plain launch.
    * The workspace may be reused by the next launch on the same stream. */
@@ -180,7 +184,8 @@ typedef struct fmha_fwd_params {
 int fmha_fwd_launch(const fmha_fwd_params *p, void *hip_stream);
 
 /* Bytes of `workspace` with which fmha_fwd_launch(p) would run its key range in pieces on the current
- * device, or 0 where it would not (p as for the launch; the pointers are not looked at). */
+ * device, or 0 where it would not (p as for the launch, sizes, kinds, strides and flags; of the pointers only whether
+ * save_softmax and save_dropout are NULL is looked at). */
 uint64_t fmha_fwd_workspace_bytes(const fmha_fwd_params *p);
 
 /*

@@ -13,7 +13,7 @@
 // form two or four banks of four lanes, the sum over the lanes leaves a different score (query row, or key where rows are fewer) in each
 // bank, and reference, exponential and sum are formed once a bank; P.V reads the probability of another bank through DPP.  Before, every
 // lane had every score, and e4m3 rows were multiplied unpacked: a workgroup alone on its compute unit took 15.5 ns a key for four rows at
-// D 128, now 13, 8.5 at D 64, now 6.3.  Whole steps of one, two and four rows at 724 drawn sizes are 1.10, 1.19 and 1.32 times as fast (with
+// D 128, now 13, 8.5 at D 64, now 6.3.  Whole steps of one, two and four rows at 746 drawn sizes are 1.09, 1.18 and 1.37 times as fast (with
 // the lengths of the pieces that follow from this).
 //
 // Work split: a workgroup of four waves owns one (head, piece of the key range); its waves take the piece's

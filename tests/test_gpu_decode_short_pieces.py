@@ -1,5 +1,5 @@
-"""Decode steps of few heads: pieces of the key range below 1024 keys (128 to 640, by head dim and query rows), down to ranges of 512 to 2047 keys,
-the merge of up to 64 pieces, and a workspace that only has room for the longer pieces."""
+"""Decode steps of few heads: pieces of the key range below 1024 keys (128 keys and more, by a model of the step's time), ranges of 513 keys and more,
+the merge of up to 64 pieces, a workspace that only has room for the longer pieces, and steps that the model keeps whole."""
 import ctypes as C
 import numpy as np
 import pytest

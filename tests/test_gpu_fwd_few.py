@@ -87,11 +87,14 @@ def test_masks_counts_and_layouts(d, sk, packed, waves, monkeypatch):
 
 @pytest.mark.parametrize("bh,sq,sk,d,causal", [(2, 200, 200, 128, False), (8, 600, 600, 64, True), (4, 96, 5000, 64, False), (17, 1000, 1000, 128, False), (3, 200, 300, 256, True)])
 def test_the_flag_decides(bh, sq, sk, d, causal, monkeypatch):
-    """Without FMHA_FLAG_SPLIT_KEYS a head's bits are those of the launch it is in alone; the operator, which sets the flag, takes this kernel where
+    """Without FMHA_FLAG_SPLIT_KEYS a launch of few workgroups does not take this kernel: at these shapes, where the other kernels have no line in the
+    number of heads, a head's bits are those it has among twelve times as many.  The operator, which sets the flag, takes this kernel where
     the rule does and agrees with the other kernels to the rounding of O.  (4 x 96 x 5000 stays in pieces, 17 x 1000 is too large.)"""
     monkeypatch.delenv("FMHA_FWD_FEW", raising=False)
     q, k, v = (t.cuda() for t in make_qkv(bh, sq, sk, d, seed=d, std=0.5))
     plain = capi.fwd(q, k, v, causal=causal, want_lse=True, workspace=False)
+    many = capi.fwd(*(t.repeat(12, 1, 1) for t in (q, k, v)), causal=causal, want_lse=True, workspace=False)
+    assert torch.equal(many[0][-bh:], plain[0]) and torch.equal(many[1][-bh:], plain[1])
     flagged = capi.fwd(q, k, v, causal=causal, want_lse=True, flags=4)
     ops = load_ops()
     got = ops.fmha_fwd(q, k, v, None, 0.0, causal, 0.0, 0, 0, None)
