@@ -1,5 +1,8 @@
 // The forward whose waves share 32 queries (fmha_fwd_few.h) for one (element type, head dim, row layout kind) triple, chosen with
 // -DFMHA_TU_BF16={0,1} -DFMHA_TU_D={32,64,96,128,256} -DFMHA_TU_STRIDED={0,1}, and its dispatcher.
+// The rules (few_waves, few_chunk) reach every build: four and eight waves each mask, causal or not, with and without dropout (training forwards), at head
+// dim 256 four only; one wave the same, at head dim 64 causal launches, dropout on many heads and query rows too far apart for the one-pass
+// kernel; pieces without causal mask and dropout from run-time row layouts (folded tensors are one).
 #include "fmha_launch.h"
 
 #if FMHA_TU_BF16
