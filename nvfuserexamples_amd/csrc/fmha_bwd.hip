@@ -47,7 +47,7 @@ template <typename K> int set_lds(K kern, int bytes) {
 }
 
 // The pipelined kernels (fmha_bwd_pipe.hip) take everything but full mask tensors and, at head dim 256, dK / dV -- at head dims 128
-// and 256 from a number of queries on, because their prologue costs more and a causal head's dQ streams are cut short by its diagonal.
+// and 256 from a number of queries on, because their prologue costs more.
 // Kernel times, us, pipelined / phase by phase, 512 heads, D 128, fp16, S queries and keys:
 //   dQ, no causal mask     S 61 13 / 11, S 128 20 / 21, S 256 58 / 62, S 512 131 / 131, S 1024 402 / 418
 //     with dropout         S 61 15 / 13, S 128 22 / 22, S 256 59 / 59, S 512 147 / 152, S 1024 455 / 471
@@ -62,20 +62,12 @@ template <typename K> int set_lds(K kern, int bytes) {
 // 228; BH 576 S 120 56 / 49).
 template <int MASK, bool CAUSAL, int DROP> constexpr bool pipe_built() { return FMHA_TU_D != 256 && MASK != kMaskFull; }
 static inline bool pipe_wanted(const BwdArgs &a) { return FMHA_TU_D <= 64 || a.sq >= 128; }
-// dQ of causal heads at head dim 128 has a line of its own: a pass pays the prologue with all compute units in step, and
-// workgroups take pairs of short streams.  Same measurement (us, pipelined / phase by phase, 512 heads, fp16, in brackets
-// bf16): S 384 107 / 93, S 512 134 / 126 (144 / 117), S 640 170 / 161, S 768 198 / 198 (204 / 195), S 896 257 / 256
-// (265 / 254), S 1024 292 / 303 (293 / 289), S 1536 534 / 571 (529 / 558); with dropout S 512 142 / 129, S 768 230 / 216,
-// S 896 300 / 292, S 1024 336 / 335; BH 256 S 2048 438 / 484, with dropout BH 128 S 2048 271 / 281: level to 4 % either way
-// from 896 to 1024, ahead beyond.  (At few heads ahead earlier, BH 64 S 512 23 / 25, but a head's gradients do not depend
-// on how many others there are.)
+// dQ of causal heads at head dim 128 follows the same line (backward, us, phase by phase / pipelined, 512 heads: S 160 bf16 73.1 / 72.1,
+// S 256 106.8 / 105.7, S 384 169.4 / 163.8, S 512 248 / 244, S 768 446 / 418, S 895 fp16 627 / 573; with dropout S 200 107 / 103, S 640
+// fp16 423 / 387; BH 64 S 512 47.9 / 41.4, BH 100 S 700 87.6 / 87.7, BH 40 S 800 with dropout 76.4 / 61.3).
 // dQ at head dim 256, one wave per SIMD: from 128 queries on as well (us, pipelined / phase by phase: BH 128 S 2048 750 / 1041,
 // causal 440 / 616; BH 64 S 1000 with dropout 118 / 140; BH 300 S 512 bf16 causal with dropout 174 / 244; BH 512 S 256 119 / 126,
 // causal 113 / 126, S 128 42.6 / 43.7; BH 1000 S 129 causal 164 / 174; BH 8 S 1750 59 / 102).
-template <bool CAUSAL> bool pipe_wanted_dq(const BwdArgs &a) {
-  return pipe_wanted(a) && !(FMHA_TU_D == 128 && CAUSAL && a.sq < 896);
-}
-
 template <typename K> int launch_one(K kern, BwdArgs &a, long long nblk, int threads, int lds, hipStream_t s) {
   if (nblk > 0x7fffffffLL) return 2;
   hipLaunchKernelGGL(kern, dim3((unsigned)nblk), dim3(threads), lds, s, a);
@@ -84,7 +76,7 @@ template <typename K> int launch_one(K kern, BwdArgs &a, long long nblk, int thr
 
 template <int MASK, bool CAUSAL, int DROP> int launch_dq(BwdArgs &a, const BwdVariant &v, long long nblk, hipStream_t s) {
   if constexpr (MASK != kMaskFull) { // (pipe_built, or head dim 256, where it is built for dQ only)
-    if (pipe_wanted_dq<CAUSAL>(a)) return FMHA_PIPE_NAME(FMHA_TU_TNAME, FMHA_TU_D)(a, v, false, nblk, s);
+    if (pipe_wanted(a)) return FMHA_PIPE_NAME(FMHA_TU_TNAME, FMHA_TU_D)(a, v, false, nblk, s);
   }
   if constexpr (!(pipe_built<MASK, CAUSAL, DROP>() && FMHA_TU_D <= 64)) { // (there the pipelined kernel takes all)
     constexpr int kLds = BwdCfg<FMHA_TU_D, bwd_dq_tile_rows<FMHA_TU_D>()>::LDS_BYTES;

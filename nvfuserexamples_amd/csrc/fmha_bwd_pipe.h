@@ -170,6 +170,12 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(bwd_dq_
   };
 
   for (int pass = 0; pass < npass; ++pass) {
+    // (At head dim 128 set up for each pass, from an index that the compiler cannot trace: kept from one pass to the next, what a lane
+    // addresses had 33 to 59 registers spilled into the stream.  Backward, us: BH 512 S 1024 bf16 698 -> 649, with dropout 836 -> 776,
+    // BH 128 S 900 167 -> 154, BH 32 S 4096 497 -> 485.  Where nothing spills it costs the second pass 1 to 2 %.)
+    int tid = threadIdx.x;
+    if (CAUSAL && D > 64) asm volatile("" : "+v"(tid));
+    const int w = tid >> 6, l = tid & 63, ql = l & 31, h = l >> 5;
     const int qt = CAUSAL ? (pass == 0 ? a.ntile - 1 - pi : pi) : pi;
     const int q0w = qt * QT + w * 32;
     const int q = q0w + ql;
@@ -527,6 +533,10 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(bwd_dkd
   };
 
   for (int pass = 0; pass < npass; ++pass) {
+    // (where registers spilled set up for each pass, see dQ: BH 600 S 380 D 64 packed with dropout, backward 134.6 -> 131.8 us)
+    int tid = threadIdx.x;
+    if (CAUSAL && (D > 64 || STRIDED)) asm volatile("" : "+v"(tid));
+    const int w = tid >> 6, l = tid & 63, kl = l & 31, h = l >> 5;
     const int ktile = pass == 0 ? pi : a.ntile - 1 - pi;
     const int k0w = ktile * KT + w * 32;
     const int key = k0w + kl;
