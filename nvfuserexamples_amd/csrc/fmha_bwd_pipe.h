@@ -38,7 +38,10 @@ template <int D> struct BwdPipeCfg {
   static constexpr int BT = 32, NST = 4; // rows per tile, tiles resident per operand
   static constexpr int KS = D / 16, DB = D / 32;
   static constexpr int TILEB = BT * tile_cols(D) * 2, STAGEB = 2 * TILEB;
-  static constexpr int OFF_X = NST * STAGEB;
+  static constexpr bool TURNED = D == 64 || D == 128;                       // register operands are read as whole rows (load_row_operands)
+  static constexpr int OFF_T = (NST - 1) * STAGEB, TURNB = 32 * kPanelRowB; // ... and turned here, in the last stage, a panel per wave
+  static constexpr int OFF_X = D == 64 ? OFF_T + 4 * TURNB : NST * STAGEB;
+  static_assert(!TURNED || 4 * TURNB + OFF_T <= OFF_X, "a panel for each of four waves");
   static_assert(4 * RowStore<D>::BYTES <= OFF_X, "the output rows are turned in the tiles' LDS");
   static constexpr int MSEG = 4096;             // per-key mask terms staged at once
   static constexpr int QSEG = 1024;             // queries whose extra-step rows are staged at once (dK / dV)
@@ -72,6 +75,38 @@ template <typename T, int D, int NT> struct PipeCopy {
   FMHA_DEV void issue(const T *base, int tile, uint32_t lds_tile, int i) const {
     const uint32_t o = voff[i] + (uint32_t)tile * tile_step;
     dma_global_to_lds_b128(base, o < lim[i] ? o : lim[i], lds_tile + dst + (uint32_t)(i * NT * 16));
+  }
+};
+
+// A wave's 32 rows as register operands: lane (row l % 32, half l / 32) gets columns 16 ks + 8 (l / 32) .. +7.  Loaded as they are
+// wanted, an instruction touches 32 rows, 32 bytes of each.  Here whole panel rows are loaded, eight lanes a row, and turned through a
+// panel of the wave's own LDS.  Backward, us, loaded as wanted / so: D 128 BH 512 S 1024 bf16 causal 642 / 623, S 384 169 / 166, packed
+// with dropout S 512 369 / 358; D 64 BH 512 S 1024 causal 343 / 331, packed S 512 170 / 166, BH 256 S 800 with dropout 234 / 229,
+// BH 100 S 400 31.8 / 30.6; level to 1.5 % behind on whole rows without mask and dropout, BH 512 S 512 157 / 158.
+template <typename T, int D> struct RowOperands {
+  static constexpr int NI = 32 * tile_cols(D) / 8 / 64;
+  u32x4 v[NI];
+  FMHA_DEV void load(const T *base, uint32_t ss, int row0, int rend, int cols, int l) {
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      int row, col;
+      TileCopy<T, D, 32, 64>::slot(l + i * 64, row, col);
+      int r = row0 + row;
+      r = r < rend ? r : rend - 1;
+      v[i] = *(const u32x4 *)(base + (size_t)(uint32_t)r * ss + (col * 8 < cols ? col * 8 : 0)); // (as in PipeCopy)
+    }
+  }
+  FMHA_DEV void turn(char *panel, const PanelLane &pl, int l, u32x4 (&out)[D / 16]) const {
+#pragma unroll
+    for (int p = 0; p < NI / 4; ++p) {
+      asm volatile("" ::: "memory"); // (a wave's LDS accesses execute in order)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) *(u32x4 *)(panel + (l + i * 64) * 16) = v[4 * p + i];
+      asm volatile("" ::: "memory");
+#pragma unroll
+      for (int ks = 4 * p; ks < 4 * p + 4 && ks < D / 16; ++ks) out[ks] = as_u32x4(panel_read_rows<T, 32>(panel, pl, 0, ks & 3));
+    }
+    asm volatile("" ::: "memory");
   }
 };
 
@@ -197,24 +232,39 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(bwd_dq_
 #pragma unroll
     for (int t = 0; t < NST - 1; ++t) dma_kv(t);
 
+    PanelLane pl;
+    pl.init(l);
     // ---- per-row operands (all loads unconditional, see fmha_bwd_dq_kernel)
     v8 qreg[KS], doreg[KS], bxs, bxd;
     float delta, nlse;
     {
       const int qc = q < a.sq ? q : a.sq - 1;
       u32x4 tq[KS], td[KS], to[KS];
+      RowOperands<T, D> rq, rd, ro;
+      if constexpr (C::TURNED) {
+        rq.load(Qb, RW::ss(a.mq), q0w, a.sq, RW::cols(a), l);
+        rd.load(dOb, RW::ss(a.mdo), q0w, a.sq, RW::cols(a), l);
+        ro.load(Ob, RW::ss(a.mo), q0w, a.sq, RW::cols(a), l);
+      } else {
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        const size_t col = ks * 16 + h * 8 < RW::cols(a) ? ks * 16 + h * 8 : 0;
-        tq[ks] = *(const u32x4 *)(Qb + (size_t)qc * RW::ss(a.mq) + col);
-        td[ks] = *(const u32x4 *)(dOb + (size_t)qc * RW::ss(a.mdo) + col);
-        to[ks] = *(const u32x4 *)(Ob + (size_t)qc * RW::ss(a.mo) + col);
+        for (int ks = 0; ks < KS; ++ks) {
+          const size_t col = ks * 16 + h * 8 < RW::cols(a) ? ks * 16 + h * 8 : 0;
+          tq[ks] = *(const u32x4 *)(Qb + (size_t)qc * RW::ss(a.mq) + col);
+          td[ks] = *(const u32x4 *)(dOb + (size_t)qc * RW::ss(a.mdo) + col);
+          to[ks] = *(const u32x4 *)(Ob + (size_t)qc * RW::ss(a.mo) + col);
+        }
       }
       const float lse_q = a.lse[(size_t)bh * a.sq + qc];
       if (MASK == kMaskPerKey && (pass == 0 || a.sk > C::MSEG)) { // (with more than one segment the first pass leaves a later one)
         const int n = stage_mask(0); // (its loads share the trip to memory)
         const bool trim = a.sk > 128 && a.sk <= C::MSEG && !(a.flags & kBwdFlagNoTrim);
         if (trim && n > 0 && n < skv) skv = n; // a row without any live key keeps all its keys
+      }
+      if constexpr (C::TURNED) {
+        char *panel = lds + C::OFF_T + w * C::TURNB;
+        rq.turn(panel, pl, l, tq);
+        rd.turn(panel, pl, l, td);
+        ro.turn(panel, pl, l, to);
       }
       float dsum = 0.f;
 #pragma unroll
@@ -274,8 +324,6 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(bwd_dq_
       nktw = own < nkt ? own : nkt;
     }
 
-    PanelLane pl;
-    pl.init(l);
     constexpr uint32_t ONES = std::is_same<T, _Float16>::value ? 0x3c003c00u : 0x3f803f80u;
     constexpr uint32_t BIGPAIR = std::is_same<T, _Float16>::value ? 0x0000fb53u : 0x0000c76au; // (-60000 in T, 0)
     auto hl_of = [&](int kt) -> uint32_t { // (mask_hi, mask_lo) of key (l % 32) of a tile
@@ -400,19 +448,32 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(bwd_dq_
     using No = std::false_type;
 
     // ---- first products of tile 0 (its wait covers the loads above too: they are younger than its copies)
+    uint32_t wd0[4];
+    if (DROP == 1) drop_words_q(a.drop, (uint32_t)bh, (uint32_t)q, 0u, h, l, wd0); // (while the tiles are on their way)
     bwd_vm_wait<0>();
     bwd_lds_barrier();
-    auto first = [&](f32x16 &x, f32x16 &g) {
+    auto first = [&](f32x16 &x, f32x16 &g, uint32_t (&wd)[4]) {
+#pragma unroll
+      for (int i = 0; i < 4 && DROP == 1; ++i) wd[i] = wd0[i];
       const v8 xa = xa_of(hl_of(0));
       f32x16 z;
 #pragma unroll
       for (int r = 0; r < 16; ++r) z[r] = 0.f;
+      constexpr int AHEAD = 2; // (operand pairs asked for ahead of their products)
+      v8 ox[KS], og[KS];
+      auto fetch = [&](int ks) {
+        ox[ks] = panel_read_rows<T, BT>(lds, pl, 0, ks);
+        og[ks] = panel_read_rows<T, BT>(lds + TILEB, pl, 0, ks);
+      };
+#pragma unroll
+      for (int ks = 0; ks < AHEAD && ks < KS; ++ks) fetch(ks);
       x = XS ? E::mfma(xa, bxs, z) : z;
       g = GS ? E::mfma(xa, bxd, z) : z;
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
-        x = E::mfma(panel_read_rows<T, BT>(lds, pl, 0, ks), qreg[ks], x);
-        g = E::mfma(panel_read_rows<T, BT>(lds + TILEB, pl, 0, ks), doreg[ks], g);
+        if (ks + AHEAD < KS) fetch(ks + AHEAD);
+        x = E::mfma(ox[ks], qreg[ks], x);
+        g = E::mfma(og[ks], doreg[ks], g);
         __builtin_amdgcn_sched_barrier(0);
       }
     };
@@ -433,13 +494,11 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(bwd_dq_
     int kt = 0;
     const int nmid = nktw - 1;
     if (nmid & 1) {
-      if (DROP == 1) drop_words_q(a.drop, (uint32_t)bh, (uint32_t)q, 0u, h, l, wdB);
-      first(xB, gB);
+      first(xB, gB, wdB);
       mid(0, xB, gB, wdB, xA, gA, wdA);
       kt = 1;
     } else {
-      if (DROP == 1) drop_words_q(a.drop, (uint32_t)bh, (uint32_t)q, 0u, h, l, wdA);
-      first(xA, gA);
+      first(xA, gA, wdA);
     }
     for (; kt < nmid; kt += 2) {
       mid(kt, xA, gA, wdA, xB, gB, wdB);
@@ -561,20 +620,33 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(bwd_dkd
 #pragma unroll
     for (int t = 0; t < NST - 1; ++t) dma_qdo(qt0 + t);
 
+    PanelLane pl;
+    pl.init(l);
     // ---- per-key operands
     v8 kreg[KS], vreg[KS], bxs, bxd;
     {
       const int kc = key < a.sk ? key : a.sk - 1;
       u32x4 tk[KS], tv[KS];
+      RowOperands<T, D> rk, rv;
+      if constexpr (C::TURNED) {
+        rk.load(Kb, RW::ss(a.mk), k0w, a.sk, RW::cols(a), l);
+        rv.load(Vb, RW::ss(a.mv), k0w, a.sk, RW::cols(a), l);
+      } else {
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        const size_t col = ks * 16 + h * 8 < RW::cols(a) ? ks * 16 + h * 8 : 0;
-        tk[ks] = *(const u32x4 *)(Kb + (size_t)kc * RW::ss(a.mk) + col);
-        tv[ks] = *(const u32x4 *)(Vb + (size_t)kc * RW::ss(a.mv) + col);
+        for (int ks = 0; ks < KS; ++ks) {
+          const size_t col = ks * 16 + h * 8 < RW::cols(a) ? ks * 16 + h * 8 : 0;
+          tk[ks] = *(const u32x4 *)(Kb + (size_t)kc * RW::ss(a.mk) + col);
+          tv[ks] = *(const u32x4 *)(Vb + (size_t)kc * RW::ss(a.mv) + col);
+        }
       }
       T mraw = (T)0.f;
       if (MASK == kMaskPerKey) mraw = ((const T *)a.mask)[(size_t)(bh / a.mask_div) * a.mask_sb + kc];
       if (pass == 0 || a.sq > C::QSEG) stage_rows(qt0 * BT / C::QSEG * C::QSEG);
+      if constexpr (C::TURNED) {
+        char *panel = lds + C::OFF_T + w * C::TURNB; // (the first tiles go to the other stages: qt0 is a multiple of four)
+        rk.turn(panel, pl, l, tk);
+        rv.turn(panel, pl, l, tv);
+      }
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
         const bool live = ks * 16 + h * 8 < RW::cols(a);
@@ -617,8 +689,6 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(bwd_dkd
         dv[db][r] = 0.f;
       }
 
-    PanelLane pl;
-    pl.init(l);
     f32x16 xA, gA, xB, gB;
     uint32_t rbA[4], rbB[4];
     PhiloxSlices ph;
@@ -730,19 +800,33 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(bwd_dkd
     using No = std::false_type;
     using Guard = std::integral_constant<bool, CAUSAL>;
 
+    // causal: query tiles ahead of the one that holds this wave's own diagonal see none of its keys
+    const int t_own = CAUSAL ? (ktile * KT + __builtin_amdgcn_readfirstlane(w) * 32) / BT : qt0;
+    uint32_t rb0[4];
+    if (DROP == 1) drop_bytes_k(a.drop, (uint32_t)bh, (uint32_t)(t_own * BT), (uint32_t)key, h, l, rb0); // (while the tiles are on their way)
     auto first = [&](int qt, f32x16 &x, f32x16 &g, uint32_t (&rb)[4]) {
       const char *t = lds + (qt & (NST - 1)) * STAGEB;
-      if (DROP == 1) drop_bytes_k(a.drop, (uint32_t)bh, (uint32_t)(qt * BT), (uint32_t)key, h, l, rb);
+#pragma unroll
+      for (int i = 0; i < 4 && DROP == 1; ++i) rb[i] = rb0[i];
       const v8 xa = xrow(qt);
       f32x16 z;
 #pragma unroll
       for (int r = 0; r < 16; ++r) z[r] = 0.f;
+      constexpr int AHEAD = 2; // (operand pairs asked for ahead of their products)
+      v8 ox[KS], og[KS];
+      auto fetch = [&](int ks) {
+        ox[ks] = panel_read_rows<T, BT>(t, pl, 0, ks);
+        og[ks] = panel_read_rows<T, BT>(t + TILEB, pl, 0, ks);
+      };
+#pragma unroll
+      for (int ks = 0; ks < AHEAD && ks < KS; ++ks) fetch(ks);
       x = E::mfma(xa, bxs, z);
       g = E::mfma(xa, bxd, z);
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
-        x = E::mfma(panel_read_rows<T, BT>(t, pl, 0, ks), kreg[ks], x);
-        g = E::mfma(panel_read_rows<T, BT>(t + TILEB, pl, 0, ks), vreg[ks], g);
+        if (ks + AHEAD < KS) fetch(ks + AHEAD);
+        x = E::mfma(ox[ks], kreg[ks], x);
+        g = E::mfma(og[ks], vreg[ks], g);
         __builtin_amdgcn_sched_barrier(0);
       }
     };
@@ -758,11 +842,9 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(bwd_dkd
     bwd_vm_wait<0>();
     bwd_lds_barrier();
     if (!dead && qt0 < nqt) {
-      // causal: query tiles ahead of the one that holds this wave's own diagonal see none of its keys
       int t0 = qt0;
       if (CAUSAL) {
-        const int own = (ktile * KT + __builtin_amdgcn_readfirstlane(w) * 32) / BT;
-        const int stop = own < nqt ? own : nqt; // (no query at all may see them)
+        const int stop = t_own < nqt ? t_own : nqt; // (no query at all may see them)
         for (; t0 < stop; ++t0) {
           turn(t0);
           dma_qdo(t0 + NST - 1);
