@@ -50,6 +50,7 @@ template <typename T, int D, int NW, bool CAUSAL, int DROP, bool STRIDED>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(1, 1))) void fmha_bwd_dkdv_persist_kernel(const BwdArgs a) {
   using RW = Rows<STRIDED, D>;
   using E = Elem<T>;
+  using M = MfmaV<T>;
   using v8 = typename E::v8;
   using C = BwdPersistCfg<D>;
   constexpr int BT = C::BT, NST = C::NST, KS = C::KS, DB = C::DB, TILEB = C::TILEB, STAGEB = C::STAGEB;
@@ -390,18 +391,15 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(1, 1)))
 #pragma unroll
       for (int m = 0; m < NM; ++m) {
         if (m < NX) {
-          f32x16 z;
-#pragma unroll
-          for (int r = 0; r < 16; ++r) z[r] = 0.f;
-          if (m == 0) xn = E::mfma(xa, bxs, z);
-          else gn = E::mfma(xa, bxd, z);
+          if (m == 0) M::start(xa, bxs, xn);
+          else M::start(xa, bxd, gn);
         } else {
           const int j = m - NX;
           if (j + AHEAD < NO) opnd[j + AHEAD] = fetch(j + AHEAD);
           const int u = j ^ 1; // (the later one of a pair first: its wait covers the other)
           if (u < NA) {
-            if ((u & 1) == 0) xn = E::mfma(opnd[u], kreg[u >> 1], xn);
-            else gn = E::mfma(opnd[u], vreg[u >> 1], gn);
+            if ((u & 1) == 0) M::add(opnd[u], kreg[u >> 1], xn);
+            else M::add(opnd[u], vreg[u >> 1], gn);
           } else {
             const int i = u - NA, db = (i >> 1) % DB, c = (i >> 1) / DB;
             f32x16 &acc = (i & 1) ? dk[db] : dv[db];
@@ -427,17 +425,25 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(1, 1)))
       const char *t = stage_of(tj);
       if (DROP == 1) drop_bytes_k(a.drop, (uint32_t)bh, (uint32_t)((qt0 + tj) * BT), (uint32_t)key, h, l, rb);
       const v8 xa = xrow(tj);
-      f32x16 z;
+      constexpr int AHEAD = 2; // (operand pairs asked for ahead of their products)
+      v8 ox[KS], og[KS];
+      auto fetch = [&](int ks) {
+        ox[ks] = panel_read_rows<T, BT>(t, pl, 0, ks);
+        og[ks] = panel_read_rows<T, BT>(t + TILEB, pl, 0, ks);
+      };
 #pragma unroll
-      for (int r = 0; r < 16; ++r) z[r] = 0.f;
-      x = E::mfma(xa, bxs, z);
-      g = E::mfma(xa, bxd, z);
+      for (int ks = 0; ks < AHEAD; ++ks) fetch(ks);
+      asm volatile("s_nop 4"); // (the operands may just have been written)
+      M::start(xa, bxs, x);
+      M::start(xa, bxd, g);
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
-        x = E::mfma(panel_read_rows<T, BT>(t, pl, 0, ks), kreg[ks], x);
-        g = E::mfma(panel_read_rows<T, BT>(t + TILEB, pl, 0, ks), vreg[ks], g);
+        if (ks + AHEAD < KS) fetch(ks + AHEAD);
+        M::add(ox[ks], kreg[ks], x);
+        M::add(og[ks], vreg[ks], g);
         __builtin_amdgcn_sched_barrier(0);
       }
+      settle(x, g);
       if (CAUSAL) { // the wave's first tile is the one on its diagonal
 #pragma unroll
         for (int r = 0; r < 16; ++r) x[r] = key <= (qt0 + tj) * BT + 8 * (r / 4) + 4 * h + r % 4 ? x[r] : BIGNEG;

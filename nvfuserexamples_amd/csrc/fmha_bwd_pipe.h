@@ -110,6 +110,22 @@ template <typename T, int D> struct RowOperands {
   }
 };
 
+// Products on score / dP accumulators that stay in the first half of the register file, where the vector pipe reads them.  Left to
+// the compiler, all accumulators of a kernel that needs both halves go to the second one, and 32 moves a tile bring these back
+// (backward at head dim 128, us, so / with these: BH 512 S 1024 causal bf16 637 / 606, with dropout 769 / 722, BH 256 S 1024 482 / 469,
+// BH 32 S 4096 821 / 803, BH 512 S 512 under a padding mask with dropout 339 / 329).  The compiler does not see into them: behind
+// the last one `settle` before anything but another product reads the result.
+template <typename T> struct MfmaV;
+template <> struct MfmaV<_Float16> {
+  static FMHA_DEV void start(f16x8 a, f16x8 b, f32x16 &c) { asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, 0" : "=&v"(c) : "v"(a), "v"(b)); }
+  static FMHA_DEV void add(f16x8 a, f16x8 b, f32x16 &c) { asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b)); }
+};
+template <> struct MfmaV<__bf16> {
+  static FMHA_DEV void start(bf16x8 a, bf16x8 b, f32x16 &c) { asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(c) : "v"(a), "v"(b)); }
+  static FMHA_DEV void add(bf16x8 a, bf16x8 b, f32x16 &c) { asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b)); }
+};
+FMHA_DEV void settle(f32x16 &x, f32x16 &g) { asm volatile("s_nop 15" : "+v"(x), "+v"(g)); } // (eleven wait states are due)
+
 // One Philox4x32-10 call in slices that can be spread over an instruction stream.
 struct PhiloxSlices {
   uint32_t c[4];
@@ -694,6 +710,21 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(bwd_dkd
     PhiloxSlices ph;
     const uint32_t sel1 = (l & 1) ? 0x03070105u : 0x06020400u, sel2 = (l & 2) ? 0x03020706u : 0x05040100u; // see drop_bytes_k
 
+    constexpr bool VFORM = D > 64;
+    auto begin = [&](const v8 &p, const v8 &q, f32x16 &c) {
+      if constexpr (VFORM) {
+        MfmaV<T>::start(p, q, c);
+      } else {
+        f32x16 z;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) z[r] = 0.f;
+        c = E::mfma(p, q, z);
+      }
+    };
+    auto add = [&](const v8 &p, const v8 &q, f32x16 &c) {
+      if constexpr (VFORM) MfmaV<T>::add(p, q, c);
+      else c = E::mfma(p, q, c);
+    };
     auto xrow = [&](int qt) -> v8 { return as_v8<T>(ldsX[(qt * BT + kl) & (C::QSEG - 1)]); };
     auto step = [&](auto next_tag, auto guard_tag, int qt, const f32x16 &xc, const f32x16 &gc, const uint32_t (&rc)[4],
                     f32x16 &xn, f32x16 &gn, uint32_t (&rn)[4]) {
@@ -767,18 +798,15 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(bwd_dkd
 #pragma unroll
       for (int m = 0; m < NM; ++m) {
         if (m < NX) {
-          f32x16 z;
-#pragma unroll
-          for (int r = 0; r < 16; ++r) z[r] = 0.f;
-          if (m == 0) xn = E::mfma(xa, bxs, z);
-          else gn = E::mfma(xa, bxd, z);
+          if (m == 0) begin(xa, bxs, xn);
+          else begin(xa, bxd, gn);
         } else {
           const int j = m - NX;
           if (j + AHEAD < NO) opnd[j + AHEAD] = fetch(j + AHEAD);
           const int u = SWAP ? j ^ 1 : j; // (the later one of a pair first: its wait covers the other)
           if (u < NA) {
-            if ((u & 1) == 0) xn = E::mfma(opnd[u], kreg[u >> 1], xn);
-            else gn = E::mfma(opnd[u], vreg[u >> 1], gn);
+            if ((u & 1) == 0) add(opnd[u], kreg[u >> 1], xn);
+            else add(opnd[u], vreg[u >> 1], gn);
           } else {
             const int i = u - NA, db = (i >> 1) % DB, c = (i >> 1) / DB;
             f32x16 &acc = (i & 1) ? dk[db] : dv[db];
@@ -809,9 +837,6 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(bwd_dkd
 #pragma unroll
       for (int i = 0; i < 4 && DROP == 1; ++i) rb[i] = rb0[i];
       const v8 xa = xrow(qt);
-      f32x16 z;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) z[r] = 0.f;
       constexpr int AHEAD = 2; // (operand pairs asked for ahead of their products)
       v8 ox[KS], og[KS];
       auto fetch = [&](int ks) {
@@ -820,15 +845,17 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(bwd_dkd
       };
 #pragma unroll
       for (int ks = 0; ks < AHEAD && ks < KS; ++ks) fetch(ks);
-      x = E::mfma(xa, bxs, z);
-      g = E::mfma(xa, bxd, z);
+      if (VFORM) asm volatile("s_nop 4"); // (the operands may just have been written)
+      begin(xa, bxs, x);
+      begin(xa, bxd, g);
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
         if (ks + AHEAD < KS) fetch(ks + AHEAD);
-        x = E::mfma(ox[ks], kreg[ks], x);
-        g = E::mfma(og[ks], vreg[ks], g);
+        add(ox[ks], kreg[ks], x);
+        add(og[ks], vreg[ks], g);
         __builtin_amdgcn_sched_barrier(0);
       }
+      if (VFORM) settle(x, g);
     };
     // top of the iteration of tile qt: tile qt + 1 has landed, tile qt - 1 is no longer read
     auto turn = [&](int qt) {
