@@ -129,6 +129,13 @@ FMHA_DEV void settle(f32x16 &x, f32x16 &g) { asm volatile("s_nop 15" : "+v"(x), 
 // One Philox4x32-10 call in slices that can be spread over an instruction stream.
 struct PhiloxSlices {
   uint32_t c[4];
+  // Both halves of a product are wanted, one round apart: said so, it is one v_mad_u64_u32 (the compiler made v_mul_lo and v_mul_hi,
+  // each as dear, of half of them).
+  static FMHA_DEV uint64_t product(uint32_t c, uint32_t m) {
+    uint64_t p = (uint64_t)c * m;
+    asm volatile("" ::"v"(p));
+    return p;
+  }
   FMHA_DEV void start(const DropCtx &d, uint32_t bh, uint32_t q4, uint32_t k4) {
     const uint64_t blk = ((uint64_t)bh * d.qb4 + q4) * d.kb4 + k4;
     c[0] = d.off_lo;
@@ -138,7 +145,7 @@ struct PhiloxSlices {
   }
   FMHA_DEV void round(const DropCtx &d, int r) {
     const uint32_t k0 = d.seed_lo + (uint32_t)r * Philox::W0, k1 = d.seed_hi + (uint32_t)r * Philox::W1;
-    const uint64_t p0 = (uint64_t)Philox::M0 * c[0], p1 = (uint64_t)Philox::M1 * c[2];
+    const uint64_t p0 = product(c[0], Philox::M0), p1 = product(c[2], Philox::M1);
     const uint32_t n0 = __builtin_amdgcn_bitop3_b32((uint32_t)(p1 >> 32), c[1], k0, 0x96);
     const uint32_t n2 = __builtin_amdgcn_bitop3_b32((uint32_t)(p0 >> 32), c[3], k1, 0x96);
     c[0] = n0;
