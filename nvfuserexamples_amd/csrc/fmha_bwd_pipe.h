@@ -136,15 +136,22 @@ struct PhiloxSlices {
     asm volatile("" ::"v"(p));
     return p;
   }
+  // With round 0: its offset is the same for all lanes like the key, and so is what round 1 adds to c[3].  These scalars meet here: the
+  // instruction of `round` reads one scalar at most, and copies of the others in vector registers, kept across the loop around it, made
+  // dQ at head dim 128 reload five spilled registers a turn, each behind all copies in flight (backward with dropout, us, as copies / so:
+  // D 128 BH 96 S 700 causal packed under a padding mask 97.9 / 95.0, BH 64 S 2048 causal 314 / 309, BH 256 S 1024 556 / 550; D 64 BH 512
+  // S 512 under a padding mask 184.6 / 180.1; D 32 BH 512 S 512 135 / 132).
   FMHA_DEV void start(const DropCtx &d, uint32_t bh, uint32_t q4, uint32_t k4) {
     const uint64_t blk = ((uint64_t)bh * d.qb4 + q4) * d.kb4 + k4;
-    c[0] = d.off_lo;
-    c[1] = d.off_hi;
-    c[2] = (uint32_t)blk;
-    c[3] = (uint32_t)(blk >> 32);
+    const uint64_t p0 = (uint64_t)Philox::M0 * d.off_lo, p1 = product((uint32_t)blk, Philox::M1);
+    c[0] = (uint32_t)(p1 >> 32) ^ (d.off_hi ^ d.seed_lo);
+    c[1] = (uint32_t)p1;
+    c[2] = (uint32_t)(blk >> 32) ^ ((uint32_t)(p0 >> 32) ^ d.seed_hi);
+    c[3] = (uint32_t)p0 ^ (d.seed_hi + Philox::W1);
   }
   FMHA_DEV void round(const DropCtx &d, int r) {
-    const uint32_t k0 = d.seed_lo + (uint32_t)r * Philox::W0, k1 = d.seed_hi + (uint32_t)r * Philox::W1;
+    if (r == 0) return;
+    const uint32_t k0 = d.seed_lo + (uint32_t)r * Philox::W0, k1 = r == 1 ? 0u : d.seed_hi + (uint32_t)r * Philox::W1;
     const uint64_t p0 = product(c[0], Philox::M0), p1 = product(c[2], Philox::M1);
     const uint32_t n0 = __builtin_amdgcn_bitop3_b32((uint32_t)(p1 >> 32), c[1], k0, 0x96);
     const uint32_t n2 = __builtin_amdgcn_bitop3_b32((uint32_t)(p0 >> 32), c[3], k1, 0x96);
@@ -615,9 +622,10 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(bwd_dkd
   };
 
   for (int pass = 0; pass < npass; ++pass) {
-    // (where registers spilled set up for each pass, see dQ: BH 600 S 380 D 64 packed with dropout, backward 134.6 -> 131.8 us)
+    // (where registers spilled set up for each pass, see dQ: backward, us, BH 600 S 380 D 64 packed with dropout 134.6 -> 131.8; BH 512 S 512
+    // with dropout 146 -> 142, S 1024 bf16 405 -> 398; on whole rows without dropout, where nothing spills, 1 to 2 % behind)
     int tid = threadIdx.x;
-    if (CAUSAL && (D > 64 || STRIDED)) asm volatile("" : "+v"(tid));
+    if (CAUSAL && (D > 64 || STRIDED || DROP == 1)) asm volatile("" : "+v"(tid));
     const int w = tid >> 6, l = tid & 63, kl = l & 31, h = l >> 5;
     const int ktile = pass == 0 ? pi : a.ntile - 1 - pi;
     const int k0w = ktile * KT + w * 32;
