@@ -99,12 +99,17 @@ template <int MASK, bool CAUSAL, int DROP> int launch_dkdv(BwdArgs &a, const Bwd
   return attr ? 2 : launch_one(kern, a, nblk, Cfg::NW * 64, Cfg::LDS_BYTES, s);
 #else
   constexpr bool kPipe = pipe_built<MASK, CAUSAL, DROP>();
-  // One exception: under a mask or key counts, without causal mask and dropout, dK / dV at head dim 128 stays on 32-row tiles at
-  // two waves per SIMD, which overlap one workgroup's start and stores with another's arithmetic as the persistent kernel
-  // does where there is neither (plain pipelined kernel / this: BH 256 S 1024 343 / 335 us on one card, 347 / 359-369 on another).
+  // One exception: under a mask or key counts, without causal mask and dropout, short heads' dK / dV at head dim 128 stays on 32-row
+  // tiles at two waves per SIMD, which overlap one workgroup's start and stores with another's arithmetic as the persistent
+  // kernel does where there is neither: below 192 queries, and up to 384 of rows shorter than the kernel's.  Backward under padding
+  // masks / key counts, us, so / pipelined: BH 512 S 128 48.3 / 51.0, 45.6 / 50.8, S 160 level; S 197 110.9 / 100.3, S 258 156 / 133, 135
+  // / 129, S 512 417 / 329, 316 / 307, packed 464 / 342, 460 / 325; BH 256 S 1024 702 / 524, 503 / 491, packed 796 / 527, 785 / 503; 112
+  // to 120 columns BH 192 S 320 65.3 / 66.6, 65.9 / 64.4, S 384 87.7 / 92.2, 84.5 / 87.5, BH 512 S 416 270 / 251, 278 / 245, BH 64 S 2048
+  // 502 / 430, 476 / 377.
   constexpr bool kTwoWaves = bwd_dkdv_small_tiles<FMHA_TU_D, CAUSAL, DROP>();
   if constexpr (kPipe && FMHA_TU_D != 96) { // (see pipe_wanted)
-    if (pipe_wanted(a) && !(kTwoWaves && (MASK != kMaskNone || a.kv_len))) {
+    const bool two_waves = kTwoWaves && (MASK != kMaskNone || a.kv_len) && (a.dcols < FMHA_TU_D ? a.sq <= 384 : a.sq < 192);
+    if (pipe_wanted(a) && !two_waves) {
       const int rc = FMHA_PIPE_NAME(FMHA_TU_TNAME, FMHA_TU_D)(a, v, true, nblk, s);
       if (FMHA_TU_D <= 64 || rc != kBwdNotHere) return rc;
     }

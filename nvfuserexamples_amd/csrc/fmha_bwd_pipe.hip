@@ -75,14 +75,11 @@ template <int MASK, bool CAUSAL, int DROP> int launch(const BwdArgs &a, bool dkd
     // BH 350 43.4 / 40.6; under a padding mask BH 512 S 128 54.2 / 51.2, S 176 95.1 / 91.3, S 160 level; S 200 103.4 / 105.5).
     if (CAUSAL && a.sq < 192) return kBwdNotHere;
 #endif
-    if constexpr (bwd_dkdv_small_tiles<FMHA_TU_D, CAUSAL, DROP>() && MASK != kMaskNone) return kBwdNotHere; // (see fmha_bwd.hip)
-    else {
-      auto kern = fmha_bwd_dkdv_pipe_kernel<FMHA_TU_T, FMHA_TU_D, kNW, MASK, CAUSAL, DROP, kStrided>;
-      static const bool ready = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                    Cfg::dkdv_lds_bytes(DROP, Cfg::QSEG)) == hipSuccess;
-      if (!ready) return 2;
-      hipLaunchKernelGGL(kern, dim3((unsigned)nblk), dim3(kNW * 64), Cfg::dkdv_lds_bytes(DROP, a.sq), s, a);
-    }
+    auto kern = fmha_bwd_dkdv_pipe_kernel<FMHA_TU_T, FMHA_TU_D, kNW, MASK, CAUSAL, DROP, kStrided>;
+    static const bool ready = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                  Cfg::dkdv_lds_bytes(DROP, Cfg::QSEG)) == hipSuccess;
+    if (!ready) return 2;
+    hipLaunchKernelGGL(kern, dim3((unsigned)nblk), dim3(kNW * 64), Cfg::dkdv_lds_bytes(DROP, a.sq), s, a);
   } else
 #endif
   {
