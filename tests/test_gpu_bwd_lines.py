@@ -1,0 +1,55 @@
+"""The backward on both sides of the lines where its kernels change, with ragged last tiles and numbers of heads that do not divide
+over the compute dies: causal dQ at head dim 128 (pipelined from 128 queries on), dK / dV at head dim 128 under masks and key counts
+without dropout (from 192, of shorter rows from 385), heads left over behind groups of eight, against the oracle."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from conftest import f32, make_qkv, pad_mask
+from nvfuserexamples_amd import capi
+
+pytestmark = pytest.mark.gpu
+
+TDT = {"fp16": torch.float16, "bf16": torch.bfloat16}
+UNIT = {"fp16": 2.0 ** -11, "bf16": 2.0 ** -8}  # one rounding of a value to the element type
+
+CASES = [
+    # bh, sq, sk, d, dtype, mask, causal, p
+    (3, 127, 127, 128, "fp16", None, True, 0.0),
+    (9, 128, 128, 128, "bf16", None, True, 0.1),
+    (3, 129, 161, 128, "fp16", "pad", True, 0.1),
+    (2, 225, 97, 112, "bf16", "len", True, 0.0),
+    (2, 415, 415, 128, "fp16", None, True, 0.1),
+    (3, 191, 65, 128, "bf16", "pad", False, 0.0),
+    (9, 192, 193, 128, "fp16", "len", False, 0.0),
+    (11, 193, 31, 128, "bf16", "pad", False, 0.0),
+    (3, 384, 129, 104, "fp16", "pad", False, 0.0),
+    (3, 385, 129, 104, "fp16", "len", False, 0.0),
+    (13, 70, 333, 64, "fp16", "pad", False, 0.1),  # five heads left over behind the eight of a group
+]
+
+
+@pytest.mark.parametrize("bh,sq,sk,d,dtype,mask,causal,p", CASES)
+def test_backward_on_both_sides_of_its_lines(bh, sq, sk, d, dtype, mask, causal, p):
+    q, k, v, do = make_qkv(bh, sq, sk, d, seed=sq + sk + d, std=0.7, dtype=dtype, with_dout=True)
+    kw, okw, m, om = dict(causal=causal), dict(causal=causal), None, None
+    if mask == "pad":
+        m = pad_mask(1, sk, max(1, sk // 2), sk, seed=5).to(TDT[dtype])
+        om = f32(m)
+    elif mask == "len":
+        n = sk - sk // 3
+        kw["kv_len"] = torch.tensor([n], dtype=torch.int32, device="cuda")
+        om = f32(torch.where(torch.arange(sk) < n, 0.0, float("-inf")).view(1, 1, sk))
+    if p > 0:
+        kw.update(drop_kind=capi.DROP_PHILOX, p_drop=p, seed=99, offset=12)
+        okw.update(philox=True, p_drop=p, seed=99, offset=12)
+    qc, kc, vc, mc = q.cuda(), k.cuda(), v.cuda(), (None if m is None else m.cuda())
+    o, lse, _, _ = capi.fwd(qc, kc, vc, mask=mc, want_lse=True, **kw)
+    got = capi.bwd(do.cuda(), qc, kc, vc, o, lse, mask=mc, **kw)
+    torch.cuda.synchronize()
+    ref = oracle.attention(f32(q), f32(k), f32(v), mask=om, dout=f32(do), want=("dq", "dk", "dv"), **okw)
+    # P, dS, O (in delta) and the result are rounded once each, by one unit of their size at most, and dP - delta may lose part of its
+    # size to the subtraction: twice the four units bound the norm of the error.
+    for name, t in zip(("dq", "dk", "dv"), got):
+        assert np.linalg.norm(f32(t.cpu()) - ref[name]) <= 8 * UNIT[dtype] * np.linalg.norm(ref[name]), name
