@@ -166,6 +166,13 @@ struct PhiloxSlices {
 // (waves per SIMD: at head dim 256 a wave needs about 400 registers, and the tiles leave room for one workgroup; at 32 without a
 // causal mask three waves have the 150 it needs: with dK / dV at three as well BH 512 S 512 backward 96 -> 89 us, BH 1760 S 64 under a padding mask 35 -> 29)
 template <int D, bool CAUSAL> constexpr int bwd_dq_pipe_occ() { return D == 256 ? 1 : D == 32 && !CAUSAL ? 3 : 2; }
+// A query's LSE and delta are constants of its lane: where registers have room for 32 copies, the products of x and g start from them,
+// and neither an extra contraction step (two of a tile's 14 matrix instructions at head dim 64, and the only one left is a mask's) nor
+// a subtraction per element brings them in.  Backward, us, before / so: D 64 BH 64 S 2048 239.6 / 234.4, with dropout 295.7 / 290.7, key
+// counts 201.3 / 196.4, BH 512 S 512 packed with dropout 184.9 / 182.2, BH 192 S 1024 bf16 causal 120.4 / 118.0; D 96 BH 64 S 2048 363.7 /
+// 353.2, BH 512 S 512 under a padding mask 220.3 / 213.3; D 32 BH 512 S 512 causal 77.7 / 75.8; up to 700 queries of 24 heads level.
+// No room: D 32 at three waves and D 96, each with dropout (16 to 20 registers spill), and D 128.
+template <int D, bool CAUSAL, int DROP> constexpr bool bwd_dq_pipe_constants() { return D == 64 || (D == 96 && DROP == 0) || (D == 32 && (CAUSAL || DROP == 0)); }
 template <typename T, int D, int NW, int MASK, bool CAUSAL, int DROP, bool STRIDED>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(bwd_dq_pipe_occ<D, CAUSAL>(), bwd_dq_pipe_occ<D, CAUSAL>()))) void fmha_bwd_dq_pipe_kernel(const BwdArgs a) {
   using RW = Rows<STRIDED, D>;
@@ -177,9 +184,12 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(bwd_dq_
   constexpr float NEG_INF = -__builtin_inff();
   constexpr float BIGNEG = -60000.f;
   static_assert(MASK != kMaskFull, "full mask tensors: fmha_bwd_dq_kernel");
-  // Rank-one terms: at head dim 64 the vector pipe is the busier one and they ride in an extra contraction step (XS, GS);
-  // at head dim 128 it is the matrix pipe, and a subtraction per element costs less: there only a per-key mask does.
-  constexpr bool XS = D <= 64 || MASK == kMaskPerKey, GS = D <= 64, LS = D <= 64; // (LS: the LSE rides in the extra step)
+  // Rank-one terms that the products do not start from (CI): at head dims up to 64 the vector pipe is the busier one and they ride in
+  // an extra contraction step (XS, GX); above it is the matrix pipe, and a subtraction per element costs less.  A per-key mask always
+  // rides in one.
+  constexpr bool CI = bwd_dq_pipe_constants<D, CAUSAL, DROP>();
+  constexpr bool XS = (D <= 64 && !CI) || MASK == kMaskPerKey, GX = D <= 64 && !CI; // x, g have an extra step
+  constexpr bool GS = D <= 64 || CI, LS = GS;                                       // they come with delta, with the LSE
 
   extern __shared__ __attribute__((aligned(16))) char lds[];
   uint32_t *ldsM = (uint32_t *)(lds + C::OFF_X + 64); // (mask_hi, mask_lo) per key of the current segment
@@ -235,11 +245,11 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(bwd_dq_
   };
 
   for (int pass = 0; pass < npass; ++pass) {
-    // (At head dim 128 set up for each pass, from an index that the compiler cannot trace: kept from one pass to the next, what a lane
-    // addresses had 33 to 59 registers spilled into the stream.  Backward, us: BH 512 S 1024 bf16 698 -> 649, with dropout 836 -> 776,
+    // (From head dim 64 on set up for each pass, from an index that the compiler cannot trace: kept from one pass to the next, what a lane
+    // addresses had 33 to 59 registers spilled into the stream at 128, and would have up to 9 at 64.  Backward, us: BH 512 S 1024 bf16 698 -> 649, with dropout 836 -> 776,
     // BH 128 S 900 167 -> 154, BH 32 S 4096 497 -> 485.  Where nothing spills it costs the second pass 1 to 2 %.)
     int tid = threadIdx.x;
-    if (CAUSAL && D > 64) asm volatile("" : "+v"(tid));
+    if (CAUSAL && D >= 64) asm volatile("" : "+v"(tid));
     const int w = tid >> 6, l = tid & 63, ql = l & 31, h = l >> 5;
     const int qt = CAUSAL ? (pass == 0 ? a.ntile - 1 - pi : pi) : pi;
     const int q0w = qt * QT + w * 32;
@@ -325,7 +335,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(bwd_dq_
       }
       if (h == 0) {
         T hi, lo;
-        split_hi_lo<T>(LS ? nl : 0.f, hi, lo);
+        split_hi_lo<T>(LS && !CI ? nl : 0.f, hi, lo);
         bxs[0] = hi;
         bxs[1] = lo;
         bxs[2] = (T)1.f;
@@ -366,6 +376,14 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(bwd_dq_
     };
     auto xa_of = [&](uint32_t hl) -> v8 { return as_v8<T>(u32x4{ONES, hl, 0u, 0u}); };
 
+    f32x16 cx, cg; // what the products of x and g start from
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      cx[r] = CI ? nlse : 0.f;
+      cg[r] = CI ? -delta : 0.f;
+    }
+    if (CI) asm volatile("" : "+v"(cx), "+v"(cg)); // (left alone the compiler forms them anew for each tile)
+
     f32x16 dq[DB];
 #pragma unroll
     for (int db = 0; db < DB; ++db)
@@ -381,7 +399,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(bwd_dq_
     auto step = [&](auto next_tag, auto guard_tag, int kt, uint32_t hl, const f32x16 &xc, const f32x16 &gc,
                     const uint32_t (&wc)[4], f32x16 &xn, f32x16 &gn, uint32_t (&wn)[4]) {
       constexpr bool NEXT = decltype(next_tag)::value, GUARD = decltype(guard_tag)::value;
-      constexpr int NX = NEXT ? (XS ? 1 : 0) + (GS ? 1 : 0) : 0, NA = NEXT ? 2 * KS : 0, NC = 2 * DB, NO = NA + NC, NM = NX + NO;
+      constexpr int NX = NEXT ? (XS ? 1 : 0) + (GX ? 1 : 0) : 0, NA = NEXT ? 2 * KS : 0, NC = 2 * DB, NO = NA + NC, NM = NX + NO;
       constexpr int AHEAD = 3;
       constexpr int NS = 10;                                  // softmax slots: 8 pairs, two to drain
       constexpr int NP = DROP == 1 && NEXT ? 14 : 0;          // Philox slots
@@ -445,20 +463,14 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(bwd_dq_
       for (int m = 0; m < NM; ++m) {
         if (m < NX) {
           const v8 xa = xa_of(hl);
-          f32x16 z;
-#pragma unroll
-          for (int r = 0; r < 16; ++r) z[r] = 0.f;
-          if (XS && m == 0) xn = E::mfma(xa, bxs, z);
-          else gn = E::mfma(xa, bxd, z);
+          if (XS && m == 0) xn = E::mfma(xa, bxs, cx);
+          else gn = E::mfma(xa, bxd, cg);
         } else {
           const int j = m - NX;
           if (j + AHEAD < NO) opnd[j + AHEAD] = fetch(j + AHEAD);
           if (j < NA) {
-            f32x16 z;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) z[r] = 0.f;
-            if ((j & 1) == 0) xn = E::mfma(opnd[j], qreg[j >> 1], !XS && j == 0 ? z : xn);
-            else gn = E::mfma(opnd[j], doreg[j >> 1], !GS && j == 1 ? z : gn);
+            if ((j & 1) == 0) xn = E::mfma(opnd[j], qreg[j >> 1], !XS && j == 0 ? cx : xn);
+            else gn = E::mfma(opnd[j], doreg[j >> 1], !GX && j == 1 ? cg : gn);
           } else {
             const int i = j - NA;
             dq[i % DB] = E::mfma(opnd[j], frag[i / DB], dq[i % DB]);
@@ -486,9 +498,6 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(bwd_dq_
 #pragma unroll
       for (int i = 0; i < 4 && DROP == 1; ++i) wd[i] = wd0[i];
       const v8 xa = xa_of(hl_of(0));
-      f32x16 z;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) z[r] = 0.f;
       constexpr int AHEAD = 2; // (operand pairs asked for ahead of their products)
       v8 ox[KS], og[KS];
       auto fetch = [&](int ks) {
@@ -497,8 +506,8 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(bwd_dq_
       };
 #pragma unroll
       for (int ks = 0; ks < AHEAD && ks < KS; ++ks) fetch(ks);
-      x = XS ? E::mfma(xa, bxs, z) : z;
-      g = GS ? E::mfma(xa, bxd, z) : z;
+      x = XS ? E::mfma(xa, bxs, cx) : cx;
+      g = GX ? E::mfma(xa, bxd, cg) : cg;
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
         if (ks + AHEAD < KS) fetch(ks + AHEAD);

@@ -1,6 +1,7 @@
 """The backward on both sides of the lines where its kernels change, with ragged last tiles and numbers of heads that do not divide
 over the compute dies: causal dQ at head dim 128 (pipelined from 128 queries on), dK / dV at head dim 128 under masks and key counts
-without dropout (from 192, of shorter rows from 385), heads left over behind groups of eight, against the oracle."""
+without dropout (from 192, of shorter rows from 385), heads left over behind groups of eight, dQ at head dims up to 96 whose products
+start from LSE and delta (only a mask has an extra step: the last tile's missing keys are a test per score), against the oracle."""
 import numpy as np
 import pytest
 import torch
@@ -27,6 +28,13 @@ CASES = [
     (3, 384, 129, 104, "fp16", "pad", False, 0.0),
     (3, 385, 129, 104, "fp16", "len", False, 0.0),
     (13, 70, 333, 64, "fp16", "pad", False, 0.1),  # five heads left over behind the eight of a group
+    (3, 257, 289, 64, "fp16", None, False, 0.0),
+    (9, 257, 290, 64, "bf16", "len", False, 0.1),
+    (3, 300, 287, 64, "bf16", None, True, 0.1),
+    (2, 290, 321, 96, "fp16", None, False, 0.0),
+    (3, 257, 299, 80, "bf16", "len", True, 0.0),
+    (5, 300, 299, 32, "fp16", "len", True, 0.1),
+    (3, 129, 161, 32, "bf16", None, False, 0.0),
 ]
 
 
