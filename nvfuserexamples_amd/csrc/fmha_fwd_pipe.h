@@ -372,6 +372,11 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu((QB == 
     st.mraw = (T)0.f;
     if (MASK == kMaskPerKey) st.mraw = mk[st.mvalid ? kr : (kend > 0 ? kend - 1 : 0)];
   };
+  // Whether the second half of a row, all zeros, is written in the prologue only.  Where two waves per SIMD fill the registers, its four
+  // zeros were reloaded from scratch at the top of every causal iteration, ahead of the copies (us, written with each tile / once: head
+  // dim 128 causal BH 512 S 1024 bf16 206.2 / 200.5, fp16 217.3 / 212.0, packed 228.8 / 225.1, BH 32 S 4001 151.3 / 149.7, with dropout
+  // BH 512 S 512 111.0 / 107.9; head dim 96 causal BH 60 S 1000 28.3 / 27.5).  At head dim 64 nothing spills: level.
+  constexpr bool ZONCE = D == 96 || D == 128;
   auto lstoreX = [&](int tile, const XStage &st) {
     if (tid < BK) {
       float mk = 0.f;
@@ -380,19 +385,16 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu((QB == 
       const T hi = (T)mk;
       const bool fin = (float)hi != NEG_INF;
       const T lo = fin ? (T)(mk - (float)hi) : (T)0.f;
-      v8 x0, x1;
+      v8 x0;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        x0[j] = (T)0.f;
-        x1[j] = (T)0.f;
-      }
+      for (int j = 0; j < 8; ++j) x0[j] = (T)0.f;
       x0[0] = (T)1.f;
       x0[1] = hi;
       x0[2] = lo;
       x0[3] = (T)1.f;
       v8 *dst = (v8 *)(ldsXb + (tile & 1) * BK * XROWB + tid * XROWB);
       dst[0] = x0;
-      dst[1] = x1;
+      if (!ZONCE) dst[1] = as_v8<T>(u32x4{0u, 0u, 0u, 0u});
     }
   };
 
@@ -916,6 +918,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu((QB == 
     }
     lstoreX(0, x0);
     lstoreX(1, x1);
+    if (ZONCE && tid < 2 * BK) *(u32x4 *)(ldsXb + tid * XROWB + 16) = u32x4{0u, 0u, 0u, 0u}; // (see lstoreX)
   }
 
   for (int idx = lb, ord = 0;;) {
