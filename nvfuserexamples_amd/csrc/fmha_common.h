@@ -211,11 +211,14 @@ template <bool STRIDED, int D> struct Rows {
   }
 };
 
-template <typename T, int D, int BT, int NT> struct TileCopy {
+// APART: a lane keeps the offset of its first chunk only; the others are a uniform distance away, which the scalar unit adds to the base.
+template <typename T, int D, int BT, int NT, bool APART = false> struct TileCopy {
   static constexpr int CHUNKS = BT * tile_cols(D) / 8;
   static constexpr int CPT = CHUNKS / NT;
   static_assert(D % 32 == 0 && CHUNKS % NT == 0, "tile must divide evenly over the workgroup");
-  uint32_t voff[CPT];
+  static constexpr int ROWS = NT / 8; // rows of a panel that the workgroup copies at once
+  static_assert(!APART || (D % 64 == 0 && ROWS % 16 == 0 && BT % ROWS == 0), "no uniform distance");
+  uint32_t voff[APART ? 1 : CPT];
   uint32_t ss; // elements between rows of the source tensor
 
   // chunk slot c of a tile: panel c / (8*BT), row (c / 8) % BT, position c % 8, which holds the
@@ -229,7 +232,7 @@ template <typename T, int D, int BT, int NT> struct TileCopy {
   FMHA_DEV void init(int tid, int64_t row_stride, int dv = D) {
     ss = (uint32_t)row_stride;
 #pragma unroll
-    for (int i = 0; i < CPT; ++i) {
+    for (int i = 0; i < (APART ? 1 : CPT); ++i) {
       int row, col;
       slot(tid + i * NT, row, col);
       voff[i] = (uint32_t)row * ss * 2u + (D % 64 == 0 || col * 8 < dv ? (uint32_t)(col * 16) : 0u);
@@ -287,7 +290,12 @@ template <typename T, int D, int BT, int NT> struct TileCopy {
     if (row0 + BT <= rend) { // wave-uniform: a full tile needs no per-lane address arithmetic
       const T *tb = base + (uint32_t)row0 * ss;
 #pragma unroll
-      for (int i = 0; i < CPT; ++i) dma_global_to_lds_b128(tb, voff[i], wave_dst + (uint32_t)(i * NT * 16));
+      for (int i = 0; i < CPT; ++i) {
+        if constexpr (APART) // (i * ROWS rows on, counted panel by panel)
+          dma_global_to_lds_b128(tb + ((uint32_t)(i * ROWS % BT) * ss + (uint32_t)(i * ROWS / BT * 64)), voff[0], wave_dst + (uint32_t)(i * NT * 16));
+        else
+          dma_global_to_lds_b128(tb, voff[i], wave_dst + (uint32_t)(i * NT * 16));
+      }
     } else {
 #pragma unroll
       for (int i = 0; i < CPT; ++i) {
