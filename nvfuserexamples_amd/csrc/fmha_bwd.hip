@@ -157,6 +157,10 @@ template <int MASK, bool CAUSAL, int DROP> int launch(BwdArgs &a, const BwdVaria
     else if (CAUSAL && by_head) a.pair = kTilesByHead;
     a.lg = head_groups_log2(a.bh);
     a.units = !CAUSAL || a.pair == kTilesByHead ? ntile : a.pair == kTilesPaired ? (ntile + 1) / 2 : a.bh >> a.lg;
+    const bool uneven = !CAUSAL && (MASK == kMaskPerKey || (MASK == kMaskNone && a.kv_len));
+    const bool share = rows_share_lines(a.mq.heads, a.mq.sh, a.mq.ss) || rows_share_lines(a.mk.heads, a.mk.sh, a.mk.ss);
+    a.dealt = uneven ? bwd_dealt_blocks(FMHA_TU_D == 256 && tiles >= 4LL * cus, share, a.bh, ntile) : 0;
+    a.range = bwd_range_blocks(a.pair == kTilesPaired ? pairs : tiles, a.dealt);
     return a.pair == kTilesPaired ? pairs : tiles;
   };
   // dQ first: it also writes delta, which the dK/dV kernel reads (same stream => ordered)

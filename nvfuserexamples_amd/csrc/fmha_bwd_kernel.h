@@ -61,7 +61,38 @@ struct BwdArgs {
   int32_t dcols; // elements per row that exist (<= the kernel's head dim; run-time layouts only)
   int32_t units; // what a block's number is divided by (bwd_item): a head's tiles or pairs of tiles; kTilesByLength: heads of a group
   int32_t lg; // head_groups_log2 of the heads
+  int32_t dealt; // blocks at the front of the launch whose heads go to the XCDs one by one (bwd_dealt_blocks)
+  int32_t range; // neighbours of an XCD among the blocks behind those (bwd_range_blocks)
 };
+
+// Workgroups go to the 8 XCDs by turns, and a head's tiles should share an XCD, whose L2 then reads the head's rows once.  Where the number
+// of workgroups divides by 8 each XCD can take a range of neighbouring heads.  Where a per-key mask or key counts may make heads differ in
+// length, of every 8 heads each XCD takes one instead (`dealt`: the first blocks of the launch, whole groups of 8 heads; those left over
+// follow as ranges).  Backward, us, ranges / dealt: padded batches of 16 heads a sequence, D 64 BH 160 S 600 68.6 / 62.2, BH 512
+// S 640 199 / 188, packed with dropout 261 / 240, BH 512 S 512 level to 1 % ahead, D 128 BH 256 S 512 139.7 / 132.3, packed with dropout
+// 176.7 / 168.6 (but BH 200 S 300 of 4 heads a sequence D 64 35.9 / 37.9, of 8 heads 0.92 of the ranges' time); without ranges to be
+// had, a head's tiles on all XCDs / dealt, BH 300 S 300 D 64 52.3 / 46.8, D 128 97.0 / 86.9.
+// Up to two tiles a head stay ranges where they can: there is little to even out, and dealt D 32 BH 512 S 40 is 2 % behind, S 200 and D 128 level.
+// Interleaved rows of neighbouring heads that meet inside a cache line, which two XCDs then read and write, stay ranges up to seven
+// tiles: packed D 32 BH 512 S 128 21.2 / 26.0, S 200 42.1 / 47.9, S 512 129.7 / 133.8, D 80 BH 256 S 512 136 / 141, S 640 198 / 207,
+// S 1024 443 / 439.  Full mask tensors are not dealt, their heads are equally long: D 128 BH 256 S 512 245 / 254, D 64 BH 512 S 512 210 / 217.
+FMHA_HOST_DEV bool rows_share_lines(int32_t heads, int64_t sh, int64_t ss) { return heads > 1 && sh < ss && (sh == 0 || sh % 64 != 0); }
+// Heads of one tile (`one`) at head dim 256 are dealt from four rounds of workgroups on (S 128 BH 512 1.5 % behind, BH 1024 3 to 6 % ahead,
+// BH 2240 S 56 1.5 to 4 % ahead, S 24 1 % behind; two tiles, BH 768 S 250, 1 to 4 % behind).
+FMHA_HOST_DEV int bwd_dealt_blocks(bool one, bool share_lines, int bh, int units) {
+  const int64_t nb = (int64_t)bh * units;
+  const bool deal = units >= (nb % 8 != 0 ? 2 : share_lines ? 8 : 3) || (one && !share_lines && units == 1);
+  return deal ? (int)((int64_t)(bh & ~7) * units) : 0;
+}
+FMHA_HOST_DEV int bwd_range_blocks(int64_t nb, int dealt) { return (nb - dealt) % 8 == 0 ? (int)((nb - dealt) / 8) : 0; } // (0: as they come)
+FMHA_HOST_DEV void bwd_head_and_unit(int bid, int dealt, int range, int units, int &bh, int &pi) {
+  const int r = bid - dealt, behind = range ? (r & 7) * range + (r >> 3) : r;
+  const bool deal = r < 0;
+  const uint32_t n = deal ? bid >> 3 : dealt + behind;
+  const uint32_t head = n / (uint32_t)units;
+  pi = (int)(n - head * (uint32_t)units);
+  bh = (int)(deal ? head * 8 + (bid & 7) : head);
+}
 
 // BT: rows per LDS tile (keys in the dQ kernel, queries in the dK/dV kernel).  The dK/dV kernel
 // at head dim 128 holds 128 accumulator registers; walking the queries 32 at a time brings its
@@ -104,35 +135,18 @@ FMHA_DEV int bwd_valid_keys(const BwdArgs &a, int bh) {
 // and a compute unit's second workgroup is as short as its first is long (us, head by head / so, dQ and dK / dV: D 64 BH 88 S 1368
 // with dropout 62.0 / 53.9, 81.8 / 67.5, BH 40 S 1088 30.3 / 24.6, 38.1 / 31.7, BH 128 S 512 17.6 / 15.2, 21.0 / 17.1; D 128 BH 12
 // S 3584 101 / 83 and, persistent, 99; a single tile a compute unit, BH 16 S 2816, level).
-// TWO: two workgroups share a compute unit.
-template <bool CAUSAL, bool TWO> FMHA_DEV void bwd_item(const BwdArgs &a, int &bh, int &pi, int &npass) {
-  int bid = blockIdx.x;
-  const int nb = gridDim.x;
+// TWO: two workgroups share a compute unit.  DEALT: some heads may be (BwdArgs::dealt).
+template <bool CAUSAL, bool TWO, bool DEALT> FMHA_DEV void bwd_item(const BwdArgs &a, int &bh, int &pi, int &npass) {
+  const int bid = blockIdx.x;
   if (CAUSAL && a.pair == kTilesByLength) {
-    const int lg = a.lg, m = TWO ? by_length(bid, nb, lg) : bid >> lg;
+    const int lg = a.lg, m = TWO ? by_length(bid, gridDim.x, lg) : bid >> lg;
     pi = m / a.units;
     bh = ((m - pi * a.units) << lg) + (bid & ((1 << lg) - 1));
     npass = 1;
     return;
   }
-  // Workgroups go to the 8 XCDs by turns, and all tiles of a head to one of them: under a mask or key counts of every 8 heads one, so that
-  // heads of different lengths are spread evenly (backward, us, a range of neighbours / so: padded batches of 16 heads a sequence,
-  // D 64 BH 512 S 512 154.8 / 149.9, with dropout 184.4 / 178.1, BH 1024 S 300 149.5 / 142.3, BH 96 S 1024 with dropout 123.0 / 118.6, D 128
-  // BH 512 S 512 with dropout 355.6 / 349.0), else, and for the heads left over, a range of neighbours.
-  if (!CAUSAL && (a.mask || a.kv_len)) {
-    const int grouped = (a.bh & ~7) * a.units;
-    if (bid < grouped) {
-      const int head = (bid >> 3) / a.units;
-      bh = head * 8 + (bid & 7);
-      pi = (bid >> 3) - head * a.units;
-      npass = 1;
-      return;
-    }
-  } else if ((nb & 7) == 0) {
-    bid = (bid & 7) * (nb >> 3) + (bid >> 3);
-  }
-  bh = bid / a.units;
-  pi = bid - bh * a.units;
+  const int dealt = DEALT ? a.dealt : 0, range = a.range, units = a.units;
+  bwd_head_and_unit(bid, dealt, range, units, bh, pi);
   npass = CAUSAL && a.pair == kTilesPaired && a.ntile - 1 - pi != pi ? 2 : 1;
 }
 
@@ -219,7 +233,7 @@ __global__ __launch_bounds__(NW * 64)
   const int w = tid >> 6, l = tid & 63, ql = l & 31, h = l >> 5;
 
   int bh, pi, npass;
-  bwd_item<CAUSAL, D != 256>(a, bh, pi, npass);
+  bwd_item<CAUSAL, D != 256, !CAUSAL && MASK != kMaskFull>(a, bh, pi, npass);
   MaskTail<T, NT> tail;
   int live_keys = a.sk; // the mask's own count of keys worth visiting
   if (MASK == kMaskPerKey) tail.issue(a, (const T *)a.mask + (size_t)(bh / a.mask_div) * a.mask_sb, tid);
@@ -555,7 +569,7 @@ __global__ __launch_bounds__(NW * 64)
   stamp();
 #endif
   int bh, pi, npass;
-  bwd_item<CAUSAL, D != 256>(a, bh, pi, npass);
+  bwd_item<CAUSAL, D != 256, !CAUSAL && MASK != kMaskFull>(a, bh, pi, npass);
   MaskTail<T, NT> tail;
   int live_keys = a.sk; // the mask's own count of keys worth visiting
   if (MASK == kMaskPerKey) tail.issue(a, (const T *)a.mask + (size_t)(bh / a.mask_div) * a.mask_sb, tid);

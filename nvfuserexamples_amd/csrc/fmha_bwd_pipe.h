@@ -199,7 +199,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(bwd_dq_
   const int w = tid >> 6, l = tid & 63, ql = l & 31, h = l >> 5;
 
   int bh, pi, npass;
-  bwd_item<CAUSAL, bwd_dq_pipe_occ<D, CAUSAL>() == 2>(a, bh, pi, npass);
+  bwd_item<CAUSAL, bwd_dq_pipe_occ<D, CAUSAL>() == 2, !CAUSAL>(a, bh, pi, npass);
 
   const T *Qb = (const T *)a.q + RW::head(a.mq, bh, a.sq);
   const T *Ob = (const T *)a.o + RW::head(a.mo, bh, a.sq);
@@ -588,7 +588,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(bwd_dkd
   const int w = tid >> 6, l = tid & 63, kl = l & 31, h = l >> 5;
 
   int bh, pi, npass;
-  bwd_item<CAUSAL, bwd_dkdv_pipe_occ<D, CAUSAL, DROP>() == 2>(a, bh, pi, npass);
+  bwd_item<CAUSAL, bwd_dkdv_pipe_occ<D, CAUSAL, DROP>() == 2, !CAUSAL>(a, bh, pi, npass);
 
   const T *Qb = (const T *)a.q + RW::head(a.mq, bh, a.sq);
   const T *dOb = (const T *)a.dout + RW::head(a.mdo, bh, a.sq);

@@ -61,7 +61,7 @@ __global__ __launch_bounds__(bwd_wide_threads<D>()) __attribute__((amdgpu_waves_
   u32x4 *exch = (u32x4 *)(lds + W::OFF_EXCH) + pairi * (NSB * 2 * 64) + l;
 
   int bh, pi, npass;
-  bwd_item<CAUSAL, false>(a, bh, pi, npass);
+  bwd_item<CAUSAL, false, !CAUSAL && MASK != kMaskFull>(a, bh, pi, npass);
   MaskTail<T, NT> tail;
   int live_keys = a.sk;
   if (MASK == kMaskPerKey) tail.issue(a, (const T *)a.mask + (size_t)(bh / a.mask_div) * a.mask_sb, tid);

@@ -30,6 +30,7 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 #define FMHA_LOG2E 1.4426950408889634f
 #define FMHA_LN2 0.6931471805599453f
 #define FMHA_DEV __device__ __forceinline__
+#define FMHA_HOST_DEV __host__ __device__ __forceinline__
 
 template <typename T> struct Elem;
 

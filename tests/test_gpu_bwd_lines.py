@@ -28,6 +28,9 @@ CASES = [
     (3, 384, 129, 104, "fp16", "pad", False, 0.0),
     (3, 385, 129, 104, "fp16", "len", False, 0.0),
     (13, 70, 333, 64, "fp16", "pad", False, 0.1),  # five heads left over behind the eight of a group
+    (12, 385, 300, 64, "fp16", "len", False, 0.0),  # the four left over are ranges of each die
+    (20, 260, 257, 128, "bf16", "pad", False, 0.1),
+    (7, 300, 400, 96, "bf16", "pad", False, 0.0),   # fewer than eight heads
     (3, 257, 289, 64, "fp16", None, False, 0.0),
     (9, 257, 290, 64, "bf16", "len", False, 0.1),
     (3, 300, 287, 64, "bf16", None, True, 0.1),
