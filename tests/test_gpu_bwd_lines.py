@@ -64,3 +64,45 @@ def test_backward_on_both_sides_of_its_lines(bh, sq, sk, d, dtype, mask, causal,
     # size to the subtraction: twice the four units bound the norm of the error.
     for name, t in zip(("dq", "dk", "dv"), got):
         assert np.linalg.norm(f32(t.cpu()) - ref[name]) <= 8 * UNIT[dtype] * np.linalg.norm(ref[name]), name
+
+
+MASKED = [
+    # b, h, sq, sk, dtype, mask, packed: dK / dV at head dim 128 without dropout and causal mask, pipelined
+    (3, 2, 1056, 130, "fp16", "pad", False),   # rows (-LSE, -delta) in two segments
+    (3, 1, 1100, 1100, "bf16", "len", True),
+    (2, 4, 200, 200, "fp16", "pad", True),
+    (4, 3, 192, 257, "bf16", "len", False),
+]
+
+
+@pytest.mark.parametrize("b,h,sq,sk,dtype,mask,packed", MASKED)
+def test_masked_dk_dv_at_head_dim_128(b, h, sq, sk, dtype, mask, packed):
+    """More than one segment of queries, packed rows, and lengths that differ between the sequences: none, one key, half, all."""
+    d = 128
+    q, k, v, do = make_qkv(b * h, sq, sk, d, seed=sq + sk, std=0.7, dtype=dtype, with_dout=True)
+    lens = [0 if mask == "len" else 2, sk, sk // 2, 1][:b]
+    live = torch.arange(sk)[None] < torch.tensor(lens)[:, None]
+    kw = dict(kv_len=torch.tensor(lens, dtype=torch.int32).cuda()) if mask == "len" else dict(mask=torch.where(live, 0.0, -10000.0).to(TDT[dtype]).view(b, 1, 1, sk).cuda())
+    if packed:
+        qkv = torch.stack([t.view(b, h, sq, d).transpose(1, 2) for t in (q, k, v)], 2).cuda()  # [B, S, 3, H, D]
+        dev = [qkv[:, :, i].transpose(1, 2) for i in range(3)] + [do.view(b, h, sq, d).transpose(1, 2).contiguous().cuda().transpose(1, 2)]
+    else:
+        dev = [t.cuda() for t in (q, k, v, do)]
+    o, lse, _, _ = capi.fwd(*dev[:3], want_lse=True, **kw)
+    got = [f32(t.reshape(b * h, -1, d).cpu()) for t in capi.bwd(dev[3], *dev[:3], o, lse, **kw)]
+    torch.cuda.synchronize()
+    shown = live | (torch.tensor(lens) == 0)[:, None]  # (a sequence without keys: no gradient at all, below)
+    om = torch.where(shown, 0.0, float("-inf")).repeat_interleave(h, 0).unsqueeze(1).expand(b * h, sq, sk).contiguous()
+    ref = oracle.attention(f32(q), f32(k), f32(v), mask=f32(om), dout=f32(do), want=("dq", "dk", "dv"))
+    for name, t in zip(("dq", "dk", "dv"), got):
+        for i, n in enumerate(lens):
+            a, r = t[i * h:(i + 1) * h], ref[name][i * h:(i + 1) * h]
+            if n == 0:
+                assert not a.any(), (name, i)
+                continue
+            if name != "dq":
+                assert not a[:, n:].any(), (name, i)
+            # the bound of the test above; with one key dS is what rounding leaves of dP = dO V, 0.7^2 sqrt(d), times Q or K, 0.7 sqrt(d)
+            # a row, times the scale, over rows that add up at random
+            floor = 0.7 ** 3 * d * d ** -0.5 * np.sqrt(h * sq) if n == 1 and name != "dv" else 0.0
+            assert np.linalg.norm(a - r) <= 8 * UNIT[dtype] * max(np.linalg.norm(r), floor), (name, i)
