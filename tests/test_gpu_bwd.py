@@ -148,6 +148,32 @@ def test_causal_tile_pairing_is_bit_identical(bh, sq, sk, d, dtype, p, monkeypat
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("bh,sq,sk,d,dtype,p", [(3, 400, 333, 128, "fp16", 0.0), (2, 520, 520, 128, "bf16", 0.1), (3, 300, 400, 64, "fp16", 0.1)])
+def test_causal_tile_pairing_under_a_full_mask(bh, sq, sk, d, dtype, p, monkeypatch):
+    """Pairs of tiles in the kernels that work phase by phase, which causal heads of more than one tile reach with a full mask
+    tensor: the same bits as one tile a workgroup, and the oracle's gradients."""
+    q, k, v, do = make_qkv(bh, sq, sk, d, seed=sq + sk, std=0.5 if d == 128 else 1.0, dtype=dtype, with_dout=True)
+    m = (torch.rand(bh, sq, sk, generator=torch.Generator().manual_seed(2)) < 0.1).to(TDT[dtype]) * -10000.0
+    qc, kc, vc, doc, mc = (t.cuda() for t in (q, k, v, do, m))
+    kw, okw = dict(causal=True), dict(causal=True)
+    if p:
+        kw.update(drop_kind=capi.DROP_PHILOX, p_drop=p, seed=7, offset=3)
+        okw.update(philox=True, p_drop=p, seed=7, offset=3)
+    o, lse, _, _ = capi.fwd(qc, kc, vc, mask=mc, want_lse=True, **kw)
+    outs = []
+    for pair in ("0", "1"):
+        monkeypatch.setenv("FMHA_BWD_PAIR", pair)
+        outs.append([t.clone() for t in capi.bwd(doc, qc, kc, vc, o, lse, mask=mc, **kw)])
+        torch.cuda.synchronize()
+    for a, b in zip(*outs):
+        assert torch.equal(a, b)
+    ref = oracle.attention(f32(q), f32(k), f32(v), mask=f32(m), dout=f32(do), want=("dq", "dk", "dv"), **okw)
+    unit = {"fp16": 2.0 ** -11, "bf16": 2.0 ** -8}[dtype]
+    # P, dS, O (in delta) and the result are rounded once each; twice their four units for what dP - delta loses
+    for name, t in zip(("dq", "dk", "dv"), outs[1]):
+        assert np.linalg.norm(f32(t.cpu()) - ref[name]) <= 8 * unit * np.linalg.norm(ref[name]), name
+
+
 FULL_SIZE = [
     # B, H, S, D, dtype, causal, p_drop, std          (the other train configurations, at full size)
     (4, 16, 2048, 64, "fp16", False, 0.1, 1.0),       # long sequences, Philox dropout, no mask

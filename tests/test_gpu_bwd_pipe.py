@@ -50,11 +50,12 @@ def test_pipelined_backward_at_its_edges(bh, sq, sk, d, dtype, pad, causal, p):
         assert rel_to_max(f32(t.cpu()), ref[name], floor=1e-2) <= TOL[dtype], name
 
 
-@pytest.mark.parametrize("bh,sq,sk,dtype,pad,p", [(2, 384, 384, "fp16", False, 0.0), (2, 400, 333, "bf16", True, 0.1),
+@pytest.mark.parametrize("bh,sq,sk,dtype,pad,p", [(3, 129, 300, "bf16", False, 0.0), (2, 384, 384, "fp16", False, 0.0), (2, 400, 333, "bf16", True, 0.1),
                                                   (1, 895, 900, "fp16", False, 0.1), (1, 896, 896, "fp16", True, 0.0)])
-def test_causal_pairs_at_head_dim_128_in_either_dq_kernel(bh, sq, sk, dtype, pad, p, monkeypatch):
-    """The dQ kernel changes at 896 queries (here with pairs of tiles, as launches of many heads have them); the dK / dV
-    kernel and the delta it reads are the same on both sides."""
+def test_causal_pairs_at_head_dim_128(bh, sq, sk, dtype, pad, p, monkeypatch):
+    """Pairs of causal tiles, as launches of many heads have them: two query tiles and up, even and odd numbers of them, the
+    second tile of a pair on lane constants that are set up anew.  (The kernels phase by phase take pairs under full mask tensors
+    only: test_causal_tile_pairing_under_a_full_mask.)"""
     monkeypatch.setenv("FMHA_BWD_PAIR", "1")
     capi.lib().fmha_reload_overrides()
     try:
