@@ -19,6 +19,8 @@ def test_dealt_packed_rows_give_what_folded_rows_give(b, h, s, d):
     o2, lse2, _, _ = capi.fwd(*folded, **kw)
     torch.cuda.synchronize()
     a, c = o.reshape(b * h, s, d).float().cpu(), o2.float().cpu()
-    # the two round the same probabilities and outputs, but may take another reference exponent: one unit of each
-    assert (a - c).norm() <= 2 * 2.0 ** -8 * c.norm()
+    # The two round the same probabilities and outputs, but may take another reference exponent: half a unit for each of the four, row
+    # by row, so that the keys of the last tile count: the last row's output without them is off by sqrt(8 / 1800), 1 / sqrt(1345) and
+    # sqrt(12 / 1100) of its size.
+    assert ((a - c).norm(dim=-1) <= 2 * 2.0 ** -8 * c.norm(dim=-1)).all()
     assert torch.allclose(lse.reshape(b * h, s).cpu(), lse2.cpu(), rtol=0, atol=2.0 ** -8)
