@@ -56,7 +56,7 @@ template <typename K> int set_lds(K kern, int bytes) {
 //   dK+dV, causal          S 128 27 / 30, S 192 43 / 56, S 256 55 / 71, 2048 heads S 128 with dropout 101 / 126
 //   dK+dV of few heads (one round of workgroups, the plain pipelined kernel): 64 heads S 200 12 / 17, causal 14 / 16
 // The line is 128 queries (192 for causal dK / dV that is not persistent, see fmha_bwd_pipe.hip).
-// At head dim 96 dQ has no line of its own for causal heads, and dK / dV is never pipelined: phase by phase on 32-row tiles it has the
+// At head dim 96 dK / dV is never pipelined: phase by phase on 32-row tiles it has the
 // registers for two waves per SIMD, pipelined it does not (backward, us, persistent or pipelined / so: BH 512 S 512 padding mask and
 // dropout 316 / 270, without either 265 / 245; causal BH 608 S 365 181 / 158, BH 128 S 1024 with dropout 171 / 154, BH 32 S 3000 232 /
 // 228; BH 576 S 120 56 / 49).

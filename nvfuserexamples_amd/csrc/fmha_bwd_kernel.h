@@ -97,9 +97,10 @@ FMHA_HOST_DEV void bwd_head_and_unit(int bid, int dealt, int range, int units, i
 // BT: rows per LDS tile (keys in the dQ kernel, queries in the dK/dV kernel).  The dK/dV kernel
 // at head dim 128 holds 128 accumulator registers; walking the queries 32 at a time brings its
 // score / dP tiles and their fragments close enough to a two-waves-per-SIMD register budget
-// that forcing that occupancy pays (+11 % measured) -- for the plain variant only: with a causal
+// that forcing that occupancy pays (+11 % measured) -- without causal mask and dropout only: with a causal
 // mask the shorter tiles lose more to the uneven tile counts, and the dropout variant spills
-// too much, so those keep 64-row tiles at one wave per SIMD.
+// too much, so those keep 64-row tiles at one wave per SIMD.  (What reaches these builds at head dim 128: full mask tensors, heads of
+// fewer than 128 queries, and short heads under a per-key mask or key counts, see fmha_bwd.hip.)
 template <int D> constexpr int bwd_dq_tile_rows() { return 64; }
 // (Head dim 256 has a dK/dV kernel of its own, fmha_bwd_wide.h.)
 template <int D, bool CAUSAL, int DROP> constexpr bool bwd_dkdv_small_tiles() { return D == 96 || (D == 128 && !CAUSAL && DROP == 0); }

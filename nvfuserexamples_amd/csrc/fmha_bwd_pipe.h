@@ -1,4 +1,4 @@
-// Software-pipelined backward kernels for head dims 64 and 128, and dQ at 256 (no mask or a per-key mask; full mask tensors stay on
+// Software-pipelined backward kernels for head dims up to 128 (96: dQ), and dQ at 256 (no mask or a per-key mask; full mask tensors stay on
 // fmha_bwd_kernel.h).  Mathematics, register layouts and the extra contraction step are those of fmha_bwd_kernel.h, whose
 // header describes them; what changes is the order of work and how tiles arrive:
 //
@@ -21,7 +21,8 @@
 // Measured against the two-stage, phase-by-phase kernels on one card (kernel times, us, dQ / dK+dV, fp16 unless said): BH 64
 // S 2048 D 64 without dropout 126.9 / 159.3 -> 116.6 / 153.1, with dropout 140.0 / 194.5 -> 135.9 / 174.7; BH 192 S 1024 D 64
 // causal 84.3 / 98.2 -> 66.4 / 81.9; BH 32 S 4096 D 128 causal 280 / 335 -> 225 / 304 (bf16 272 / 329 -> 214 / 275); BH 512
-// S 1024 D 128 causal bf16 285 / 455 -> 293 / 413 (the lines between the two at head dim 128: fmha_bwd.hip).
+// S 1024 D 128 causal bf16 285 / 455 -> 293 / 413, before dQ there lost the registers that spilled into its stream (308 -> 252 on another
+// card; the lines between the two kinds of kernel at head dim 128: fmha_bwd.hip).
 // What bounds them: at head dim 64 the issue slots (a matrix instruction takes the vector pipe for about 21 cycles, a
 // vector instruction for 2.5, and the sum of both is what two waves per SIMD need); at head dim 128 the board's power
 // (dQ on random data: 1.57 GHz, on zeros 2.19 GHz) and, for dK / dV at one wave per SIMD, the start and the stores of
@@ -38,7 +39,7 @@ template <int D> struct BwdPipeCfg {
   static constexpr int BT = 32, NST = 4; // rows per tile, tiles resident per operand
   static constexpr int KS = D / 16, DB = D / 32;
   static constexpr int TILEB = BT * tile_cols(D) * 2, STAGEB = 2 * TILEB;
-  static constexpr bool TURNED = D == 64 || D == 128;                       // register operands are read as whole rows (load_row_operands)
+  static constexpr bool TURNED = D == 64 || D == 128;                       // register operands are read as whole rows (RowOperands)
   static constexpr int OFF_T = (NST - 1) * STAGEB, TURNB = 32 * kPanelRowB; // ... and turned here, in the last stage, a panel per wave
   static constexpr int OFF_X = D == 64 ? OFF_T + 4 * TURNB : NST * STAGEB;
   static_assert(!TURNED || 4 * TURNB + OFF_T <= OFF_X, "a panel for each of four waves");
@@ -124,7 +125,7 @@ template <> struct MfmaV<__bf16> {
   static FMHA_DEV void start(bf16x8 a, bf16x8 b, f32x16 &c) { asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(c) : "v"(a), "v"(b)); }
   static FMHA_DEV void add(bf16x8 a, bf16x8 b, f32x16 &c) { asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b)); }
 };
-FMHA_DEV void settle(f32x16 &x, f32x16 &g) { asm volatile("s_nop 15" : "+v"(x), "+v"(g)); } // (eleven wait states are due)
+FMHA_DEV void settle(f32x16 &x, f32x16 &g) { asm volatile("s_nop 15" : "+v"(x), "+v"(g)); } // (twelve wait states are due, this is sixteen)
 
 // One Philox4x32-10 call in slices that can be spread over an instruction stream.
 struct PhiloxSlices {

@@ -305,9 +305,11 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu((QB == 
   // Copy tile `tile` of `base` (K or V of a head) into stage (tile & 1) of the LDS area at byte
   // offset area_off.  Rows past kend re-read the last valid row: their scores get -inf through
   // the extra step, and finite garbage in V is multiplied by P = 0.
-  // (APART where else three of the lane's four offsets were reloaded from scratch ahead of each copy, behind the copies before: dealt causal
-  // packed bf16 rows with dropout at head dim 128, BH 24 S 1800 95.1 -> 62.1 us, BH 32 S 1500 79.0 -> 49.5, at 112 columns, whose copies do without these offsets, BH 40
-  // S 1100 41.2 -> 42.3.  Where they are not reloaded it costs up to 3 %: without dropout 45.1 -> 46.7, fp16 level.)
+  // (APART in the one build whose allocation reloaded three of the lane's four offsets from scratch ahead of each copy, behind the copies before:
+  // dealt causal packed bf16 rows with dropout at head dim 128, BH 24 S 1800 95.1 -> 62.1 us, BH 32 S 1500 79.0 -> 49.5; at 112 columns, whose copies
+  // do without these offsets, BH 40 S 1100 41.2 -> 42.3.  In all builds for run-time rows at head dim 128 it costs the others: dealt causal BH 24
+  // S 1800 without dropout bf16 44.7 -> 46.0, fp16 43.7 -> 44.9, with dropout fp16 55.1 -> 56.4; the distances added by the vector pipe leave
+  // 99.0 and 82.9 there.  Which build it is depends on the compiler: to be measured again with another one.)
   TileCopy<T, D, BK, NT, D == 128 && STRIDED && DEAL && DROP == 1 && std::is_same<T, __bf16>::value> tcopy;
   tcopy.init(tid, RW::ss(a.mk), RW::cols(a)); // K and V rows are equally far apart
   auto dma_tile = [&](const T *base, int kend, int tile, uint32_t area_off, bool any_past) {
