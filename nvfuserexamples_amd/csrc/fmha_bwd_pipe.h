@@ -295,7 +295,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(bwd_dq_
           to[ks] = *(const u32x4 *)(Ob + (size_t)qc * RW::ss(a.mo) + col);
         }
       }
-      const float lse_q = a.lse[(size_t)bh * a.sq + qc];
+      float lse_q = a.lse[(size_t)bh * a.sq + qc];
       if (MASK == kMaskPerKey && (pass == 0 || a.sk > C::MSEG)) { // (with more than one segment the first pass leaves a later one)
         const int n = stage_mask(0); // (its loads share the trip to memory)
         const bool trim = a.sk > 128 && a.sk <= C::MSEG && !(a.flags & kBwdFlagNoTrim);
@@ -307,6 +307,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(bwd_dq_
         rd.turn(panel, pl, l, td);
         ro.turn(panel, pl, l, to);
       }
+      asm volatile("" : "+v"(lse_q));
       float dsum = 0.f;
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
@@ -495,7 +496,8 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(bwd_dq_
     if (DROP == 1) drop_words_q(a.drop, (uint32_t)bh, (uint32_t)q, 0u, h, l, wd0); // (while the tiles are on their way)
     bwd_vm_wait<0>();
     bwd_lds_barrier();
-    auto first = [&](f32x16 &x, f32x16 &g, uint32_t (&wd)[4]) {
+    auto first = [&](auto odd, f32x16 &x, f32x16 &g, uint32_t (&wd)[4]) {
+      asm volatile("" ::"n"(decltype(odd)::value) : "memory"); // (its reads stay on either side of the branch below: ahead of it they spill)
 #pragma unroll
       for (int i = 0; i < 4 && DROP == 1; ++i) wd[i] = wd0[i];
       const v8 xa = xa_of(hl_of(0));
@@ -534,11 +536,11 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(bwd_dq_
     int kt = 0;
     const int nmid = nktw - 1;
     if (nmid & 1) {
-      first(xB, gB, wdB);
+      first(Yes{}, xB, gB, wdB);
       mid(0, xB, gB, wdB, xA, gA, wdA);
       kt = 1;
     } else {
-      first(xA, gA, wdA);
+      first(No{}, xA, gA, wdA);
     }
     for (; kt < nmid; kt += 2) {
       mid(kt, xA, gA, wdA, xB, gB, wdB);

@@ -1,10 +1,15 @@
-"""A compile-time property of the products that the dK / dV kernels at head dim 128 write as instructions, checked on their assembly.
+"""Compile-time properties of the pipelined backward kernels, checked on their assembly.
+
+Products that the dK / dV kernels at head dim 128 write as instructions:
 
 The compiler does not see into these instructions, so it adds no wait states behind them: their result may be read by anything but the
 next product on the same accumulator, or overwritten, twelve wait states later at the earliest (eight passes of a 32x32x16 product on
 gfx950), and an operand written by the vector pipe may be read two wait states later (by another product: twelve).  This follows every
 path from and to every such instruction and counts each instruction as one wait state (device side only, no GPU needed), in each of
 the four builds that have them: registers are allocated, and instructions ordered, anew in each.
+
+The stream of dQ: copies of the next tiles are on their way all the time and are waited for with a count, so nothing in it may wait for
+a load of its own -- neither for a spilled register nor for one that the compiler believes still to be loading from the prologue.
 """
 import concurrent.futures as cf
 import os
@@ -17,6 +22,7 @@ from nvfuserexamples_amd import build as B
 
 RESULT, OPERAND = 12, 2  # wait states
 BUILDS = ["fmha_bwd_pipe_f16_d128", "fmha_bwd_pipe_bf16_d128", "fmha_bwd_pipe_f16_d128_strided", "fmha_bwd_pipe_bf16_d128_strided"]
+STREAMS = BUILDS + ["fmha_bwd_pipe_f16_d64", "fmha_bwd_pipe_bf16_d64_strided"]
 
 
 def registers(operand):
@@ -132,8 +138,8 @@ def listings(tmp_path_factory):
                        capture_output=True)
         return open(out).read()
 
-    with cf.ThreadPoolExecutor(len(BUILDS)) as ex:
-        return dict(zip(BUILDS, ex.map(compiled, BUILDS)))
+    with cf.ThreadPoolExecutor(len(STREAMS)) as ex:
+        return dict(zip(STREAMS, ex.map(compiled, STREAMS)))
 
 
 @pytest.mark.skipif(not os.path.exists(B.HIPCC), reason="needs hipcc")
@@ -142,6 +148,41 @@ def test_written_products_are_left_alone_until_they_are_done(name, listings):
     found, broken = check(listings[name])
     assert broken is None, broken
     assert found > 1000
+
+
+def streams(text, kernel):
+    """(function, lines) of the stream of every function of that name: the blocks that hold matrix instructions, of the innermost loop
+    that copies and passes two barriers (two tiles a turn)."""
+    lines, found = text.split("\n"), []
+    for start in (i for i, line in enumerate(lines) if re.match(r"_Z\S*%s\S*:" % kernel, line)):
+        body = lines[start:next(i for i in range(start, len(lines)) if lines[i].startswith(".Lfunc_end"))]
+        labels = {m[1]: i for i, line in enumerate(body) if (m := re.match(r"(\.LBB\S+):", line))}
+        spans = [(labels[m[1]], i) for i, line in enumerate(body) if (m := re.match(r"\s+s_c?branch\w*\s+(\.LBB\S+)", line)) and labels[m[1]] <= i]
+        turns = []
+        for a, b in spans:
+            blocks, inside = [[]], False
+            for line in body[a:b + 1]:
+                if line.startswith(".LBB"):
+                    blocks.append([])
+                inside = "#ASMSTART" in line or (inside and "#ASMEND" not in line)
+                blocks[-1].append((inside, line.split(";")[0].strip()))
+                if re.match(r"\s+s_c?branch", line):
+                    blocks.append([])
+            blocks = [x for block in blocks if any(line.startswith("v_mfma") for _, line in block) for x in block]
+            if sum("global_load_lds" in line for _, line in blocks) and sum("s_barrier" in line for _, line in blocks) >= 2:
+                turns.append((a, b, blocks))
+        found += [(body[0], blocks) for a, b, blocks in turns if not any((c, d) != (a, b) and a <= c and d <= b for c, d, _ in turns)]
+    return found
+
+
+@pytest.mark.skipif(not os.path.exists(B.HIPCC), reason="needs hipcc")
+@pytest.mark.parametrize("name", STREAMS)
+def test_streams_of_dq_wait_for_nothing_but_their_copies(name, listings):
+    found = streams(listings[name], "fmha_bwd_dq_pipe_kernel")
+    assert len({function for function, _ in found}) == 8  # no / per-key mask, causal or not, with dropout or not
+    for function, lines in found:
+        own = [line for inside, line in lines if not inside and ("vmcnt" in line or line.startswith("scratch_"))]
+        assert not own, (function, own)
 
 
 PRODUCT = "\t;#ASMSTART\n\tv_mfma_f32_32x32x16_f16 v[0:15], v[16:19], v[20:23], 0\n\t;#ASMEND\n"
