@@ -105,7 +105,8 @@ template <int MASK, bool CAUSAL, int DROP> int launch_dkdv(BwdArgs &a, const Bwd
   // masks / key counts, us, so / pipelined: BH 512 S 128 48.3 / 51.0, 45.6 / 50.8, S 160 level; S 197 110.9 / 100.3, S 258 156 / 133, 135
   // / 129, S 512 417 / 329, 316 / 307, packed 464 / 342, 460 / 325; BH 256 S 1024 702 / 524, 503 / 491, packed 796 / 527, 785 / 503; 112
   // to 120 columns BH 192 S 320 65.3 / 66.6, 65.9 / 64.4, S 384 87.7 / 92.2, 84.5 / 87.5, BH 512 S 416 270 / 251, 278 / 245, BH 64 S 2048
-  // 502 / 430, 476 / 377.
+  // 502 / 430, 476 / 377.  (Whole folded rows under key counts of 192 to 256 queries: 64 to 128 heads a fifth less, BH 256 S 256 50.2 / 52.1, BH 512
+  // S 256 95.8 / 100.3; the line must not depend on the number of heads, with which a head's gradients would change.)
   constexpr bool kTwoWaves = bwd_dkdv_small_tiles<FMHA_TU_D, CAUSAL, DROP>();
   if constexpr (kPipe && FMHA_TU_D != 96) { // (see pipe_wanted)
     const bool two_waves = kTwoWaves && (MASK != kMaskNone || a.kv_len) && (a.dcols < FMHA_TU_D ? a.sq <= 384 : a.sq < 192);
@@ -147,6 +148,13 @@ template <int MASK, bool CAUSAL, int DROP> int launch(BwdArgs &a, const BwdVaria
       n = 0;
     return n;
   }();
+  const int qtiles = (a.sq + QT - 1) / QT, ktiles = (a.sk + KT - 1) / KT;
+  const bool uneven = !CAUSAL && (MASK == kMaskPerKey || (MASK == kMaskNone && a.kv_len));
+  const bool share = rows_share_lines(a.mq.heads, a.mq.sh, a.mq.ss) || rows_share_lines(a.mk.heads, a.mk.sh, a.mk.ss);
+  const bool dealt = uneven && bwd_heads_dealt(share, a.bh, qtiles, ktiles);
+  // dQ of short heads at head dim 256 is dealt alone from four rounds of workgroups on (backward, us, ranges / so: BH 1024 S 128 1.5 to 4 %
+  // less, BH 2240 S 56 and S 24 level).
+  const bool one = FMHA_TU_D == 256 && uneven && !share && qtiles == 1 && a.bh >= 4 * cus;
   auto blocks = [&](int ntile, bool dq) -> long long {
     const long long tiles = (long long)a.bh * ntile, pairs = (long long)a.bh * ((ntile + 1) / 2), over = tiles - 2LL * cus;
     const bool by_head = (ntile == 3 || ntile == 5) && ((tiles >= (ntile + 1LL) * cus && (dq || DROP == 0)) || (FMHA_TU_D <= 64 && over > 0 && 16 * over <= cus));
@@ -157,16 +165,14 @@ template <int MASK, bool CAUSAL, int DROP> int launch(BwdArgs &a, const BwdVaria
     else if (CAUSAL && by_head) a.pair = kTilesByHead;
     a.lg = head_groups_log2(a.bh);
     a.units = !CAUSAL || a.pair == kTilesByHead ? ntile : a.pair == kTilesPaired ? (ntile + 1) / 2 : a.bh >> a.lg;
-    const bool uneven = !CAUSAL && (MASK == kMaskPerKey || (MASK == kMaskNone && a.kv_len));
-    const bool share = rows_share_lines(a.mq.heads, a.mq.sh, a.mq.ss) || rows_share_lines(a.mk.heads, a.mk.sh, a.mk.ss);
-    a.dealt = uneven ? bwd_dealt_blocks(FMHA_TU_D == 256 && tiles >= 4LL * cus, share, a.bh, ntile) : 0;
+    a.dealt = dealt || (one && dq) ? bwd_dealt_blocks(a.bh, ntile) : 0;
     a.range = bwd_range_blocks(a.pair == kTilesPaired ? pairs : tiles, a.dealt);
     return a.pair == kTilesPaired ? pairs : tiles;
   };
   // dQ first: it also writes delta, which the dK/dV kernel reads (same stream => ordered)
-  const long long nq = blocks((a.sq + QT - 1) / QT, true);
+  const long long nq = blocks(qtiles, true);
   if (const int rc = launch_dq<MASK, CAUSAL, DROP>(a, v, nq, s)) return rc;
-  const long long nk = blocks((a.sk + KT - 1) / KT, false);
+  const long long nk = blocks(ktiles, false);
   return launch_dkdv<MASK, CAUSAL, DROP>(a, v, nk, s);
 }
 

@@ -61,7 +61,7 @@ struct BwdArgs {
   int32_t dcols; // elements per row that exist (<= the kernel's head dim; run-time layouts only)
   int32_t units; // what a block's number is divided by (bwd_item): a head's tiles or pairs of tiles; kTilesByLength: heads of a group
   int32_t lg; // head_groups_log2 of the heads
-  int32_t dealt; // blocks at the front of the launch whose heads go to the XCDs one by one (bwd_dealt_blocks)
+  int32_t dealt; // blocks at the front of the launch whose heads go to the XCDs one by one (bwd_heads_dealt)
   int32_t range; // neighbours of an XCD among the blocks behind those (bwd_range_blocks)
 };
 
@@ -72,18 +72,19 @@ struct BwdArgs {
 // S 640 199 / 188, packed with dropout 261 / 240, BH 512 S 512 level to 1 % ahead, D 128 BH 256 S 512 139.7 / 132.3, packed with dropout
 // 176.7 / 168.6 (but BH 200 S 300 of 4 heads a sequence D 64 35.9 / 37.9, of 8 heads 0.92 of the ranges' time); without ranges to be
 // had, a head's tiles on all XCDs / dealt, BH 300 S 300 D 64 52.3 / 46.8, D 128 97.0 / 86.9.
-// Up to two tiles a head stay ranges where they can: there is little to even out, and dealt D 32 BH 512 S 40 is 2 % behind, S 200 and D 128 level.
-// Interleaved rows of neighbouring heads that meet inside a cache line, which two XCDs then read and write, stay ranges up to seven
-// tiles: packed D 32 BH 512 S 128 21.2 / 26.0, S 200 42.1 / 47.9, S 512 129.7 / 133.8, D 80 BH 256 S 512 136 / 141, S 640 198 / 207,
-// S 1024 443 / 439.  Full mask tensors are not dealt, their heads are equally long: D 128 BH 256 S 512 245 / 254, D 64 BH 512 S 512 210 / 217.
+// One order for dQ and dK / dV: what one leaves in an XCD's L2 the other reads there (only one of them dealt: 2 % behind both and neither as a
+// geometric mean over 700 masked launches, where this rule is 1.9 % ahead of ranges alone and 0.3 % of dealing all).
+// Heads of up to two tiles of queries and of keys stay ranges where they can: there is little to even out, and dealt D 32 BH 512 S 40 is
+// 2 % behind, S 200 and D 128 level.  Interleaved rows of neighbouring heads that meet inside a cache line, which two XCDs then read and write,
+// stay ranges up to four tiles: packed D 32 BH 512 S 128 21.2 / 26.0, S 200 42.1 / 47.9, S 512 129.7 / 133.8, D 80 BH 256 S 512 136 / 141, S 640 198
+// / 207, but D 96 BH 96 S 688 102.5 / 85.1.  Full mask tensors are not dealt, their heads are equally long: D 128 BH 256 S 512 245 / 254, D 64 BH
+// 512 S 512 210 / 217.
 FMHA_HOST_DEV bool rows_share_lines(int32_t heads, int64_t sh, int64_t ss) { return heads > 1 && sh < ss && (sh == 0 || sh % 64 != 0); }
-// Heads of one tile (`one`) at head dim 256 are dealt from four rounds of workgroups on (S 128 BH 512 1.5 % behind, BH 1024 3 to 6 % ahead,
-// BH 2240 S 56 1.5 to 4 % ahead, S 24 1 % behind; two tiles, BH 768 S 250, 1 to 4 % behind).
-FMHA_HOST_DEV int bwd_dealt_blocks(bool one, bool share_lines, int bh, int units) {
-  const int64_t nb = (int64_t)bh * units;
-  const bool deal = units >= (nb % 8 != 0 ? 2 : share_lines ? 8 : 3) || (one && !share_lines && units == 1);
-  return deal ? (int)((int64_t)(bh & ~7) * units) : 0;
+FMHA_HOST_DEV bool bwd_heads_dealt(bool share_lines, int bh, int qtiles, int ktiles) {
+  const bool ranges = (int64_t)bh * qtiles % 8 == 0 && (int64_t)bh * ktiles % 8 == 0;
+  return (qtiles > ktiles ? qtiles : ktiles) >= (!ranges ? 2 : share_lines ? 5 : 3);
 }
+FMHA_HOST_DEV int bwd_dealt_blocks(int bh, int units) { return (int)((int64_t)(bh & ~7) * units); }
 FMHA_HOST_DEV int bwd_range_blocks(int64_t nb, int dealt) { return (nb - dealt) % 8 == 0 ? (int)((nb - dealt) / 8) : 0; } // (0: as they come)
 FMHA_HOST_DEV void bwd_head_and_unit(int bid, int dealt, int range, int units, int &bh, int &pi) {
   const int r = bid - dealt, behind = range ? (r & 7) * range + (r >> 3) : r;

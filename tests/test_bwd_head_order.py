@@ -13,9 +13,9 @@ PROGRAM = r"""
 #include "fmha_bwd_kernel.h"
 #include <cstdio>
 int main() {
-  int kind, bh, units;
-  while (std::scanf("%d %d %d", &kind, &bh, &units) == 3) {
-    const int dealt = kind < 0 ? 0 : fmha::bwd_dealt_blocks(kind == 2, kind == 1, bh, units), nb = bh * units;
+  int kind, bh, units, others;
+  while (std::scanf("%d %d %d %d", &kind, &bh, &units, &others) == 4) {
+    const int dealt = kind >= 0 && fmha::bwd_heads_dealt(kind != 0, bh, units, others) ? fmha::bwd_dealt_blocks(bh, units) : 0, nb = bh * units;
     std::printf("%d", dealt);
     for (int bid = 0; bid < nb; ++bid) {
       int head, unit;
@@ -28,10 +28,9 @@ int main() {
   for (const auto &r : rows) std::printf("%d ", (int)fmha::rows_share_lines((int)r[0], r[1], r[2]));
 }
 """
-NO_MASK, WHOLE, SHARED, ONE = -1, 0, 1, 2  # no lengths that may differ; rows in cache lines of their own; lines shared by neighbouring
-# heads; many heads of one tile at head dim 256
-LAUNCHES = [(kind, bh, units) for kind in (NO_MASK, WHOLE, SHARED, ONE) for bh in (1, 4, 7, 8, 9, 12, 20, 36, 60, 64, 272)
-            for units in (1, 2, 3, 4, 5, 7, 8, 16, 32)]
+NOT, WHOLE, SHARED = -1, 0, 1  # no lengths that may differ; rows in cache lines of their own; lines shared by neighbouring heads
+LAUNCHES = [(kind, bh, units, others) for kind in (NOT, WHOLE, SHARED) for bh in (1, 4, 7, 8, 9, 12, 20, 36, 60, 64, 272)
+            for units in (1, 2, 3, 4, 5, 7, 8, 16, 32) for others in (1, 4, 9)]
 
 
 @pytest.mark.skipif(not os.path.exists(B.HIPCC), reason="needs hipcc")
@@ -40,13 +39,14 @@ def test_heads_of_a_backward_launch_on_the_compute_dies(tmp_path):
     src.write_text(PROGRAM)
     subprocess.run([B.HIPCC, "-x", "hip", "--cuda-host-only", "-std=c++17", "-O1", "-I", B.CSRC, str(src), "-o", exe], check=True,
                    capture_output=True)
-    text = "\n".join("%d %d %d" % x for x in LAUNCHES)
+    text = "\n".join("%d %d %d %d" % x for x in LAUNCHES)
     out = subprocess.run([exe], input=text, check=True, capture_output=True, text=True).stdout.split("\n")
-    for (kind, bh, units), line in zip(LAUNCHES, out):
+    for (kind, bh, units, others), line in zip(LAUNCHES, out):
         dealt, *item = map(int, line.split())
-        nb, name = bh * units, (kind, bh, units)
+        nb, name = bh * units, (kind, bh, units, others)
         assert sorted(item) == list(range(nb)), name
-        wanted = kind != NO_MASK and (units >= (2 if nb % 8 else 8 if kind == SHARED else 3) or (kind == ONE and units == 1))
+        ranges = nb % 8 == 0 and bh * others % 8 == 0  # to be had, for dQ and for dK / dV
+        wanted = kind != NOT and max(units, others) >= (2 if not ranges else 5 if kind == SHARED else 3)
         assert dealt == (bh // 8 * 8 * units if wanted else 0), name
         dies = [{i & 7 for i in range(nb) if item[i] // units == head} for head in range(bh)]
         assert all(len(d) == 1 for d in dies[:dealt // units]), name
