@@ -21,7 +21,7 @@
 // Measured against the two-stage, phase-by-phase kernels on one card (kernel times, us, dQ / dK+dV, fp16 unless said): BH 64
 // S 2048 D 64 without dropout 126.9 / 159.3 -> 116.6 / 153.1, with dropout 140.0 / 194.5 -> 135.9 / 174.7; BH 192 S 1024 D 64
 // causal 84.3 / 98.2 -> 66.4 / 81.9; BH 32 S 4096 D 128 causal 280 / 335 -> 225 / 304 (bf16 272 / 329 -> 214 / 275); BH 512
-// S 1024 D 128 causal bf16 285 / 455 -> 293 / 413, before dQ there lost the registers that spilled into its stream (308 -> 252 on another
+// S 1024 D 128 causal bf16 285 / 455 -> 293 / 413, before dQ there lost the registers that spilled into its stream (300 -> 246 on another
 // card; the lines between the two kinds of kernel at head dim 128: fmha_bwd.hip).
 // What bounds them: at head dim 64 the issue slots (a matrix instruction takes the vector pipe for about 21 cycles, a
 // vector instruction for 2.5, and the sum of both is what two waves per SIMD need); at head dim 128 the board's power
