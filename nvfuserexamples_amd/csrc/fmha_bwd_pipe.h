@@ -84,6 +84,10 @@ template <typename T, int D, int NT> struct PipeCopy {
 // panel of the wave's own LDS.  Backward, us, loaded as wanted / so: D 128 BH 512 S 1024 bf16 causal 642 / 623, S 384 169 / 166, packed
 // with dropout S 512 369 / 358; D 64 BH 512 S 1024 causal 343 / 331, packed S 512 170 / 166, BH 256 S 800 with dropout 234 / 229,
 // BH 100 S 400 31.8 / 30.6; level to 1.5 % behind on whole rows without mask and dropout, BH 512 S 512 157 / 158.
+// Rows of 33 to 63 columns that follow on each other (heads folded) fill the lines they are in as they are, and short heads of them pay for
+// the way through LDS: without a causal mask they are loaded as wanted (D 48, 16 to 128
+// heads of 64 to 320 rows 4 to 6 % less, 512 heads level).  Under one the kernels have no registers for both ways (D 48
+// and 112 10 to 12 % behind), and at head dim 128 the way through LDS is level to 1 % ahead.
 template <typename T, int D> struct RowOperands {
   static constexpr int NI = 32 * tile_cols(D) / 8 / 64;
   u32x4 v[NI];
@@ -281,8 +285,9 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(bwd_dq_
     {
       const int qc = q < a.sq ? q : a.sq - 1;
       u32x4 tq[KS], td[KS], to[KS];
+      const bool turned = C::TURNED && (CAUSAL || D != 64 || !STRIDED || RW::ss(a.mq) != (uint32_t)RW::cols(a)); // (see RowOperands)
       RowOperands<T, D> rq, rd, ro;
-      if constexpr (C::TURNED) {
+      if (turned) {
         rq.load(Qb, RW::ss(a.mq), q0w, a.sq, RW::cols(a), l);
         rd.load(dOb, RW::ss(a.mdo), q0w, a.sq, RW::cols(a), l);
         ro.load(Ob, RW::ss(a.mo), q0w, a.sq, RW::cols(a), l);
@@ -301,7 +306,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(bwd_dq_
         const bool trim = a.sk > 128 && a.sk <= C::MSEG && !(a.flags & kBwdFlagNoTrim);
         if (trim && n > 0 && n < skv) skv = n; // a row without any live key keeps all its keys
       }
-      if constexpr (C::TURNED) {
+      if (turned) {
         char *panel = lds + C::OFF_T + w * C::TURNB;
         rq.turn(panel, pl, l, tq);
         rd.turn(panel, pl, l, td);
@@ -670,8 +675,9 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(bwd_dkd
     {
       const int kc = key < a.sk ? key : a.sk - 1;
       u32x4 tk[KS], tv[KS];
+      const bool turned = C::TURNED && (CAUSAL || D != 64 || !STRIDED || RW::ss(a.mk) != (uint32_t)RW::cols(a)); // (see RowOperands)
       RowOperands<T, D> rk, rv;
-      if constexpr (C::TURNED) {
+      if (turned) {
         rk.load(Kb, RW::ss(a.mk), k0w, a.sk, RW::cols(a), l);
         rv.load(Vb, RW::ss(a.mv), k0w, a.sk, RW::cols(a), l);
       } else {
@@ -685,7 +691,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(bwd_dkd
       T mraw = (T)0.f;
       if (MASK == kMaskPerKey) mraw = ((const T *)a.mask)[(size_t)(bh / a.mask_div) * a.mask_sb + kc];
       if (pass == 0 || a.sq > C::QSEG) stage_rows(qt0 * BT / C::QSEG * C::QSEG);
-      if constexpr (C::TURNED) {
+      if (turned) {
         char *panel = lds + C::OFF_T + w * C::TURNB; // (the first tiles go to the other stages: qt0 is a multiple of four)
         rk.turn(panel, pl, l, tk);
         rv.turn(panel, pl, l, tv);

@@ -1,7 +1,7 @@
 """The backward on both sides of the lines where its kernels change, with ragged last tiles and numbers of heads that do not divide
 over the compute dies: causal dQ at head dim 128 (pipelined from 128 queries on), dK / dV at head dim 128 under masks and key counts
 without dropout (from 192, of shorter rows from 385), heads left over behind groups of eight, dQ at head dims up to 96 whose products
-start from LSE and delta (only a mask has an extra step: the last tile's missing keys are a test per score), against the oracle."""
+start from LSE and delta (only a mask has an extra step: the last tile's missing keys are a test per score), rows narrower than the kernel's, against the oracle."""
 import numpy as np
 import pytest
 import torch
@@ -38,6 +38,9 @@ CASES = [
     (3, 257, 299, 80, "bf16", "len", True, 0.0),
     (5, 300, 299, 32, "fp16", "len", True, 0.1),
     (3, 129, 161, 32, "bf16", None, False, 0.0),
+    (3, 70, 100, 48, "fp16", "pad", False, 0.1),   # narrow rows one behind the other: register operands loaded as wanted
+    (2, 290, 257, 40, "bf16", None, False, 0.0),
+    (2, 201, 230, 56, "fp16", "len", True, 0.1),   # ... and turned
 ]
 
 
