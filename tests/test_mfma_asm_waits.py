@@ -199,6 +199,6 @@ PRODUCT = "\t;#ASMSTART\n\tv_mfma_f32_32x32x16_f16 v[0:15], v[16:19], v[20:23], 
     ("\tv_mfma_f32_32x32x16_f16 v[16:31], v[40:43], v[44:47], 0\n\ts_nop 5\n{}\ts_nop 15\n", False),
     ("\tv_cmp_gt_f32_e32 vcc, v17, v18\n\tv_readfirstlane_b32 s3, v17\n{}\ts_nop 15\n", True),
 ])
-def test_the_checker_itself(around, fine):
+def test_the_check_itself(around, fine):
     found, broken = check(around.format(PRODUCT) + "\ts_endpgm\n")
     assert found == 1 and (broken is None) == fine, broken
