@@ -152,8 +152,8 @@ template <int MASK, bool CAUSAL, int DROP> int launch(BwdArgs &a, const BwdVaria
   const bool uneven = !CAUSAL && (MASK == kMaskPerKey || (MASK == kMaskNone && a.kv_len));
   const bool share = rows_share_lines(a.mq.heads, a.mq.sh, a.mq.ss) || rows_share_lines(a.mk.heads, a.mk.sh, a.mk.ss);
   const bool dealt = uneven && bwd_heads_dealt(share, a.bh, qtiles, ktiles);
-  // dQ of short heads at head dim 256 is dealt alone from four rounds of workgroups on (backward, us, ranges / so: BH 1024 S 128 1.5 to 4 %
-  // less, BH 2240 S 56 and S 24 level).
+  // dQ of short heads at head dim 256 is dealt alone from four rounds of workgroups on (backward: BH 1024 S 128 both kernels dealt 3 to 6 % less
+  // than ranges, dQ alone 1.5 to 4 % less than both; BH 2240 S 56 and S 24 level).
   const bool one = FMHA_TU_D == 256 && uneven && !share && qtiles == 1 && a.bh >= 4 * cus;
   auto blocks = [&](int ntile, bool dq) -> long long {
     const long long tiles = (long long)a.bh * ntile, pairs = (long long)a.bh * ((ntile + 1) / 2), over = tiles - 2LL * cus;
